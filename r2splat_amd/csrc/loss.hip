@@ -5,136 +5,256 @@
 #include "common.hpp"
 #include "raster_common.hpp"
 
+#include <type_traits>
+
 namespace r2s {
 
+// The losses stream their buffers: a thread takes VEC consecutive elements of
+// a row (16-byte loads; VEC = 1 where a row's length or a pointer is not a
+// multiple of 16 bytes), and what bounds them is memory traffic as long as
+// three things stay small, each of which the first form of these kernels paid
+// for: the sums end in one atomic per workgroup, and same-address atomics
+// retire one every 12.7 ns, so the grid is capped (65536 workgroups took 833
+// us for a 256^3 float volume, the capped one 24 us, 5.6 TB/s); row and plane
+// indices come from 32-bit divisions per VEC elements instead of 64-bit ones
+// per element (anisotropic gradient 91 -> 30 us); and the isotropic gradient
+// marches along z, so that a voxel costs 2.25 square roots instead of four
+// (126 -> 66 us, bound by the correctly rounded square roots and divisions).
 constexpr int kLossThreads = 256;
+constexpr int kSumThreads = 1024;
+constexpr uint32_t kSumBlocks = 512;  // two per CU: at most 512 same-address atomics (6.5 us)
+constexpr uint32_t kMarch = 8;        // planes per thread of the isotropic gradient
 
 template <typename S>
 __device__ __forceinline__ S sgn(S x) { return x > S(0) ? S(1) : (x < S(0) ? S(-1) : S(0)); }
 
-// Block sum of one value per thread, then one atomic per block.
+// Block sum of one value per thread (in double), then one atomic per block.
 template <typename S>
 __device__ __forceinline__ void block_sum_atomic(S v, S* out) {
-    __shared__ S part[kLossThreads / kWave];
-    v = wave_sum(v);
-    if (lane_id() == 0) part[threadIdx.x / kWave] = v;
+    __shared__ double part[kSumThreads / kWave];
+    const double w = wave_sum(double(v));
+    if (lane_id() == 0) part[threadIdx.x / kWave] = w;
     __syncthreads();
     if (threadIdx.x == 0) {
-        S t = S(0);
-        for (int w = 0; w < kLossThreads / kWave; ++w) t += part[w];
-        atomic_add(out, t);
+        double t = 0.0;
+        for (int k = 0; k < kSumThreads / kWave; ++k) t += part[k];
+        atomic_add(out, S(t));
     }
 }
 
-template <typename S>
-__global__ void __launch_bounds__(kLossThreads)
-tv_fwd_kernel(const S* __restrict__ vol, uint32_t B, uint32_t D, uint32_t H, uint32_t W,
-              S* __restrict__ tv_map, S* __restrict__ tv_sum) {
-    const size_t total = size_t(B) * D * H * W;
-    const size_t idx = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    S tv = S(0);
-    if (idx < total) {
-        const uint32_t w = uint32_t(idx % W), h = uint32_t((idx / W) % H), d = uint32_t((idx / (size_t(W) * H)) % D);
-        const S v = vol[idx];
-        if (d + 1 < D) tv += fabs(vol[idx + size_t(H) * W] - v);
-        if (h + 1 < H) tv += fabs(vol[idx + W] - v);
-        if (w + 1 < W) tv += fabs(vol[idx + 1] - v);
-        tv_map[idx] = tv;
+template <typename S, int VEC>
+struct __align__(VEC * sizeof(S)) Pack {
+    S v[VEC];
+};
+
+template <typename S, int VEC>
+__device__ __forceinline__ Pack<S, VEC> load_pack(const S* __restrict__ p) {
+    return *reinterpret_cast<const Pack<S, VEC>*>(p);
+}
+template <typename S, int VEC>
+__device__ __forceinline__ void store_pack(S* __restrict__ p, const Pack<S, VEC>& x) {
+    *reinterpret_cast<Pack<S, VEC>*>(p) = x;
+}
+
+// A volume [B, D, H, W] as rows of `quads` = W / VEC packs; I is the index type
+// (32-bit unless the pack count needs 64).
+template <typename I>
+struct Volume {
+    I quads, total;  // packs per row, packs in all
+    uint32_t D, H, W;
+};
+
+// Pack i -> its first element, and its place: x (first column), h, d.
+template <typename I, int VEC>
+__device__ __forceinline__ size_t locate(const Volume<I>& g, I i, uint32_t& x, uint32_t& h, uint32_t& d) {
+    const I row = i / g.quads;
+    const I plane = row / I(g.H);
+    x = uint32_t(i - row * g.quads) * VEC;
+    h = uint32_t(row - plane * I(g.H));
+    d = uint32_t(plane % I(g.D));
+    return size_t(row) * g.W + x;
+}
+
+// One pack's forward differences along z, y and x (0 past the last index of an
+// axis); `right` is the element after the pack in its row.
+template <typename S, int VEC>
+__device__ __forceinline__ void differences(const Pack<S, VEC>& c, const Pack<S, VEC>& zn, const Pack<S, VEC>& yn,
+                                            S right, bool has_z, bool has_y, bool has_x, S (&dz)[VEC], S (&dy)[VEC],
+                                            S (&dx)[VEC]) {
+#pragma unroll
+    for (int k = 0; k < VEC; ++k) {
+        dz[k] = has_z ? zn.v[k] - c.v[k] : S(0);
+        dy[k] = has_y ? yn.v[k] - c.v[k] : S(0);
+        if (k + 1 < VEC)
+            dx[k] = c.v[k + 1 < VEC ? k + 1 : k] - c.v[k];
+        else
+            dx[k] = has_x ? right - c.v[k] : S(0);
     }
-    block_sum_atomic(tv, tv_sum);
+}
+
+// tv_map and its sum: anisotropic |dz| + |dy| + |dx|, or (ISO) the isotropic
+// sqrt(dz^2 + dy^2 + dx^2 + eps), with forward differences.
+template <typename S, typename I, int VEC, bool ISO>
+__global__ void __launch_bounds__(kSumThreads)
+tv_fwd_kernel(const S* __restrict__ vol, Volume<I> g, S eps, S* __restrict__ tv_map, S* __restrict__ tv_sum) {
+    S sum = S(0);
+    const size_t sd = size_t(g.H) * g.W, sh = g.W;
+    for (I i = I(blockIdx.x) * kSumThreads + threadIdx.x; i < g.total; i += I(gridDim.x) * kSumThreads) {
+        uint32_t x, h, d;
+        const size_t o = locate<I, VEC>(g, i, x, h, d);
+        const bool has_z = d + 1 < g.D, has_y = h + 1 < g.H, has_x = x + VEC < g.W;
+        const Pack<S, VEC> c = load_pack<S, VEC>(vol + o);
+        const Pack<S, VEC> zn = has_z ? load_pack<S, VEC>(vol + o + sd) : c;
+        const Pack<S, VEC> yn = has_y ? load_pack<S, VEC>(vol + o + sh) : c;
+        const S right = has_x ? vol[o + VEC] : S(0);
+        S dz[VEC], dy[VEC], dx[VEC];
+        differences<S, VEC>(c, zn, yn, right, has_z, has_y, has_x, dz, dy, dx);
+        Pack<S, VEC> t;
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) {
+            if constexpr (ISO) t.v[k] = sqrt(dz[k] * dz[k] + dy[k] * dy[k] + dx[k] * dx[k] + eps);
+            else t.v[k] = fabs(dz[k]) + fabs(dy[k]) + fabs(dx[k]);
+            sum += t.v[k];
+        }
+        store_pack<S, VEC>(tv_map + o, t);
+    }
+    block_sum_atomic(sum, tv_sum);
 }
 
 // grad = ((sign sum) * (g / edges)) * lambda: the reference's rounding order
 // (the kernel's g / edges product, then the host-side multiply by lambda).
-template <typename S>
+template <typename S, typename I, int VEC>
 __global__ void __launch_bounds__(kLossThreads)
-tv_bwd_kernel(const S* __restrict__ vol, const S* __restrict__ grad_out, uint32_t B, uint32_t D, uint32_t H,
-              uint32_t W, S edges, S lambda, S* __restrict__ grad) {
-    const size_t total = size_t(B) * D * H * W;
-    const size_t idx = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (idx >= total) return;
-    const uint32_t w = uint32_t(idx % W), h = uint32_t((idx / W) % H), d = uint32_t((idx / (size_t(W) * H)) % D);
-    const S v = vol[idx];
-    const size_t sd = size_t(H) * W, sh = W;
-    S g = S(0);
-    if (d + 1 < D) g -= sgn(vol[idx + sd] - v);
-    if (d > 0) g += sgn(v - vol[idx - sd]);
-    if (h + 1 < H) g -= sgn(vol[idx + sh] - v);
-    if (h > 0) g += sgn(v - vol[idx - sh]);
-    if (w + 1 < W) g -= sgn(vol[idx + 1] - v);
-    if (w > 0) g += sgn(v - vol[idx - 1]);
+tv_bwd_kernel(const S* __restrict__ vol, const S* __restrict__ grad_out, Volume<I> g, S edges, S lambda,
+              S* __restrict__ grad) {
+    const I i = I(blockIdx.x) * kLossThreads + threadIdx.x;
+    if (i >= g.total) return;
+    uint32_t x, h, d;
+    const size_t o = locate<I, VEC>(g, i, x, h, d), sd = size_t(g.H) * g.W, sh = g.W;
+    const bool has_zn = d + 1 < g.D, has_zp = d > 0, has_yn = h + 1 < g.H, has_yp = h > 0;
+    const Pack<S, VEC> c = load_pack<S, VEC>(vol + o);
+    // a missing neighbour equals the voxel: its sign is 0
+    const Pack<S, VEC> zn = has_zn ? load_pack<S, VEC>(vol + o + sd) : c;
+    const Pack<S, VEC> zp = has_zp ? load_pack<S, VEC>(vol + o - sd) : c;
+    const Pack<S, VEC> yn = has_yn ? load_pack<S, VEC>(vol + o + sh) : c;
+    const Pack<S, VEC> yp = has_yp ? load_pack<S, VEC>(vol + o - sh) : c;
+    const bool has_xn = x + VEC < g.W, has_xp = x > 0;
+    const S right = has_xn ? vol[o + VEC] : S(0), left = has_xp ? vol[o - 1] : S(0);
     const S per_edge = grad_out[0] / edges;
-    grad[idx] = (g * per_edge) * lambda;
+    Pack<S, VEC> out;
+#pragma unroll
+    for (int k = 0; k < VEC; ++k) {
+        const S v = c.v[k];
+        S s = S(0);
+        if (has_zn) s -= sgn(zn.v[k] - v);
+        if (has_zp) s += sgn(v - zp.v[k]);
+        if (has_yn) s -= sgn(yn.v[k] - v);
+        if (has_yp) s += sgn(v - yp.v[k]);
+        if (k + 1 < VEC) s -= sgn(c.v[k + 1 < VEC ? k + 1 : k] - v);
+        else if (has_xn) s -= sgn(right - v);
+        if (k > 0) s += sgn(v - c.v[k > 0 ? k - 1 : k]);
+        else if (has_xp) s += sgn(v - left);
+        out.v[k] = (s * per_edge) * lambda;
+    }
+    store_pack<S, VEC>(grad + o, out);
 }
 
-// Isotropic TV: t(v) = sqrt(dz^2 + dy^2 + dx^2 + eps) with forward differences
-// (zero past the last index of an axis); tv_map = t, tv_sum = sum of t.
-template <typename S>
-__device__ __forceinline__ S iso_term(const S* __restrict__ vol, size_t idx, uint32_t d, uint32_t h, uint32_t w,
-                                      uint32_t D, uint32_t H, uint32_t W, S eps, S& dz, S& dy, S& dx) {
-    const S v = vol[idx];
-    dz = d + 1 < D ? vol[idx + size_t(H) * W] - v : S(0);
-    dy = h + 1 < H ? vol[idx + W] - v : S(0);
-    dx = w + 1 < W ? vol[idx + 1] - v : S(0);
-    return sqrt(dz * dz + dy * dy + dx * dx + eps);
-}
-
-template <typename S>
+// d/dV(v) of sum_u t(u), t the isotropic term: -(dz + dy + dx)(v) / t(v) plus
+// dz(v - ez) / t(v - ez), dy(v - ey) / t(v - ey) and dx(v - ex) / t(v - ex)
+// where those voxels exist. A thread takes a pack's column over kMarch planes:
+// plane d's dz / t is what plane d + 1 needs, and the pack's own dx / t what
+// its next columns need, so a voxel costs its own term, the one below it in y
+// and 1 / VEC of the one to its left. `total` counts (plane chunk, row, pack).
+template <typename S, typename I, int VEC>
 __global__ void __launch_bounds__(kLossThreads)
-tv_iso_fwd_kernel(const S* __restrict__ vol, uint32_t B, uint32_t D, uint32_t H, uint32_t W, S eps,
-                  S* __restrict__ tv_map, S* __restrict__ tv_sum) {
-    const size_t total = size_t(B) * D * H * W;
-    const size_t idx = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    S t = S(0);
-    if (idx < total) {
-        const uint32_t w = uint32_t(idx % W), h = uint32_t((idx / W) % H), d = uint32_t((idx / (size_t(W) * H)) % D);
-        S dz, dy, dx;
-        t = iso_term(vol, idx, d, h, w, D, H, W, eps, dz, dy, dx);
-        tv_map[idx] = t;
+tv_iso_bwd_kernel(const S* __restrict__ vol, const S* __restrict__ grad_out, Volume<I> g, uint32_t chunks, S eps,
+                  S scale, S* __restrict__ grad) {
+    const I i = I(blockIdx.x) * kLossThreads + threadIdx.x;
+    if (i >= g.total) return;
+    const I row = i / g.quads, slab = row / I(g.H);
+    const uint32_t x = uint32_t(i - row * g.quads) * VEC, h = uint32_t(row - slab * I(g.H));
+    const I b = slab / I(chunks);
+    const uint32_t d0 = uint32_t(slab - b * I(chunks)) * kMarch, d1 = min(g.D, d0 + kMarch);
+    const size_t sd = size_t(g.H) * g.W, sh = g.W;
+    const bool has_yn = h + 1 < g.H, has_yp = h > 0, has_xn = x + VEC < g.W, has_xp = x > 0;
+    const S gs = grad_out[0] * scale;
+    size_t o = ((size_t(b) * g.D + d0) * g.H + h) * g.W + x;
+    Pack<S, VEC> c = load_pack<S, VEC>(vol + o);
+    S below[VEC];  // dz / t of the plane below
+#pragma unroll
+    for (int k = 0; k < VEC; ++k) below[k] = S(0);
+    if (d0 > 0) {
+        const size_t q = o - sd;
+        const Pack<S, VEC> p = load_pack<S, VEC>(vol + q);
+        const Pack<S, VEC> yn = has_yn ? load_pack<S, VEC>(vol + q + sh) : p;
+        const S right = has_xn ? vol[q + VEC] : S(0);
+        S dz[VEC], dy[VEC], dx[VEC];
+        differences<S, VEC>(p, c, yn, right, true, has_yn, has_xn, dz, dy, dx);
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) below[k] = dz[k] / sqrt(dz[k] * dz[k] + dy[k] * dy[k] + dx[k] * dx[k] + eps);
     }
-    block_sum_atomic(t, tv_sum);
+    for (uint32_t d = d0; d < d1; ++d, o += sd) {
+        const bool has_z = d + 1 < g.D;
+        const Pack<S, VEC> zn = has_z ? load_pack<S, VEC>(vol + o + sd) : c;
+        const Pack<S, VEC> yn = has_yn ? load_pack<S, VEC>(vol + o + sh) : c;
+        const S right = has_xn ? vol[o + VEC] : S(0);
+        S dz[VEC], dy[VEC], dx[VEC];
+        differences<S, VEC>(c, zn, yn, right, has_z, has_yn, has_xn, dz, dy, dx);
+        S carry_x = S(0);  // dx / t of the voxel to the left
+        if (has_xp) {
+            const S l = vol[o - 1];
+            const S lz = has_z ? vol[o + sd - 1] - l : S(0), ly = has_yn ? vol[o + sh - 1] - l : S(0);
+            const S lx = c.v[0] - l;
+            carry_x = lx / sqrt(lz * lz + ly * ly + lx * lx + eps);
+        }
+        S from_y[VEC];  // dy / t of the voxel at y - 1
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) from_y[k] = S(0);
+        if (has_yp) {
+            const size_t q = o - sh;
+            const Pack<S, VEC> p = load_pack<S, VEC>(vol + q);
+            const Pack<S, VEC> pz = has_z ? load_pack<S, VEC>(vol + q + sd) : p;
+            const S pr = has_xn ? vol[q + VEC] : S(0);
+            S az[VEC], ay[VEC], ax[VEC];
+            differences<S, VEC>(p, pz, c, pr, has_z, true, has_xn, az, ay, ax);
+#pragma unroll
+            for (int k = 0; k < VEC; ++k)
+                from_y[k] = ay[k] / sqrt(az[k] * az[k] + ay[k] * ay[k] + ax[k] * ax[k] + eps);
+        }
+        Pack<S, VEC> out;
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) {
+            const S t = sqrt(dz[k] * dz[k] + dy[k] * dy[k] + dx[k] * dx[k] + eps);
+            S s = -(dz[k] + dy[k] + dx[k]) / t;
+            s += below[k];
+            s += from_y[k];
+            s += carry_x;
+            out.v[k] = s * gs;
+            below[k] = dz[k] / t;
+            carry_x = dx[k] / t;
+        }
+        store_pack<S, VEC>(grad + o, out);
+        c = zn;
+    }
 }
 
-// d/dV(v) of sum_u t(u): -(dz + dy + dx)(v) / t(v) plus dz(v - ez) / t(v - ez),
-// dy(v - ey) / t(v - ey) and dx(v - ex) / t(v - ex) where those voxels exist.
-template <typename S>
-__global__ void __launch_bounds__(kLossThreads)
-tv_iso_bwd_kernel(const S* __restrict__ vol, const S* __restrict__ grad_out, uint32_t B, uint32_t D, uint32_t H,
-                  uint32_t W, S eps, S scale, S* __restrict__ grad) {
-    const size_t total = size_t(B) * D * H * W;
-    const size_t idx = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (idx >= total) return;
-    const uint32_t w = uint32_t(idx % W), h = uint32_t((idx / W) % H), d = uint32_t((idx / (size_t(W) * H)) % D);
-    const size_t sd = size_t(H) * W, sh = W;
-    S dz, dy, dx;
-    S t = iso_term(vol, idx, d, h, w, D, H, W, eps, dz, dy, dx);
-    S g = -(dz + dy + dx) / t;
-    if (d > 0) {
-        t = iso_term(vol, idx - sd, d - 1, h, w, D, H, W, eps, dz, dy, dx);
-        g += dz / t;
-    }
-    if (h > 0) {
-        t = iso_term(vol, idx - sh, d, h - 1, w, D, H, W, eps, dz, dy, dx);
-        g += dy / t;
-    }
-    if (w > 0) {
-        t = iso_term(vol, idx - 1, d, h, w - 1, D, H, W, eps, dz, dy, dx);
-        g += dx / t;
-    }
-    grad[idx] = g * (grad_out[0] * scale);
-}
-
-template <typename S>
-__global__ void __launch_bounds__(kLossThreads)
+template <typename S, int VEC>
+__global__ void __launch_bounds__(kSumThreads)
 l1_fwd_kernel(const S* __restrict__ p, const S* __restrict__ t, uint64_t n, S* __restrict__ map,
               S* __restrict__ sum) {
-    const size_t idx = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    S a = S(0);
-    if (idx < n) {
-        a = fabs(p[idx] - t[idx]);
-        map[idx] = a;
+    S s = S(0);
+    for (uint64_t i = uint64_t(blockIdx.x) * kSumThreads + threadIdx.x; i < n / VEC;
+         i += uint64_t(gridDim.x) * kSumThreads) {
+        const Pack<S, VEC> a = load_pack<S, VEC>(p + i * VEC), b = load_pack<S, VEC>(t + i * VEC);
+        Pack<S, VEC> m;
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) {
+            m.v[k] = fabs(a.v[k] - b.v[k]);
+            s += m.v[k];
+        }
+        store_pack<S, VEC>(map + i * VEC, m);
     }
-    block_sum_atomic(a, sum);
+    block_sum_atomic(s, sum);
 }
 
 template <typename S>
@@ -144,6 +264,45 @@ l1_bwd_kernel(const S* __restrict__ p, const S* __restrict__ t, const S* __restr
     const size_t idx = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (idx >= n) return;
     out[idx] = g[0] * lambda * sgn(p[idx] - t[idx]) / S(n);  // the reference's operation order
+}
+
+// Whether `length` and the pointers allow 16-byte packs of S.
+template <typename S>
+static bool packed16(uint64_t length, const void* a, const void* b, const void* c = nullptr) {
+    const uintptr_t bits = reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b) |
+                           reinterpret_cast<uintptr_t>(c);
+    return length % (16 / sizeof(S)) == 0 && bits % 16 == 0;
+}
+
+static uint32_t sum_blocks(uint64_t items) {
+    return std::min<uint32_t>(kSumBlocks, std::max<uint32_t>(1u, ceil_div(items, kSumThreads)));
+}
+
+// Calls f(I{}, std::integral_constant<int, VEC>{}) with the pack width that W
+// and the pointers allow and 32-bit indices where `rows` packed rows fit them
+// (grid-stride loops step up to 2^19 past the last index).
+template <typename S, typename F>
+static int with_packs(uint64_t rows, uint32_t W, const void* a, const void* b, F&& f) {
+    constexpr int kWide = 16 / int(sizeof(S));
+    const bool wide = packed16<S>(W, a, b);
+    const bool small = rows * (wide ? W / kWide : W) < (1ull << 32) - (1ull << 20);
+    if (wide && small) return f(uint32_t{}, std::integral_constant<int, kWide>{});
+    if (wide) return f(uint64_t{}, std::integral_constant<int, kWide>{});
+    if (small) return f(uint32_t{}, std::integral_constant<int, 1>{});
+    return f(uint64_t{}, std::integral_constant<int, 1>{});
+}
+
+template <typename S, bool ISO>
+static int launch_tv_fwd(const S* vol, uint32_t B, uint32_t D, uint32_t H, uint32_t W, S eps, S* map, S* sum,
+                         hipStream_t stream, const char* where) {
+    const uint64_t rows = uint64_t(B) * D * H;
+    return with_packs<S>(rows, W, vol, map, [&](auto index, auto vec) {
+        using I = decltype(index);
+        constexpr int VEC = decltype(vec)::value;
+        const Volume<I> g{I(W / VEC), I(rows * (W / VEC)), D, H, W};
+        tv_fwd_kernel<S, I, VEC, ISO><<<sum_blocks(g.total), kSumThreads, 0, stream>>>(vol, g, eps, map, sum);
+        return check_launch(where);
+    });
 }
 
 }  // namespace r2s
@@ -157,9 +316,8 @@ extern "C" int r2s_volume_tv_fwd(int dtype, const void* volume, uint32_t B, uint
         using S = decltype(tag);
         if (int rc = fill_zero<S>((S*)tv_sum, 1, stream)) return rc;
         if (total == 0) return R2S_OK;
-        tv_fwd_kernel<S><<<ceil_div(total, kLossThreads), kLossThreads, 0, stream>>>(
-            (const S*)volume, B, D, H, W, (S*)tv_map, (S*)tv_sum);
-        return check_launch("volume_tv_fwd");
+        return launch_tv_fwd<S, false>((const S*)volume, B, D, H, W, S(0), (S*)tv_map, (S*)tv_sum, stream,
+                                       "volume_tv_fwd");
     });
 }
 
@@ -173,9 +331,15 @@ extern "C" int r2s_volume_tv_bwd(int dtype, const void* volume, const void* grad
     const int64_t edges = edges64 < 1 ? 1 : edges64;
     return dispatch_dtype(dtype, [&](auto tag) {
         using S = decltype(tag);
-        tv_bwd_kernel<S><<<ceil_div(total, kLossThreads), kLossThreads, 0, stream>>>(
-            (const S*)volume, (const S*)grad_output, B, D, H, W, S(edges), S(lambda_tv), (S*)grad_volume);
-        return check_launch("volume_tv_bwd");
+        const uint64_t rows = uint64_t(B) * D * H;
+        return with_packs<S>(rows, W, volume, grad_volume, [&](auto index, auto vec) {
+            using I = decltype(index);
+            constexpr int VEC = decltype(vec)::value;
+            const Volume<I> g{I(W / VEC), I(rows * (W / VEC)), D, H, W};
+            tv_bwd_kernel<S, I, VEC><<<ceil_div(g.total, kLossThreads), kLossThreads, 0, stream>>>(
+                (const S*)volume, (const S*)grad_output, g, S(edges), S(lambda_tv), (S*)grad_volume);
+            return check_launch("volume_tv_bwd");
+        });
     });
 }
 
@@ -187,9 +351,8 @@ extern "C" int r2s_volume_tv_iso_fwd(int dtype, const void* volume, uint32_t B, 
         using S = decltype(tag);
         if (int rc = fill_zero<S>((S*)tv_sum, 1, stream)) return rc;
         if (total == 0) return R2S_OK;
-        tv_iso_fwd_kernel<S><<<ceil_div(total, kLossThreads), kLossThreads, 0, stream>>>(
-            (const S*)volume, B, D, H, W, S(eps), (S*)tv_map, (S*)tv_sum);
-        return check_launch("volume_tv_iso_fwd");
+        return launch_tv_fwd<S, true>((const S*)volume, B, D, H, W, S(eps), (S*)tv_map, (S*)tv_sum, stream,
+                                      "volume_tv_iso_fwd");
     });
 }
 
@@ -201,10 +364,17 @@ extern "C" int r2s_volume_tv_iso_bwd(int dtype, const void* volume, const void* 
     if (total == 0) return R2S_OK;
     return dispatch_dtype(dtype, [&](auto tag) {
         using S = decltype(tag);
-        tv_iso_bwd_kernel<S><<<ceil_div(total, kLossThreads), kLossThreads, 0, stream>>>(
-            (const S*)volume, (const S*)grad_output, B, D, H, W, S(eps), S(lambda_tv / double(total)),
-            (S*)grad_volume);
-        return check_launch("volume_tv_iso_bwd");
+        const uint32_t chunks = ceil_div(D, kMarch);
+        const uint64_t rows = uint64_t(B) * chunks * H;  // one per (plane chunk, row)
+        return with_packs<S>(rows, W, volume, grad_volume, [&](auto index, auto vec) {
+            using I = decltype(index);
+            constexpr int VEC = decltype(vec)::value;
+            const Volume<I> g{I(W / VEC), I(rows * (W / VEC)), D, H, W};
+            tv_iso_bwd_kernel<S, I, VEC><<<ceil_div(g.total, kLossThreads), kLossThreads, 0, stream>>>(
+                (const S*)volume, (const S*)grad_output, g, chunks, S(eps), S(lambda_tv / double(total)),
+                (S*)grad_volume);
+            return check_launch("volume_tv_iso_bwd");
+        });
     });
 }
 
@@ -214,8 +384,13 @@ extern "C" int r2s_image_l1_fwd(int dtype, const void* prediction, const void* t
         using S = decltype(tag);
         if (int rc = fill_zero<S>((S*)l1_sum, 1, stream)) return rc;
         if (n == 0) return R2S_OK;
-        l1_fwd_kernel<S><<<ceil_div(n, kLossThreads), kLossThreads, 0, stream>>>(
-            (const S*)prediction, (const S*)target, n, (S*)l1_map, (S*)l1_sum);
+        constexpr int kWide = 16 / int(sizeof(S));
+        if (packed16<S>(n, prediction, target, l1_map))
+            l1_fwd_kernel<S, kWide><<<sum_blocks(n / kWide), kSumThreads, 0, stream>>>(
+                (const S*)prediction, (const S*)target, n, (S*)l1_map, (S*)l1_sum);
+        else
+            l1_fwd_kernel<S, 1><<<sum_blocks(n), kSumThreads, 0, stream>>>(
+                (const S*)prediction, (const S*)target, n, (S*)l1_map, (S*)l1_sum);
         return check_launch("image_l1_fwd");
     });
 }

@@ -1,0 +1,64 @@
+"""Volume and image loss kernels at the edges of their packing: row lengths
+that are and are not a multiple of a 16-byte pack, pointers off that boundary,
+plane counts around the gradient's march, and more packs than one sweep."""
+
+import pytest
+import torch
+
+from oracle import splat as O
+from r2splat_amd import hip as ops
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(1, 1, 1, 1), (1, 8, 2, 4), (2, 9, 3, 8), (1, 17, 5, 3), (3, 7, 1, 12), (1, 130, 128, 132)]
+
+
+def _place(x, device, offset):
+    """x on the device, its first element `offset` elements past an allocation's start."""
+    flat = torch.empty(x.numel() + offset, dtype=x.dtype, device=device)
+    out = flat[offset:].view(x.shape)
+    out.copy_(x)
+    return out
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_tv_losses_at_pack_edges(shape, offset, dtype):
+    device = torch.device("cuda:0")
+    g = torch.Generator().manual_seed(sum(shape) + offset)
+    vol = torch.randn(*shape, generator=g, dtype=torch.float64).to(dtype)
+    ref = vol.double().requires_grad_()
+    x = _place(vol, device, offset)
+    one = torch.ones(1, device=device, dtype=dtype)
+    # one rounding per operation of a short chain; the sums of n terms of one
+    # sign in chains of at most 512 partial sums
+    t = 2e-6 if dtype == torch.float32 else 1e-12
+    for fwd, bwd, oracle in ((ops.volume_loss_fwd, ops.volume_loss_bwd, O.volume_tv(ref)),
+                             (ops.volume_loss_iso_fwd, ops.volume_loss_iso_bwd, O.volume_tv_iso(ref, 1e-8))):
+        (grad,) = torch.autograd.grad(oracle, ref)
+        _, tv, tv_map = fwd(x, 1.0)
+        assert abs(tv.item() - oracle.item()) <= t * abs(oracle.item())
+        n = max(sum(s1 for s1 in _edge_counts(shape)), 1) if fwd is ops.volume_loss_fwd else vol.numel()
+        assert abs(tv_map.double().sum().item() / n - oracle.item()) <= t * abs(oracle.item())
+        got = bwd(x, one, 1.0)
+        assert O.relative_error(got, grad) <= 5 * t
+
+
+def _edge_counts(shape):
+    B, D, H, W = shape
+    return B * (D - 1) * H * W, B * D * (H - 1) * W, B * D * H * (W - 1)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("n,offset", [(1, 0), (4, 0), (1023, 0), (4096, 1), (2_200_000, 0)])
+def test_image_l1_at_pack_edges(n, offset, dtype):
+    device = torch.device("cuda:0")
+    g = torch.Generator().manual_seed(n)
+    p = torch.randn(1, 1, n, generator=g, dtype=torch.float64).to(dtype)
+    q = torch.randn(1, 1, n, generator=g, dtype=torch.float64).to(dtype)
+    _, l1, l1_map = ops.image_loss_l1_fwd(_place(p, device, offset), _place(q, device, offset), 1.0)
+    expected = (p - q).abs()
+    assert torch.equal(l1_map.cpu(), expected)
+    t = 2e-6 if dtype == torch.float32 else 1e-12
+    assert abs(l1.item() - expected.double().mean().item()) <= t * expected.double().mean().item()

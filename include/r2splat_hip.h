@@ -126,6 +126,13 @@ int r2s_conics_mu_bwd(int dtype, const void* cov2d, double eps, const void* coni
                       const void* mus, const void* v_conics, const void* v_mus,
                       void* v_cov2d, uint32_t total, r2s_stream_t stream);
 
+/* betas [n] -> ratio [n] = B(1/2, beta + 1) / sqrt(2 pi), the line-integral factor
+ * of a Beta primitive, and log_grad [n] = d log ratio / d beta, evaluated in
+ * double (either output may be NULL). The reference computes them in Python
+ * (r2splat/_beta.py:10-49). */
+int r2s_beta_factors(int dtype, const void* betas, uint64_t n, void* ratio, void* log_grad,
+                     r2s_stream_t stream);
+
 /* means [N,3], covars [N,6], max_scales [N] (unused metadata), ranges [3],
  * centers [3] -> means3d_v [N,3] voxel coordinates, conics [N,6] (inverse voxel
  * covariance, packed), radii int32 [N,3]. The 3x3 inversion runs in double.

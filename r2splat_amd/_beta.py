@@ -19,6 +19,8 @@ import math
 
 import torch
 
+from .hip import _backend as be
+
 _SWITCH = 20.0
 # (power of 1/z, coefficient) of log Gamma(z) - log Gamma(z + 1/2) + 1/2 log z.
 _SERIES = ((1, 1.0 / 8.0), (3, -1.0 / 192.0), (5, 1.0 / 640.0), (7, -17.0 / 14336.0), (9, 31.0 / 18432.0))
@@ -54,4 +56,20 @@ def beta_path_log_grad(gamma: torch.Tensor) -> torch.Tensor:
     return torch.where(value < _SWITCH, direct, derivative).to(gamma.dtype)
 
 
-__all__ = ["beta_path_ratio", "beta_path_log_grad"]
+def beta_factors(gamma: torch.Tensor, ratio: torch.Tensor | None = None, log_grad: torch.Tensor | None = None):
+    """(beta_path_ratio, beta_path_log_grad) of constant exponents, into the
+    given buffers if any. On the GPU one native launch evaluates both in
+    double; elsewhere (and for exponents that autograd follows) the forms above."""
+    if not gamma.is_cuda or (gamma.requires_grad and torch.is_grad_enabled()):
+        values = (beta_path_ratio(gamma).contiguous(), beta_path_log_grad(gamma).contiguous())
+        return tuple(v if out is None else out.copy_(v) for v, out in zip(values, (ratio, log_grad)))
+    gamma = gamma.contiguous()
+    ratio = torch.empty_like(gamma) if ratio is None else ratio
+    log_grad = torch.empty_like(gamma) if log_grad is None else log_grad
+    with torch.cuda.device(gamma.device):
+        be.call("r2s_beta_factors", be.dtype_code(gamma.dtype), be.ptr(gamma), gamma.numel(), be.ptr(ratio),
+                be.ptr(log_grad), be.stream_of(gamma.device))
+    return ratio, log_grad
+
+
+__all__ = ["beta_factors", "beta_path_ratio", "beta_path_log_grad"]

@@ -138,19 +138,6 @@ __device__ __forceinline__ uint32_t qlim_of(float w) {
 
 __device__ __forceinline__ bool contributes(float q, uint32_t qlim) { return __float_as_uint(q) < qlim; }
 
-// The Beta line-integral factor r(beta) = Gamma(beta + 1) / (sqrt(2)
-// Gamma(beta + 3/2)) in double, as the host computes it (lgamma below 20; from
-// 20 the Stirling series of log Gamma(z) - log Gamma(z + 1/2) + 1/2 log z, z =
-// beta + 1, which avoids the cancellation of two large lgamma values).
-__device__ __forceinline__ double beta_ratio_f64(double beta) {
-    constexpr double kHalfLn2 = 0.34657359027997264;
-    if (beta < 20.0) return exp(lgamma(beta + 1.0) - lgamma(beta + 1.5) - kHalfLn2);
-    const double z = beta + 1.0, w = 1.0 / z, w2 = w * w;
-    const double series = w * (1.0 / 8.0 + w2 * (-1.0 / 192.0 + w2 * (1.0 / 640.0 + w2 * (-17.0 / 14336.0 +
-                                                                                          w2 * (31.0 / 18432.0)))));
-    return exp(series - 0.5 * (2.0 * kHalfLn2 + log(z)));
-}
-
 // The Beta cut-off in double: the largest d^2 with |w| (1 - d^2)^b2d >= 1e-5
 // (-1 when |w| < 1e-5), and the qlim of its float32 rounding.
 // Takes inv_b2d = 1 / b2d (NaN when b2d <= 0) and forms the bound as
@@ -455,7 +442,11 @@ permute_params_kernel(const uint32_t* __restrict__ perm, uint32_t N, const float
     PrimFrame f;
     covariance_from(R, s, f.cov);
     const double b2d = betas ? double(betas[n]) + 0.5 : 0.0;
-    f.ratio = betas ? beta_ratio_f64(double(betas[n])) : 0.0;
+    f.ratio = 0.0;
+    if (betas) {
+        double log_grad;
+        beta_factors_f64(double(betas[n]), f.ratio, log_grad);
+    }
     f.inv_b2d = b2d > 0.0 ? 1.0 / b2d : __builtin_nan("");
     o_frames[p] = f;
 }

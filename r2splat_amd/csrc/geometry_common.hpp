@@ -362,6 +362,46 @@ __device__ __forceinline__ void conic_mu_vjp_f64(const double c[6], const double
 }
 
 // ---------------------------------------------------------------------------
+// Beta line-integral factor r(beta) = Gamma(beta + 1) / (sqrt(2) Gamma(beta +
+// 3/2)) and d log r / d beta = psi(beta + 1) - psi(beta + 3/2), in double
+// (r2splat/_beta.py:10-49). With a = beta + 1 the argument is raised to z = a +
+// n >= 10 by the recurrences of Gamma and psi, every term of which has one
+// sign (no cancellation of two large values), and the rest is the asymptotic
+// series log Gamma(z) - log Gamma(z + 1/2) + 1/2 log z = sum_k (2 - 2^-k)
+// B_(k+1) / (k (k+1) z^k), k = 1, 3, .., 13 (the next term is below 1e-16).
+// beta <= -1 (outside the primitives' domain) goes through lgamma and the
+// reflection of psi.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ void beta_factors_f64(double beta, double& ratio, double& log_grad) {
+    constexpr double kC[7] = {1.0 / 8.0, -1.0 / 192.0, 1.0 / 640.0, -17.0 / 14336.0, 31.0 / 18432.0,
+                              -691.0 / 180224.0, 5461.0 / 425984.0};
+    const bool below = beta <= -1.0;
+    const double a = beta + 1.0, start = below ? 0.5 - a : a;
+    double num = 1.0, den = 1.0, shift = 0.0, z = start;
+    while (z < 10.0) {
+        num *= z + 0.5;
+        den *= z;
+        shift -= 0.5 / (z * (z + 0.5));
+        z += 1.0;
+    }
+    const double w = 1.0 / z, w2 = w * w;
+    double series = 0.0, slope = 0.0;
+#pragma unroll
+    for (int i = 6; i >= 0; --i) {
+        series = fma(series, w2, kC[i]);
+        slope = fma(slope, w2, double(2 * i + 1) * kC[i]);
+    }
+    ratio = (num / den) * exp(series * w) / ::sqrt(2.0 * z);
+    log_grad = shift - w * (0.5 + slope * w);
+    if (below) {
+        ratio = exp(lgamma(a) - lgamma(a + 0.5) - 0.34657359027997264);  // ln 2 / 2
+        double s, c;
+        sincospi(a, &s, &c);
+        log_grad = -log_grad - M_PI * (c / s + s / c);
+    }
+}
+
+// ---------------------------------------------------------------------------
 // World -> volume mapping (WorldToVolumeMappingFwd.cu:57-157,
 // WorldToVolumeMappingBwd.cu:51-167, CovarianceMath.cuh:10-68).
 // ---------------------------------------------------------------------------

@@ -24,7 +24,7 @@ from . import fused
 from . import hip as ops
 from .hip import _backend as be
 from .hip import _wrapper as _ops_impl
-from ._beta import beta_path_log_grad, beta_path_ratio
+from ._beta import beta_factors
 from .profiling import stage
 
 Tensor = torch.Tensor
@@ -258,9 +258,9 @@ def _raster_state(prims, viewmats, Ks, width, height, eps, radius_clip) -> dict:
                                                                  radius_clip)
         conics, base_mus = ops.conics_mu_fwd(cov2d, eps)
     opacity = densities.unsqueeze(0).expand(C, -1).contiguous()
-    mus, beta2d, ratio = base_mus, None, None
+    mus, beta2d, ratio, log_grad = base_mus, None, None, None
     if beta is not None:
-        ratio = beta_path_ratio(beta)
+        ratio, log_grad = beta_factors(beta)
         mus = base_mus * ratio.unsqueeze(0)
         beta2d = (beta + 0.5).unsqueeze(0).expand(C, -1).contiguous()
     tiles_x, tiles_y = (width + T - 1) // T, (height + T - 1) // T
@@ -268,7 +268,7 @@ def _raster_state(prims, viewmats, Ks, width, height, eps, radius_clip) -> dict:
         _, isect_ids, flatten_ids = ops.isect_tiles(mapped, radii, T, tiles_x, tiles_y)
         offsets = ops.isect_offset_encode(isect_ids, C, tiles_x, tiles_y)
     return dict(covars=covars, mapped=mapped, cov2d=cov2d, conics=conics, base_mus=base_mus, mus=mus,
-                opacity=opacity, beta2d=beta2d, ratio=ratio, offsets=offsets, isect_ids=isect_ids,
+                opacity=opacity, beta2d=beta2d, ratio=ratio, log_grad=log_grad, offsets=offsets, isect_ids=isect_ids,
                 flatten_ids=flatten_ids)
 
 
@@ -381,7 +381,7 @@ def rasterize_bwd(context: _Context, v_image: Optional[Tensor], v_variance: Opti
     v_beta = None
     if beta is not None:
         # mu_beta = mu_gauss * ratio(beta) and the projected exponent is beta + 1/2.
-        v_beta = grads[5].sum(dim=0) + (v_mus * b["mus"]).sum(dim=0) * beta_path_log_grad(beta)
+        v_beta = grads[5].sum(dim=0) + (v_mus * b["mus"]).sum(dim=0) * b["log_grad"]
         v_mus = (v_mus * b["ratio"].unsqueeze(0)).contiguous()
     with stage("project_bwd"):
         v_cov2d = ops.conics_mu_bwd(b["cov2d"], context.eps, b["conics"], b["base_mus"], v_conics.contiguous(),

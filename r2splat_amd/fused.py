@@ -21,7 +21,7 @@ from typing import Optional
 
 import torch
 
-from ._beta import beta_path_log_grad, beta_path_ratio
+from ._beta import beta_factors
 from .hip import _backend as be
 from .hip._backend import call, ptr
 from .profiling import stage
@@ -117,11 +117,6 @@ def _kind(beta, uncertainty) -> int:
 def _scratch(C, N, width, height, tile_size, capacity, beta, device):
     nbytes = be.lib().r2s_fused_scratch_bytes(C, N, width, height, tile_size, capacity, beta)
     return torch.empty((nbytes,), dtype=torch.uint8, device=device)
-
-
-def beta_factors(beta: torch.Tensor):
-    """(ratio, log_grad) of float32 betas, as the explicit path computes them."""
-    return beta_path_ratio(beta).contiguous(), beta_path_log_grad(beta).contiguous()
 
 
 def prepare(means, quats, scales, densities, viewmats, Ks, width, height, eps, radius_clip, *, capacity=None,

@@ -58,6 +58,7 @@ SIGNATURES = {
     "r2s_world_to_image_projection_bwd": [I32, P, P, P, P, U32, U32, P, P, P, P, U32, U32, P],
     "r2s_conics_mu_fwd": [I32, P, D, P, P, U32, P],
     "r2s_conics_mu_bwd": [I32, P, D, P, P, P, P, P, U32, P],
+    "r2s_beta_factors": [I32, P, U64, P, P, P],
     "r2s_world_to_volume_mapping_fwd": [I32, P, P, P, P, P, U32, U32, U32, D, D, P, P, P, U32, P],
     "r2s_world_to_volume_mapping_bwd": [I32, P, P, P, P, U32, U32, U32, D, P, P, P, P, U32, P],
     "r2s_scan_workspace_bytes": [U64],

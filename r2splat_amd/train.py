@@ -29,7 +29,7 @@ from typing import Optional
 import torch
 
 from . import fused
-from ._beta import beta_path_log_grad, beta_path_ratio
+from ._beta import beta_factors
 from .hip import _backend as be
 from .hip._backend import call, ptr
 
@@ -205,8 +205,7 @@ class GaussianFit:
         s = be.stream_of(self.device)
         ws = self.ws
         if self.kind:  # line-integral factors of the current betas (float64 math, as the explicit path)
-            self.beta_ratio.copy_(beta_path_ratio(self.beta))
-            self.beta_log_grad.copy_(beta_path_log_grad(self.beta))
+            beta_factors(self.beta, self.beta_ratio, self.beta_log_grad)
         call("r2s_fused_prepare", ptr(self.means), ptr(self.quats), ptr(self.scales), ptr(self.densities),
              ptr(self.beta), ptr(self.beta_ratio), None, ptr(self.viewmats), ptr(self.Ks), self.C, self.N, self.W,
              self.H, self.tile_size, self.eps, self.radius_clip, self.capacity,

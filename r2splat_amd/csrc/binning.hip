@@ -11,6 +11,9 @@
 #include "common.hpp"
 #include "binning.hpp"
 
+#include <type_traits>
+#include <utility>
+
 namespace r2s {
 
 // ---------------------------------------------------------------------------
@@ -111,21 +114,11 @@ constexpr int kScanBigThreads = 1024;
 constexpr int kScanBigItems = 16;
 constexpr uint32_t kScanBigTile = kScanBigThreads * kScanBigItems;
 
-__device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t x) {
-    const int lane = lane_id();
-#pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) {
-        const uint32_t y = __shfl_up(x, off, kWave);
-        if (lane >= off) x += y;
-    }
-    return x;
-}
-
 // Block-wide exclusive scan of one value per thread; returns the block total.
 __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t x, uint32_t& excl, uint32_t* lds_waves) {
     const int lane = lane_id(), wave = threadIdx.x / kWave;
     const int n_waves = blockDim.x / kWave;
-    const uint32_t incl = wave_inclusive_scan(x);
+    const uint32_t incl = wave_scan(x);
     if (lane == kWave - 1) lds_waves[wave] = incl;
     __syncthreads();
     uint32_t base = 0, total = 0;
@@ -228,12 +221,11 @@ size_t scan_workspace_bytes(uint64_t n) { return scan_levels_bytes(n); }
 // ---------------------------------------------------------------------------
 // Stable LSD radix sort of (uint32 key, uint32 value) pairs.
 // ---------------------------------------------------------------------------
-constexpr int kSortThreads = 256;
+constexpr int kSortThreads = kRadixThreads;
 constexpr int kSortWaves = kSortThreads / kWave;
-constexpr int kSortRounds = 16;  // rounds of 64 keys per wave
-constexpr uint32_t kSortTile = kSortThreads * kSortRounds;  // 4096 keys per block
 constexpr int kRadixBits = 8;
 constexpr int kRadix = 1 << kRadixBits;
+static_assert(kRadix == kRadixDigits, "the interface states the digits");
 
 // `n` is the element count, or the capacity when `d_n` (device count) is given.
 // A device count above the capacity means the emitted records are incomplete:
@@ -245,27 +237,24 @@ __device__ __forceinline__ uint32_t live_count(uint32_t n, const uint32_t* d_n) 
 // Per-block digit histogram. Lanes of a wave holding the same digit are
 // grouped with ballots and counted once by their lowest lane, so runs of equal
 // keys (common in emission order) cost one LDS atomic per run, not per key.
+template <int ROUNDS>  // rounds of 64 keys per wave: a tile of ROUNDS * kSortThreads keys
 __global__ void __launch_bounds__(kSortThreads)
 radix_upsweep_kernel(const uint32_t* __restrict__ keys, uint32_t n, const uint32_t* __restrict__ d_n,
                      uint32_t shift, uint32_t nbits, uint32_t n_blocks, uint32_t* __restrict__ hist) {
     __shared__ uint32_t h[kRadix];
+    constexpr uint32_t kSortTile = kSortThreads * ROUNDS;
     n = live_count(n, d_n);
     h[threadIdx.x] = 0;
     __syncthreads();
     const uint32_t mask = (1u << nbits) - 1u;
     const int lane = lane_id();
     const size_t base = size_t(blockIdx.x) * kSortTile;
-    for (int k = 0; k < kSortRounds; ++k) {
+    for (int k = 0; k < ROUNDS; ++k) {
         const size_t i = base + size_t(k) * kSortThreads + threadIdx.x;
         const bool valid = i < n;
         const uint32_t d = valid ? (keys[i] >> shift) & mask : 0u;
-        uint64_t peers = __ballot(valid);
-        if (!peers) continue;  // wave-uniform
-        for (uint32_t b = 0; b < nbits; ++b) {
-            const bool bit = (d >> b) & 1u;
-            const uint64_t m = __ballot(bit);
-            peers &= bit ? m : ~m;
-        }
+        if (__ballot(valid) == 0ull) continue;  // wave-uniform
+        const uint64_t peers = wave_match(d, nbits, __ballot(valid));
         const int leader = __ffsll((unsigned long long)peers) - 1;
         if (valid && lane == leader) atomicAdd(&h[d], uint32_t(__popcll(peers)));
     }
@@ -273,12 +262,13 @@ radix_upsweep_kernel(const uint32_t* __restrict__ keys, uint32_t n, const uint32
     hist[size_t(threadIdx.x) * n_blocks + blockIdx.x] = h[threadIdx.x];
 }
 
-template <typename KOut>
+template <typename KOut, int ROUNDS>
 __global__ void __launch_bounds__(kSortThreads)
 radix_downsweep_kernel(const uint32_t* __restrict__ keys_in, const uint32_t* __restrict__ vals_in,
                        KOut* __restrict__ keys_out, uint32_t* __restrict__ vals_out, uint32_t n,
                        const uint32_t* __restrict__ d_n, uint32_t shift, uint32_t nbits,
                        uint32_t n_blocks, const uint32_t* __restrict__ hist_scanned) {
+    constexpr uint32_t kSortTile = kSortThreads * ROUNDS;
     n = live_count(n, d_n);
     if (size_t(blockIdx.x) * kSortTile >= n) return;  // whole block beyond the live count
     __shared__ uint32_t wave_cnt[kSortWaves][kRadix];
@@ -294,22 +284,17 @@ radix_downsweep_kernel(const uint32_t* __restrict__ keys_in, const uint32_t* __r
     __syncthreads();
 
     const size_t tile0 = size_t(blockIdx.x) * kSortTile;
-    const size_t wave0 = tile0 + size_t(wave) * (kSortRounds * kWave);
+    const size_t wave0 = tile0 + size_t(wave) * (ROUNDS * kWave);
     const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    uint32_t key[kSortRounds], val[kSortRounds], rank[kSortRounds];
+    uint32_t key[ROUNDS], val[ROUNDS], rank[ROUNDS];
 #pragma unroll
-    for (int r = 0; r < kSortRounds; ++r) {
+    for (int r = 0; r < ROUNDS; ++r) {
         const size_t i = wave0 + size_t(r) * kWave + lane;
         const bool valid = i < n;
         key[r] = valid ? keys_in[i] : 0u;
         val[r] = valid ? vals_in[i] : 0u;
         const uint32_t d = (key[r] >> shift) & mask;
-        uint64_t peers = __ballot(valid);
-        for (uint32_t b = 0; b < nbits; ++b) {
-            const bool bit = (d >> b) & 1u;
-            const uint64_t m = __ballot(bit);
-            peers &= bit ? m : ~m;
-        }
+        const uint64_t peers = wave_match(d, nbits, __ballot(valid));
         uint32_t old = 0;
         const int leader = peers ? (__ffsll((unsigned long long)peers) - 1) : 0;
         if (valid && lane == leader) old = atomicAdd(&wave_cnt[wave][d], uint32_t(__popcll(peers)));
@@ -333,7 +318,7 @@ radix_downsweep_kernel(const uint32_t* __restrict__ keys_in, const uint32_t* __r
     }
     __syncthreads();
 #pragma unroll
-    for (int r = 0; r < kSortRounds; ++r) {
+    for (int r = 0; r < ROUNDS; ++r) {
         const size_t i = wave0 + size_t(r) * kWave + lane;
         if (i < n) {
             const uint32_t d = (key[r] >> shift) & mask;
@@ -361,14 +346,15 @@ static size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
 static SortLayout sort_layout(uint64_t n) {
     SortLayout L;
-    L.n_blocks = uint32_t((n + kSortTile - 1) / kSortTile);
+    L.n_blocks = ceil_div(n, radix_tile(n));
     size_t o = 0;
     const size_t kb = align256(size_t(n) * 4 + 4);
     L.off_a_keys = o; o += kb;
     L.off_a_vals = o; o += kb;
     L.off_b_keys = o; o += kb;
     L.off_b_vals = o; o += kb;
-    const size_t hist_n = size_t(kRadix) * L.n_blocks;
+    // (a workspace never shrinks as n grows past 2^20, where the tiles get larger)
+    const size_t hist_n = size_t(kRadix) * std::max<size_t>(L.n_blocks, n > (1u << 20) ? 1024 : 0);
     L.off_hist = o; o += align256((hist_n + 1) * 4);
     L.off_scan = o; o += align256(scan_levels_bytes(hist_n));
     L.total = o;
@@ -382,12 +368,17 @@ uint32_t* sort_vals_buffer(void* ws, uint64_t n) {
     return reinterpret_cast<uint32_t*>(static_cast<char*>(ws) + sort_layout(n).off_a_vals);
 }
 
+uint32_t* sort_hist_buffer(void* ws, uint64_t n) {
+    return reinterpret_cast<uint32_t*>(static_cast<char*>(ws) + sort_layout(n).off_hist);
+}
+
 // Sorts the pairs held in the workspace's A buffers (written by an emit kernel).
+// `counted`: the first pass's histogram is in the workspace already.
 // `n` is the element count, or a capacity when the live count is on the device
 // (`d_n`); the last pass writes keys as KOut and values to the final outputs.
 template <typename KOut>
 static int sort_pairs_impl(void* ws, size_t ws_bytes, uint32_t n, const uint32_t* d_n, uint32_t end_bit,
-                           KOut* keys_out, uint32_t* vals_out, hipStream_t stream) {
+                           KOut* keys_out, uint32_t* vals_out, hipStream_t stream, bool counted = false) {
     const SortLayout L = sort_layout(n);
     R2S_REQUIRE(ws_bytes >= L.total, "sort workspace too small: %zu < %zu bytes", ws_bytes, L.total);
     if (n == 0) return R2S_OK;
@@ -404,19 +395,29 @@ static int sort_pairs_impl(void* ws, size_t ws_bytes, uint32_t n, const uint32_t
     for (uint32_t p = 0; p < passes; ++p) {
         const uint32_t shift = p * kRadixBits;
         const uint32_t nb = std::min<uint32_t>(kRadixBits, bits - shift);
-        radix_upsweep_kernel<<<L.n_blocks, kSortThreads, 0, stream>>>(ka, n, d_n, shift, nb, L.n_blocks, hist);
-        if (int rc = check_launch("radix_upsweep")) return rc;
-        if (int rc = scan_exclusive(hist, hist_n, hist, nullptr, scan_ws, stream)) return rc;
-        if (p + 1 == passes) {
-            radix_downsweep_kernel<KOut><<<L.n_blocks, kSortThreads, 0, stream>>>(
-                ka, va, keys_out, vals_out, n, d_n, shift, nb, L.n_blocks, hist);
-        } else {
-            radix_downsweep_kernel<uint32_t><<<L.n_blocks, kSortThreads, 0, stream>>>(
-                ka, va, kb, vb, n, d_n, shift, nb, L.n_blocks, hist);
-            uint32_t* t = ka; ka = kb; kb = t;
-            t = va; va = vb; vb = t;
-        }
-        if (int rc = check_launch("radix_downsweep")) return rc;
+        const auto pass = [&](auto rounds) -> int {
+            constexpr int R = decltype(rounds)::value;
+            if (p > 0 || !counted) {
+                radix_upsweep_kernel<R><<<L.n_blocks, kSortThreads, 0, stream>>>(ka, n, d_n, shift, nb, L.n_blocks,
+                                                                                 hist);
+                if (int rc = check_launch("radix_upsweep")) return rc;
+            }
+            if (int rc = scan_exclusive(hist, hist_n, hist, nullptr, scan_ws, stream)) return rc;
+            if (p + 1 == passes)
+                radix_downsweep_kernel<KOut, R><<<L.n_blocks, kSortThreads, 0, stream>>>(
+                    ka, va, keys_out, vals_out, n, d_n, shift, nb, L.n_blocks, hist);
+            else
+                radix_downsweep_kernel<uint32_t, R><<<L.n_blocks, kSortThreads, 0, stream>>>(
+                    ka, va, kb, vb, n, d_n, shift, nb, L.n_blocks, hist);
+            return check_launch("radix_downsweep");
+        };
+        const uint32_t tile = radix_tile(n);
+        if (int rc = tile == 1024   ? pass(std::integral_constant<int, 4>{})
+                     : tile == 2048 ? pass(std::integral_constant<int, 8>{})
+                                    : pass(std::integral_constant<int, 16>{}))
+            return rc;
+        std::swap(ka, kb);
+        std::swap(va, vb);
     }
     return R2S_OK;
 }
@@ -428,8 +429,8 @@ int sort_pairs_to_output(void* ws, size_t ws_bytes, uint32_t n, uint32_t end_bit
 }
 
 int sort_pairs_u32(void* ws, size_t ws_bytes, uint32_t capacity, const uint32_t* d_n, uint32_t end_bit,
-                   uint32_t* keys_out, uint32_t* vals_out, hipStream_t stream) {
-    return sort_pairs_impl<uint32_t>(ws, ws_bytes, capacity, d_n, end_bit, keys_out, vals_out, stream);
+                   uint32_t* keys_out, uint32_t* vals_out, hipStream_t stream, bool counted) {
+    return sort_pairs_impl<uint32_t>(ws, ws_bytes, capacity, d_n, end_bit, keys_out, vals_out, stream, counted);
 }
 
 uint32_t key_end_bit(uint64_t max_key) {

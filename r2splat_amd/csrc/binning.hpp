@@ -47,15 +47,30 @@ size_t scan_workspace_bytes(uint64_t n);
 int scan_exclusive(const uint32_t* in, uint32_t n, uint32_t* out, uint32_t* d_total, void* ws,
                    hipStream_t stream);
 
+// The sort's threads per workgroup and digits per pass, and the keys of a
+// workgroup (its radix tile) when n are sorted: 4096 from 2^20 keys on; below
+// that a launch of 4096-key tiles has fewer workgroups than the GPU has compute
+// units and takes as long as one workgroup's 16 rounds (15 us at 30k keys), so
+// the tiles are smaller (1024: 6 us), with 2048 where that keeps the histogram
+// within the one-launch scan.
+constexpr uint32_t kRadixThreads = 256, kRadixDigits = 256;
+inline uint32_t radix_tile(uint64_t n) {
+    if (n > (1u << 20)) return 4096;
+    return n > (1u << 16) && n <= (1u << 17) ? 2048 : 1024;
+}
+
 size_t sort_workspace_bytes(uint64_t n);
 uint32_t* sort_keys_buffer(void* ws);
 uint32_t* sort_vals_buffer(void* ws, uint64_t n);
+// The first pass's histogram: digit d of tile b at d n_tiles + b.
+uint32_t* sort_hist_buffer(void* ws, uint64_t n);
 uint32_t key_end_bit(uint64_t max_key);
 int sort_pairs_to_output(void* ws, size_t ws_bytes, uint32_t n, uint32_t end_bit, int64_t* keys_out,
                          int32_t* vals_out, hipStream_t stream);
 // Capacity-bounded variant: sorts min(*d_n, capacity) pairs, grids sized for
-// `capacity`, so the launch sequence needs no host-side count.
+// `capacity`, so the launch sequence needs no host-side count. `counted`: the
+// caller has written the first pass's histogram (sort_hist_buffer).
 int sort_pairs_u32(void* ws, size_t ws_bytes, uint32_t capacity, const uint32_t* d_n, uint32_t end_bit,
-                   uint32_t* keys_out, uint32_t* vals_out, hipStream_t stream);
+                   uint32_t* keys_out, uint32_t* vals_out, hipStream_t stream, bool counted = false);
 
 }  // namespace r2s

@@ -92,6 +92,36 @@ __device__ __forceinline__ T wave_sum(T v) {
 
 __device__ __forceinline__ int lane_id() { return __lane_id(); }
 
+// Inclusive scan over the 64 lanes by data-parallel-primitive moves (within
+// rows of 16, then across rows): no LDS traffic, every lane active.
+__device__ __forceinline__ uint32_t wave_scan(uint32_t x) {
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);  // row_shr:1
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);  // row_shr:2
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);  // row_shr:4
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);  // row_shr:8
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast:15
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31
+    return x;
+}
+
+// Lanes of `among` that hold the same value as this lane, for values of up to
+// `bits` bits: each ballot keeps the lanes that agree with this lane's bit
+// (four bits per loop: bits past the value are 0 in every lane).
+__device__ __forceinline__ uint64_t wave_match(uint32_t value, uint32_t bits, uint64_t among) {
+    uint32_t lo = uint32_t(among), hi = uint32_t(among >> 32);
+    for (uint32_t b = 0; b < bits; b += 4) {
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) {
+            const uint32_t own = uint32_t(__builtin_amdgcn_sbfe(int(value >> j), 0, 1));  // all ones where set
+            const uint64_t m = __ballot(own != 0u);
+            lo &= ~(uint32_t(m) ^ own);
+            hi &= ~(uint32_t(m >> 32) ^ own);
+        }
+        value >>= 4;
+    }
+    return (uint64_t(hi) << 32) | lo;
+}
+
 // Device atomics on float / double with hardware fp atomics (-munsafe-fp-atomics).
 template <typename S>
 __device__ __forceinline__ void atomic_add(S* p, S v) { atomicAdd(p, v); }

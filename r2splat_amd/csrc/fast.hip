@@ -296,23 +296,12 @@ __device__ __forceinline__ uint32_t rows_reached(float my, float ext, float y_ba
 // ---------------------------------------------------------------------------
 constexpr uint32_t kOrderThreads = 1024;
 
-// Floats as unsigned integers of the same order (for min/max atomics).
-__device__ __forceinline__ uint32_t order_bits(float f) {
-    const uint32_t b = __float_as_uint(f);
-    return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
-}
-__device__ __forceinline__ float order_float(uint32_t u) {
-    return __uint_as_float((u & 0x80000000u) ? (u & 0x7fffffffu) : ~u);
-}
-
-// bounds (ordered bits) = {min x, min y, min z, max x, max y, max z} of the
-// finite means; bounds starts at {~0 x3, 0 x3} (morton_bounds_init_kernel).
-__global__ void morton_bounds_init_kernel(uint32_t* __restrict__ bounds) {
-    if (threadIdx.x < 6) bounds[threadIdx.x] = threadIdx.x < 3 ? 0xffffffffu : 0u;
-}
+// Per-workgroup bounds {min x, min y, min z, max x, max y, max z} of the finite
+// means (+inf / -inf where a workgroup has none).
+constexpr uint32_t kOrderBlocks = 256;
 
 __global__ void __launch_bounds__(kOrderThreads)
-morton_bounds_kernel(const float* __restrict__ means, uint32_t N, uint32_t* __restrict__ bounds) {
+morton_bounds_kernel(const float* __restrict__ means, uint32_t N, float* __restrict__ partial) {
     __shared__ float red[6][kOrderThreads / kWave];
     float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
     for (uint32_t n = blockIdx.x * kOrderThreads + threadIdx.x; n < N; n += gridDim.x * kOrderThreads) {
@@ -342,12 +331,10 @@ morton_bounds_kernel(const float* __restrict__ means, uint32_t N, uint32_t* __re
     }
     __syncthreads();
     if (threadIdx.x < 6) {
-        const bool is_lo = threadIdx.x < 3;
         float v = red[threadIdx.x][0];
         for (uint32_t w = 1; w < kOrderThreads / kWave; ++w)
-            v = is_lo ? fminf(v, red[threadIdx.x][w]) : fmaxf(v, red[threadIdx.x][w]);
-        if (is_lo) atomicMin(bounds + threadIdx.x, order_bits(v));
-        else atomicMax(bounds + threadIdx.x, order_bits(v));
+            v = threadIdx.x < 3 ? fminf(v, red[threadIdx.x][w]) : fmaxf(v, red[threadIdx.x][w]);
+        partial[6 * blockIdx.x + threadIdx.x] = v;
     }
 }
 
@@ -363,23 +350,159 @@ __device__ __forceinline__ uint32_t spread_bits3(uint32_t v) {  // up to 10 bits
     return v;
 }
 
-__global__ void __launch_bounds__(256)
-morton_keys_kernel(const float* __restrict__ means, uint32_t N, const uint32_t* __restrict__ bounds,
-                   uint32_t drop, uint32_t* __restrict__ keys, uint32_t* __restrict__ vals) {
-    const uint32_t n = blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= N) return;
+// The code of mean n over the box [lo, lo + ext] (an axis without extent, or
+// without a finite mean, counts as 0).
+__device__ __forceinline__ uint32_t morton_key(const float* __restrict__ means, uint32_t n, const float (&lo)[3],
+                                               const float (&ext)[3]) {
     uint32_t key = 0;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-        // no finite mean: lo = NaN and every key 0
-        const float lo = order_float(bounds[k]), ext = order_float(bounds[3 + k]) - lo;
-        const float t = ext > 0.f ? (means[3 * size_t(n) + k] - lo) / ext : 0.f;
+        const float t = ext[k] > 0.f ? (means[3 * size_t(n) + k] - lo[k]) / ext[k] : 0.f;
         constexpr float kCells = float(1u << kMortonAxisBits);
         const float q = fminf(fmaxf(t * kCells, 0.f), kCells - 1.f);  // NaN -> 0
         key |= spread_bits3(uint32_t(q)) << (2 - k);
     }
-    keys[n] = key >> drop;
-    vals[n] = n;
+    return key;
+}
+
+// Codes (the top bits: code >> drop) and input indices of a radix tile of means,
+// and the tile's histogram of the first radix digit (what the sort's first
+// pass would count by itself in a launch of its own). Every workgroup reduces
+// the n_partial bounds.
+__global__ void __launch_bounds__(kRadixThreads)
+morton_keys_kernel(const float* __restrict__ means, uint32_t N, const float* __restrict__ partial,
+                   uint32_t n_partial, uint32_t drop, uint32_t tile, uint32_t n_blocks, uint32_t* __restrict__ keys,
+                   uint32_t* __restrict__ vals, uint32_t* __restrict__ hist) {
+    __shared__ float bounds[6][kRadixThreads / kWave];
+    __shared__ uint32_t h[kRadixDigits];
+    const uint32_t lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    static_assert(kOrderBlocks <= kRadixThreads && kRadixDigits == kRadixThreads, "one partial and digit per thread");
+    h[threadIdx.x] = 0u;
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+        float v = k < 3 ? INFINITY : -INFINITY;
+        if (threadIdx.x < n_partial) v = partial[6 * threadIdx.x + k];
+        for (uint32_t off = kWave / 2; off > 0; off >>= 1) {
+            const float y = __shfl_xor(v, off, kWave);
+            v = k < 3 ? fminf(v, y) : fmaxf(v, y);
+        }
+        if (lane == 0) bounds[k][wave] = v;
+    }
+    __syncthreads();
+    float lo[3], ext[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        float a = bounds[k][0], b = bounds[3 + k][0];
+        for (uint32_t w = 1; w < kRadixThreads / kWave; ++w) {
+            a = fminf(a, bounds[k][w]);
+            b = fmaxf(b, bounds[3 + k][w]);
+        }
+        lo[k] = a;
+        ext[k] = b - a;
+    }
+    for (uint32_t i = threadIdx.x; i < tile; i += kRadixThreads) {
+        const uint32_t n = blockIdx.x * tile + i;
+        if (n >= N) break;
+        const uint32_t key = morton_key(means, n, lo, ext) >> drop;
+        keys[n] = key;
+        vals[n] = n;
+        atomicAdd(&h[key % kRadixDigits], 1u);
+    }
+    __syncthreads();
+    hist[size_t(threadIdx.x) * n_blocks + blockIdx.x] = h[threadIdx.x];
+}
+
+// The whole primitive order of up to kOrderSmall primitives in one workgroup:
+// bounds, 8-bit codes, and a stable counting sort of one radix digit (each
+// wave ranks a contiguous run of the input with ballots; the waves' digit
+// counts are summed in LDS). A call of 1000 primitives spends 6 us here
+// instead of 27 us in six launches of a few workgroups each.
+constexpr uint32_t kOrderSmall = 16384, kOrderWaves = kOrderThreads / kWave;
+constexpr int kOrderRounds = kOrderSmall / kOrderThreads;
+
+__global__ void __launch_bounds__(kOrderThreads)
+morton_order_small_kernel(const float* __restrict__ means, uint32_t N, uint32_t drop, uint32_t* __restrict__ perm) {
+    __shared__ float red[6][kOrderWaves];
+    __shared__ uint32_t cnt[kOrderWaves][kRadixDigits];  // per wave and digit: counts, then first positions
+    __shared__ uint32_t digit_sum[kRadixDigits / kWave];
+    const uint32_t lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    float lo[3], ext[3];
+    {
+        float a[3] = {INFINITY, INFINITY, INFINITY}, b[3] = {-INFINITY, -INFINITY, -INFINITY};
+        for (uint32_t n = threadIdx.x; n < N; n += kOrderThreads) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const float x = means[3 * size_t(n) + k];
+                if (isfinite(x)) {
+                    a[k] = fminf(a[k], x);
+                    b[k] = fmaxf(b[k], x);
+                }
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            for (uint32_t off = kWave / 2; off > 0; off >>= 1) {
+                a[k] = fminf(a[k], __shfl_xor(a[k], off, kWave));
+                b[k] = fmaxf(b[k], __shfl_xor(b[k], off, kWave));
+            }
+            if (lane == 0) {
+                red[k][wave] = a[k];
+                red[3 + k][wave] = b[k];
+            }
+        }
+        for (uint32_t i = threadIdx.x; i < kOrderWaves * kRadixDigits; i += kOrderThreads) (&cnt[0][0])[i] = 0u;
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            float u = red[k][0], v = red[3 + k][0];
+            for (uint32_t w = 1; w < kOrderWaves; ++w) {
+                u = fminf(u, red[k][w]);
+                v = fmaxf(v, red[3 + k][w]);
+            }
+            lo[k] = u;
+            ext[k] = v - u;
+        }
+    }
+    // wave w ranks inputs [w run, (w + 1) run), run a multiple of the wave size
+    const uint32_t rounds = (N + kOrderThreads - 1) / kOrderThreads, first = wave * rounds * kWave;
+    const uint64_t below = (uint64_t(1) << lane) - 1u;
+    uint32_t key[kOrderRounds], rank[kOrderRounds];
+#pragma unroll
+    for (int r = 0; r < kOrderRounds; ++r) {
+        if (uint32_t(r) >= rounds) break;
+        const uint32_t n = first + uint32_t(r) * kWave + lane;
+        const bool valid = n < N;
+        key[r] = valid ? morton_key(means, n, lo, ext) >> drop : 0u;
+        const uint64_t peers = wave_match(key[r], 8, __ballot(valid));
+        rank[r] = valid ? cnt[wave][key[r]] + uint32_t(__popcll(peers & below)) : 0u;
+        wave_lds_sync();  // every lane has read its digit's count
+        if (valid && (peers >> lane) == 1u) cnt[wave][key[r]] = rank[r] + 1u;
+        wave_lds_sync();
+    }
+    __syncthreads();
+    uint32_t total = 0, incl = 0;
+    if (threadIdx.x < kRadixDigits) {
+        for (uint32_t w = 0; w < kOrderWaves; ++w) {
+            const uint32_t c = cnt[w][threadIdx.x];
+            cnt[w][threadIdx.x] = total;
+            total += c;
+        }
+        incl = wave_scan(total);
+        if (lane == kWave - 1) digit_sum[wave] = incl;
+    }
+    __syncthreads();
+    if (threadIdx.x < kRadixDigits) {
+        uint32_t before = incl - total;
+        for (uint32_t w = 0; w < wave; ++w) before += digit_sum[w];
+        for (uint32_t w = 0; w < kOrderWaves; ++w) cnt[w][threadIdx.x] += before;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kOrderRounds; ++r) {
+        if (uint32_t(r) >= rounds) break;
+        const uint32_t n = first + uint32_t(r) * kWave + lane;
+        if (n < N) perm[cnt[wave][key[r]] + rank[r]] = n;
+    }
 }
 
 // The camera-independent double-precision terms of one primitive's
@@ -410,9 +533,9 @@ __device__ __forceinline__ void camera_frame(const float* __restrict__ viewmats,
 
 // Copies of the primitive parameters in the sorted order (perm[p] = input
 // index), and each primitive's PrimFrame; workgroup 0 also writes the C
-// camera frames.
+// camera frames and clears the counters.
 __global__ void __launch_bounds__(256)
-permute_params_kernel(const uint32_t* __restrict__ perm, uint32_t N, const float* __restrict__ means,
+permute_params_kernel(const uint32_t* __restrict__ perm, uint32_t* __restrict__ counters, uint32_t N, const float* __restrict__ means,
                       const float* __restrict__ quats, const float* __restrict__ scales,
                       const float* __restrict__ dens, const float* __restrict__ betas,
                       const float* __restrict__ ratio, const float* __restrict__ unc, float* __restrict__ o_means,
@@ -420,8 +543,10 @@ permute_params_kernel(const uint32_t* __restrict__ perm, uint32_t N, const float
                       float* __restrict__ o_unc, PrimFrame* __restrict__ o_frames,
                       const float* __restrict__ viewmats, const float* __restrict__ Ks, uint32_t C, uint32_t W,
                       uint32_t H, CamFrame* __restrict__ cams) {
-    if (blockIdx.x == 0)
+    if (blockIdx.x == 0) {
+        if (threadIdx.x < 2) counters[threadIdx.x] = 0u;
         for (uint32_t c = threadIdx.x; c < C; c += blockDim.x) camera_frame(viewmats, Ks, c, W, H, cams);
+    }
     const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= N) return;
     const size_t n = perm[p];
@@ -549,7 +674,7 @@ fused_project_kernel(const float* __restrict__ means, const PrimFrame* __restric
             recs[idx] = rec;
         rects[idx] = rect;
         if (reach) reach[idx] = rr;
-        counts[idx] = count;
+        if (counts) counts[idx] = count;
     }
 }
 
@@ -820,8 +945,9 @@ fused_pack_kernel(const uint2* __restrict__ rects, const float2* __restrict__ re
 // walks the records' tile rectangles in step (pair k of every lane's
 // rectangle, row-major, at step k):
 //   count: per range, the number of intersections in each bin (LDS counters);
-//   scan:  per (camera, bin) an exclusive scan over the ranges, then one over
-//          (camera, bin): every (range, bin) gets its first packed slot;
+//   scan:  per (camera, bin) an exclusive scan over the ranges and one over
+//          the (camera, range) totals, then per camera one over its bins: every
+//          (range, bin) gets its first packed slot;
 //   place: the same walk, each (record, tile) pair's list entry {record
 //          index, emission index} written straight to its slot; pairs of one
 //          step that share a bin are ranked by lane (ballots on the bin's
@@ -831,9 +957,10 @@ fused_pack_kernel(const uint2* __restrict__ rects, const float2* __restrict__ re
 // ---------------------------------------------------------------------------
 constexpr uint32_t kBinClasses = 9;  // heights ceil(8 h / T) = 8 .. 1, then h = 0
 
+// (T is 8, 16 or 32: the division is a shift)
 __device__ __forceinline__ uint32_t height_class(const SpanRect& r, uint32_t ty, uint32_t T) {
     const uint32_t h = rows_reached(r.my, r.ext, float(ty * T), T);
-    return h == 0u ? kBinClasses - 1u : kBinClasses - 1u - (8u * h + T - 1u) / T;
+    return h == 0u ? kBinClasses - 1u : kBinClasses - 1u - ((8u * h + T - 1u) >> (__builtin_ctz(T)));
 }
 
 // A lane's walk over its record's tile rectangle, row-major.
@@ -860,63 +987,159 @@ struct RectWalk {
     }
 };
 
-// grid (n_ranges, C), one wave; dynamic LDS: n_bins counters.
+// grid (n_ranges, C), one wave; dynamic LDS: n_bins counters. range_totals:
+// the intersections of each (camera, range).
 __global__ void __launch_bounds__(kWave)
 fused_bin_count_kernel(const uint2* __restrict__ rects, const float2* __restrict__ reach, uint32_t N,
                        uint32_t range_len, uint32_t n_ranges, uint32_t ntx, uint32_t T, uint32_t n_bins,
-                       uint32_t* __restrict__ range_counts, uint32_t* __restrict__ counters, uint32_t capacity) {
+                       uint32_t* __restrict__ range_counts, uint32_t* __restrict__ range_totals) {
     extern __shared__ uint32_t hist[];
     const uint32_t range = blockIdx.x, cam = blockIdx.y, lane = threadIdx.x;
-    // counters = {intersections (the scan's total), overflow}: the flag is
-    // raised when the count exceeds the capacity
-    if (range == 0 && cam == 0 && lane == 0) counters[1] = counters[0] > capacity ? 1u : 0u;
     for (uint32_t b = lane; b < n_bins; b += kWave) hist[b] = 0u;
     __syncthreads();
     const uint32_t n0 = range * range_len, n1 = min(N, n0 + range_len);
+    uint32_t total = 0;
     for (uint32_t n = n0 + lane; n < n1; n += kWave) {
         const SpanRect sr = load_span(rects, reach, size_t(cam) * N + n);
         RectWalk w;
         w.start(sr, ntx, T);
+        total += w.cnt;
         for (uint32_t k = 0; k < w.cnt; ++k) {
             atomicAdd(&hist[w.bin()], 1u);
             w.advance(sr, ntx, T);
         }
     }
+    total = wave_sum(total);
+    if (lane == 0) range_totals[size_t(cam) * n_ranges + range] = total;
     __syncthreads();
     uint32_t* out = range_counts + (size_t(cam) * n_ranges + range) * n_bins;
     for (uint32_t b = lane; b < n_bins; b += kWave) out[b] = hist[b];
 }
 
-// Per (camera, bin): exclusive scan of its counts over the ranges (in place);
-// the column total goes to totals[cam * n_bins + bin].
-__global__ void __launch_bounds__(256)
-fused_bin_scan_ranges_kernel(uint32_t* __restrict__ range_counts, uint32_t C, uint32_t n_ranges, uint32_t n_bins,
-                             uint32_t* __restrict__ totals) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= C * n_bins) return;
-    const uint32_t cam = i / n_bins, b = i - cam * n_bins;
-    uint32_t* col = range_counts + size_t(cam) * n_ranges * n_bins + b;
-    uint32_t run = 0;
-    for (uint32_t r = 0; r < n_ranges; ++r) {
-        const uint32_t v = col[size_t(r) * n_bins];
-        col[size_t(r) * n_bins] = run;
-        run += v;
+// Exclusive scan of `n` values by one workgroup, in place, kScanPer per thread
+// and round; returns the total (every thread).
+constexpr uint32_t kScanThreads = 512, kScanPer = 8;
+
+__device__ __forceinline__ uint32_t scan_in_place(uint32_t* __restrict__ v, uint32_t n, uint32_t base,
+                                                  uint32_t* lds_waves) {
+    const uint32_t lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    uint32_t carry = base;
+    for (uint32_t r = 0; r < n; r += kScanThreads * kScanPer) {
+        const uint32_t i0 = r + threadIdx.x * kScanPer;
+        uint32_t x[kScanPer], sum = 0;
+#pragma unroll
+        for (uint32_t j = 0; j < kScanPer; ++j) {
+            x[j] = i0 + j < n ? v[i0 + j] : 0u;
+            sum += x[j];
+        }
+        const uint32_t incl = wave_scan(sum);
+        if (lane == kWave - 1) lds_waves[wave] = incl;
+        __syncthreads();
+        uint32_t before = 0, total = 0;
+#pragma unroll
+        for (uint32_t w = 0; w < kScanThreads / kWave; ++w) {
+            before += w < wave ? lds_waves[w] : 0u;
+            total += lds_waves[w];
+        }
+        uint32_t run = carry + before + incl - sum;
+#pragma unroll
+        for (uint32_t j = 0; j < kScanPer; ++j) {
+            if (i0 + j < n) v[i0 + j] = run;
+            run += x[j];
+        }
+        carry += total;
+        __syncthreads();  // lds_waves is reused
     }
-    totals[i] = run;
+    return carry;
 }
 
-// grid (n_ranges, C), one wave; dynamic LDS: the n_bins next free slots.
+// Column scans: workgroup b < gridDim.x - 1 takes kScanCols (camera, bin)
+// columns, each an exclusive scan of its counts over the ranges (in place), the
+// ranges split over kScanSplit threads whose partial sums meet in LDS; the
+// column total goes to totals[cam * n_bins + bin]. (One thread per column
+// walked its ranges one dependent load after another: 42 us for 22k columns of
+// 157 ranges, now 8 us.) The last workgroup scans the (camera, range) totals in
+// place, giving the first emission index of each, and writes counters =
+// {intersections, overflow} and the end of the record offsets.
+constexpr uint32_t kScanCols = 64, kScanSplit = kScanThreads / kScanCols;
+
+__global__ void __launch_bounds__(kScanThreads)
+fused_bin_scan_ranges_kernel(uint32_t* __restrict__ range_counts, uint32_t C, uint32_t n_ranges, uint32_t n_bins,
+                             uint32_t* __restrict__ totals, uint32_t* __restrict__ range_totals, uint32_t capacity,
+                             uint32_t* __restrict__ counters, uint32_t* __restrict__ cum_end) {
+    __shared__ uint32_t lds[kScanThreads];
+    if (blockIdx.x + 1 == gridDim.x) {
+        const uint32_t total = scan_in_place(range_totals, C * n_ranges, 0u, lds);
+        if (threadIdx.x == 0) {
+            counters[0] = total;
+            counters[1] = total > capacity ? 1u : 0u;
+            *cum_end = total;
+        }
+        return;
+    }
+    const uint32_t col = threadIdx.x % kScanCols, part = threadIdx.x / kScanCols;
+    const uint32_t i = blockIdx.x * kScanCols + col;
+    const bool valid = i < C * n_bins;
+    const uint32_t cam = valid ? i / n_bins : 0u, b = i - cam * n_bins;
+    uint32_t* column = range_counts + size_t(cam) * n_ranges * n_bins + b;
+    const uint32_t per = (n_ranges + kScanSplit - 1) / kScanSplit;
+    const uint32_t r0 = min(n_ranges, part * per), r1 = valid ? min(n_ranges, r0 + per) : r0;
+    constexpr uint32_t kBatch = 8;  // loads in flight
+    uint32_t sum = 0;
+    for (uint32_t r = r0; r < r1; r += kBatch) {
+        uint32_t v[kBatch];
+#pragma unroll
+        for (uint32_t j = 0; j < kBatch; ++j) v[j] = r + j < r1 ? column[size_t(r + j) * n_bins] : 0u;
+#pragma unroll
+        for (uint32_t j = 0; j < kBatch; ++j) sum += v[j];
+    }
+    lds[threadIdx.x] = sum;
+    __syncthreads();
+    uint32_t run = 0, total = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < kScanSplit; ++k) {
+        const uint32_t x = lds[k * kScanCols + col];
+        run += k < part ? x : 0u;
+        total += x;
+    }
+    for (uint32_t r = r0; r < r1; r += kBatch) {
+        uint32_t v[kBatch];
+#pragma unroll
+        for (uint32_t j = 0; j < kBatch; ++j) v[j] = r + j < r1 ? column[size_t(r + j) * n_bins] : 0u;
+#pragma unroll
+        for (uint32_t j = 0; j < kBatch; ++j) {
+            if (r + j < r1) column[size_t(r + j) * n_bins] = run;
+            run += v[j];
+        }
+    }
+    if (valid && part == 0) totals[i] = total;
+}
+
+// One workgroup per camera: its bins' totals -> their first packed slots (an
+// exclusive scan from the camera's first emission index).
+__global__ void __launch_bounds__(kScanThreads)
+fused_bin_starts_kernel(uint32_t* __restrict__ totals, uint32_t n_bins, const uint32_t* __restrict__ range_starts,
+                        uint32_t n_ranges) {
+    __shared__ uint32_t lds[kScanThreads / kWave];
+    const uint32_t base = n_ranges ? range_starts[size_t(blockIdx.x) * n_ranges] : 0u;
+    scan_in_place(totals + size_t(blockIdx.x) * n_bins, n_bins, base, lds);
+}
+
+// grid (n_ranges, C), one wave; dynamic LDS: the n_bins next free slots. Also
+// writes the record offsets: first_isect, the (camera, range)'s first emission
+// index, and a wave scan of the records' tile counts.
 __global__ void __launch_bounds__(kWave)
 fused_bin_place_kernel(const uint2* __restrict__ rects, const float2* __restrict__ reach,
-                       const uint32_t* __restrict__ cum, uint32_t N, uint32_t range_len, uint32_t n_ranges,
+                       uint32_t* __restrict__ cum, uint32_t N, uint32_t range_len, uint32_t n_ranges,
                        uint32_t ntx, uint32_t T, uint32_t n_bins, uint32_t bin_bits,
                        const uint32_t* __restrict__ range_starts, const uint32_t* __restrict__ bin_starts,
-                       uint32_t capacity, uint2* __restrict__ entries) {
+                       const uint32_t* __restrict__ first_isect, uint32_t capacity, uint2* __restrict__ entries) {
     extern __shared__ uint32_t next_slot[];
     const uint32_t range = blockIdx.x, cam = blockIdx.y, lane = threadIdx.x;
     const uint32_t* rs = range_starts + (size_t(cam) * n_ranges + range) * n_bins;
     const uint32_t* bs = bin_starts + size_t(cam) * n_bins;
     for (uint32_t b = lane; b < n_bins; b += kWave) next_slot[b] = bs[b] + rs[b];
+    uint32_t emitted = first_isect[size_t(cam) * n_ranges + range];
     __syncthreads();
     const uint64_t below = (uint64_t(1) << lane) - 1u;
     const uint32_t n0 = range * range_len, n1 = min(N, n0 + range_len);
@@ -927,17 +1150,15 @@ fused_bin_place_kernel(const uint2* __restrict__ rects, const float2* __restrict
         if (n < n1) sr = load_span(rects, reach, idx);
         RectWalk w;
         w.start(sr, ntx, T);
-        const uint32_t g = w.cnt ? cum[idx] : 0u;
+        const uint32_t incl = wave_scan(w.cnt);
+        const uint32_t g = emitted + incl - w.cnt;
+        emitted += __builtin_amdgcn_readlane(incl, kWave - 1);
+        if (n < n1) cum[idx] = g;
         for (uint32_t k = 0; __ballot(k < w.cnt); ++k) {
             const bool act = k < w.cnt;
             const uint32_t bin = act ? w.bin() : 0u;
             // lanes of this step with the same bin, ranked by lane
-            uint64_t same = __ballot(act);
-            for (uint32_t bit = 0; bit < bin_bits; ++bit) {
-                const bool one = (bin >> bit) & 1u;
-                const uint64_t m = __ballot(one);
-                same &= one ? m : ~m;
-            }
+            const uint64_t same = wave_match(bin, bin_bits, __ballot(act));
             if (act) {
                 // every lane reads its bin's slot before the group's last lane advances it
                 const uint32_t pos = next_slot[bin] + uint32_t(__popcll(same & below));
@@ -1682,7 +1903,7 @@ struct FusedScratch {
     // direct placement (place = true) or sort + pack
     bool place;
     uint32_t range_len, n_ranges, n_bins, bin_bits;
-    size_t reach, range_counts, bin_totals, bin_scan;
+    size_t reach, range_counts, range_totals, bin_totals;
     // primitive order: bounds, key sort, and the permuted parameter copies
     size_t order_bounds, order_sort_n, order_sort_n_bytes, order_sorted_keys, params, frames, cams;
 };
@@ -1704,16 +1925,26 @@ static size_t packed_bytes(uint32_t C, uint32_t N, uint32_t capacity, int kind) 
     return entries_bytes(capacity) + al(size_t(C) * N * record_bytes(kind));
 }
 
-// Largest bin table of the direct placement (its waves hold one table each in
-// LDS, so larger tables cost occupancy; larger tile grids sort and pack).
-constexpr size_t kPlaceLdsBytes = 16384;
+// Bin tables of the direct placement: its waves hold one table each in LDS, so
+// larger tables cost occupancy. Up to kPlaceLdsBytes every call places; up to
+// kPlaceLargeBytes (1024 tiles a camera) those whose waves are all resident at
+// once do (one view of 333 x 517 with 30k primitives: 100 us of binning kernels
+// against 145 us of sort and pack), and larger grids or more waves sort and pack (500k
+// primitives x 256 views of 512^2 took 49.6 ms a step placing, 44.7 sorting).
+// Calls of the middle kind have scratch for either.
+constexpr size_t kPlaceLdsBytes = 16384, kPlaceLargeBytes = 40960, kLdsBytes = 163840;
+constexpr uint64_t kComputeUnits = 256;
 constexpr uint32_t kPlaceWaves = 4096;  // target number of ranges (waves) per binning pass
+// Bytes of count tables up to which ranges shorter than 256 records pay: a wave
+// walks its range's rectangles one step after another (0.4 us a step), while a
+// table is written, scanned twice and read once.
+constexpr uint64_t kRangeTables = 8ull << 20;
 
 static FusedScratch fused_scratch(uint32_t C, uint32_t N, uint32_t n_tiles, uint32_t capacity, int kind) {
     FusedScratch L = {};
     const size_t CN = size_t(C) * N;
     size_t o = 0;
-    L.order_bounds = o; o += al(8 * sizeof(float));
+    L.order_bounds = o; o += al(6 * kOrderBlocks * sizeof(float));
     L.order_sort_n_bytes = sort_workspace_bytes(N);
     L.order_sort_n = o; o += al(L.order_sort_n_bytes);
     L.order_sorted_keys = o; o += al(size_t(N) * 4 + 4);
@@ -1722,21 +1953,31 @@ static FusedScratch fused_scratch(uint32_t C, uint32_t N, uint32_t n_tiles, uint
     L.cams = o; o += al(size_t(C) * sizeof(CamFrame));
     L.rects = o; o += al(CN * sizeof(uint2));
     L.reach = o; o += al(CN * sizeof(float2));
-    L.scan = o; o += al(scan_workspace_bytes(CN));
     const uint64_t nt = C ? n_tiles / C : 0;
-    L.place = C > 0 && nt * kBinClasses * sizeof(uint32_t) <= kPlaceLdsBytes;
-    if (L.place) {
+    const size_t table = nt * kBinClasses * sizeof(uint32_t);
+    if (C > 0 && nt > 0 && table <= kPlaceLargeBytes) {
         L.n_bins = uint32_t(nt) * kBinClasses;
         L.bin_bits = 32u - uint32_t(__builtin_clz(L.n_bins - 1u));
+        // a range holds the records that make about kPlaceWaves ranges, but no fewer
+        // than 64, and 128 or 256 where the ranges' count tables would pass kRangeTables
         const uint64_t per = (CN + kPlaceWaves - 1) / kPlaceWaves;
-        L.range_len = uint32_t(std::max<uint64_t>(256, (per + 63) / 64 * 64));
+        uint64_t least = 64;
+        while (least < 256 && uint64_t(C) * ((N + least - 1) / least) * table > kRangeTables) least *= 2;
+        L.range_len = uint32_t(std::max<uint64_t>(least, (per + 63) / 64 * 64));
         L.n_ranges = (N + L.range_len - 1) / L.range_len;
-        L.range_counts = o; o += al(size_t(C) * L.n_ranges * L.n_bins * 4 + 4);
-        L.bin_totals = o; o += al(size_t(C) * L.n_bins * 4 + 4);
-        L.bin_scan = o; o += al(scan_workspace_bytes(uint64_t(C) * L.n_bins));
+        L.place = table <= kPlaceLdsBytes ||
+                  uint64_t(C) * L.n_ranges <= kComputeUnits * (kLdsBytes / table);
+        if (L.place) {
+            L.range_counts = o; o += al(size_t(C) * L.n_ranges * L.n_bins * 4 + 4);
+            L.range_totals = o; o += al(size_t(C) * L.n_ranges * 4 + 4);
+            L.bin_totals = o; o += al(size_t(C) * L.n_bins * 4 + 4);
+        }
+    }
+    if (table <= kPlaceLdsBytes && L.place) {
         L.bytes = o;
         return L;
     }
+    L.scan = o; o += al(scan_workspace_bytes(CN));
     L.sort_bytes = sort_workspace_bytes(capacity);
     L.sort = o; o += al(L.sort_bytes);
     L.keys = o; o += al(size_t(capacity) * 4 + 4);
@@ -1873,7 +2114,6 @@ static int prepare_impl(const float* means, const float* quats, const float* sca
     const FusedScratch L = fused_scratch(C, N, C * ntx * nty, capacity, (BETA ? kKindBeta : 0) | (VAR ? kKindVar : 0));
     R2S_REQUIRE(scratch_bytes >= L.bytes, "fused scratch too small: %zu < %zu", scratch_bytes, L.bytes);
     const uint32_t CN = C * N, n_tiles = C * ntx * nty;
-    if (int rc = fill_zero<uint32_t>(counters, 2, stream)) return rc;
     uint2* entries = static_cast<uint2*>(packed);
     R* recs = at<R>(packed, entries_bytes(capacity));
     uint32_t* cum = record_offsets;
@@ -1883,62 +2123,68 @@ static int prepare_impl(const float* means, const float* quats, const float* sca
     float* p_unc = pp + 6 * size_t(N);
     PrimFrame* p_frames = at<PrimFrame>(scratch, L.frames);
     if (N > 0) {
-        void* ows = at<void>(scratch, L.order_sort_n);
-        uint32_t* bounds = at<uint32_t>(scratch, L.order_bounds);
-        morton_bounds_init_kernel<<<1, kWave, 0, stream>>>(bounds);
-        if (int rc = check_launch("morton_bounds_init")) return rc;
-        morton_bounds_kernel<<<std::min(ceil_div(N, kOrderThreads), 256u), kOrderThreads, 0, stream>>>(means, N,
-                                                                                                       bounds);
-        if (int rc = check_launch("morton_bounds")) return rc;
-        // small sets sort by the code's top 8 bits only (one radix pass; 8 x 8 x 4
-        // cells still keep a range of neighbouring primitives on a few tiles),
-        // larger ones by all 15 (two passes; coarser cells cost the raster
-        // kernels' gather locality there)
+        // sets of up to 2^17 sort by the code's top 8 bits only (one radix digit; 8 x
+        // 8 x 4 cells still keep a range of neighbouring primitives on a few tiles),
+        // larger ones by all 15 (two passes; coarser cells cost the raster kernels'
+        // gather locality there)
         const uint32_t code_bits = N <= kMortonCoarseMax ? 8u : 3u * kMortonAxisBits;
-        morton_keys_kernel<<<ceil_div(N, 256), 256, 0, stream>>>(means, N, bounds, 3u * kMortonAxisBits - code_bits,
-                                                                 sort_keys_buffer(ows), sort_vals_buffer(ows, N));
-        if (int rc = check_launch("morton_keys")) return rc;
-        if (int rc = sort_pairs_u32(ows, L.order_sort_n_bytes, N, nullptr, code_bits,
-                                    at<uint32_t>(scratch, L.order_sorted_keys), perm, stream))
-            return rc;
+        const uint32_t drop = 3u * kMortonAxisBits - code_bits;
+        if (N <= kOrderSmall) {
+            morton_order_small_kernel<<<1, kOrderThreads, 0, stream>>>(means, N, drop, perm);
+            if (int rc = check_launch("morton_order_small")) return rc;
+        } else {
+            void* ows = at<void>(scratch, L.order_sort_n);
+            float* bounds = at<float>(scratch, L.order_bounds);
+            const uint32_t n_bounds = std::min(ceil_div(N, kOrderThreads), kOrderBlocks);
+            morton_bounds_kernel<<<n_bounds, kOrderThreads, 0, stream>>>(means, N, bounds);
+            if (int rc = check_launch("morton_bounds")) return rc;
+            const uint32_t tile = radix_tile(N), n_sort = ceil_div(N, tile);
+            morton_keys_kernel<<<n_sort, kRadixThreads, 0, stream>>>(means, N, bounds, n_bounds, drop, tile, n_sort,
+                                                                     sort_keys_buffer(ows), sort_vals_buffer(ows, N),
+                                                                     sort_hist_buffer(ows, N));
+            if (int rc = check_launch("morton_keys")) return rc;
+            if (int rc = sort_pairs_u32(ows, L.order_sort_n_bytes, N, nullptr, code_bits,
+                                        at<uint32_t>(scratch, L.order_sorted_keys), perm, stream, true))
+                return rc;
+        }
         permute_params_kernel<<<ceil_div(N, 256), 256, 0, stream>>>(
-            perm, N, means, quats, scales, densities, BETA ? betas : nullptr, BETA ? beta_ratio : nullptr,
-            VAR ? uncertainties : nullptr, p_means, p_dens, p_betas, p_ratio, p_unc, p_frames, viewmats, Ks, C,
-            width, height, at<CamFrame>(scratch, L.cams));
+            perm, counters, N, means, quats, scales, densities, BETA ? betas : nullptr,
+            BETA ? beta_ratio : nullptr, VAR ? uncertainties : nullptr, p_means, p_dens, p_betas, p_ratio, p_unc,
+            p_frames, viewmats, Ks, C, width, height, at<CamFrame>(scratch, L.cams));
         if (int rc = check_launch("permute_params")) return rc;
+    } else if (int rc = fill_zero<uint32_t>(counters, 2, stream)) {
+        return rc;
     }
     if (CN > 0) {  // (N > 0: the permute pass wrote the camera frames)
         const CamFrame* cams = at<CamFrame>(scratch, L.cams);
         dim3 grid(ceil_div(N, 256), ceil_div(C, kProjectCams));
         fused_project_kernel<BETA, VAR><<<grid, 256, 0, stream>>>(
             p_means, p_frames, p_dens, p_betas, p_ratio, p_unc, cams, C, width, height, eps, radius_clip,
-            tile_size, ntx, nty, N, recs, at<uint2>(scratch, L.rects), at<float2>(scratch, L.reach), cum);
+            tile_size, ntx, nty, N, recs, at<uint2>(scratch, L.rects), at<float2>(scratch, L.reach), L.place ? nullptr : cum);
         if (int rc = check_launch("fused_project")) return rc;
     }
-    if (int rc = scan_exclusive(cum, CN, cum, counters, at<void>(scratch, L.scan), stream)) return rc;
     if (L.place) {
-        // (with CN = 0 the count is 0 and the zeroed overflow flag stays 0)
         uint32_t* range_counts = at<uint32_t>(scratch, L.range_counts);
+        uint32_t* range_totals = at<uint32_t>(scratch, L.range_totals);
         uint32_t* totals = at<uint32_t>(scratch, L.bin_totals);
         const size_t lds = size_t(L.n_bins) * sizeof(uint32_t);
         const dim3 grid(L.n_ranges, C);
         if (CN > 0) {
-            fused_bin_count_kernel<<<grid, kWave, lds, stream>>>(at<uint2>(scratch, L.rects),
-                                                                 at<float2>(scratch, L.reach), N, L.range_len,
-                                                                 L.n_ranges, ntx, tile_size, L.n_bins, range_counts,
-                                                                 counters, capacity);
+            fused_bin_count_kernel<<<grid, kWave, lds, stream>>>(
+                at<uint2>(scratch, L.rects), at<float2>(scratch, L.reach), N, L.range_len, L.n_ranges, ntx, tile_size,
+                L.n_bins, range_counts, range_totals);
             if (int rc = check_launch("fused_bin_count")) return rc;
         }
-        const uint32_t n_cols = C * L.n_bins;
-        fused_bin_scan_ranges_kernel<<<ceil_div(n_cols, 256), 256, 0, stream>>>(range_counts, C, L.n_ranges, L.n_bins,
-                                                                               totals);
+        fused_bin_scan_ranges_kernel<<<ceil_div(size_t(C) * L.n_bins, kScanCols) + 1, kScanThreads, 0, stream>>>(
+            range_counts, C, L.n_ranges, L.n_bins, totals, range_totals, capacity, counters, cum + CN);
         if (int rc = check_launch("fused_bin_scan_ranges")) return rc;
-        if (int rc = scan_exclusive(totals, n_cols, totals, nullptr, at<void>(scratch, L.bin_scan), stream)) return rc;
+        fused_bin_starts_kernel<<<C, kScanThreads, 0, stream>>>(totals, L.n_bins, range_totals, L.n_ranges);
+        if (int rc = check_launch("fused_bin_starts")) return rc;
         if (CN > 0) {
             fused_bin_place_kernel<<<grid, kWave, lds, stream>>>(
                 at<uint2>(scratch, L.rects), at<float2>(scratch, L.reach), cum, N,
-                L.range_len, L.n_ranges, ntx, tile_size, L.n_bins, L.bin_bits, range_counts, totals, capacity,
-                entries);
+                L.range_len, L.n_ranges, ntx, tile_size, L.n_bins, L.bin_bits, range_counts, totals, range_totals,
+                capacity, entries);
             if (int rc = check_launch("fused_bin_place")) return rc;
         }
         if (tile_order && n_tiles > 0) {  // the tile offsets come with the tile order
@@ -1949,6 +2195,7 @@ static int prepare_impl(const float* means, const float* quats, const float* sca
         fused_bin_tile_offsets_kernel<<<ceil_div(n_tiles, 256), 256, 0, stream>>>(totals, n_tiles, tile_offsets);
         if (int rc = check_launch("fused_bin_tile_offsets")) return rc;
     } else {
+    if (int rc = scan_exclusive(cum, CN, cum, counters, at<void>(scratch, L.scan), stream)) return rc;
     void* sort_ws = at<void>(scratch, L.sort);
     if (CN > 0) {
         fused_emit_kernel<<<ceil_div(CN, 256), 256, 0, stream>>>(

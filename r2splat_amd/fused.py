@@ -148,7 +148,7 @@ def prepare(means, quats, scales, densities, viewmats, Ks, width, height, eps, r
     tile_order = torch.empty((C * nty * ntx,), dtype=torch.int32, device=device)
     # per-record intersection offsets (C*N + 1) followed by the primitive order (N)
     record_offsets = torch.empty((C * N + 1 + N,), dtype=torch.int32, device=device)
-    counters = torch.zeros((2,), dtype=torch.int32, device=device)
+    counters = torch.empty((2,), dtype=torch.int32, device=device)
     with torch.cuda.device(device):
         stream = be.stream_of(device)
         n_isects = -1

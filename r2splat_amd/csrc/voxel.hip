@@ -297,12 +297,11 @@ vox_bwd_isect_kernel(VoxArgs<S> A, const int64_t* __restrict__ isect_ids, const 
 }
 
 // ---------------------------------------------------------------------------
-// Moments form of the per-primitive VJP (float32, mean only, 8^3 tiles): each
-// workgroup takes a fixed chunk of the tile-sorted intersections (equal work
-// per workgroup, whatever the tile populations), one per lane, and visits the
-// chunk's tiles in order with each tile's adjoint staged in LDS; a lane sums its
-// primitive's moments over the 512 voxels row by row (every lane of the tile
-// reads the same row: broadcast loads, and no cross-lane reduction):
+// Moments form of the per-primitive VJP (float32, 8^3 tiles): a workgroup takes
+// a fixed chunk of the tile-sorted intersections (equal work per workgroup,
+// whatever the tile populations), with the adjoints of its tiles staged in LDS
+// kMomTiles at a time; a lane sums one intersection's moments over the rows of
+// 8 voxels that its primitive reaches, without cross-lane reduction:
 //   Gaussian, delta = voxel - mean, G = v e^-sigma (terms that pass the cut-off):
 //     M0 = sum G, M_k = sum G delta_k, M_kl = sum G delta_k delta_l,
 //     v_mean = opac P M, v_conic = -opac (M_xx/2, M_xy, M_xz, M_yy/2, M_yz, M_zz/2),
@@ -313,8 +312,18 @@ vox_bwd_isect_kernel(VoxArgs<S> A, const int64_t* __restrict__ isect_ids, const 
 // the same VJP as voxel_vjp summed over the tile. sigma is evaluated in log2
 // units (P scaled by log2 e) and the cut-off "sigma >= 0 and |opac e^-sigma| >=
 // 1e-6" (Beta: "0 <= q < 1 and |opac h^beta| >= 1e-5") is one unsigned compare
-// of the bits of q against qlim. Gradients are accumulated with one atomic per
-// field.
+// of the bits of q against qlim.
+//
+// Vector issue bounds it, so lanes must neither walk rows their primitive does
+// not reach nor wait for lanes that walk more: the reached rows are a 64-bit
+// mask per intersection (vox_row_mask), the chunk's intersections are sorted by
+// its population (a counting sort in LDS), and the waves take 64 at a time, most
+// rows first. Walking all 64 rows with only the lanes of one tile at a time
+// active took 3.40 ms for 500k Beta primitives with a variance in 256^3 (4% of
+// the pairs contribute), now 0.77, and 0.60 ms for 100k Gaussians in 128^3 (three
+// quarters of the rows are reached), now 0.48 at the full issue rate. The
+// register target is four waves a SIMD: the double-precision form at two (209
+// registers) took 0.92 ms.
 // ---------------------------------------------------------------------------
 constexpr uint32_t kMomT = 8;
 
@@ -389,7 +398,7 @@ __device__ __forceinline__ void vox_conic(const VoxArgs<float>& A, size_t G, flo
 __device__ __forceinline__ double beta_qmax(float w, float beta) {
     const double aw = fabs(double(w));
     if (!(aw >= 1e-5) || !(beta > 0.f)) return -1.0;
-    return 1.0 - pow(1e-5 / aw, 1.0 / double(beta));
+    return 1.0 - exp2(log2(1e-5 / aw) / double(beta));
 }
 
 constexpr uint32_t kVoxPartial = 12;  // floats per intersection partial (11, or 12 with a variance)
@@ -407,223 +416,386 @@ __device__ __forceinline__ uint32_t vox_qlim(float opac, float beta, bool is_bet
     return __float_as_uint(fminf(D, 0.99999994f)) + 1u;
 }
 
+// One intersection's quadratic form q = a dx^2 + bxy dx dy + bxz dx dz + cyy
+// dy^2 + cyz dy dz + czz dz^2 (Gaussian: sigma in log2 units) and its mean.
+struct VoxForm {
+    float hi[3], lo[3], P[6];  // mean as hi + lo, conic
+    float a, bxy, bxz, cyy, cyz, czz;
+    float opac, beta;
+    uint32_t qlim;  // float cut-off, or (WIDE) 1 when some term passes
+    double qmax;    // WIDE: the cut-off on d^2
+};
+
+template <bool BETA, bool WIDE>
+__device__ __forceinline__ VoxForm vox_form(const VoxArgs<float>& A, size_t G, const double* bound = nullptr) {
+    VoxForm f;
+    vox_mean_split(A, G, f.hi, f.lo);
+    vox_conic(A, G, f.P);
+    const float s = BETA ? 1.f : 0.5f * kL2E, t2 = BETA ? 2.f : kL2E;
+    f.a = s * f.P[0];
+    f.bxy = t2 * f.P[1];
+    f.bxz = t2 * f.P[2];
+    f.cyy = s * f.P[3];
+    f.cyz = t2 * f.P[4];
+    f.czz = s * f.P[5];
+    f.opac = A.opac[G];
+    f.beta = BETA ? A.betas[G] : 0.f;
+    f.qmax = -1.0;
+    if constexpr (WIDE) {
+        f.qmax = bound ? *bound : beta_qmax(f.opac, f.beta);  // (given where it was computed before)
+        f.qlim = f.qmax >= 0.0 ? 1u : 0u;
+    } else {
+        f.qlim = vox_qlim(f.opac, f.beta, BETA);
+    }
+    return f;
+}
+
+// Rows of 8 voxels (bit 8 z + y) of the tile whose first voxel centre is (x0, y0,
+// z0) that can hold a voxel with q <= S. In the plane dz the ellipsoid is an
+// ellipse in (x, y) of bound S - k dz^2 (k the Schur complement of czz) about
+// the mean shifted by (xs, ys) dz; its extent in y over the row's eight columns
+// is that of its upper and lower branches y(x) = (+-sqrt(4 cyy S - den x^2) - bxy
+// x) / 2 cyy, den = 4 a cyy - bxy^2, at their extremes clamped to the columns. S
+// is widened by 2e-3 and the columns and rows by 0.05 voxels, which covers the
+// rounding of q and of this bound where den and k do not cancel (to 1e-3);
+// other forms get every row, and a form no term of which passes none.
+__device__ __forceinline__ uint64_t vox_row_mask(const VoxForm& f, float S, float x0, float y0, float z0) {
+    if (f.qlim == 0u) return 0ull;
+    const float ac4 = 4.f * f.a * f.cyy, den = ac4 - f.bxy * f.bxy, inv = __builtin_amdgcn_rcpf(den);
+    const float xs = (f.bxy * f.cyz - 2.f * f.cyy * f.bxz) * inv, ys = (f.bxy * f.bxz - 2.f * f.a * f.cyz) * inv;
+    const float k = f.czz + 0.5f * (f.bxz * xs + f.cyz * ys);
+    const float wide = S * 1.002f;
+    if (!(f.a > 0.f) || !(f.cyy > 0.f) || !(den > 1e-3f * ac4) || !(k > 1e-3f * f.czz) || !(wide * inv < 1e30f))
+        return ~0ull;
+    const float reach_x = __builtin_amdgcn_sqrtf(4.f * f.cyy * inv) * 1.001f;      // per sqrt of the plane's bound
+    const float top = -0.5f * f.bxy * __builtin_amdgcn_rcpf(f.a) * __builtin_amdgcn_sqrtf(4.f * f.a * inv);
+    const float half_c = 0.5f * __builtin_amdgcn_rcpf(f.cyy), c4 = 4.f * f.cyy;
+    const float mx = f.hi[0] - x0, my = f.hi[1] - y0, mz = f.hi[2] - z0;  // the mean in voxels of this tile
+    uint32_t half[2] = {0u, 0u};
+#pragma unroll
+    for (int z = 0; z < int(kMomT); ++z) {
+        const float dz = float(z) - mz, Sz = fmaf(-k * dz, dz, wide);
+        const float r = __builtin_amdgcn_sqrtf(fmaxf(Sz, 0.f)), rx = reach_x * r;
+        const float cx = fmaf(xs, dz, mx), cy = fmaf(ys, dz, my);
+        const float u0 = -0.05f - cx, u1 = float(kMomT - 1) + 0.05f - cx;
+        const float xt = fminf(fmaxf(top * r, u0), u1), xb = fminf(fmaxf(-top * r, u0), u1);
+        const float yt = (__builtin_amdgcn_sqrtf(fmaxf(c4 * Sz - den * xt * xt, 0.f)) - f.bxy * xt) * half_c;
+        const float yb = -(__builtin_amdgcn_sqrtf(fmaxf(c4 * Sz - den * xb * xb, 0.f)) + f.bxy * xb) * half_c;
+        const uint32_t lo = uint32_t(fminf(fmaxf(ceilf(cy + yb - 0.05f), 0.f), float(kMomT)));
+        const uint32_t hi = uint32_t(fminf(fmaxf(floorf(cy + yt + 0.05f) + 1.f, 0.f), float(kMomT)));
+        const bool hit = Sz >= 0.f && u0 <= rx && u1 >= -rx && hi > lo;
+        half[z / 4] |= hit ? ((1u << hi) - (1u << lo)) << (8 * (z % 4)) : 0u;
+    }
+    return (uint64_t(half[1]) << 32) | half[0];
+}
+
 // VAR: the voxel adjoint becomes v + var_scale q alpha v_var (var_scale 2, or
 // 0 when the variance is detached) and the partial's twelfth slot carries
 // v_q = sum v_var alpha^2 (variance = sum q alpha^2). WIDE (Beta with a
 // frame): q and h = 1 - q are formed in double from the frame, with the
 // cut-off 0 <= q <= qmax decided in double, exactly as the fused forward does.
-template <bool BETA, bool VAR, bool WIDE = false>
-__global__ void __launch_bounds__(kMomThreads)
+// With `partials` an intersection's gradient goes to its emission index, else
+// it is added to the outputs with one atomic per field.
+// A workgroup takes 512 intersections, or 256 where those would leave most
+// compute units with a single workgroup (up to 2^19 intersections in all: 285k
+// take 30 us against 66; 2.9M take 534 us against 479, their rows sorted less
+// finely).
+constexpr uint32_t kMomFew = 1u << 19;
+constexpr uint32_t kMomTiles = 8;  // tiles whose adjoints are staged together
+
+template <uint32_t kMomChunk, bool BETA, bool VAR, bool WIDE>
+__global__ void __launch_bounds__(kMomThreads) __attribute__((amdgpu_waves_per_eu(4)))
 vox_bwd_moments_kernel(VoxArgs<float> A, const int64_t* __restrict__ isect_ids, const float* __restrict__ v_render,
                        const float* __restrict__ v_render_var, float var_scale,
                        float* __restrict__ v_xyz, float* __restrict__ v_c, float* __restrict__ v_opac,
                        float* __restrict__ v_beta, const int32_t* __restrict__ radii,
                        const uint32_t* __restrict__ cum, float* __restrict__ partials) {
-    constexpr uint32_t T = kMomT, T3 = T * T * T;
-    __shared__ __align__(16) float sv[T3];
-    __shared__ __align__(16) float svv[VAR ? T3 : 4];
-    __shared__ int64_t ids[kMomThreads];
-    // a chunk of kMomThreads consecutive (tile-sorted) intersections, one per thread; the chunk's
-    // tiles are visited in order, each one's adjoint staged in LDS in turn
-    const uint32_t e0 = blockIdx.x * kMomThreads, e1 = min(e0 + kMomThreads, A.n_isects);
-    const uint32_t e = e0 + threadIdx.x;
-    const int64_t mine = e < e1 ? isect_ids[e] : INT64_MAX;
-    ids[threadIdx.x] = mine;
-    __syncthreads();
-    const uint32_t n_here = e1 - e0;
-    const int64_t nt = int64_t(A.ntx) * A.nty * A.ntz;
+    constexpr uint32_t T = kMomT, T3 = T * T * T, kPer = kMomChunk / kMomThreads, kWaves = kMomThreads / kWave;
+    constexpr uint32_t kNoTile = 0xffffffffu, kClasses = T * T + 1;
     static_assert(!WIDE || BETA, "the double-precision form is for Beta profiles");
-    uint32_t pos = 0;  // first chunk entry of the current tile
-    while (pos < n_here) {
-        const int64_t tile = ids[pos];
-        uint32_t lo = pos, hi = n_here;  // first entry of the next tile
-        while (lo < hi) {
-            const uint32_t mid = (lo + hi) >> 1;
-            if (ids[mid] <= tile) lo = mid + 1; else hi = mid;
+    static_assert(kClasses == kWave + 1, "the row counts 64 .. 1 are scanned by one wave");
+    __shared__ __align__(16) float sv[kMomTiles * T3];
+    __shared__ __align__(16) float svv[VAR ? kMomTiles * T3 : 4];
+    __shared__ uint64_t masks[kMomChunk];
+    __shared__ double bounds[WIDE ? kMomChunk : 1];
+    __shared__ uint32_t tile_of[kMomChunk], sorted[kMomChunk];  // sorted: chunk entry | staged tile << 16
+    __shared__ uint32_t first_of[kMomChunk + 1];                // first entry of the chunk's k-th tile
+    __shared__ uint32_t hist[kClasses], first[kClasses], wave_tiles[kPer * kWaves], n_items, next_item;
+    const uint32_t lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    const uint32_t e0 = blockIdx.x * kMomChunk, n_here = min(kMomChunk, A.n_isects - e0);
+    const int64_t nt = int64_t(A.ntx) * A.nty * A.ntz;
+    uint32_t place[kPer];  // which of the chunk's tiles an entry belongs to
+#pragma unroll
+    for (uint32_t k = 0; k < kPer; ++k) {
+        const uint32_t i = k * kMomThreads + threadIdx.x;
+        int64_t id = -1;
+        if (i < n_here) id = isect_ids[e0 + i];
+        tile_of[i] = id >= 0 && id < nt ? uint32_t(id) : kNoTile;
+    }
+    __syncthreads();
+    uint64_t starts[kPer];
+#pragma unroll
+    for (uint32_t k = 0; k < kPer; ++k) {
+        const uint32_t i = k * kMomThreads + threadIdx.x;
+        starts[k] = __ballot(i < n_here && (i == 0 || tile_of[i] != tile_of[i - 1]));
+        if (lane == 0) wave_tiles[k * kWaves + wave] = uint32_t(__popcll(starts[k]));
+    }
+    __syncthreads();
+    uint32_t n_tiles = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < kPer; ++k) {
+        uint32_t before = 0;
+        for (uint32_t w = 0; w < k * kWaves + wave; ++w) before += wave_tiles[w];
+        const uint64_t upto = starts[k] & (~0ull >> (kWave - 1 - lane));
+        place[k] = before + uint32_t(__popcll(upto)) - 1u;
+        if ((starts[k] >> lane) & 1ull) first_of[place[k]] = k * kMomThreads + threadIdx.x;
+    }
+    for (uint32_t w = 0; w < kPer * kWaves; ++w) n_tiles += wave_tiles[w];
+    for (uint32_t t0 = 0; t0 < n_tiles; t0 += kMomTiles) {
+        __syncthreads();  // first_of is written; the previous tiles' adjoints are consumed
+        const uint32_t n_staged = min(kMomTiles, n_tiles - t0);
+        for (uint32_t p = threadIdx.x; p < n_staged * T3; p += kMomThreads) {
+            const uint32_t tile = tile_of[first_of[t0 + p / T3]], q = p % T3;
+            if (tile == kNoTile) continue;
+            const uint32_t tx = tile % A.ntx, rest = tile / A.ntx, ty = rest % A.nty, tz = rest / A.nty;
+            const uint32_t x = tx * T + q % T, j = ty * T + (q / T) % T, i = tz * T + q / (T * T);
+            const bool in = i < A.dz && j < A.dy && x < A.dx;
+            const size_t o = (size_t(i) * A.dy + j) * A.dx + x;
+            sv[p] = in ? v_render[o] : 0.f;
+            if constexpr (VAR) svv[p] = in ? v_render_var[o] : 0.f;
         }
-        const bool valid_tile = tile >= 0 && tile < nt;
-        const uint32_t blk = valid_tile ? uint32_t(tile) : 0u;
-        const uint32_t tx = blk % A.ntx, rest = blk / A.ntx, ty = rest % A.nty, tz = rest / A.nty;
-        if (valid_tile)
-            for (uint32_t p = threadIdx.x; p < T3; p += blockDim.x) {
-                const uint32_t k = tx * T + p % T, j = ty * T + (p / T) % T, i = tz * T + p / (T * T);
-                const bool in = i < A.dz && j < A.dy && k < A.dx;
-                const size_t o = (size_t(i) * A.dy + j) * A.dx + k;
-                sv[p] = in ? v_render[o] : 0.f;
-                if constexpr (VAR) svv[p] = in ? v_render_var[o] : 0.f;
+        for (uint32_t c = threadIdx.x; c < kClasses; c += kMomThreads) hist[c] = 0u;
+        __syncthreads();
+        uint64_t mask[kPer];
+        double bound[kPer];
+        uint32_t rank[kPer];
+        bool mine[kPer];
+#pragma unroll
+        for (uint32_t k = 0; k < kPer; ++k) {
+            const uint32_t i = k * kMomThreads + threadIdx.x;
+            mine[k] = i < n_here && place[k] >= t0 && place[k] < t0 + n_staged && tile_of[i] != kNoTile;
+            mask[k] = 0ull;
+            bound[k] = -1.0;
+            rank[k] = 0u;
+            if (mine[k]) {
+                const int32_t g = A.flatten[e0 + i];
+                mine[k] = g >= 0 && uint32_t(g) < A.N;
+                if (mine[k]) {
+                    const VoxForm f = vox_form<BETA, WIDE>(A, size_t(g));
+                    const uint32_t tile = tile_of[i], tx = tile % A.ntx, rest = tile / A.ntx;
+                    bound[k] = f.qmax;
+                    const float S = WIDE ? float(f.qmax) : __uint_as_float(f.qlim - 1u);
+                    mask[k] = vox_row_mask(f, S, float(tx * T) + 0.5f, float((rest % A.nty) * T) + 0.5f,
+                                           float((rest / A.nty) * T) + 0.5f);
+                    rank[k] = atomicAdd(&hist[T * T - uint32_t(__popcll(mask[k]))], 1u);
+                }
+            }
+        }
+        __syncthreads();
+        if (wave == 0) {  // starts of the row counts, most rows first
+            const uint32_t c = hist[lane], incl = wave_scan(c);
+            first[lane] = incl - c;
+            if (lane == kWave - 1) {
+                first[kWave] = incl;
+                n_items = incl + hist[kWave];
+                next_item = 0u;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (uint32_t k = 0; k < kPer; ++k)
+            if (mine[k]) {
+                const uint32_t at = first[T * T - uint32_t(__popcll(mask[k]))] + rank[k];
+                masks[at] = mask[k];
+                if constexpr (WIDE) bounds[at] = bound[k];
+                sorted[at] = (k * kMomThreads + threadIdx.x) | ((place[k] - t0) << 16);
             }
         __syncthreads();
-        if (valid_tile && mine == tile) {
+        for (;;) {
+            uint32_t c = 0;
+            if (lane == 0) c = atomicAdd(&next_item, uint32_t(kWave));
+            c = __builtin_amdgcn_readfirstlane(c);
+            if (c >= n_items) break;
+            const bool active = c + lane < n_items;  // the others repeat item c without rows
+            const uint32_t at = active ? c + lane : c, it = sorted[at], i = it & 0xffffu, staged = (it >> 16) * T3;
+            uint64_t rows = active ? masks[at] : 0ull;
+            const uint32_t tile = tile_of[i], tx = tile % A.ntx, rest = tile / A.ntx, ty = rest % A.nty,
+                           tz = rest / A.nty;
             const float x0 = float(tx * T) + 0.5f, y0 = float(ty * T) + 0.5f, z0 = float(tz * T) + 0.5f;
-            const int32_t g = A.flatten[e];
-            if (g >= 0 && uint32_t(g) < A.N) {
-                const size_t G = size_t(g);
-                float hi3[3], lo3[3], P[6];
-                vox_mean_split(A, G, hi3, lo3);
-                vox_conic(A, G, P);
-                const float mx = hi3[0], my = hi3[1], mz = hi3[2];
-                const float opac = A.opac[g], beta = BETA ? A.betas[g] : 0.f;
-                uint32_t qlim = vox_qlim(opac, beta, BETA);
-                double md[3] = {0.0, 0.0, 0.0}, Pd[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0}, qmax = -1.0;
-                if constexpr (WIDE) {
+            const int32_t g = A.flatten[e0 + i];
+            const size_t G = size_t(g);
+            const VoxForm f = vox_form<BETA, WIDE>(A, G, WIDE ? &bounds[at] : nullptr);
+            const float* P = f.P;
+            const float opac = f.opac, beta = f.beta;
+            double md[3] = {0.0, 0.0, 0.0}, Pd[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+            if constexpr (WIDE) {
 #pragma unroll
-                    for (int k = 0; k < 3; ++k) md[k] = A.frame[kFrame * G + k];
+                for (int k = 0; k < 3; ++k) md[k] = A.frame[kFrame * G + k];
 #pragma unroll
-                    for (int k = 0; k < 6; ++k) Pd[k] = A.frame[kFrame * G + 3 + k];
-                    qmax = beta_qmax(opac, beta);
-                    qlim = qmax >= 0.0 ? 1u : 0u;  // liveness only: the cut-off is q <= qmax
-                }
-                const double ad = Pd[0], bxyd = 2.0 * Pd[1], bxzd = 2.0 * Pd[2], cyyd = Pd[3], cyzd = 2.0 * Pd[4],
-                             czzd = Pd[5];
-                const double dx0d = double(float(tx * T) + 0.5f) - md[0];
-                const float kvar = VAR ? var_scale * A.unc[g] * opac : 0.f;  // d variance / d (alpha / w) factor
-                // q = a dx^2 + bxy dx dy + bxz dx dz + cyy dy^2 + cyz dy dz + czz dz^2
-                const float s = BETA ? 1.f : 0.5f * kL2E, t2 = BETA ? 2.f : kL2E;
-                const float a = s * P[0], bxy = t2 * P[1], bxz = t2 * P[2], cyy = s * P[3], cyz = t2 * P[4], czz = s * P[5];
-                const float bm1 = beta - 1.f;
-                float m0 = 0.f, m_x = 0.f, m_y = 0.f, m_z = 0.f, mxx = 0.f, myy = 0.f, mzz = 0.f, mxy = 0.f, mxz = 0.f,
-                      myz = 0.f, se = 0.f, sl = 0.f, vq = 0.f;
-                const float dx0 = (x0 - mx) - lo3[0];
-                if (qlim != 0u) {
-                    for (uint32_t z = 0; z < T; ++z) {
-                        const double dzd = double(z0 + float(z)) - md[2];
-                        const float dz = WIDE ? float(dzd) : ((z0 + float(z)) - mz) - lo3[2];
-                        for (uint32_t y = 0; y < T; ++y) {
-                            const double dyd = double(y0 + float(y)) - md[1];
-                            const float dy = WIDE ? float(dyd) : ((y0 + float(y)) - my) - lo3[1];
-                            const float4* row = reinterpret_cast<const float4*>(sv + (z * T + y) * T);
-                            const float4 va = row[0], vb = row[1];
-                            const float v[8] = {va.x, va.y, va.z, va.w, vb.x, vb.y, vb.z, vb.w};
-                            float vv[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+                for (int k = 0; k < 6; ++k) Pd[k] = A.frame[kFrame * G + 3 + k];
+            }
+            const double ad = Pd[0], bxyd = 2.0 * Pd[1], bxzd = 2.0 * Pd[2], cyyd = Pd[3], cyzd = 2.0 * Pd[4],
+                         czzd = Pd[5];
+            const double dx0d = double(x0) - md[0];
+            const float kvar = VAR ? var_scale * A.unc[g] * opac : 0.f;  // d variance / d (alpha / w) factor
+            const float bm1 = beta - 1.f;
+            float m0 = 0.f, m_x = 0.f, m_y = 0.f, m_z = 0.f, mxx = 0.f, myy = 0.f, mzz = 0.f, mxy = 0.f, mxz = 0.f,
+                  myz = 0.f, se = 0.f, sl = 0.f, vq = 0.f;
+            const float dx0 = (x0 - f.hi[0]) - f.lo[0];
+            // the columns' offsets and their squares are the same in every row
+            float dxc[T], dxsq[T];
+#pragma unroll
+            for (uint32_t x = 0; x < T; ++x) {
+                dxc[x] = dx0 + float(x);
+                dxsq[x] = dxc[x] * dxc[x];
+            }
+            while (rows) {
+                const uint32_t bit = uint32_t(__builtin_ctzll(rows)), z = bit / T, y = bit % T;
+                rows &= rows - 1ull;
+                const double dzd = double(z0 + float(z)) - md[2], dyd = double(y0 + float(y)) - md[1];
+                const float dz = WIDE ? float(dzd) : ((z0 + float(z)) - f.hi[2]) - f.lo[2];
+                const float dy = WIDE ? float(dyd) : ((y0 + float(y)) - f.hi[1]) - f.lo[1];
+                const float c1 = fmaf(f.bxy, dy, f.bxz * dz);
+                const float c0 = fmaf(dy, fmaf(f.cyy, dy, f.cyz * dz), f.czz * dz * dz);
+                const double c1d = fma(bxyd, dyd, bxzd * dzd);
+                const double c0d = fma(dyd, fma(cyyd, dyd, cyzd * dzd), czzd * dzd * dzd);
+                float r0 = 0.f, r1 = 0.f, r2 = 0.f, re = 0.f, rl = 0.f;
+                // four voxels at a time: with the double-precision form all eight at once
+                // take 209 registers (two waves a SIMD)
+                constexpr int kStep = WIDE ? 4 : 8;
+#pragma unroll 1
+                for (int h4 = 0; h4 < 8; h4 += kStep) {
+                    float v[kStep], vv[kStep];
+#pragma unroll
+                    for (int j = 0; j < kStep; j += 4) {
+                        const float4 w = *reinterpret_cast<const float4*>(sv + staged + bit * T + h4 + j);
+                        v[j] = w.x; v[j + 1] = w.y; v[j + 2] = w.z; v[j + 3] = w.w;
+                        if constexpr (VAR) {
+                            const float4 u = *reinterpret_cast<const float4*>(svv + staged + bit * T + h4 + j);
+                            vv[j] = u.x; vv[j + 1] = u.y; vv[j + 2] = u.z; vv[j + 3] = u.w;
+                        }
+                    }
+                    const double dx4 = dx0d + double(h4);
+#pragma unroll
+                    for (int x = 0; x < kStep; ++x) {
+                        float dx, dx2, q, h;
+                        bool in;
+                        if constexpr (WIDE) {
+                            const double dxd = dx4 + double(x);
+                            const double qd = fma(dxd, fma(ad, dxd, c1d), c0d);
+                            in = qd >= 0.0 && qd <= f.qmax;
+                            h = float(1.0 - qd);
+                            q = 0.f;
+                            dx = float(dxd);
+                            dx2 = dx * dx;
+                        } else {
+                            dx = dxc[x];
+                            dx2 = dxsq[x];
+                            q = fmaf(dx, fmaf(f.a, dx, c1), c0);
+                            in = __float_as_uint(q) < f.qlim;
+                            h = 1.f - q;
+                        }
+                        float gv;
+                        if constexpr (BETA) {
+                            const float lg = __log2f(h);
+                            const float hb = in ? __builtin_amdgcn_exp2f(bm1 * lg) : 0.f;  // h^(beta - 1)
+                            float ve;
                             if constexpr (VAR) {
-                                const float4* rowv = reinterpret_cast<const float4*>(svv + (z * T + y) * T);
-                                const float4 wa = rowv[0], wb = rowv[1];
-                                vv[0] = wa.x; vv[1] = wa.y; vv[2] = wa.z; vv[3] = wa.w;
-                                vv[4] = wb.x; vv[5] = wb.y; vv[6] = wb.z; vv[7] = wb.w;
+                                const float he = hb * h;  // h^beta = alpha / w
+                                const float vj = fmaf(kvar * he, vv[x], v[x]);
+                                gv = vj * hb;
+                                ve = vj * he;
+                                vq = fmaf(vv[x] * he, he, vq);
+                            } else {
+                                gv = v[x] * hb;
+                                ve = gv * h;
                             }
-                            const float c1 = fmaf(bxy, dy, bxz * dz);
-                            const float c0 = fmaf(dy, fmaf(cyy, dy, cyz * dz), czz * dz * dz);
-                            const double c1d = fma(bxyd, dyd, bxzd * dzd);
-                            const double c0d = fma(dyd, fma(cyyd, dyd, cyzd * dzd), czzd * dzd * dzd);
-                            float r0 = 0.f, r1 = 0.f, r2 = 0.f, re = 0.f, rl = 0.f;
-#pragma unroll
-                            for (int x = 0; x < 8; ++x) {
-                                float dx, q, h;
-                                bool in;
-                                if constexpr (WIDE) {
-                                    const double dxd = dx0d + double(x);
-                                    const double qd = fma(dxd, fma(ad, dxd, c1d), c0d);
-                                    in = qd >= 0.0 && qd <= qmax;
-                                    h = float(1.0 - qd);
-                                    q = 0.f;
-                                    dx = float(dxd);
-                                } else {
-                                    dx = dx0 + float(x);
-                                    q = fmaf(dx, fmaf(a, dx, c1), c0);
-                                    in = __float_as_uint(q) < qlim;
-                                    h = 1.f - q;
-                                }
-                                float gv;
-                                if constexpr (BETA) {
-                                    const float lg = __log2f(h);
-                                    const float hb = in ? __builtin_amdgcn_exp2f(bm1 * lg) : 0.f;  // h^(beta - 1)
-                                    float ve;
-                                    if constexpr (VAR) {
-                                        const float he = hb * h;  // h^beta = alpha / w
-                                        const float vj = fmaf(kvar * he, vv[x], v[x]);
-                                        gv = vj * hb;
-                                        ve = vj * he;
-                                        vq = fmaf(vv[x] * he, he, vq);
-                                    } else {
-                                        gv = v[x] * hb;
-                                        ve = gv * h;
-                                    }
-                                    re += ve;
-                                    rl = fmaf(ve, in ? lg : 0.f, rl);
-                                } else {
-                                    const float e = in ? __builtin_amdgcn_exp2f(-q) : 0.f;
-                                    if constexpr (VAR) {
-                                        const float vj = fmaf(kvar * e, vv[x], v[x]);
-                                        gv = vj * e;
-                                        vq = fmaf(vv[x] * e, e, vq);
-                                    } else {
-                                        gv = v[x] * e;
-                                    }
-                                }
-                                r0 += gv;
-                                const float gx = gv * dx;
-                                r1 += gx;
-                                r2 = fmaf(gx, dx, r2);
-                            }
-                            m0 += r0;
-                            m_x += r1;
-                            mxx += r2;
-                            m_y = fmaf(dy, r0, m_y);
-                            m_z = fmaf(dz, r0, m_z);
-                            myy = fmaf(dy * dy, r0, myy);
-                            mzz = fmaf(dz * dz, r0, mzz);
-                            myz = fmaf(dy * dz, r0, myz);
-                            mxy = fmaf(dy, r1, mxy);
-                            mxz = fmaf(dz, r1, mxz);
-                            if constexpr (BETA) {
-                                se += re;
-                                sl += rl;
+                            re += ve;
+                            rl = fmaf(ve, in ? lg : 0.f, rl);
+                        } else {
+                            const float e = in ? __builtin_amdgcn_exp2f(-q) : 0.f;
+                            if constexpr (VAR) {
+                                const float vj = fmaf(kvar * e, vv[x], v[x]);
+                                gv = vj * e;
+                                vq = fmaf(vv[x] * e, e, vq);
+                            } else {
+                                gv = v[x] * e;
                             }
                         }
+                        r0 += gv;
+                        r1 = fmaf(gv, dx, r1);
+                        r2 = fmaf(gv, dx2, r2);
                     }
                 }
-                const float k = BETA ? 2.f * opac * beta : opac;
-                const float gm[3] = {k * (P[0] * m_x + P[1] * m_y + P[2] * m_z), k * (P[1] * m_x + P[3] * m_y + P[4] * m_z),
-                                     k * (P[2] * m_x + P[4] * m_y + P[5] * m_z)};
-                float gc[6];
+                m0 += r0;
+                m_x += r1;
+                mxx += r2;
+                m_y = fmaf(dy, r0, m_y);
+                m_z = fmaf(dz, r0, m_z);
+                myy = fmaf(dy * dy, r0, myy);
+                mzz = fmaf(dz * dz, r0, mzz);
+                myz = fmaf(dy * dz, r0, myz);
+                mxy = fmaf(dy, r1, mxy);
+                mxz = fmaf(dz, r1, mxz);
                 if constexpr (BETA) {
-                    const float kb = -opac * beta;
-                    gc[0] = kb * mxx; gc[1] = 2.f * kb * mxy; gc[2] = 2.f * kb * mxz;
-                    gc[3] = kb * myy; gc[4] = 2.f * kb * myz; gc[5] = kb * mzz;
-                } else {
-                    gc[0] = -0.5f * opac * mxx; gc[1] = -opac * mxy; gc[2] = -opac * mxz;
-                    gc[3] = -0.5f * opac * myy; gc[4] = -opac * myz; gc[5] = -0.5f * opac * mzz;
-                }
-                const float go = BETA ? se : m0, gb = BETA ? opac * 0.6931471805599453f * sl : 0.f;
-                if (partials) {
-                    // the partial of this intersection at its emission index: the binning wrote
-                    // the primitive's tiles from cum[n] on, in z, y, x order over its tile box
-                    uint32_t lo[3], hi[3];
-                    if (box_3d(A.means3d, radii, G, T, A.ntx, A.nty, A.ntz, lo, hi) && tx >= lo[0] && tx < hi[0] &&
-                        ty >= lo[1] && ty < hi[1] && tz >= lo[2] && tz < hi[2]) {
-                        const uint32_t w = cum[G] + ((tz - lo[2]) * (hi[1] - lo[1]) + (ty - lo[1])) * (hi[0] - lo[0]) +
-                                           (tx - lo[0]);
-                        if (w < A.n_isects) {
-                            float4* out = reinterpret_cast<float4*>(partials + kVoxPartial * size_t(w));
-                            out[0] = make_float4(gm[0], gm[1], gm[2], gc[0]);
-                            out[1] = make_float4(gc[1], gc[2], gc[3], gc[4]);
-                            out[2] = make_float4(gc[5], go, gb, VAR ? opac * opac * vq : 0.f);
-                        }
-                    }
-                } else {
-#pragma unroll
-                    for (int q = 0; q < 3; ++q) atomic_add(v_xyz + 3 * G + q, gm[q]);
-#pragma unroll
-                    for (int q = 0; q < 6; ++q) atomic_add(v_c + 6 * G + q, gc[q]);
-                    atomic_add(v_opac + G, go);
-                    if constexpr (BETA) atomic_add(v_beta + G, gb);
+                    se += re;
+                    sl += rl;
                 }
             }
+            const float k = BETA ? 2.f * opac * beta : opac;
+            const float gm[3] = {k * (P[0] * m_x + P[1] * m_y + P[2] * m_z), k * (P[1] * m_x + P[3] * m_y + P[4] * m_z),
+                                 k * (P[2] * m_x + P[4] * m_y + P[5] * m_z)};
+            float gc[6];
+            if constexpr (BETA) {
+                const float kb = -opac * beta;
+                gc[0] = kb * mxx; gc[1] = 2.f * kb * mxy; gc[2] = 2.f * kb * mxz;
+                gc[3] = kb * myy; gc[4] = 2.f * kb * myz; gc[5] = kb * mzz;
+            } else {
+                gc[0] = -0.5f * opac * mxx; gc[1] = -opac * mxy; gc[2] = -opac * mxz;
+                gc[3] = -0.5f * opac * myy; gc[4] = -opac * myz; gc[5] = -0.5f * opac * mzz;
+            }
+            const float go = BETA ? se : m0, gb = BETA ? opac * 0.6931471805599453f * sl : 0.f;
+            if (!active) {
+            } else if (partials) {
+                // the partial of this intersection at its emission index: the binning wrote
+                // the primitive's tiles from cum[n] on, in z, y, x order over its tile box
+                uint32_t lo[3], hi[3];
+                if (box_3d(A.means3d, radii, G, T, A.ntx, A.nty, A.ntz, lo, hi) && tx >= lo[0] && tx < hi[0] &&
+                    ty >= lo[1] && ty < hi[1] && tz >= lo[2] && tz < hi[2]) {
+                    const uint32_t w = cum[G] + ((tz - lo[2]) * (hi[1] - lo[1]) + (ty - lo[1])) * (hi[0] - lo[0]) +
+                                       (tx - lo[0]);
+                    if (w < A.n_isects) {
+                        float4* out = reinterpret_cast<float4*>(partials + kVoxPartial * size_t(w));
+                        out[0] = make_float4(gm[0], gm[1], gm[2], gc[0]);
+                        out[1] = make_float4(gc[1], gc[2], gc[3], gc[4]);
+                        out[2] = make_float4(gc[5], go, gb, VAR ? opac * opac * vq : 0.f);
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int q = 0; q < 3; ++q) atomic_add(v_xyz + 3 * G + q, gm[q]);
+#pragma unroll
+                for (int q = 0; q < 6; ++q) atomic_add(v_c + 6 * G + q, gc[q]);
+                atomic_add(v_opac + G, go);
+                if constexpr (BETA) atomic_add(v_beta + G, gb);
+            }
         }
-        __syncthreads();  // every thread is done with this tile's adjoint
-        pos = lo;
     }
 }
 
 // ---------------------------------------------------------------------------
-// Fused float32 forward (mean only, 8^3 tiles): kVoxFwdWaves waves per tile,
-// wave k summing the k-th contiguous slice of the tile's list; lane = one
-// (y, z) row of 8 voxels. Records (mean, the quadratic form in log2 units for
-// Gaussians, qlim, opacity, beta) are built from the primitive arrays a batch
-// of 64 ahead by the lanes and read back from LDS by broadcast; per record a
-// lane forms the row terms once and evaluates q = a dx^2 + (bxy dy + bxz dz) dx
-// + c(dy, dz) for its 8 voxels. The slices' partial volumes are summed in LDS
-// in wave order, so the result does not depend on scheduling.
+// Fused float32 forward (8^3 tiles): kVoxFwdWaves waves per tile, wave k summing
+// the k-th contiguous slice of the tile's list. Records (the mean and the
+// quadratic form, the cut-off, opacity, beta) are built from the primitive
+// arrays a batch of 64 ahead by the lanes and read back from LDS by broadcast.
+// Gaussians (log2 units), which reach most of the tiles they are binned to: lane
+// = one (y, z) row of 8 voxels, a lane forms the row terms once and evaluates q
+// = a dx^2 + (bxy dy + bxz dz) dx + c(dy, dz) for its 8 voxels. Beta primitives,
+// whose support fills 4% of the voxels of its tiles at 500k primitives in
+// 256^3: lane = one voxel of each 4^3 octant, and octants that the support's
+// bounding box does not reach are skipped by scalar branches (0.97 -> 0.52 ms
+// there; 100k Gaussians in 128^3 take 0.38 ms). The slices' partial volumes are summed in LDS in wave order, so the result does
+// not depend on scheduling.
 // ---------------------------------------------------------------------------
 constexpr int kVoxFwdWaves = 4;
 
@@ -636,11 +808,11 @@ struct __align__(16) VoxRec {
 static_assert(sizeof(VoxRec) == 64, "voxel record must be 64 bytes");
 
 // Beta record: the mean and the conic (off-diagonals doubled) in double; a
-// term passes the cut-off when 0 <= d^2 <= qmax (qlim = 1 when some term can).
+// term passes the cut-off when 0 <= d^2 <= qmax; the octants it can reach.
 struct __align__(16) VoxRecB {
     double mx, my, mz, a, bxy, bxz, cyy, cyz, czz, qmax;
     float w, beta;
-    uint32_t qlim, pad;
+    uint32_t octants, pad;  // bit 4 oz + 2 oy + ox
 };
 static_assert(sizeof(VoxRecB) == 96, "Beta voxel record must be 96 bytes");
 
@@ -674,8 +846,33 @@ __device__ __forceinline__ VoxRec load_gauss_rec(const VoxArgs<float>& A, int32_
     return r;
 }
 
+// Octants of the tile at voxel (x0, y0, z0) that the ellipsoid d^2 <= qmax of a
+// record can reach: its bounding box (half-extents sqrt(qmax C_kk), C the
+// inverse of the conic), widened by 1e-3 and 0.05 voxels; every octant where
+// the conic's determinant cancels.
+__device__ __forceinline__ uint32_t vox_octants(const VoxRecB& r, float x0, float y0, float z0) {
+    if (!(r.qmax >= 0.0)) return 0u;
+    const float xx = float(r.a), yy = float(r.cyy), zz = float(r.czz), xy = 0.5f * float(r.bxy),
+                xz = 0.5f * float(r.bxz), yz = 0.5f * float(r.cyz), S = float(r.qmax);
+    const float c[3] = {yy * zz - yz * yz, xx * zz - xz * xz, xx * yy - xy * xy};
+    const float det = xx * c[0] - xy * (xy * zz - xz * yz) + xz * (xy * yz - xz * yy);
+    if (!(det > 1e-3f * xx * yy * zz)) return 0xffu;
+    const float m[3] = {float(r.mx - double(x0)), float(r.my - double(y0)), float(r.mz - double(z0))};
+    uint32_t part[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const float e = __builtin_amdgcn_sqrtf(fmaxf(S * c[k] * __builtin_amdgcn_rcpf(det), 0.f)) * 1.001f + 0.05f;
+        const float lo = m[k] - e, hi = m[k] + e;  // voxel centres of the tile at 0.5 .. 7.5
+        part[k] = (lo <= 3.5f && hi >= 0.5f ? 1u : 0u) | (lo <= 7.5f && hi >= 4.5f ? 2u : 0u);
+        if (!(e < 1e30f)) part[k] = 3u;
+    }
+    const uint32_t row = part[0], plane = (part[1] & 1u ? row : 0u) | (part[1] & 2u ? row << 2 : 0u);
+    return (part[2] & 1u ? plane : 0u) | (part[2] & 2u ? plane << 4 : 0u);
+}
+
 // Needs the frame (the fused entry points require it).
-__device__ __forceinline__ VoxRecB load_beta_rec(const VoxArgs<float>& A, int32_t i, int32_t hi) {
+__device__ __forceinline__ VoxRecB load_beta_rec(const VoxArgs<float>& A, int32_t i, int32_t hi, float x0, float y0,
+                                                 float z0) {
     VoxRecB r = {};
     if (i >= hi) return r;
     const int32_t g = A.flatten[i];
@@ -693,14 +890,16 @@ __device__ __forceinline__ VoxRecB load_beta_rec(const VoxArgs<float>& A, int32_
     r.w = A.opac[g];
     r.beta = A.betas[g];
     r.qmax = beta_qmax(r.w, r.beta);
-    r.qlim = r.qmax >= 0.0 ? 1u : 0u;
+    r.octants = vox_octants(r, x0, y0, z0);
     return r;
 }
 
+// Entry i's record for the tile whose corner is (x0, y0, z0).
 template <bool BETA>
-__device__ __forceinline__ VoxRecOf<BETA> load_vox_rec(const VoxArgs<float>& A, int32_t i, int32_t hi) {
+__device__ __forceinline__ VoxRecOf<BETA> load_vox_rec(const VoxArgs<float>& A, int32_t i, int32_t hi, float x0,
+                                                       float y0, float z0) {
     if constexpr (BETA)
-        return load_beta_rec(A, i, hi);
+        return load_beta_rec(A, i, hi, x0, y0, z0);
     else
         return load_gauss_rec(A, i, hi);
 }
@@ -717,7 +916,7 @@ __device__ __forceinline__ float load_vox_unc(const VoxArgs<float>& A, int32_t i
 // Beta terms form d^2 and 1 - d^2 in double (the record's mean and conic),
 // decide the cut-off on d^2 in double and take the power in float32.
 template <bool BETA, bool VAR>
-__global__ void __launch_bounds__(kVoxFwdWaves * kWave)
+__global__ void __launch_bounds__(kVoxFwdWaves * kWave) __attribute__((amdgpu_waves_per_eu(4)))
 vox_fwd_fused_kernel(VoxArgs<float> A, float* __restrict__ out, float* __restrict__ out_var) {
     constexpr uint32_t T = kMomT;
     using R = VoxRecOf<BETA>;
@@ -734,8 +933,17 @@ vox_fwd_fused_kernel(VoxArgs<float> A, float* __restrict__ out, float* __restric
     const int32_t per = (end - start + kVoxFwdWaves - 1) / kVoxFwdWaves;
     const int32_t lo = min(end, start + int32_t(wave) * per), hi = min(end, lo + per);
     const uint32_t tx = blk % A.ntx, rest = blk / A.ntx, ty = rest % A.nty, tz = rest / A.nty;
-    const uint32_t ly = lane % T, lz = lane / T;
-    const float py = float(ty * T + ly) + 0.5f, pz = float(tz * T + lz) + 0.5f, px0 = float(tx * T) + 0.5f;
+    // a lane's voxels: Gaussian row (0 .. 7, ly, lz); Beta (lx + 4 ox, ly + 4 oy, lz + 4 oz) for octant 4 oz + 2 oy + ox
+    constexpr uint32_t kEdge = BETA ? 4 : T;
+    const uint32_t lx = BETA ? lane % 4 : 0u, ly = BETA ? (lane / 4) % 4 : lane % T, lz = BETA ? lane / 16 : lane / T;
+    const float x0 = float(tx * T), y0 = float(ty * T), z0 = float(tz * T);
+    const float px = x0 + float(lx) + 0.5f, py = y0 + float(ly) + 0.5f, pz = z0 + float(lz) + 0.5f;
+    auto place = [&](uint32_t k) -> uint32_t {  // the tile voxel of accumulator k
+        if constexpr (BETA)
+            return ((lz + kEdge * (k >> 2)) * T + ly + kEdge * ((k >> 1) & 1u)) * T + lx + kEdge * (k & 1u);
+        else
+            return (lz * T + ly) * T + k;
+    };
     float acc[T], acc_var[T];
 #pragma unroll
     for (uint32_t x = 0; x < T; ++x) {
@@ -743,34 +951,50 @@ vox_fwd_fused_kernel(VoxArgs<float> A, float* __restrict__ out, float* __restric
         acc_var[x] = 0.f;
     }
     R* slot = stage[wave];
-    R next = load_vox_rec<BETA>(A, lo + int32_t(lane), hi);
+    R next = load_vox_rec<BETA>(A, lo + int32_t(lane), hi, x0, y0, z0);
     float next_q = VAR ? load_vox_unc(A, lo + int32_t(lane), hi) : 0.f;
     for (int32_t base = lo; base < hi; base += kWave) {
         wave_sync_lds();
         slot[lane] = next;
         if constexpr (VAR) stage_q[wave][lane] = next_q;
         wave_sync_lds();
-        next = load_vox_rec<BETA>(A, base + kWave + int32_t(lane), hi);
+        next = load_vox_rec<BETA>(A, base + kWave + int32_t(lane), hi, x0, y0, z0);
         if constexpr (VAR) next_q = load_vox_unc(A, base + kWave + int32_t(lane), hi);
         const int32_t n = min(int32_t(kWave), hi - base);
         for (int32_t j = 0; j < n; ++j) {
             const R r = slot[j];
-            if (r.qlim == 0u) continue;  // wave-uniform (every lane reads the same record)
             const float unc = VAR ? stage_q[VAR ? wave : 0][j] : 0.f;
-            float ek[T];
+            auto add = [&](uint32_t k, float e) {
+                if constexpr (VAR) {
+                    const float alpha = e * r.w;
+                    acc[k] += alpha;
+                    acc_var[k] = fmaf(unc * alpha, alpha, acc_var[k]);
+                } else {
+                    acc[k] = fmaf(e, r.w, acc[k]);
+                }
+            };
             if constexpr (BETA) {
-                const double dy = double(py) - r.my, dz = double(pz) - r.mz, dx0 = double(px0) - r.mx;
-                const double c1 = fma(r.bxy, dy, r.bxz * dz);
-                const double c0 = fma(dy, fma(r.cyy, dy, r.cyz * dz), r.czz * dz * dz);
+                const uint32_t octants = __builtin_amdgcn_readfirstlane(r.octants);  // every lane reads the same record
+                if (octants == 0u) continue;
+                const double dx0 = double(px) - r.mx, dy0 = double(py) - r.my, dz0 = double(pz) - r.mz;
 #pragma unroll
-                for (uint32_t x = 0; x < T; ++x) {
-                    const double dx = dx0 + double(x);
-                    const double q = fma(dx, fma(r.a, dx, c1), c0);
-                    const float e = __builtin_amdgcn_exp2f(r.beta * __log2f(float(1.0 - q)));
-                    ek[x] = (q >= 0.0 && q <= r.qmax) ? e : 0.f;
+                for (uint32_t o = 0; o < 8; o += 2) {
+                    if (((octants >> o) & 3u) == 0u) continue;
+                    const double dy = (o & 2u) ? dy0 + 4.0 : dy0, dz = (o & 4u) ? dz0 + 4.0 : dz0;
+                    const double c1 = fma(r.bxy, dy, r.bxz * dz);
+                    const double c0 = fma(dy, fma(r.cyy, dy, r.cyz * dz), r.czz * dz * dz);
+#pragma unroll
+                    for (uint32_t ox = 0; ox < 2; ++ox) {
+                        if (!((octants >> (o + ox)) & 1u)) continue;
+                        const double dx = ox ? dx0 + 4.0 : dx0;
+                        const double q = fma(dx, fma(r.a, dx, c1), c0);
+                        const float e = __builtin_amdgcn_exp2f(r.beta * __log2f(float(1.0 - q)));
+                        add(o + ox, (q >= 0.0 && q <= r.qmax) ? e : 0.f);
+                    }
                 }
             } else {
-                const float dy = (py - r.my) - r.ly, dz = (pz - r.mz) - r.lz, dx0 = (px0 - r.mx) - r.lx;
+                if (r.qlim == 0u) continue;  // wave-uniform
+                const float dy = (py - r.my) - r.ly, dz = (pz - r.mz) - r.lz, dx0 = (px - r.mx) - r.lx;
                 const float c1 = fmaf(r.bxy, dy, r.bxz * dz);
                 const float c0 = fmaf(dy, fmaf(r.cyy, dy, r.cyz * dz), r.czz * dz * dz);
 #pragma unroll
@@ -778,23 +1002,13 @@ vox_fwd_fused_kernel(VoxArgs<float> A, float* __restrict__ out, float* __restric
                     const float dx = dx0 + float(x);
                     const float q = fmaf(dx, fmaf(r.a, dx, c1), c0);
                     const float e = __builtin_amdgcn_exp2f(-q);
-                    ek[x] = __float_as_uint(q) < r.qlim ? e : 0.f;
-                }
-            }
-#pragma unroll
-            for (uint32_t x = 0; x < T; ++x) {
-                if constexpr (VAR) {
-                    const float alpha = ek[x] * r.w;
-                    acc[x] += alpha;
-                    acc_var[x] = fmaf(unc * alpha, alpha, acc_var[x]);
-                } else {
-                    acc[x] = fmaf(ek[x], r.w, acc[x]);
+                    add(x, __float_as_uint(q) < r.qlim ? e : 0.f);
                 }
             }
         }
     }
 #pragma unroll
-    for (uint32_t x = 0; x < T; ++x) part[wave][(lz * T + ly) * T + x] = acc[x];
+    for (uint32_t x = 0; x < T; ++x) part[wave][place(x)] = acc[x];
     __syncthreads();
     for (uint32_t p = threadIdx.x; p < T * T * T; p += blockDim.x) {
         float v = 0.f;
@@ -806,7 +1020,7 @@ vox_fwd_fused_kernel(VoxArgs<float> A, float* __restrict__ out, float* __restric
     if constexpr (VAR) {
         __syncthreads();  // the mean's partial volumes are consumed
 #pragma unroll
-        for (uint32_t x = 0; x < T; ++x) part[wave][(lz * T + ly) * T + x] = acc_var[x];
+        for (uint32_t x = 0; x < T; ++x) part[wave][place(x)] = acc_var[x];
         __syncthreads();
         for (uint32_t p = threadIdx.x; p < T * T * T; p += blockDim.x) {
             float v = 0.f;
@@ -818,30 +1032,66 @@ vox_fwd_fused_kernel(VoxArgs<float> A, float* __restrict__ out, float* __restric
     }
 }
 
-// Per-primitive sums of the intersection partials [cum[n], cum[n+1]) in
-// emission order (deterministic; no atomics).
-__global__ void __launch_bounds__(256)
+// Per-primitive sums of the intersection partials [cum[n], cum[n+1]) in a fixed
+// order (deterministic; no atomics): 16 lanes per primitive, lane 4 p + c adding
+// float4 c (of three) of the partials p, p + 4, .. in order, then the four
+// phases pairwise. (One lane per primitive read its partials one after another:
+// 65 us for 2.9M partials of 100k primitives, now 24, and 21 us for 285k of 3k,
+// now 5.)
+constexpr uint32_t kReduceLanes = 16, kReduceThreads = 256;
+
+__global__ void __launch_bounds__(kReduceThreads)
 vox_partials_reduce_kernel(const uint32_t* __restrict__ cum, const float* __restrict__ partials, uint32_t N,
                            uint32_t n_isects, float* __restrict__ v_xyz, float* __restrict__ v_c,
                            float* __restrict__ v_opac, float* __restrict__ v_beta, float* __restrict__ v_unc) {
-    const uint32_t n = blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= N) return;
-    float acc[12] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    const uint32_t lo = min(cum[n], n_isects), hi = min(cum[n + 1], n_isects);
-    for (uint32_t j = lo; j < hi; ++j) {
-        const float4* p = reinterpret_cast<const float4*>(partials + kVoxPartial * size_t(j));
-        const float4 a = p[0], b = p[1], c = p[2];
-        acc[0] += a.x; acc[1] += a.y; acc[2] += a.z; acc[3] += a.w;
-        acc[4] += b.x; acc[5] += b.y; acc[6] += b.z; acc[7] += b.w;
-        acc[8] += c.x; acc[9] += c.y; acc[10] += c.z; acc[11] += c.w;
+    constexpr uint32_t kBatch = 4, kGroups = kReduceThreads / kReduceLanes;  // loads in flight; primitives per round
+    const uint32_t column = threadIdx.x % 4, phase = (threadIdx.x % kReduceLanes) / 4;
+    const float4* part = reinterpret_cast<const float4*>(partials);
+    static_assert(kVoxPartial == 12, "a partial is three float4");
+    for (uint32_t n0 = blockIdx.x * kGroups; n0 < N; n0 += gridDim.x * kGroups) {
+        const uint32_t n = n0 + threadIdx.x / kReduceLanes;
+        float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (n < N && column < 3) {
+            const uint32_t lo = min(cum[n], n_isects), hi = min(cum[n + 1], n_isects);
+            for (uint32_t j = lo + phase; j < hi; j += 4 * kBatch) {
+                float4 p[kBatch];
+#pragma unroll
+                for (uint32_t k = 0; k < kBatch; ++k)
+                    p[k] = j + 4 * k < hi ? part[3 * size_t(j + 4 * k) + column] : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+                for (uint32_t k = 0; k < kBatch; ++k) {
+                    acc.x += p[k].x;
+                    acc.y += p[k].y;
+                    acc.z += p[k].z;
+                    acc.w += p[k].w;
+                }
+            }
+        }
+#pragma unroll
+        for (int off = 4; off < int(kReduceLanes); off *= 2) {
+            acc.x += __shfl_xor(acc.x, off, kWave);
+            acc.y += __shfl_xor(acc.y, off, kWave);
+            acc.z += __shfl_xor(acc.z, off, kWave);
+            acc.w += __shfl_xor(acc.w, off, kWave);
+        }
+        if (n >= N || phase != 0) continue;
+        if (column == 0) {  // v_mean, v_conic xx
+            v_xyz[3 * size_t(n)] = acc.x;
+            v_xyz[3 * size_t(n) + 1] = acc.y;
+            v_xyz[3 * size_t(n) + 2] = acc.z;
+            v_c[6 * size_t(n)] = acc.w;
+        } else if (column == 1) {  // v_conic xy, xz, yy, yz
+            v_c[6 * size_t(n) + 1] = acc.x;
+            v_c[6 * size_t(n) + 2] = acc.y;
+            v_c[6 * size_t(n) + 3] = acc.z;
+            v_c[6 * size_t(n) + 4] = acc.w;
+        } else if (column == 2) {  // v_conic zz, v_opac, v_beta, v_q
+            v_c[6 * size_t(n) + 5] = acc.x;
+            v_opac[n] = acc.y;
+            if (v_beta) v_beta[n] = acc.z;
+            if (v_unc) v_unc[n] = acc.w;
+        }
     }
-#pragma unroll
-    for (int k = 0; k < 3; ++k) v_xyz[3 * size_t(n) + k] = acc[k];
-#pragma unroll
-    for (int k = 0; k < 6; ++k) v_c[6 * size_t(n) + k] = acc[3 + k];
-    v_opac[n] = acc[9];
-    if (v_beta) v_beta[n] = acc[10];
-    if (v_unc) v_unc[n] = acc[11];
 }
 
 inline int check_vox_tile(uint32_t T, uint32_t ntx, uint32_t nty, uint32_t ntz, uint32_t dx,
@@ -956,8 +1206,12 @@ extern "C" int r2s_voxelize_to_voxels_bwd_per_gaussian(
         if constexpr (std::is_same<S, float>::value) {
             const uint64_t n_tiles = uint64_t(n_tiles_x) * n_tiles_y * n_tiles_z;
             if (tile_size == kMomT && !v_render_var && n_tiles < (1ull << 31)) {  // moments form
-                auto km = beta ? vox_bwd_moments_kernel<true, false> : vox_bwd_moments_kernel<false, false>;
-                km<<<ceil_div(n_isects, kMomThreads), kMomThreads, 0, stream>>>(
+                const bool few = n_isects <= kMomFew;
+                auto km = beta ? (few ? vox_bwd_moments_kernel<256, true, false, false>
+                                      : vox_bwd_moments_kernel<512, true, false, false>)
+                               : (few ? vox_bwd_moments_kernel<256, false, false, false>
+                                      : vox_bwd_moments_kernel<512, false, false, false>);
+                km<<<ceil_div(n_isects, few ? 256 : 512), kMomThreads, 0, stream>>>(
                     A, isect_ids, (const float*)v_render, nullptr, 0.f, (float*)v_means3d, (float*)v_conics,
                     (float*)v_opacities, (float*)v_betas, nullptr, nullptr, nullptr);
                 return check_launch("voxelize_to_voxels_bwd_per_gaussian");
@@ -1011,16 +1265,23 @@ extern "C" int r2s_voxelize_fused_vjp(const float* means3d, const double* frame,
         auto A = make_vox_args<float>(means3d, conics, opacities, betas, uncertainties, nullptr, flatten_ids,
                                       n_isects, N, dim_x, dim_y, dim_z, tile_size, n_tiles_x, n_tiles_y, n_tiles_z);
         A.frame = frame;
-        auto km = beta ? (var ? vox_bwd_moments_kernel<true, true, true> : vox_bwd_moments_kernel<true, false, true>)
-                       : (var ? vox_bwd_moments_kernel<false, true> : vox_bwd_moments_kernel<false, false>);
-        km<<<ceil_div(n_isects, kMomThreads), kMomThreads, 0, stream>>>(
+        const bool few = n_isects <= kMomFew;
+        auto km = beta ? (var ? (few ? vox_bwd_moments_kernel<256, true, true, true>
+                                     : vox_bwd_moments_kernel<512, true, true, true>)
+                              : (few ? vox_bwd_moments_kernel<256, true, false, true>
+                                     : vox_bwd_moments_kernel<512, true, false, true>))
+                       : (var ? (few ? vox_bwd_moments_kernel<256, false, true, false>
+                                     : vox_bwd_moments_kernel<512, false, true, false>)
+                              : (few ? vox_bwd_moments_kernel<256, false, false, false>
+                                     : vox_bwd_moments_kernel<512, false, false, false>));
+        km<<<ceil_div(n_isects, few ? 256 : 512), kMomThreads, 0, stream>>>(
             A, isect_ids, v_render, v_render_var, detach ? 0.f : 2.f, nullptr, nullptr, nullptr, nullptr, radii,
             tile_cum, partials);
         if (int rc = check_launch("voxelize_fused_vjp")) return rc;
     }
-    vox_partials_reduce_kernel<<<ceil_div(N, 256), 256, 0, stream>>>(tile_cum, partials, N, n_isects, v_means3d,
-                                                                     v_conics, v_opacities, beta ? v_betas : nullptr,
-                                                                     var ? v_uncertainties : nullptr);
+    vox_partials_reduce_kernel<<<std::min(ceil_div(N, kReduceThreads / kReduceLanes), 1u << 22), kReduceThreads, 0,
+                                 stream>>>(tile_cum, partials, N, n_isects, v_means3d, v_conics, v_opacities,
+                                           beta ? v_betas : nullptr, var ? v_uncertainties : nullptr);
     return check_launch("voxelize_fused_vjp_reduce");
 }
 

@@ -48,15 +48,16 @@ int scan_exclusive(const uint32_t* in, uint32_t n, uint32_t* out, uint32_t* d_to
                    hipStream_t stream);
 
 // The sort's threads per workgroup and digits per pass, and the keys of a
-// workgroup (its radix tile) when n are sorted: 4096 from 2^20 keys on; below
-// that a launch of 4096-key tiles has fewer workgroups than the GPU has compute
-// units and takes as long as one workgroup's 16 rounds (15 us at 30k keys), so
-// the tiles are smaller (1024: 6 us), with 2048 where that keeps the histogram
-// within the one-launch scan.
+// workgroup (its radix tile) when n are sorted. A launch of few workgroups takes
+// as long as one workgroup's rounds (4096 keys 15 us, 1024 keys 6 us at 30k), so
+// the tiles are the smallest whose histogram is scanned in one launch (64 tiles)
+// up to 2^18 keys; past that the scan takes three launches anyway, and 1024-key
+// tiles are kept until there are enough of 4096 to fill the GPU.
 constexpr uint32_t kRadixThreads = 256, kRadixDigits = 256;
 inline uint32_t radix_tile(uint64_t n) {
     if (n > (1u << 20)) return 4096;
-    return n > (1u << 16) && n <= (1u << 17) ? 2048 : 1024;
+    if (n > (1u << 18) || n <= (1u << 16)) return 1024;
+    return n <= (1u << 17) ? 2048 : 4096;
 }
 
 size_t sort_workspace_bytes(uint64_t n);

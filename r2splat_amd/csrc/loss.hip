@@ -13,24 +13,26 @@ namespace r2s {
 // a row (16-byte loads; VEC = 1 where a row's length or a pointer is not a
 // multiple of 16 bytes), and what bounds them is memory traffic as long as
 // three things stay small, each of which the first form of these kernels paid
-// for: the sums end in one atomic per workgroup, and same-address atomics
-// retire one every 12.7 ns, so the grid is capped (65536 workgroups took 833
-// us for a 256^3 float volume, the capped one 24 us, 5.6 TB/s); row and plane
+// for: the sums end in one partial per workgroup (or, without a buffer for
+// them, one atomic: same-address atomics retire one every 12.7 ns), so the grid
+// is capped (65536 workgroups took 833 us for a 256^3 float volume, the capped
+// one 24 us, 5.6 TB/s); row and plane
 // indices come from 32-bit divisions per VEC elements instead of 64-bit ones
 // per element (anisotropic gradient 91 -> 30 us); and the isotropic gradient
 // marches along z, so that a voxel costs 2.25 square roots instead of four
 // (126 -> 66 us, bound by the correctly rounded square roots and divisions).
 constexpr int kLossThreads = 256;
 constexpr int kSumThreads = 1024;
-constexpr uint32_t kSumBlocks = 512;  // two per CU: at most 512 same-address atomics (6.5 us)
+constexpr uint32_t kSumBlocks = 512;  // two per CU
 constexpr uint32_t kMarch = 8;        // planes per thread of the isotropic gradient
 
 template <typename S>
 __device__ __forceinline__ S sgn(S x) { return x > S(0) ? S(1) : (x < S(0) ? S(-1) : S(0)); }
 
-// Block sum of one value per thread (in double), then one atomic per block.
+// Block sum of one value per thread (in double): the block's entry of `partials`
+// (summed in order by loss_total_kernel), or without them one atomic per block.
 template <typename S>
-__device__ __forceinline__ void block_sum_atomic(S v, S* out) {
+__device__ __forceinline__ void block_sum(S v, S* out, double* partials) {
     __shared__ double part[kSumThreads / kWave];
     const double w = wave_sum(double(v));
     if (lane_id() == 0) part[threadIdx.x / kWave] = w;
@@ -38,7 +40,23 @@ __device__ __forceinline__ void block_sum_atomic(S v, S* out) {
     if (threadIdx.x == 0) {
         double t = 0.0;
         for (int k = 0; k < kSumThreads / kWave; ++k) t += part[k];
-        atomic_add(out, S(t));
+        if (partials) partials[blockIdx.x] = t;
+        else atomic_add(out, S(t));
+    }
+}
+
+// *out = the sum of m <= kSumBlocks partials, in double and a fixed order.
+template <typename S>
+__global__ void __launch_bounds__(kSumBlocks)
+loss_total_kernel(const double* __restrict__ partials, uint32_t m, S* __restrict__ out) {
+    __shared__ double part[kSumBlocks / kWave];
+    const double w = wave_sum(threadIdx.x < m ? partials[threadIdx.x] : 0.0);
+    if (lane_id() == 0) part[threadIdx.x / kWave] = w;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double t = 0.0;
+        for (uint32_t k = 0; k < kSumBlocks / kWave; ++k) t += part[k];
+        *out = S(t);
     }
 }
 
@@ -96,7 +114,8 @@ __device__ __forceinline__ void differences(const Pack<S, VEC>& c, const Pack<S,
 // sqrt(dz^2 + dy^2 + dx^2 + eps), with forward differences.
 template <typename S, typename I, int VEC, bool ISO>
 __global__ void __launch_bounds__(kSumThreads)
-tv_fwd_kernel(const S* __restrict__ vol, Volume<I> g, S eps, S* __restrict__ tv_map, S* __restrict__ tv_sum) {
+tv_fwd_kernel(const S* __restrict__ vol, Volume<I> g, S eps, S* __restrict__ tv_map, S* __restrict__ tv_sum,
+              double* __restrict__ partials) {
     S sum = S(0);
     const size_t sd = size_t(g.H) * g.W, sh = g.W;
     for (I i = I(blockIdx.x) * kSumThreads + threadIdx.x; i < g.total; i += I(gridDim.x) * kSumThreads) {
@@ -118,7 +137,7 @@ tv_fwd_kernel(const S* __restrict__ vol, Volume<I> g, S eps, S* __restrict__ tv_
         }
         store_pack<S, VEC>(tv_map + o, t);
     }
-    block_sum_atomic(sum, tv_sum);
+    block_sum(sum, tv_sum, partials);
 }
 
 // grad = ((sign sum) * (g / edges)) * lambda: the reference's rounding order
@@ -241,7 +260,7 @@ tv_iso_bwd_kernel(const S* __restrict__ vol, const S* __restrict__ grad_out, Vol
 template <typename S, int VEC>
 __global__ void __launch_bounds__(kSumThreads)
 l1_fwd_kernel(const S* __restrict__ p, const S* __restrict__ t, uint64_t n, S* __restrict__ map,
-              S* __restrict__ sum) {
+              S* __restrict__ sum, double* __restrict__ partials) {
     S s = S(0);
     for (uint64_t i = uint64_t(blockIdx.x) * kSumThreads + threadIdx.x; i < n / VEC;
          i += uint64_t(gridDim.x) * kSumThreads) {
@@ -254,7 +273,7 @@ l1_fwd_kernel(const S* __restrict__ p, const S* __restrict__ t, uint64_t n, S* _
         }
         store_pack<S, VEC>(map + i * VEC, m);
     }
-    block_sum_atomic(s, sum);
+    block_sum(s, sum, partials);
 }
 
 template <typename S>
@@ -292,16 +311,52 @@ static int with_packs(uint64_t rows, uint32_t W, const void* a, const void* b, F
     return f(uint64_t{}, std::integral_constant<int, 1>{});
 }
 
-template <typename S, bool ISO>
-static int launch_tv_fwd(const S* vol, uint32_t B, uint32_t D, uint32_t H, uint32_t W, S eps, S* map, S* sum,
-                         hipStream_t stream, const char* where) {
+// The sum of a loss forward: cleared for atomics, or finished from `blocks` partials.
+template <typename S>
+static int begin_sum(S* sum, double* partials, uint64_t total, hipStream_t stream) {
+    return partials && total ? R2S_OK : fill_zero<S>(sum, 1, stream);
+}
+template <typename S>
+static int end_sum(S* sum, const double* partials, uint32_t blocks, hipStream_t stream, const char* where) {
+    if (partials) loss_total_kernel<S><<<1, kSumBlocks, 0, stream>>>(partials, blocks, sum);
+    return check_launch(where);
+}
+
+static int tv_fwd(int dtype, bool iso, const void* volume, uint32_t B, uint32_t D, uint32_t H, uint32_t W, double eps,
+                  void* tv_map, void* tv_sum, double* partials, hipStream_t stream, const char* where) {
     const uint64_t rows = uint64_t(B) * D * H;
-    return with_packs<S>(rows, W, vol, map, [&](auto index, auto vec) {
-        using I = decltype(index);
-        constexpr int VEC = decltype(vec)::value;
-        const Volume<I> g{I(W / VEC), I(rows * (W / VEC)), D, H, W};
-        tv_fwd_kernel<S, I, VEC, ISO><<<sum_blocks(g.total), kSumThreads, 0, stream>>>(vol, g, eps, map, sum);
-        return check_launch(where);
+    return dispatch_dtype(dtype, [&](auto tag) {
+        using S = decltype(tag);
+        const S* vol = (const S*)volume;
+        if (int rc = begin_sum<S>((S*)tv_sum, partials, rows * W, stream)) return rc;
+        if (rows * W == 0) return R2S_OK;
+        return with_packs<S>(rows, W, volume, tv_map, [&](auto index, auto vec) {
+            using I = decltype(index);
+            constexpr int VEC = decltype(vec)::value;
+            const Volume<I> g{I(W / VEC), I(rows * (W / VEC)), D, H, W};
+            const uint32_t blocks = sum_blocks(g.total);
+            auto k = iso ? tv_fwd_kernel<S, I, VEC, true> : tv_fwd_kernel<S, I, VEC, false>;
+            k<<<blocks, kSumThreads, 0, stream>>>(vol, g, S(eps), (S*)tv_map, (S*)tv_sum, partials);
+            if (int rc = check_launch(where)) return rc;
+            return end_sum<S>((S*)tv_sum, partials, blocks, stream, where);
+        });
+    });
+}
+
+static int l1_fwd(int dtype, const void* prediction, const void* target, uint64_t n, void* l1_map, void* l1_sum,
+                  double* partials, hipStream_t stream) {
+    return dispatch_dtype(dtype, [&](auto tag) {
+        using S = decltype(tag);
+        constexpr int kWide = 16 / int(sizeof(S));
+        if (int rc = begin_sum<S>((S*)l1_sum, partials, n, stream)) return rc;
+        if (n == 0) return R2S_OK;
+        const bool wide = packed16<S>(n, prediction, target, l1_map);
+        const uint32_t blocks = sum_blocks(wide ? n / kWide : n);
+        auto k = wide ? l1_fwd_kernel<S, kWide> : l1_fwd_kernel<S, 1>;
+        k<<<blocks, kSumThreads, 0, stream>>>((const S*)prediction, (const S*)target, n, (S*)l1_map, (S*)l1_sum,
+                                              partials);
+        if (int rc = check_launch("image_l1_fwd")) return rc;
+        return end_sum<S>((S*)l1_sum, partials, blocks, stream, "image_l1_fwd");
     });
 }
 
@@ -311,14 +366,7 @@ using namespace r2s;
 
 extern "C" int r2s_volume_tv_fwd(int dtype, const void* volume, uint32_t B, uint32_t D, uint32_t H,
                                  uint32_t W, void* tv_map, void* tv_sum, r2s_stream_t stream) {
-    const size_t total = size_t(B) * D * H * W;
-    return dispatch_dtype(dtype, [&](auto tag) {
-        using S = decltype(tag);
-        if (int rc = fill_zero<S>((S*)tv_sum, 1, stream)) return rc;
-        if (total == 0) return R2S_OK;
-        return launch_tv_fwd<S, false>((const S*)volume, B, D, H, W, S(0), (S*)tv_map, (S*)tv_sum, stream,
-                                       "volume_tv_fwd");
-    });
+    return tv_fwd(dtype, false, volume, B, D, H, W, 0.0, tv_map, tv_sum, nullptr, stream, "volume_tv_fwd");
 }
 
 extern "C" int r2s_volume_tv_bwd(int dtype, const void* volume, const void* grad_output, uint32_t B,
@@ -346,14 +394,7 @@ extern "C" int r2s_volume_tv_bwd(int dtype, const void* volume, const void* grad
 extern "C" int r2s_volume_tv_iso_fwd(int dtype, const void* volume, uint32_t B, uint32_t D, uint32_t H,
                                      uint32_t W, double eps, void* tv_map, void* tv_sum, r2s_stream_t stream) {
     R2S_REQUIRE(eps > 0.0, "isotropic TV needs eps > 0 (got %g)", eps);
-    const size_t total = size_t(B) * D * H * W;
-    return dispatch_dtype(dtype, [&](auto tag) {
-        using S = decltype(tag);
-        if (int rc = fill_zero<S>((S*)tv_sum, 1, stream)) return rc;
-        if (total == 0) return R2S_OK;
-        return launch_tv_fwd<S, true>((const S*)volume, B, D, H, W, S(eps), (S*)tv_map, (S*)tv_sum, stream,
-                                      "volume_tv_iso_fwd");
-    });
+    return tv_fwd(dtype, true, volume, B, D, H, W, eps, tv_map, tv_sum, nullptr, stream, "volume_tv_iso_fwd");
 }
 
 extern "C" int r2s_volume_tv_iso_bwd(int dtype, const void* volume, const void* grad_output, uint32_t B,
@@ -380,19 +421,7 @@ extern "C" int r2s_volume_tv_iso_bwd(int dtype, const void* volume, const void* 
 
 extern "C" int r2s_image_l1_fwd(int dtype, const void* prediction, const void* target, uint64_t n,
                                 void* l1_map, void* l1_sum, r2s_stream_t stream) {
-    return dispatch_dtype(dtype, [&](auto tag) {
-        using S = decltype(tag);
-        if (int rc = fill_zero<S>((S*)l1_sum, 1, stream)) return rc;
-        if (n == 0) return R2S_OK;
-        constexpr int kWide = 16 / int(sizeof(S));
-        if (packed16<S>(n, prediction, target, l1_map))
-            l1_fwd_kernel<S, kWide><<<sum_blocks(n / kWide), kSumThreads, 0, stream>>>(
-                (const S*)prediction, (const S*)target, n, (S*)l1_map, (S*)l1_sum);
-        else
-            l1_fwd_kernel<S, 1><<<sum_blocks(n), kSumThreads, 0, stream>>>(
-                (const S*)prediction, (const S*)target, n, (S*)l1_map, (S*)l1_sum);
-        return check_launch("image_l1_fwd");
-    });
+    return l1_fwd(dtype, prediction, target, n, l1_map, l1_sum, nullptr, stream);
 }
 
 extern "C" int r2s_image_l1_bwd(int dtype, const void* prediction, const void* target,
@@ -406,4 +435,21 @@ extern "C" int r2s_image_l1_bwd(int dtype, const void* prediction, const void* t
             (S*)grad_prediction);
         return check_launch("image_l1_bwd");
     });
+}
+
+extern "C" size_t r2s_loss_partials_bytes(void) { return kSumBlocks * sizeof(double); }
+
+extern "C" int r2s_volume_tv_fwd_ordered(int dtype, int isotropic, const void* volume, uint32_t B, uint32_t D,
+                                         uint32_t H, uint32_t W, double eps, void* tv_map, void* tv_sum,
+                                         void* partials, r2s_stream_t stream) {
+    R2S_REQUIRE(partials != nullptr, "volume_tv_fwd_ordered: partials is null");
+    R2S_REQUIRE(!isotropic || eps > 0.0, "isotropic TV needs eps > 0 (got %g)", eps);
+    return tv_fwd(dtype, isotropic != 0, volume, B, D, H, W, eps, tv_map, tv_sum, static_cast<double*>(partials),
+                  stream, "volume_tv_fwd_ordered");
+}
+
+extern "C" int r2s_image_l1_fwd_ordered(int dtype, const void* prediction, const void* target, uint64_t n,
+                                        void* l1_map, void* l1_sum, void* partials, r2s_stream_t stream) {
+    R2S_REQUIRE(partials != nullptr, "image_l1_fwd_ordered: partials is null");
+    return l1_fwd(dtype, prediction, target, n, l1_map, l1_sum, static_cast<double*>(partials), stream);
 }

@@ -110,6 +110,9 @@ SIGNATURES = {
     "r2s_volume_tv_iso_bwd": [I32, P, P, U32, U32, U32, U32, D, D, P, P],
     "r2s_image_l1_fwd": [I32, P, P, U64, P, P, P],
     "r2s_image_l1_bwd": [I32, P, P, P, U64, F, P, P],
+    "r2s_loss_partials_bytes": [],
+    "r2s_volume_tv_fwd_ordered": [I32, I32, P, U32, U32, U32, U32, D, P, P, P, P],
+    "r2s_image_l1_fwd_ordered": [I32, P, P, U64, P, P, P, P],
 }
 
 _RESTYPES = {
@@ -122,6 +125,7 @@ _RESTYPES = {
     "r2s_fused_param_workspace_bytes": SZ,
     "r2s_voxel_partials_bytes": SZ,
     "r2s_mse_partials": SZ,
+    "r2s_loss_partials_bytes": SZ,
 }
 
 

@@ -694,6 +694,10 @@ def _f32(x) -> float:
     return struct.unpack("f", struct.pack("f", float(x)))[0]
 
 
+def _loss_partials(device) -> Tensor:
+    return torch.empty((be.lib().r2s_loss_partials_bytes(),), dtype=torch.uint8, device=device)
+
+
 def volume_loss_fwd(volume, lambda_tv):
     """Anisotropic TV over (B,D,H,W) -> (lambda * tv, tv, tv_map)."""
     _check("volume", volume, 4)
@@ -702,7 +706,9 @@ def volume_loss_fwd(volume, lambda_tv):
     tv_map = torch.empty_like(volume)
     tv_sum = volume.new_empty((1,))
     with _Launch(volume) as L:
-        call("r2s_volume_tv_fwd", dt, ptr(volume), B, Dd, H, W, ptr(tv_map), ptr(tv_sum), L.stream)
+        partials = _loss_partials(volume.device)
+        call("r2s_volume_tv_fwd_ordered", dt, 0, ptr(volume), B, Dd, H, W, 0.0, ptr(tv_map), ptr(tv_sum), ptr(partials),
+             L.stream)
     edges = max(B * ((Dd - 1) * H * W + Dd * (H - 1) * W + Dd * H * (W - 1)), 1)
     # the reference divides by float(edge_count) and scales by a float lambda (Loss.cpp:115-153)
     tv = (tv_sum / _f32(edges)).squeeze()
@@ -735,7 +741,9 @@ def volume_loss_iso_fwd(volume, lambda_tv, eps=1e-8):
     tv_map = torch.empty_like(volume)
     tv_sum = volume.new_empty((1,))
     with _Launch(volume) as L:
-        call("r2s_volume_tv_iso_fwd", dt, ptr(volume), B, Dd, H, W, float(eps), ptr(tv_map), ptr(tv_sum), L.stream)
+        partials = _loss_partials(volume.device)
+        call("r2s_volume_tv_fwd_ordered", dt, 1, ptr(volume), B, Dd, H, W, float(eps), ptr(tv_map), ptr(tv_sum),
+             ptr(partials), L.stream)
     tv = (tv_sum / max(volume.numel(), 1)).squeeze()
     return (float(lambda_tv) * tv), tv, tv_map
 
@@ -766,8 +774,9 @@ def image_loss_l1_fwd(prediction, target, lambda_l1):
     l1_map = torch.empty_like(prediction)
     l1_sum = prediction.new_empty((1,))
     with _Launch(prediction) as L:
-        call("r2s_image_l1_fwd", dt, ptr(prediction), ptr(target), prediction.numel(), ptr(l1_map), ptr(l1_sum),
-             L.stream)
+        partials = _loss_partials(prediction.device)
+        call("r2s_image_l1_fwd_ordered", dt, ptr(prediction), ptr(target), prediction.numel(), ptr(l1_map),
+             ptr(l1_sum), ptr(partials), L.stream)
     l1 = (l1_sum / max(prediction.numel(), 1)).squeeze()
     return _f32(lambda_l1) * l1, l1, l1_map
 

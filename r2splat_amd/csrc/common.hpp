@@ -61,6 +61,7 @@ template <> struct Math<float> {
     static __device__ __forceinline__ float log(float x) { return __logf(x); }
     static __device__ __forceinline__ float pow(float b, float e) { return __expf(e * __logf(b)); }
     static __device__ __forceinline__ float sqrt(float x) { return sqrtf(x); }
+    static __device__ __forceinline__ float fma(float a, float b, float c) { return fmaf(a, b, c); }
 };
 
 template <> struct Math<double> {
@@ -68,6 +69,7 @@ template <> struct Math<double> {
     static __device__ __forceinline__ double log(double x) { return ::log(x); }
     static __device__ __forceinline__ double pow(double b, double e) { return ::pow(b, e); }
     static __device__ __forceinline__ double sqrt(double x) { return ::sqrt(x); }
+    static __device__ __forceinline__ double fma(double a, double b, double c) { return ::fma(a, b, c); }
 };
 
 // Type-dispatch helper for the C-ABI dtype code.

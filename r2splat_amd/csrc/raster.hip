@@ -2,17 +2,23 @@
 // primitives binned to its tile (additive line integrals, no compositing).
 //
 // Operator-level kernels for every tile size and both float/double:
-//  * tile-parallel forward (mean, mean+variance), staging the tile's primitive
-//    list through LDS in batches;
+//  * tile-parallel forward (mean, mean+variance): tiles of 8, 16 and 32 pixels
+//    share their list over several waves and skip the rows a primitive does not
+//    reach; other sizes stage the list through LDS in batches, a pixel per thread;
 //  * tile-parallel ("pixel" mode) VJP and the uncertainty VJP: one wave64
 //    reduction per (wave, primitive) followed by one atomic per field;
-//  * intersection-parallel ("primitive" mode) VJP: one wave64 per
-//    intersection, lanes stride the tile's pixels, one atomic per field.
+//  * intersection-parallel ("primitive" mode) VJP: tiles of 8, 16 and 32 pixels
+//    one lane per intersection, walking the rows it reaches; other sizes and
+//    absolute gradients one wave64 per intersection, lanes striding the tile's
+//    pixels; one atomic per field.
 // Profiles follow r2splat/cuda/csrc/RasterizeToPixelsFwd.cu:155-180 (Gaussian)
 // and :664-680 (Beta), and the VJPs RasterizeToPixelsBwd.cu:169-265,421-501,
 // 674-706,909-945.
 #include "common.hpp"
 #include "raster_common.hpp"
+#include "sorted_chunk.hpp"
+
+#include <type_traits>
 
 namespace r2s {
 
@@ -234,6 +240,314 @@ raster_bwd_isect_kernel(RasterArgs<S> A, const int64_t* __restrict__ isect_ids,
 }
 
 // ---------------------------------------------------------------------------
+// Tiles of T = 8, 16 and 32 pixels: forward and per-intersection VJP that
+// evaluate only the rows of a tile a primitive can reach. In double precision
+// the exponential (and, for Beta primitives, the power) is most of a pair's
+// cost, so rows outside the footprint are what there is to save: 20k Gaussians
+// on 8 views of 128^2 touch 9.8 of 16 rows per tile. A pixel per thread over
+// the whole list took 688 us there (four waves a tile, two a SIMD), a wave per
+// intersection with its nine wave reductions 494 us; these take 206 and 157. What
+// bounds them is double arithmetic in the few tiles that the object covers.
+// ---------------------------------------------------------------------------
+// Rows [lo, hi) of a T-row tile (first pixel centre at row y_base + 1/2) in which
+// |alpha| can reach 1e-5: dy^2 <= 4 A S / (4 A C - B^2) for the form A dx^2 + B dx
+// dy + C dy^2 <= S, widened by 1e-3 and 0.05 px (the bound is formed in float).
+// Forms that are flat, not positive definite or not finite get every row; only a
+// weight surely below the cut-off gets none.
+template <typename S, bool BETA>
+__device__ __forceinline__ void reached_rows(const Prim2D<S>& p, S y_base, int T, int& lo, int& hi) {
+    lo = 0;
+    hi = T;
+    const float w = fabsf(float(p.opac * p.mu));
+    if (w < 0.999e-5f) {
+        hi = 0;
+        return;
+    }
+    float A, B, C, bound;
+    if (BETA) {
+        A = float(p.a);
+        B = 2.f * float(p.b);
+        C = float(p.c);
+        const float D = 1.f - __builtin_amdgcn_exp2f(__log2f(1e-5f / w) / float(p.beta));
+        bound = p.beta > S(0) ? fminf(1.f, 1.002f * D + 1e-4f) : 1.f;
+    } else {
+        A = 0.5f * float(p.a);
+        B = float(p.b);
+        C = 0.5f * float(p.c);
+        bound = 1.001f * __logf(w * 1e5f) + 1e-4f;
+    }
+    const float ac4 = 4.f * A * C, den = ac4 - B * B;
+    const float e2 = 4.f * A * bound * __builtin_amdgcn_rcpf(den);
+    if (!(A > 0.f) || !(den > 1e-3f * ac4) || !(e2 >= 0.f) || !(e2 < 1e30f)) return;
+    const float ext = __builtin_amdgcn_sqrtf(e2) * 1.001f + 0.05f;
+    const float c = float(p.my - y_base) - 0.5f;
+    if (!(fabsf(c) < 1e9f)) return;
+    lo = int(fminf(fmaxf(ceilf(c - ext), 0.f), float(T)));
+    hi = max(lo, int(fminf(fmaxf(floorf(c + ext) + 1.f, 0.f), float(T))));
+}
+
+// The form at a pixel, from a dx, dx, b dx (twice that for Beta), c and dy, in the
+// roundings eval_profile compiles to: a thin footprint's float32 terms cancel, and any other order would give
+// such a primitive an exponent that differs from the general kernel's.
+template <typename S, bool BETA>
+__device__ __forceinline__ S pair_form(S adx, S dx, S bdx, S c, S dy) {
+    if constexpr (BETA) return Math<S>::fma(c * dy, dy, Math<S>::fma(adx, dx, bdx * dy));
+    return Math<S>::fma(bdx, dy, S(0.5) * Math<S>::fma(adx, dx, c * dy * dy));
+}
+
+template <typename S>
+__device__ __forceinline__ Prim2D<S> load_prim(const RasterArgs<S>& A, int32_t g, bool beta) {
+    Prim2D<S> p;
+    p.mx = A.means2d[2 * size_t(g)];
+    p.my = A.means2d[2 * size_t(g) + 1];
+    p.a = A.conics[3 * size_t(g)];
+    p.b = A.conics[3 * size_t(g) + 1];
+    p.c = A.conics[3 * size_t(g) + 2];
+    p.opac = A.opac[g];
+    p.mu = A.mus[g];
+    p.beta = beta ? A.betas[g] : S(0);
+    return p;
+}
+
+// Forward: WAVES waves share a tile, wave k taking batches k, k + WAVES, ... of 64
+// records; each lane stages one record of a batch in the wave's LDS slot with
+// the row groups it reaches, and the wave reads the records back by broadcast.
+// Lane = column and row group (PX rows STEP apart); groups not reached are
+// skipped by scalar branches. The waves' partial images are summed in wave order.
+// SPLIT: a workgroup renders one row group of a tile (PX workgroups a tile), for
+// launches of few tiles, whose lists are long where the object is: 20k Gaussians
+// on 8 views of 128^2 have 128 tiles that matter, half the compute units.
+template <typename S>
+struct OpRec {
+    S mx, my, a, b, c, w, beta, q;
+};
+
+template <int T, bool SPLIT>
+constexpr int op_waves() { return (T == 32 ? 4 : 8) * (SPLIT ? 2 : 1); }
+
+constexpr uint64_t kSplitTiles = 4096;  // tiles of a launch up to which they are split
+
+template <typename S, int T, bool BETA, bool VAR, bool SPLIT>
+__global__ void __launch_bounds__((op_waves<T, SPLIT>() * kWave))
+raster_fwd_rows_kernel(RasterArgs<S> A, S* __restrict__ out, S* __restrict__ out_var) {
+    constexpr int WAVES = op_waves<T, SPLIT>(), STEP = kWave / T, GROUPS = T * T / kWave, PX = SPLIT ? 1 : GROUPS;
+    constexpr uint32_t kPixels = PX * kWave;
+    __shared__ OpRec<S> stage[WAVES][kWave];
+    __shared__ S part[WAVES][kPixels];
+    uint32_t cam, ty, tx;
+    int32_t start, end;
+    const uint32_t group = SPLIT ? blockIdx.x % GROUPS : 0u, y0 = group * STEP;  // the workgroup's first row
+    tile_range(A, SPLIT ? blockIdx.x / GROUPS : blockIdx.x, cam, ty, tx, start, end);
+    const uint32_t lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const uint32_t col = lane % T, row0 = lane / T;
+    const S px = S(tx * T + col) + S(0.5);
+    S py[PX], acc[PX], acc_var[PX];
+#pragma unroll
+    for (int k = 0; k < PX; ++k) {
+        py[k] = S(ty * T + y0 + row0 + STEP * k) + S(0.5);
+        acc[k] = S(0);
+        acc_var[k] = S(0);
+    }
+    OpRec<S>* slot = stage[wave];
+    for (int32_t base = start + int32_t(wave) * kWave; base < end; base += WAVES * kWave) {
+        uint32_t groups = 0;
+        OpRec<S> r = {};
+        if (base + int32_t(lane) < end) {
+            const int32_t g = A.flatten[base + int32_t(lane)];
+            if (g >= 0 && uint32_t(g) < A.C * A.N) {  // out-of-range ids contribute nothing
+                const Prim2D<S> p = load_prim(A, g, BETA);
+                int lo, hi;
+                reached_rows<S, BETA>(p, S(ty * T), T, lo, hi);
+                const int k_lo = lo / STEP, k_hi = (hi + STEP - 1) / STEP;
+                if (lo < hi) groups = (((1u << k_hi) - 1u) & ~((1u << k_lo) - 1u)) >> group;
+                if constexpr (SPLIT) groups &= 1u;
+                r = OpRec<S>{p.mx, p.my, p.a, p.b, p.c, p.opac * p.mu, p.beta, VAR ? A.unc[uint32_t(g) % A.N] : S(0)};
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();  // every lane is done with the previous batch
+        slot[lane] = r;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        const auto splat = [&](const OpRec<S>& s, uint32_t rows) {
+            const S dx = px - s.mx, adx = s.a * dx, bdx = (BETA ? S(2) : S(1)) * s.b * dx;
+#pragma unroll
+            for (int k = 0; k < PX; ++k) {
+                if (PX > 1 && !((rows >> k) & 1u)) continue;
+                const S dy = py[k] - s.my;
+                S alpha;
+                bool keep;
+                if constexpr (BETA) {
+                    const S q = pair_form<S, BETA>(adx, dx, bdx, s.c, dy);
+                    keep = !(q < S(0) || q >= S(1));
+                    alpha = s.w * (keep ? Math<S>::pow(S(1) - q, s.beta) : S(0));
+                } else {
+                    const S sigma = pair_form<S, BETA>(adx, dx, bdx, s.c, dy);
+                    alpha = s.w * Math<S>::exp(-sigma);
+                    keep = !(sigma < S(0));
+                }
+                if (!keep || fabs(alpha) < S(1e-5)) alpha = S(0);
+                acc[k] += alpha;
+                if constexpr (VAR) acc_var[k] += s.q * alpha * alpha;
+            }
+        };
+        // the batch's records that reach a group, the next one read from LDS while
+        // this one is evaluated (two registers that alternate roles)
+        uint64_t todo = __ballot(groups != 0u);
+        if (todo == 0ull) continue;
+        const auto pop = [&]() -> int {
+            const int j = __builtin_ctzll(todo);
+            todo &= todo - 1ull;
+            return j;
+        };
+        int ja = pop();
+        OpRec<S> a = slot[ja];
+        for (;;) {
+            const bool more_b = todo != 0ull;
+            const int jb = more_b ? pop() : ja;
+            const OpRec<S> b = slot[jb];
+            splat(a, __builtin_amdgcn_readlane(groups, ja));
+            if (!more_b) break;
+            const bool more_a = todo != 0ull;
+            ja = more_a ? pop() : jb;
+            a = slot[ja];
+            splat(b, __builtin_amdgcn_readlane(groups, jb));
+            if (!more_a) break;
+        }
+    }
+#pragma unroll
+    for (int o = 0; o < (VAR ? 2 : 1); ++o) {
+#pragma unroll
+        for (int k = 0; k < PX; ++k) part[wave][(row0 + STEP * k) * T + col] = o ? acc_var[k] : acc[k];
+        __syncthreads();
+        for (uint32_t p = threadIdx.x; p < kPixels; p += WAVES * kWave) {
+            S v = S(0);
+#pragma unroll
+            for (int k = 0; k < WAVES; ++k) v += part[k][p];
+            const uint32_t x = tx * T + p % T, y = ty * T + y0 + p / T;
+            if (x < A.W && y < A.H) (o ? out_var : out)[(size_t(cam) * A.H + y) * A.W + x] = v;
+        }
+        if (VAR && o == 0) __syncthreads();  // the mean's partial images are consumed
+    }
+}
+
+// VJP: one lane per intersection (sorted_chunk: a chunk's tiles staged together,
+// most rows first), summing its moments over the rows it reaches:
+//   Gaussian, delta = pixel - mean, g = v alpha: v_mean = (a Mx + b My, b Mx + c My),
+//     v_conic = -(Mxx / 2, Mxy, Myy / 2), v_opac = mu sum v vis, v_mu = opac sum v vis;
+//   Beta, delta = mean - pixel, G = v vis / h, k = -opac mu beta: v_mean = 2k (a Mx +
+//     b My, b Mx + c My), v_conic = k (Mxx, 2 Mxy, Myy), v_beta = sum v alpha log h.
+template <int T>
+constexpr uint32_t op_tiles() { return T == 8 ? 16 : T == 16 ? 8 : 2; }
+
+template <typename S, int T, uint32_t CHUNK, bool BETA, bool VAR>
+__global__ void __launch_bounds__(kChunkThreads) __attribute__((amdgpu_waves_per_eu(3)))
+raster_bwd_rows_kernel(RasterArgs<S> A, const int64_t* __restrict__ isect_ids, const S* __restrict__ v_render,
+                       const S* __restrict__ v_var, const S* __restrict__ unc, S* __restrict__ v_xy,
+                       S* __restrict__ v_conic, S* __restrict__ v_opac, S* __restrict__ v_mu,
+                       S* __restrict__ v_beta, S* __restrict__ v_q) {
+    constexpr uint32_t kPixels = T * T;
+    __shared__ __align__(16) S sv[op_tiles<T>() * kPixels];
+    __shared__ __align__(16) S svv[VAR ? op_tiles<T>() * kPixels : 2];
+    const uint32_t nt = A.ntx * A.nty;
+    sorted_chunk<CHUNK, op_tiles<T>(), kPixels, false>(
+        isect_ids, A.n_isects, int64_t(A.C) * nt,
+        [&](uint32_t slot, uint32_t key, uint32_t p) {
+            const uint32_t cam = key / nt, t = key - cam * nt, ty = t / A.ntx, tx = t - ty * A.ntx;
+            const uint32_t x = tx * T + p % T, y = ty * T + p / T;
+            const bool in = x < A.W && y < A.H;
+            const size_t o = (size_t(cam) * A.H + y) * A.W + x;
+            sv[slot * kPixels + p] = in ? v_render[o] : S(0);
+            if constexpr (VAR) svv[slot * kPixels + p] = in ? v_var[o] : S(0);
+        },
+        [&](uint32_t e, uint32_t key, uint64_t& mask, double&) {
+            const int32_t g = A.flatten[e];
+            if (g < 0 || uint32_t(g) >= A.C * A.N) return false;
+            int lo, hi;
+            reached_rows<S, BETA>(load_prim(A, g, BETA), S(((key % nt) / A.ntx) * T), T, lo, hi);
+            mask = ((1ull << hi) - 1ull) & ~((1ull << lo) - 1ull);
+            return hi > lo;
+        },
+        [&](uint32_t e, uint32_t key, uint32_t slot, uint64_t rows, double, bool active) {
+            const uint32_t t = key % nt, ty = t / A.ntx, tx = t - ty * A.ntx;
+            const int32_t g = A.flatten[e];
+            const Prim2D<S> p = load_prim(A, g, BETA);
+            const uint32_t n = uint32_t(g) % A.N;
+            const S w = p.opac * p.mu, q2 = VAR && unc ? S(2) * unc[n] : S(0);
+            S m0 = S(0), mx = S(0), my = S(0), mxx = S(0), mxy = S(0), myy = S(0), sl = S(0), vq = S(0);
+            while (rows) {
+                const uint32_t r = uint32_t(__builtin_ctzll(rows));
+                rows &= rows - 1ull;
+                const S py = S(ty * T + r) + S(0.5), dy = BETA ? p.my - py : py - p.my;
+                S r0 = S(0), r1 = S(0), r2 = S(0);
+                const S* row = sv + slot * kPixels + r * T;
+                const S* rowv = svv + (VAR ? slot * kPixels + r * T : 0);
+#pragma unroll 2
+                for (uint32_t j = 0; j < uint32_t(T); ++j) {
+                    const S px = S(tx * T + j) + S(0.5), dx = BETA ? p.mx - px : px - p.mx;
+                    S v = row[j];
+                    const S vv = VAR ? rowv[VAR ? j : 0] : S(0);
+                    if constexpr (BETA) {
+                        const S q = pair_form<S, BETA>(p.a * dx, dx, S(2) * p.b * dx, p.c, dy);
+                        if (q < S(0) || q >= S(1)) continue;
+                        const S h = S(1) - q, vis = Math<S>::pow(h, p.beta), alpha = w * vis;
+                        if (fabs(alpha) < S(1e-5)) continue;
+                        if constexpr (VAR) {
+                            vq += vv * alpha * alpha;
+                            v += q2 * alpha * vv;
+                        }
+                        const S gv = v * (vis / h);
+                        m0 += v * vis;
+                        sl += v * alpha * Math<S>::log(h);
+                        r0 += gv;
+                        r1 += gv * dx;
+                        r2 += gv * dx * dx;
+                    } else {
+                        const S sigma = pair_form<S, BETA>(p.a * dx, dx, p.b * dx, p.c, dy);
+                        const S vis = Math<S>::exp(-sigma), alpha = w * vis;
+                        const bool keep = !(sigma < S(0) || fabs(alpha) < S(1e-5));
+                        if constexpr (VAR) {
+                            vq += keep ? vv * alpha * alpha : S(0);
+                            v += q2 * alpha * vv;
+                        }
+                        const S gv = keep ? v * alpha : S(0);
+                        m0 += keep ? v * vis : S(0);
+                        r0 += gv;
+                        r1 += gv * dx;
+                        r2 += gv * dx * dx;
+                    }
+                }
+                mx += r1;
+                mxx += r2;
+                my += dy * r0;
+                mxy += dy * r1;
+                myy += dy * dy * r0;
+            }
+            if (!active) return;
+            const size_t G = size_t(g);
+            if constexpr (BETA) {
+                const S k = -w * p.beta;
+                atomic_add(v_xy + 2 * G, S(2) * k * (p.a * mx + p.b * my));
+                atomic_add(v_xy + 2 * G + 1, S(2) * k * (p.b * mx + p.c * my));
+                atomic_add(v_conic + 3 * G, k * mxx);
+                atomic_add(v_conic + 3 * G + 1, S(2) * k * mxy);
+                atomic_add(v_conic + 3 * G + 2, k * myy);
+                atomic_add(v_beta + G, sl);
+            } else {
+                atomic_add(v_xy + 2 * G, p.a * mx + p.b * my);
+                atomic_add(v_xy + 2 * G + 1, p.b * mx + p.c * my);
+                atomic_add(v_conic + 3 * G, S(-0.5) * mxx);
+                atomic_add(v_conic + 3 * G + 1, -mxy);
+                atomic_add(v_conic + 3 * G + 2, S(-0.5) * myy);
+            }
+            atomic_add(v_opac + G, p.mu * m0);
+            atomic_add(v_mu + G, p.opac * m0);
+            if constexpr (VAR)
+                if (v_q) atomic_add(v_q + n, vq);
+        });
+}
+
+// ---------------------------------------------------------------------------
 // Host launchers
 // ---------------------------------------------------------------------------
 inline int check_tile(uint32_t T, uint32_t ntx, uint32_t nty, uint32_t W, uint32_t H) {
@@ -269,6 +583,23 @@ int launch_fwd(int dtype, bool beta, bool var, const void* means2d, const void* 
         using S = decltype(tag);
         auto A = make_args<S>(means2d, conics, opac, mus, betas, unc, offsets, flatten, n_isects, C,
                               N, W, H, T, ntx, nty);
+        const auto rows = [&](auto tile) {
+            constexpr int TILE = decltype(tile)::value;
+            const auto launch = [&](auto split) {
+                constexpr bool SPLIT = decltype(split)::value;
+                auto k = beta ? (var ? raster_fwd_rows_kernel<S, TILE, true, true, SPLIT>
+                                     : raster_fwd_rows_kernel<S, TILE, true, false, SPLIT>)
+                              : (var ? raster_fwd_rows_kernel<S, TILE, false, true, SPLIT>
+                                     : raster_fwd_rows_kernel<S, TILE, false, false, SPLIT>);
+                k<<<uint32_t(blocks) * (SPLIT ? TILE * TILE / kWave : 1), op_waves<TILE, SPLIT>() * kWave, 0, stream>>>(
+                    A, (S*)out, (S*)out_var);
+                return check_launch("rasterize_to_pixels_fwd");
+            };
+            return blocks <= kSplitTiles ? launch(std::true_type{}) : launch(std::false_type{});
+        };
+        if (T == 8) return rows(std::integral_constant<int, 8>{});
+        if (T == 16) return rows(std::integral_constant<int, 16>{});
+        if (T == 32) return rows(std::integral_constant<int, 32>{});
         auto k = beta ? (var ? raster_fwd_kernel<S, true, true> : raster_fwd_kernel<S, true, false>)
                       : (var ? raster_fwd_kernel<S, false, true> : raster_fwd_kernel<S, false, false>);
         k<<<uint32_t(blocks), threads, shm, stream>>>(A, (S*)out, (S*)out_var);
@@ -404,6 +735,29 @@ extern "C" int r2s_rasterize_to_pixels_bwd_per_gaussian(
         if (n_isects == 0 || CN == 0) return R2S_OK;
         auto A = make_args<S>(means2d, conics, opacities, mus, betas, nullptr, nullptr, flatten_ids,
                               n_isects, C, N, width, height, tile_size, n_tiles_x, n_tiles_y);
+        const bool var = v_render_var != nullptr;
+        const auto rows = [&](auto tile) {
+            constexpr int TILE = decltype(tile)::value;
+            const bool few = n_isects <= kFewIsects;
+            const auto launch = [&](auto chunk) {
+                constexpr uint32_t CHUNK = decltype(chunk)::value;
+                auto k = beta ? (var ? raster_bwd_rows_kernel<S, TILE, CHUNK, true, true>
+                                     : raster_bwd_rows_kernel<S, TILE, CHUNK, true, false>)
+                              : (var ? raster_bwd_rows_kernel<S, TILE, CHUNK, false, true>
+                                     : raster_bwd_rows_kernel<S, TILE, CHUNK, false, false>);
+                k<<<ceil_div(n_isects, CHUNK), kChunkThreads, 0, stream>>>(
+                    A, isect_ids, (const S*)v_render, (const S*)v_render_var, (const S*)uncertainties, (S*)v_means2d,
+                    (S*)v_conics, (S*)v_opacities, (S*)v_mus, (S*)v_betas, (S*)v_uncertainties);
+            };
+            if (few) launch(std::integral_constant<uint32_t, 256>{});
+            else launch(std::integral_constant<uint32_t, 512>{});
+            return check_launch("rasterize_to_pixels_bwd_per_gaussian");
+        };
+        if (!v_means2d_abs && uint64_t(C) * n_tiles_x * n_tiles_y < (1ull << 32) - 1) {
+            if (tile_size == 8) return rows(std::integral_constant<int, 8>{});
+            if (tile_size == 16) return rows(std::integral_constant<int, 16>{});
+            if (tile_size == 32) return rows(std::integral_constant<int, 32>{});
+        }
         constexpr uint32_t waves = 4;
         auto k = beta ? raster_bwd_isect_kernel<S, true> : raster_bwd_isect_kernel<S, false>;
         k<<<std::min<uint32_t>(ceil_div(n_isects, waves), kIsectBlocks), waves * kWave, 0, stream>>>(

@@ -1,7 +1,8 @@
 // 3D voxelization: each voxel sums opacity * profile over the primitives binned
 // to its 3D tile. Tile-parallel forward / VJP (LDS-staged batches) and the
 // intersection-parallel VJP (one wave64 per intersection), for any tile size
-// with tile_size^3 <= 1024 and both float/double.
+// with tile_size^3 <= 1024 and both float/double; 8^3 tiles have forms that skip
+// what a primitive does not reach (octants in the forward, rows in the VJP).
 // Profiles follow r2splat/cuda/csrc/VoxelizeToVoxelsFwd.cu:181-219 (Gaussian,
 // threshold 1e-6) and the Beta kernels (threshold 1e-5); the VJPs follow
 // VoxelizeToVoxelsBwd.cu:387-434 and the Beta per-primitive kernel.
@@ -11,6 +12,7 @@
 #include "binning.hpp"
 #include "geometry_common.hpp"
 #include "raster_common.hpp"
+#include "sorted_chunk.hpp"
 
 namespace r2s {
 
@@ -402,7 +404,7 @@ __device__ __forceinline__ double beta_qmax(float w, float beta) {
 }
 
 constexpr uint32_t kVoxPartial = 12;  // floats per intersection partial (11, or 12 with a variance)
-constexpr uint32_t kMomThreads = 256;
+constexpr uint32_t kMomThreads = kChunkThreads;
 constexpr float kL2E = 1.4426950408889634f;
 
 __device__ __forceinline__ uint32_t vox_qlim(float opac, float beta, bool is_beta) {
@@ -496,11 +498,6 @@ __device__ __forceinline__ uint64_t vox_row_mask(const VoxForm& f, float S, floa
 // cut-off 0 <= q <= qmax decided in double, exactly as the fused forward does.
 // With `partials` an intersection's gradient goes to its emission index, else
 // it is added to the outputs with one atomic per field.
-// A workgroup takes 512 intersections, or 256 where those would leave most
-// compute units with a single workgroup (up to 2^19 intersections in all: 285k
-// take 30 us against 66; 2.9M take 534 us against 479, their rows sorted less
-// finely).
-constexpr uint32_t kMomFew = 1u << 19;
 constexpr uint32_t kMomTiles = 8;  // tiles whose adjoints are staged together
 
 template <uint32_t kMomChunk, bool BETA, bool VAR, bool WIDE>
@@ -510,121 +507,38 @@ vox_bwd_moments_kernel(VoxArgs<float> A, const int64_t* __restrict__ isect_ids, 
                        float* __restrict__ v_xyz, float* __restrict__ v_c, float* __restrict__ v_opac,
                        float* __restrict__ v_beta, const int32_t* __restrict__ radii,
                        const uint32_t* __restrict__ cum, float* __restrict__ partials) {
-    constexpr uint32_t T = kMomT, T3 = T * T * T, kPer = kMomChunk / kMomThreads, kWaves = kMomThreads / kWave;
-    constexpr uint32_t kNoTile = 0xffffffffu, kClasses = T * T + 1;
+    constexpr uint32_t T = kMomT, T3 = T * T * T;
     static_assert(!WIDE || BETA, "the double-precision form is for Beta profiles");
-    static_assert(kClasses == kWave + 1, "the row counts 64 .. 1 are scanned by one wave");
     __shared__ __align__(16) float sv[kMomTiles * T3];
     __shared__ __align__(16) float svv[VAR ? kMomTiles * T3 : 4];
-    __shared__ uint64_t masks[kMomChunk];
-    __shared__ double bounds[WIDE ? kMomChunk : 1];
-    __shared__ uint32_t tile_of[kMomChunk], sorted[kMomChunk];  // sorted: chunk entry | staged tile << 16
-    __shared__ uint32_t first_of[kMomChunk + 1];                // first entry of the chunk's k-th tile
-    __shared__ uint32_t hist[kClasses], first[kClasses], wave_tiles[kPer * kWaves], n_items, next_item;
-    const uint32_t lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-    const uint32_t e0 = blockIdx.x * kMomChunk, n_here = min(kMomChunk, A.n_isects - e0);
-    const int64_t nt = int64_t(A.ntx) * A.nty * A.ntz;
-    uint32_t place[kPer];  // which of the chunk's tiles an entry belongs to
-#pragma unroll
-    for (uint32_t k = 0; k < kPer; ++k) {
-        const uint32_t i = k * kMomThreads + threadIdx.x;
-        int64_t id = -1;
-        if (i < n_here) id = isect_ids[e0 + i];
-        tile_of[i] = id >= 0 && id < nt ? uint32_t(id) : kNoTile;
-    }
-    __syncthreads();
-    uint64_t starts[kPer];
-#pragma unroll
-    for (uint32_t k = 0; k < kPer; ++k) {
-        const uint32_t i = k * kMomThreads + threadIdx.x;
-        starts[k] = __ballot(i < n_here && (i == 0 || tile_of[i] != tile_of[i - 1]));
-        if (lane == 0) wave_tiles[k * kWaves + wave] = uint32_t(__popcll(starts[k]));
-    }
-    __syncthreads();
-    uint32_t n_tiles = 0;
-#pragma unroll
-    for (uint32_t k = 0; k < kPer; ++k) {
-        uint32_t before = 0;
-        for (uint32_t w = 0; w < k * kWaves + wave; ++w) before += wave_tiles[w];
-        const uint64_t upto = starts[k] & (~0ull >> (kWave - 1 - lane));
-        place[k] = before + uint32_t(__popcll(upto)) - 1u;
-        if ((starts[k] >> lane) & 1ull) first_of[place[k]] = k * kMomThreads + threadIdx.x;
-    }
-    for (uint32_t w = 0; w < kPer * kWaves; ++w) n_tiles += wave_tiles[w];
-    for (uint32_t t0 = 0; t0 < n_tiles; t0 += kMomTiles) {
-        __syncthreads();  // first_of is written; the previous tiles' adjoints are consumed
-        const uint32_t n_staged = min(kMomTiles, n_tiles - t0);
-        for (uint32_t p = threadIdx.x; p < n_staged * T3; p += kMomThreads) {
-            const uint32_t tile = tile_of[first_of[t0 + p / T3]], q = p % T3;
-            if (tile == kNoTile) continue;
+    sorted_chunk<kMomChunk, kMomTiles, T3, WIDE>(
+        isect_ids, A.n_isects, int64_t(A.ntx) * A.nty * A.ntz,
+        [&](uint32_t slot, uint32_t tile, uint32_t p) {
             const uint32_t tx = tile % A.ntx, rest = tile / A.ntx, ty = rest % A.nty, tz = rest / A.nty;
-            const uint32_t x = tx * T + q % T, j = ty * T + (q / T) % T, i = tz * T + q / (T * T);
+            const uint32_t x = tx * T + p % T, j = ty * T + (p / T) % T, i = tz * T + p / (T * T);
             const bool in = i < A.dz && j < A.dy && x < A.dx;
             const size_t o = (size_t(i) * A.dy + j) * A.dx + x;
-            sv[p] = in ? v_render[o] : 0.f;
-            if constexpr (VAR) svv[p] = in ? v_render_var[o] : 0.f;
-        }
-        for (uint32_t c = threadIdx.x; c < kClasses; c += kMomThreads) hist[c] = 0u;
-        __syncthreads();
-        uint64_t mask[kPer];
-        double bound[kPer];
-        uint32_t rank[kPer];
-        bool mine[kPer];
-#pragma unroll
-        for (uint32_t k = 0; k < kPer; ++k) {
-            const uint32_t i = k * kMomThreads + threadIdx.x;
-            mine[k] = i < n_here && place[k] >= t0 && place[k] < t0 + n_staged && tile_of[i] != kNoTile;
-            mask[k] = 0ull;
-            bound[k] = -1.0;
-            rank[k] = 0u;
-            if (mine[k]) {
-                const int32_t g = A.flatten[e0 + i];
-                mine[k] = g >= 0 && uint32_t(g) < A.N;
-                if (mine[k]) {
-                    const VoxForm f = vox_form<BETA, WIDE>(A, size_t(g));
-                    const uint32_t tile = tile_of[i], tx = tile % A.ntx, rest = tile / A.ntx;
-                    bound[k] = f.qmax;
-                    const float S = WIDE ? float(f.qmax) : __uint_as_float(f.qlim - 1u);
-                    mask[k] = vox_row_mask(f, S, float(tx * T) + 0.5f, float((rest % A.nty) * T) + 0.5f,
-                                           float((rest / A.nty) * T) + 0.5f);
-                    rank[k] = atomicAdd(&hist[T * T - uint32_t(__popcll(mask[k]))], 1u);
-                }
-            }
-        }
-        __syncthreads();
-        if (wave == 0) {  // starts of the row counts, most rows first
-            const uint32_t c = hist[lane], incl = wave_scan(c);
-            first[lane] = incl - c;
-            if (lane == kWave - 1) {
-                first[kWave] = incl;
-                n_items = incl + hist[kWave];
-                next_item = 0u;
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (uint32_t k = 0; k < kPer; ++k)
-            if (mine[k]) {
-                const uint32_t at = first[T * T - uint32_t(__popcll(mask[k]))] + rank[k];
-                masks[at] = mask[k];
-                if constexpr (WIDE) bounds[at] = bound[k];
-                sorted[at] = (k * kMomThreads + threadIdx.x) | ((place[k] - t0) << 16);
-            }
-        __syncthreads();
-        for (;;) {
-            uint32_t c = 0;
-            if (lane == 0) c = atomicAdd(&next_item, uint32_t(kWave));
-            c = __builtin_amdgcn_readfirstlane(c);
-            if (c >= n_items) break;
-            const bool active = c + lane < n_items;  // the others repeat item c without rows
-            const uint32_t at = active ? c + lane : c, it = sorted[at], i = it & 0xffffu, staged = (it >> 16) * T3;
-            uint64_t rows = active ? masks[at] : 0ull;
-            const uint32_t tile = tile_of[i], tx = tile % A.ntx, rest = tile / A.ntx, ty = rest % A.nty,
-                           tz = rest / A.nty;
+            sv[slot * T3 + p] = in ? v_render[o] : 0.f;
+            if constexpr (VAR) svv[slot * T3 + p] = in ? v_render_var[o] : 0.f;
+        },
+        [&](uint32_t e, uint32_t tile, uint64_t& mask, double& bound) {
+            const int32_t g = A.flatten[e];
+            if (g < 0 || uint32_t(g) >= A.N) return false;
+            const VoxForm f = vox_form<BETA, WIDE>(A, size_t(g));
+            const uint32_t tx = tile % A.ntx, rest = tile / A.ntx;
+            const float S = WIDE ? float(f.qmax) : __uint_as_float(f.qlim - 1u);
+            bound = f.qmax;
+            mask = vox_row_mask(f, S, float(tx * T) + 0.5f, float((rest % A.nty) * T) + 0.5f,
+                                float((rest / A.nty) * T) + 0.5f);
+            return true;
+        },
+        [&](uint32_t e, uint32_t tile, uint32_t slot, uint64_t rows, double bound, bool active) {
+            const uint32_t staged = slot * T3;
+            const uint32_t tx = tile % A.ntx, rest = tile / A.ntx, ty = rest % A.nty, tz = rest / A.nty;
             const float x0 = float(tx * T) + 0.5f, y0 = float(ty * T) + 0.5f, z0 = float(tz * T) + 0.5f;
-            const int32_t g = A.flatten[e0 + i];
+            const int32_t g = A.flatten[e];
             const size_t G = size_t(g);
-            const VoxForm f = vox_form<BETA, WIDE>(A, G, WIDE ? &bounds[at] : nullptr);
+            const VoxForm f = vox_form<BETA, WIDE>(A, G, &bound);
             const float* P = f.P;
             const float opac = f.opac, beta = f.beta;
             double md[3] = {0.0, 0.0, 0.0}, Pd[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
@@ -779,8 +693,7 @@ vox_bwd_moments_kernel(VoxArgs<float> A, const int64_t* __restrict__ isect_ids, 
                 atomic_add(v_opac + G, go);
                 if constexpr (BETA) atomic_add(v_beta + G, gb);
             }
-        }
-    }
+        });
 }
 
 // ---------------------------------------------------------------------------
@@ -1094,6 +1007,269 @@ vox_partials_reduce_kernel(const uint32_t* __restrict__ cum, const float* __rest
     }
 }
 
+// ---------------------------------------------------------------------------
+// Operator kernels for 8^3 tiles that skip what a primitive does not reach (the
+// exponential or power in double is most of a pair's cost; 20k Gaussians in 72 x
+// 64 x 56 contribute to a sixth of the voxels of their tiles). One voxel per
+// thread over the whole list took 210 us there and a wave per intersection 373 us;
+// these take 166 and 160.
+// ---------------------------------------------------------------------------
+// The float form of a primitive and the bound S on its q (Gaussian: q = sigma)
+// beyond which no term passes the cut-off; false when none can (its weight is
+// surely below it).
+template <typename S, bool BETA>
+__device__ __forceinline__ bool op_form(const Prim3D<S>& p, VoxForm& f, float& bound) {
+    const float w = fabsf(float(p.opac)), cut = BETA ? 1e-5f : 1e-6f;
+    if (w < 0.999f * cut) return false;
+    const float s = BETA ? 1.f : 0.5f, t2 = BETA ? 2.f : 1.f;
+    f.hi[0] = float(p.x);
+    f.hi[1] = float(p.y);
+    f.hi[2] = float(p.z);
+    f.a = s * float(p.c[0]);
+    f.bxy = t2 * float(p.c[1]);
+    f.bxz = t2 * float(p.c[2]);
+    f.cyy = s * float(p.c[3]);
+    f.cyz = t2 * float(p.c[4]);
+    f.czz = s * float(p.c[5]);
+    f.qlim = 1u;
+    if (BETA) {
+        const float D = 1.f - __builtin_amdgcn_exp2f(__log2f(cut / w) / float(p.beta));
+        bound = p.beta > S(0) ? fminf(1.f, 1.002f * D + 1e-4f) : 1.f;
+    } else {
+        bound = 1.001f * __logf(w / cut) + 1e-4f;
+    }
+    return true;
+}
+
+// Octants (bit 4 oz + 2 oy + ox) of the tile whose first voxel is (x0, y0, z0) that
+// the ellipsoid q <= S can reach, by its bounding box; every octant of forms
+// that cancel or are not finite.
+__device__ __forceinline__ uint32_t form_octants(const VoxForm& f, float S, float x0, float y0, float z0) {
+    const float xy = 0.5f * f.bxy, xz = 0.5f * f.bxz, yz = 0.5f * f.cyz;
+    const float c[3] = {f.cyy * f.czz - yz * yz, f.a * f.czz - xz * xz, f.a * f.cyy - xy * xy};
+    const float det = f.a * c[0] - xy * (xy * f.czz - xz * yz) + xz * (xy * yz - xz * f.cyy);
+    if (!(f.a > 0.f) || !(det > 1e-3f * f.a * f.cyy * f.czz) || !(S >= 0.f)) return 0xffu;
+    const float m[3] = {f.hi[0] - x0, f.hi[1] - y0, f.hi[2] - z0};
+    uint32_t part[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const float e = __builtin_amdgcn_sqrtf(S * c[k] * __builtin_amdgcn_rcpf(det)) * 1.002f + 0.05f;
+        const float lo = m[k] - e, hi = m[k] + e;  // voxel centres of the tile at 0.5 .. 7.5
+        part[k] = (lo <= 3.5f && hi >= 0.5f ? 1u : 0u) | (lo <= 7.5f && hi >= 4.5f ? 2u : 0u);
+        if (!(e < 1e9f) || !(fabsf(m[k]) < 1e9f)) part[k] = 3u;
+    }
+    const uint32_t row = part[0], plane = (part[1] & 1u ? row : 0u) | (part[1] & 2u ? row << 2 : 0u);
+    return (part[2] & 1u ? plane : 0u) | (part[2] & 2u ? plane << 4 : 0u);
+}
+
+template <typename S>
+__device__ __forceinline__ Prim3D<S> load_prim3(const VoxArgs<S>& A, int32_t g, bool beta) {
+    Prim3D<S> p;
+    const size_t G = size_t(g);
+    p.x = A.means3d[3 * G];
+    p.y = A.means3d[3 * G + 1];
+    p.z = A.means3d[3 * G + 2];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) p.c[k] = A.conics[6 * G + k];
+    p.opac = A.opac[g];
+    p.beta = beta ? A.betas[g] : S(0);
+    return p;
+}
+
+// Forward: kVoxFwdWaves waves share a tile's list as in the fused forward; lane =
+// one voxel of each 4^3 octant, octants not reached skipped by scalar branches.
+template <typename S, bool BETA, bool VAR>
+__global__ void __launch_bounds__(kVoxFwdWaves * kWave) __attribute__((amdgpu_waves_per_eu(3)))
+vox_fwd_octants_kernel(VoxArgs<S> A, S* __restrict__ out, S* __restrict__ out_var) {
+    constexpr uint32_t T = kMomT;
+    __shared__ Prim3D<S> stage[kVoxFwdWaves][kWave];
+    __shared__ S stage_q[VAR ? kVoxFwdWaves : 1][kWave];
+    __shared__ S part[kVoxFwdWaves][T * T * T];
+    const uint32_t blk = blockIdx.x, nt = A.ntx * A.nty * A.ntz;
+    int32_t start = A.offsets[blk];
+    int32_t end = (blk + 1 == nt) ? int32_t(A.n_isects) : A.offsets[blk + 1];
+    start = max(0, min(start, int32_t(A.n_isects)));
+    end = max(start, min(end, int32_t(A.n_isects)));
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+    const uint32_t tx = blk % A.ntx, rest = blk / A.ntx, ty = rest % A.nty, tz = rest / A.nty;
+    const uint32_t lx = lane % 4, ly = (lane / 4) % 4, lz = lane / 16;
+    const S px = S(tx * T + lx) + S(0.5), py = S(ty * T + ly) + S(0.5), pz = S(tz * T + lz) + S(0.5);
+    S acc[8], acc_var[8];
+#pragma unroll
+    for (int o = 0; o < 8; ++o) acc[o] = acc_var[o] = S(0);
+    for (int32_t base = start + int32_t(wave) * kWave; base < end; base += kVoxFwdWaves * kWave) {
+        uint32_t octants = 0;
+        Prim3D<S> r = {};
+        S q = S(0);
+        if (base + int32_t(lane) < end) {
+            const int32_t g = A.flatten[base + int32_t(lane)];
+            if (g >= 0 && uint32_t(g) < A.N) {  // out-of-range ids contribute nothing
+                r = load_prim3(A, g, BETA);
+                if constexpr (VAR) q = A.unc[g];
+                VoxForm f;
+                float bound;
+                if (op_form<S, BETA>(r, f, bound))
+                    octants = form_octants(f, bound, float(tx * T), float(ty * T), float(tz * T));
+            }
+        }
+        wave_sync_lds();
+        stage[wave][lane] = r;
+        if constexpr (VAR) stage_q[wave][lane] = q;
+        wave_sync_lds();
+        const int32_t n = min(int32_t(kWave), end - base);
+        for (int32_t j = 0; j < n; ++j) {
+            const uint32_t reach = __builtin_amdgcn_readlane(octants, j);
+            if (reach == 0u) continue;
+            const Prim3D<S> p = stage[wave][j];
+            const S unc = VAR ? stage_q[VAR ? wave : 0][j] : S(0);
+#pragma unroll
+            for (uint32_t o = 0; o < 8; ++o) {
+                if (!((reach >> o) & 1u)) continue;
+                S vis, alpha;
+                if (!eval_profile3<S, BETA>(p, px + S(4 * (o & 1u)), py + S(2 * (o & 2u)), pz + S(o & 4u), vis, alpha))
+                    alpha = S(0);
+                acc[o] += alpha;
+                if constexpr (VAR) acc_var[o] += unc * alpha * alpha;
+            }
+        }
+    }
+#pragma unroll
+    for (int v = 0; v < (VAR ? 2 : 1); ++v) {
+#pragma unroll
+        for (uint32_t o = 0; o < 8; ++o)
+            part[wave][((lz + (o & 4u)) * T + ly + 2 * (o & 2u)) * T + lx + 4 * (o & 1u)] = v ? acc_var[o] : acc[o];
+        __syncthreads();
+        for (uint32_t p = threadIdx.x; p < T * T * T; p += kVoxFwdWaves * kWave) {
+            S sum = S(0);
+#pragma unroll
+            for (int k = 0; k < kVoxFwdWaves; ++k) sum += part[k][p];
+            const uint32_t k = tx * T + p % T, j = ty * T + (p / T) % T, i = tz * T + p / (T * T);
+            if (i < A.dz && j < A.dy && k < A.dx) (v ? out_var : out)[(size_t(i) * A.dy + j) * A.dx + k] = sum;
+        }
+        if (VAR && v == 0) __syncthreads();  // the mean's partial volumes are consumed
+    }
+}
+
+// Gaussian: sigma, Beta: q, in the roundings eval_profile3 compiles to: the float32
+// terms of a thin primitive cancel, and another order would give it another exponent.
+template <typename S, bool BETA>
+__device__ __forceinline__ S triple_form(const Prim3D<S>& p, S dx, S dy, S dz) {
+    const S sq = Math<S>::fma(p.c[5] * dz, dz, Math<S>::fma(p.c[0] * dx, dx, p.c[3] * dy * dy));
+    const S xy = p.c[1] * dx, xz = p.c[2] * dx, yz = p.c[4] * dy;
+    if constexpr (BETA) return sq + S(2) * Math<S>::fma(yz, dz, Math<S>::fma(xy, dy, xz * dz));
+    return Math<S>::fma(yz, dz, Math<S>::fma(xz, dz, Math<S>::fma(xy, dy, S(0.5) * sq)));
+}
+
+// VJP: one lane per intersection over the rows it reaches (sorted_chunk), the
+// moments of vox_bwd_moments_kernel in S, one atomic per field.
+constexpr uint32_t kOpTiles = 4;
+
+template <typename S, uint32_t CHUNK, bool BETA, bool VAR>
+__global__ void __launch_bounds__(kChunkThreads) __attribute__((amdgpu_waves_per_eu(3)))
+vox_bwd_rows_kernel(VoxArgs<S> A, const int64_t* __restrict__ isect_ids, const S* __restrict__ v_render,
+                    const S* __restrict__ v_var, const S* __restrict__ unc, S* __restrict__ v_xyz,
+                    S* __restrict__ v_c, S* __restrict__ v_opac, S* __restrict__ v_beta, S* __restrict__ v_q) {
+    constexpr uint32_t T = kMomT, T3 = T * T * T;
+    __shared__ __align__(16) S sv[kOpTiles * T3];
+    __shared__ __align__(16) S svv[VAR ? kOpTiles * T3 : 2];
+    sorted_chunk<CHUNK, kOpTiles, T3, false>(
+        isect_ids, A.n_isects, int64_t(A.ntx) * A.nty * A.ntz,
+        [&](uint32_t slot, uint32_t tile, uint32_t p) {
+            const uint32_t tx = tile % A.ntx, rest = tile / A.ntx, ty = rest % A.nty, tz = rest / A.nty;
+            const uint32_t x = tx * T + p % T, j = ty * T + (p / T) % T, i = tz * T + p / (T * T);
+            const bool in = i < A.dz && j < A.dy && x < A.dx;
+            const size_t o = (size_t(i) * A.dy + j) * A.dx + x;
+            sv[slot * T3 + p] = in ? v_render[o] : S(0);
+            if constexpr (VAR) svv[slot * T3 + p] = in ? v_var[o] : S(0);
+        },
+        [&](uint32_t e, uint32_t tile, uint64_t& mask, double&) {
+            const int32_t g = A.flatten[e];
+            if (g < 0 || uint32_t(g) >= A.N) return false;
+            VoxForm f;
+            float bound;
+            if (!op_form<S, BETA>(load_prim3(A, g, BETA), f, bound)) return false;
+            const uint32_t tx = tile % A.ntx, rest = tile / A.ntx;
+            mask = vox_row_mask(f, bound, float(tx * T) + 0.5f, float((rest % A.nty) * T) + 0.5f,
+                                float((rest / A.nty) * T) + 0.5f);
+            return mask != 0ull;
+        },
+        [&](uint32_t e, uint32_t tile, uint32_t slot, uint64_t rows, double, bool active) {
+            const uint32_t tx = tile % A.ntx, rest = tile / A.ntx, ty = rest % A.nty, tz = rest / A.nty;
+            const int32_t g = A.flatten[e];
+            const Prim3D<S> p = load_prim3(A, g, BETA);
+            const S q2 = VAR && unc ? S(2) * unc[g] : S(0);
+            S m0 = S(0), m_x = S(0), m_y = S(0), m_z = S(0), mxx = S(0), myy = S(0), mzz = S(0), mxy = S(0), mxz = S(0),
+              myz = S(0), sl = S(0), vq = S(0);
+            while (rows) {
+                const uint32_t bit = uint32_t(__builtin_ctzll(rows)), z = bit / T, y = bit % T;
+                rows &= rows - 1ull;
+                const S dy = (S(ty * T + y) + S(0.5)) - p.y, dz = (S(tz * T + z) + S(0.5)) - p.z;
+                S r0 = S(0), r1 = S(0), r2 = S(0);
+                const S* row = sv + slot * T3 + bit * T;
+                const S* rowv = svv + (VAR ? slot * T3 + bit * T : 0);
+#pragma unroll 2
+                for (uint32_t j = 0; j < T; ++j) {
+                    const S dx = (S(tx * T + j) + S(0.5)) - p.x;
+                    const S q = triple_form<S, BETA>(p, dx, dy, dz);
+                    S v = row[j];
+                    const S vv = VAR ? rowv[VAR ? j : 0] : S(0);
+                    if constexpr (BETA) {
+                        if (q < S(0) || q >= S(1)) continue;
+                        const S h = S(1) - q, vis = Math<S>::pow(h, p.beta), alpha = p.opac * vis;
+                        if (fabs(alpha) < S(1e-5)) continue;
+                        if constexpr (VAR) {
+                            vq += vv * alpha * alpha;
+                            v += q2 * alpha * vv;
+                        }
+                        const S gv = v * (vis / h);
+                        m0 += v * vis;
+                        sl += v * alpha * Math<S>::log(h);
+                        r0 += gv;
+                        r1 += gv * dx;
+                        r2 += gv * dx * dx;
+                    } else {
+                        const S vis = Math<S>::exp(-q), alpha = p.opac * vis;
+                        const bool keep = !(q < S(0) || fabs(alpha) < S(1e-6));
+                        if constexpr (VAR) {
+                            vq += keep ? vv * alpha * alpha : S(0);
+                            v += q2 * alpha * vv;
+                        }
+                        const S gv = keep ? v * vis : S(0);
+                        r0 += gv;
+                        r1 += gv * dx;
+                        r2 += gv * dx * dx;
+                    }
+                }
+                if constexpr (!BETA) m0 += r0;
+                m_x += r1;
+                mxx += r2;
+                m_y += dy * r0;
+                m_z += dz * r0;
+                myy += dy * dy * r0;
+                mzz += dz * dz * r0;
+                myz += dy * dz * r0;
+                mxy += dy * r1;
+                mxz += dz * r1;
+            }
+            if (!active) return;
+            const size_t G = size_t(g);
+            const S k = BETA ? S(2) * p.opac * p.beta : p.opac, kc = BETA ? -p.opac * p.beta : S(-0.5) * p.opac;
+            atomic_add(v_xyz + 3 * G, k * (p.c[0] * m_x + p.c[1] * m_y + p.c[2] * m_z));
+            atomic_add(v_xyz + 3 * G + 1, k * (p.c[1] * m_x + p.c[3] * m_y + p.c[4] * m_z));
+            atomic_add(v_xyz + 3 * G + 2, k * (p.c[2] * m_x + p.c[4] * m_y + p.c[5] * m_z));
+            atomic_add(v_c + 6 * G, kc * mxx);
+            atomic_add(v_c + 6 * G + 1, S(2) * kc * mxy);
+            atomic_add(v_c + 6 * G + 2, S(2) * kc * mxz);
+            atomic_add(v_c + 6 * G + 3, kc * myy);
+            atomic_add(v_c + 6 * G + 4, S(2) * kc * myz);
+            atomic_add(v_c + 6 * G + 5, kc * mzz);
+            atomic_add(v_opac + G, m0);
+            if constexpr (BETA) atomic_add(v_beta + G, sl);
+            if constexpr (VAR)
+                if (v_q) atomic_add(v_q + G, vq);
+        });
+}
+
 inline int check_vox_tile(uint32_t T, uint32_t ntx, uint32_t nty, uint32_t ntz, uint32_t dx,
                           uint32_t dy, uint32_t dz) {
     R2S_REQUIRE(T >= 1 && T * T * T <= 1024, "tile_size %u must satisfy 1 <= tile_size^3 <= 1024", T);
@@ -1138,6 +1314,12 @@ extern "C" int r2s_voxelize_to_voxels_fwd(int dtype, const void* means3d, const 
         auto A = make_vox_args<S>(means3d, conics, opacities, betas, uncertainties, tile_offsets,
                                   flatten_ids, n_isects, N, dim_x, dim_y, dim_z, tile_size,
                                   n_tiles_x, n_tiles_y, n_tiles_z);
+        if (tile_size == kMomT) {
+            auto k = beta ? (var ? vox_fwd_octants_kernel<S, true, true> : vox_fwd_octants_kernel<S, true, false>)
+                          : (var ? vox_fwd_octants_kernel<S, false, true> : vox_fwd_octants_kernel<S, false, false>);
+            k<<<uint32_t(blocks), kVoxFwdWaves * kWave, 0, stream>>>(A, (S*)render, (S*)render_var);
+            return check_launch("voxelize_to_voxels_fwd");
+        }
         auto k = beta ? (var ? vox_fwd_kernel<S, true, true> : vox_fwd_kernel<S, true, false>)
                       : (var ? vox_fwd_kernel<S, false, true> : vox_fwd_kernel<S, false, false>);
         k<<<uint32_t(blocks), threads, shm, stream>>>(A, (S*)render, (S*)render_var);
@@ -1206,7 +1388,7 @@ extern "C" int r2s_voxelize_to_voxels_bwd_per_gaussian(
         if constexpr (std::is_same<S, float>::value) {
             const uint64_t n_tiles = uint64_t(n_tiles_x) * n_tiles_y * n_tiles_z;
             if (tile_size == kMomT && !v_render_var && n_tiles < (1ull << 31)) {  // moments form
-                const bool few = n_isects <= kMomFew;
+                const bool few = n_isects <= kFewIsects;
                 auto km = beta ? (few ? vox_bwd_moments_kernel<256, true, false, false>
                                       : vox_bwd_moments_kernel<512, true, false, false>)
                                : (few ? vox_bwd_moments_kernel<256, false, false, false>
@@ -1216,6 +1398,21 @@ extern "C" int r2s_voxelize_to_voxels_bwd_per_gaussian(
                     (float*)v_opacities, (float*)v_betas, nullptr, nullptr, nullptr);
                 return check_launch("voxelize_to_voxels_bwd_per_gaussian");
             }
+        }
+        if (tile_size == kMomT && uint64_t(n_tiles_x) * n_tiles_y * n_tiles_z < (1ull << 31)) {
+            const bool var = v_render_var != nullptr;
+            const auto launch = [&](auto chunk) {
+                constexpr uint32_t CHUNK = decltype(chunk)::value;
+                auto k = beta ? (var ? vox_bwd_rows_kernel<S, CHUNK, true, true> : vox_bwd_rows_kernel<S, CHUNK, true, false>)
+                              : (var ? vox_bwd_rows_kernel<S, CHUNK, false, true>
+                                     : vox_bwd_rows_kernel<S, CHUNK, false, false>);
+                k<<<ceil_div(n_isects, CHUNK), kChunkThreads, 0, stream>>>(
+                    A, isect_ids, (const S*)v_render, (const S*)v_render_var, (const S*)uncertainties, (S*)v_means3d,
+                    (S*)v_conics, (S*)v_opacities, (S*)v_betas, (S*)v_uncertainties);
+            };
+            if (n_isects <= kFewIsects) launch(std::integral_constant<uint32_t, 256>{});
+            else launch(std::integral_constant<uint32_t, 512>{});
+            return check_launch("voxelize_to_voxels_bwd_per_gaussian");
         }
         constexpr uint32_t waves = 4;
         auto k = beta ? vox_bwd_isect_kernel<S, true> : vox_bwd_isect_kernel<S, false>;
@@ -1265,7 +1462,7 @@ extern "C" int r2s_voxelize_fused_vjp(const float* means3d, const double* frame,
         auto A = make_vox_args<float>(means3d, conics, opacities, betas, uncertainties, nullptr, flatten_ids,
                                       n_isects, N, dim_x, dim_y, dim_z, tile_size, n_tiles_x, n_tiles_y, n_tiles_z);
         A.frame = frame;
-        const bool few = n_isects <= kMomFew;
+        const bool few = n_isects <= kFewIsects;
         auto km = beta ? (var ? (few ? vox_bwd_moments_kernel<256, true, true, true>
                                      : vox_bwd_moments_kernel<512, true, true, true>)
                               : (few ? vox_bwd_moments_kernel<256, true, false, true>

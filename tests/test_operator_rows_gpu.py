@@ -1,0 +1,138 @@
+"""The operator rasterizer's kernels for 8, 16 and 32 pixel tiles (rows a primitive
+does not reach skipped; tiles split over workgroups in small launches) and the
+operator voxelizer's for 8^3 tiles against their general kernels: every primitive
+is binned to every tile, so the tile edge changes nothing but the kernel."""
+
+import pytest
+import torch
+
+from oracle import splat as O
+from r2splat_amd import hip as ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(device, dtype, C, N, W, H, seed, beta, var):
+    g = torch.Generator().manual_seed(seed)
+    r = lambda *s: torch.rand(*s, generator=g, dtype=torch.float64)  # noqa: E731
+    means = torch.stack([r(C, N) * (W + 20) - 10, r(C, N) * (H + 20) - 10], -1)
+    theta, s1, s2 = r(C, N) * 3.1416, torch.exp(r(C, N) * 4 - 1.5), torch.exp(r(C, N) * 4 - 1.5)
+    c, s = torch.cos(theta), torch.sin(theta)
+    conics = torch.stack([c * c / s1**2 + s * s / s2**2, c * s * (1 / s1**2 - 1 / s2**2),
+                          s * s / s1**2 + c * c / s2**2], -1)
+    opac, mus = r(C, N), r(C, N) + 0.05
+    opac[:, :2] = 1e-7  # never above the cut-off
+    if N > 6:
+        conics[:, 2] = torch.tensor([0.0, 0.0, 0.0])  # flat: reaches every pixel
+        conics[:, 3] = torch.tensor([1.0, 1.5, 1.0])  # indefinite
+    out = [t.to(device, dtype) for t in (means, conics, opac, mus)]
+    betas = (0.6 + 3 * r(C, N)).to(device, dtype) if beta else None
+    unc = (0.1 * r(N)).to(device, dtype) if var else None
+    v = (r(C, H, W) - 0.5).to(device, dtype)
+    vv = (r(C, H, W) - 0.5).to(device, dtype) if var else None
+    return out, betas, unc, v, vv
+
+
+def _run(case, W, H, T):
+    (means, conics, opac, mus), betas, unc, v, vv = case
+    C, N = opac.shape
+    nx, ny = -(-W // T), -(-H // T)
+    radii = torch.full((C, N, 2), 4 * (W + H), dtype=torch.int32, device=means.device)
+    _, ids, flat = ops.isect_tiles(means, radii, T, nx, ny)
+    assert ids.numel() == C * N * nx * ny
+    off = ops.isect_offset_encode(ids, C, nx, ny)
+    args = (means, conics, opac, mus) + (() if betas is None else (betas,))
+    pre = "" if betas is None else "beta_"
+    if unc is None:
+        img = (getattr(ops, pre + "rasterize_to_pixels_fwd")(*args, off, flat, W, H, T),)
+        grads = getattr(ops, pre + "rasterize_to_pixels_bwd_per_gaussian")(*args, off, ids, flat, v, W, H, T, False)
+    else:
+        img = getattr(ops, pre + "rasterize_to_pixels_mean_var_fwd")(*args, unc, off, flat, W, H, T)
+        grads = getattr(ops, pre + "rasterize_to_pixels_mean_var_bwd_per_gaussian")(
+            *args, off, ids, flat, v, vv, unc, False, W, H, T, False)
+    return img, [g for g in grads if g is not None]
+
+
+# (cameras, primitives, width, height, tile): launches that are split and that
+# are not, more than 2^19 intersections, ragged edges, fewer records than a wave
+SHAPES = [(2, 7, 40, 24, 8), (12, 100, 200, 160, 8), (1, 70, 61, 47, 16), (36, 9, 190, 160, 16), (2, 300, 70, 33, 32),
+          (33, 20, 512, 384, 32)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("beta,var", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("C,N,W,H,T", SHAPES)
+def test_row_kernels_match_the_general_kernel(device, C, N, W, H, T, beta, var, dtype):
+    case = _case(device, dtype, C, N, W, H, C + N, beta, var)
+    _compare(lambda c, t: _run(c, W, H, t), case, T, 10)
+
+
+def _compare(run, case, tile, other):
+    got, general = run(case, tile), run(case, other)
+    dtype = case[0][0].dtype
+    assert len(got[1]) == len(general[1])
+    if dtype == torch.float64:  # the same terms summed in another order
+        for tol, new, old in ((1e-12, got[0], general[0]), (1e-11, got[1], general[1])):
+            for k, (a, b) in enumerate(zip(new, old)):
+                assert O.relative_error(a, b) <= tol, k
+        return
+    # float32 forms of thin footprints cancel, so both kernels are a few roundings
+    # of terms far above the exponent away from float64: as near as the general one
+    wide = [t.double() for t in case[0]], *(None if t is None else t.double() for t in case[1:])
+    exact = run(wide, other)
+    for tol, new, old, ref in ((1e-5, got[0], general[0], exact[0]), (1e-4, got[1], general[1], exact[1])):
+        for k, (a, b, r) in enumerate(zip(new, old, ref)):
+            e_new, e_old = O.relative_error(a.double(), r), O.relative_error(b.double(), r)
+            print(f"output {k}: {e_new:.2e}, general kernel {e_old:.2e}")
+            assert e_new <= tol + 2.0 * e_old, k
+
+
+def _voxel_case(device, dtype, N, dims, seed, beta, var):
+    g = torch.Generator().manual_seed(seed)
+    r = lambda *s: torch.rand(*s, generator=g, dtype=torch.float64)  # noqa: E731
+    means = r(N, 3) * (torch.tensor(dims, dtype=torch.float64) + 6) - 3
+    q, _ = torch.linalg.qr(r(N, 3, 3) - 0.5)
+    m = q @ torch.diag_embed(torch.exp(4 - 8 * r(N, 3)) * 0.2) @ q.transpose(1, 2)
+    conics = torch.stack([m[:, 0, 0], m[:, 0, 1], m[:, 0, 2], m[:, 1, 1], m[:, 1, 2], m[:, 2, 2]], -1)
+    opac = r(N)
+    opac[:2] = 1e-8
+    if N > 6:
+        conics[2] = 0.0
+        conics[3] = torch.tensor([1.0, 1.5, 0.2, 1.0, 0.1, 1.0])  # indefinite
+    out = [t.to(device, dtype) for t in (means, conics, opac)]
+    betas = (0.6 + 3 * r(N)).to(device, dtype) if beta else None
+    unc = (0.1 * r(N)).to(device, dtype) if var else None
+    v, vv = ((r(*dims[::-1]) - 0.5).to(device, dtype) for _ in range(2))
+    return out, betas, unc, v, vv if var else None
+
+
+def _voxel_run(case, dims, T):
+    (means, conics, opac), betas, unc, v, vv = case
+    n = [-(-d // T) for d in dims]
+    radii = torch.full((opac.numel(), 3), 4 * sum(dims), dtype=torch.int32, device=means.device)
+    _, ids, flat = ops.isect_tiles_3d(means, radii, T, *n)
+    off = ops.isect_offset_encode_3d(ids, *n)
+    args = (means, conics, opac) + (() if betas is None else (betas,))
+    pre = "" if betas is None else "beta_"
+    if unc is None:
+        img = (getattr(ops, pre + "voxelize_to_voxels_fwd")(*args, off, flat, *dims, T),)
+        grads = getattr(ops, pre + "voxelize_to_voxels_bwd_per_gaussian")(*args, off, ids, flat, v, *dims, T)
+    else:
+        img = getattr(ops, pre + "voxelize_to_voxels_mean_var_fwd")(*args, unc, off, flat, *dims, T)
+        grads = getattr(ops, pre + "voxelize_to_voxels_mean_var_bwd_per_gaussian")(
+            *args, off, ids, flat, v, vv, unc, False, *dims, T)
+    return img, [g for g in grads if g is not None]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("beta,var", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("N,dims", [(5, (16, 8, 9)), (90, (37, 21, 30)), (1100, (64, 64, 60))])
+def test_voxel_8_tiles_match_the_general_kernel(device, N, dims, beta, var, dtype):
+    case = _voxel_case(device, dtype, N, dims, N, beta, var)
+    moments = dtype == torch.float32 and not (beta or var)  # its VJP is another kernel
+
+    def run(c, t):
+        img, grads = _voxel_run(c, dims, t)
+        return img, [] if moments else grads
+
+    _compare(run, case, 8, 7)

@@ -643,16 +643,17 @@ int r2s_image_l1_bwd(int dtype, const void* prediction, const void* target,
                      void* grad_prediction, r2s_stream_t stream);
 
 /* The TV (isotropic = 0: anisotropic, eps unused) and L1 forwards with a caller
- * buffer of r2s_loss_partials_bytes() for their workgroup sums: *tv_sum / *l1_sum
- * is summed in double in a fixed order instead of by atomics, so it is
- * reproducible. The maps are those of r2s_volume_tv_fwd, r2s_volume_tv_iso_fwd
- * and r2s_image_l1_fwd. */
+ * buffer of r2s_loss_partials_bytes() for their workgroup sums, added in double in
+ * a fixed order instead of by atomics: *tv / *l1 = sum / divisor and *loss =
+ * lambda * that mean, reproducible. The maps are those of r2s_volume_tv_fwd,
+ * r2s_volume_tv_iso_fwd and r2s_image_l1_fwd. */
 size_t r2s_loss_partials_bytes(void);
 int r2s_volume_tv_fwd_ordered(int dtype, int isotropic, const void* volume, uint32_t B, uint32_t D,
-                              uint32_t H, uint32_t W, double eps, void* tv_map, void* tv_sum,
-                              void* partials, r2s_stream_t stream);
+                              uint32_t H, uint32_t W, double eps, double divisor, double lambda,
+                              void* tv_map, void* tv, void* loss, void* partials, r2s_stream_t stream);
 int r2s_image_l1_fwd_ordered(int dtype, const void* prediction, const void* target, uint64_t n,
-                             void* l1_map, void* l1_sum, void* partials, r2s_stream_t stream);
+                             double divisor, double lambda, void* l1_map, void* l1, void* loss,
+                             void* partials, r2s_stream_t stream);
 
 #ifdef __cplusplus
 }

@@ -111,8 +111,8 @@ SIGNATURES = {
     "r2s_image_l1_fwd": [I32, P, P, U64, P, P, P],
     "r2s_image_l1_bwd": [I32, P, P, P, U64, F, P, P],
     "r2s_loss_partials_bytes": [],
-    "r2s_volume_tv_fwd_ordered": [I32, I32, P, U32, U32, U32, U32, D, P, P, P, P],
-    "r2s_image_l1_fwd_ordered": [I32, P, P, U64, P, P, P, P],
+    "r2s_volume_tv_fwd_ordered": [I32, I32, P, U32, U32, U32, U32, D, D, D, P, P, P, P, P],
+    "r2s_image_l1_fwd_ordered": [I32, P, P, U64, D, D, P, P, P, P, P],
 }
 
 _RESTYPES = {

@@ -694,8 +694,10 @@ def _f32(x) -> float:
     return struct.unpack("f", struct.pack("f", float(x)))[0]
 
 
-def _loss_partials(device) -> Tensor:
-    return torch.empty((be.lib().r2s_loss_partials_bytes(),), dtype=torch.uint8, device=device)
+def _loss_buffers(x: Tensor):
+    """(mean, loss, workspace of the ordered sum) of a loss of x."""
+    partials = torch.empty((be.lib().r2s_loss_partials_bytes(),), dtype=torch.uint8, device=x.device)
+    return x.new_empty(()), x.new_empty(()), partials
 
 
 def volume_loss_fwd(volume, lambda_tv):
@@ -704,15 +706,13 @@ def volume_loss_fwd(volume, lambda_tv):
     dt = _floating(volume)
     B, Dd, H, W = volume.shape
     tv_map = torch.empty_like(volume)
-    tv_sum = volume.new_empty((1,))
-    with _Launch(volume) as L:
-        partials = _loss_partials(volume.device)
-        call("r2s_volume_tv_fwd_ordered", dt, 0, ptr(volume), B, Dd, H, W, 0.0, ptr(tv_map), ptr(tv_sum), ptr(partials),
-             L.stream)
+    tv, loss, partials = _loss_buffers(volume)
     edges = max(B * ((Dd - 1) * H * W + Dd * (H - 1) * W + Dd * H * (W - 1)), 1)
     # the reference divides by float(edge_count) and scales by a float lambda (Loss.cpp:115-153)
-    tv = (tv_sum / _f32(edges)).squeeze()
-    return _f32(lambda_tv) * tv, tv, tv_map
+    with _Launch(volume) as L:
+        call("r2s_volume_tv_fwd_ordered", dt, 0, ptr(volume), B, Dd, H, W, 0.0, _f32(edges), _f32(lambda_tv),
+             ptr(tv_map), ptr(tv), ptr(loss), ptr(partials), L.stream)
+    return loss, tv, tv_map
 
 
 def volume_loss_bwd(volume, grad_output, lambda_tv):
@@ -739,13 +739,11 @@ def volume_loss_iso_fwd(volume, lambda_tv, eps=1e-8):
     _require(float(eps) > 0.0, "eps must be positive")
     B, Dd, H, W = volume.shape
     tv_map = torch.empty_like(volume)
-    tv_sum = volume.new_empty((1,))
+    tv, loss, partials = _loss_buffers(volume)
     with _Launch(volume) as L:
-        partials = _loss_partials(volume.device)
-        call("r2s_volume_tv_fwd_ordered", dt, 1, ptr(volume), B, Dd, H, W, float(eps), ptr(tv_map), ptr(tv_sum),
-             ptr(partials), L.stream)
-    tv = (tv_sum / max(volume.numel(), 1)).squeeze()
-    return (float(lambda_tv) * tv), tv, tv_map
+        call("r2s_volume_tv_fwd_ordered", dt, 1, ptr(volume), B, Dd, H, W, float(eps), float(max(volume.numel(), 1)),
+             float(lambda_tv), ptr(tv_map), ptr(tv), ptr(loss), ptr(partials), L.stream)
+    return loss, tv, tv_map
 
 
 def volume_loss_iso_bwd(volume, grad_output, lambda_tv, eps=1e-8):
@@ -772,13 +770,12 @@ def image_loss_l1_fwd(prediction, target, lambda_l1):
     _require(prediction.shape == target.shape, "prediction and target must have same shape")
     dt = _floating(prediction)
     l1_map = torch.empty_like(prediction)
-    l1_sum = prediction.new_empty((1,))
+    l1, loss, partials = _loss_buffers(prediction)
     with _Launch(prediction) as L:
-        partials = _loss_partials(prediction.device)
-        call("r2s_image_l1_fwd_ordered", dt, ptr(prediction), ptr(target), prediction.numel(), ptr(l1_map),
-             ptr(l1_sum), ptr(partials), L.stream)
-    l1 = (l1_sum / max(prediction.numel(), 1)).squeeze()
-    return _f32(lambda_l1) * l1, l1, l1_map
+        call("r2s_image_l1_fwd_ordered", dt, ptr(prediction), ptr(target), prediction.numel(),
+             float(max(prediction.numel(), 1)), _f32(lambda_l1), ptr(l1_map), ptr(l1), ptr(loss), ptr(partials),
+             L.stream)
+    return loss, l1, l1_map
 
 
 def image_loss_l1_bwd(prediction, target, grad_output, lambda_l1):

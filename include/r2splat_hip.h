@@ -75,6 +75,17 @@ typedef struct r2s_value_check {
 int r2s_value_checks(const r2s_value_check* checks, uint32_t n_checks, uint32_t* flags,
                      r2s_stream_t stream);
 
+/* Words handed to the host while the stream goes on. `host` is pinned memory of
+ * 1 + n words that the GPU can write; it belongs to the call until
+ * r2s_fetch_wait returns. r2s_fetch_begin copies n (at most 64) words of device
+ * memory to host[1..n] once the work launched before it has ended;
+ * r2s_value_checks_begin leaves the flags of a batch of checks there.
+ * r2s_fetch_wait returns when the words have arrived (or the stream failed). */
+int r2s_fetch_begin(const uint32_t* src, uint32_t n, uint32_t* host, r2s_stream_t stream);
+int r2s_value_checks_begin(const r2s_value_check* checks, uint32_t n_checks, uint32_t* host,
+                           r2s_stream_t stream);
+int r2s_fetch_wait(const uint32_t* host, r2s_stream_t stream);
+
 /* ------------------------------------------------------------------------ */
 /* Per-primitive geometry                                                    */
 /* ------------------------------------------------------------------------ */

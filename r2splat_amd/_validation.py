@@ -74,9 +74,15 @@ class ValueChecks:
         self.element(f"{name} must contain only finite values", value, be.CHECK_NONFINITE)
 
     def run(self) -> None:
+        self.begin().report()
+
+    def begin(self) -> "PendingChecks":
+        """Launches the predicates. The caller may launch work that is safe on
+        any values before ``report()``, within a ``with`` block of the result
+        (which waits for the flags also when that work raises)."""
         pending, self._pending = self._pending, []
         if not pending or capturing():
-            return
+            return PendingChecks([], [], [], None)
         native = [i for i, (_, c) in enumerate(pending) if isinstance(c, tuple)]
         device = pending[native[0]][1][0].device if native else None
         for i in list(native):
@@ -85,9 +91,9 @@ class ValueChecks:
                 native.remove(i)
                 pending[i] = (pending[i][0], functools.partial(_element_predicate, value, kind, row))
         reduced = [i for i, (_, c) in enumerate(pending) if callable(c)]
-        parts = []
+        flags = torch.stack([pending[i][1]().reshape(()) for i in reduced]).to(torch.int32) if reduced else None
+        words = []
         if native:
-            flags = torch.empty((len(native),), dtype=torch.int32, device=device)
             with torch.cuda.device(device):
                 for lo in range(0, len(native), be.MAX_VALUE_CHECKS):
                     chunk = native[lo: lo + be.MAX_VALUE_CHECKS]
@@ -96,14 +102,35 @@ class ValueChecks:
                         value, kind, row = pending[i][1]
                         entry.data, entry.n, entry.dtype = value.data_ptr(), value.numel(), be.dtype_code(value.dtype)
                         entry.kind, entry.row = kind, row
-                    be.call("r2s_value_checks", ctypes.addressof(table), len(chunk), flags[lo:].data_ptr(),
-                            be.stream_of(device))
-            parts.append(flags)
-        if reduced:
-            parts.append(torch.stack([pending[i][1]().reshape(()) for i in reduced]).to(torch.int32))
-        values = (torch.cat(parts) if len(parts) > 1 else parts[0]).tolist() if parts else []
-        bad = dict(zip(native + reduced, values))
-        for i, (message, c) in enumerate(pending):
+                    batch = be.HostWords(len(chunk), device)
+                    be.call("r2s_value_checks_begin", ctypes.addressof(table), len(chunk), batch.ptr, batch.stream)
+                    words.append(batch)
+        return PendingChecks(pending, native + reduced, words, flags)
+
+
+class PendingChecks:
+    """A launched batch of ValueChecks: ``report()`` waits for the flags and
+    raises ValueError with the message of the first predicate that holds."""
+
+    def __init__(self, pending, order, words, flags):
+        self._pending, self._order, self._words, self._flags = pending, order, words, flags
+        self._values = []
+
+    def __enter__(self):
+        return self
+
+    def __exit__(self, *exc):
+        self._wait()
+
+    def _wait(self) -> None:
+        while self._words:
+            self._values += self._words.pop(0).wait()
+
+    def report(self) -> None:
+        self._wait()
+        values = self._values + (self._flags.tolist() if self._flags is not None else [])
+        bad = dict(zip(self._order, values))
+        for i, (message, c) in enumerate(self._pending):
             if (c if isinstance(c, bool) else bad[i]):
                 raise ValueError(message)
 

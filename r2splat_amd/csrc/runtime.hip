@@ -1,8 +1,10 @@
 // Error reporting and small utility kernels shared by every entry point.
 #include "common.hpp"
 
+#include <chrono>
 #include <cstdarg>
 #include <limits>
+#include <thread>
 
 namespace r2s {
 
@@ -88,17 +90,18 @@ __global__ void __launch_bounds__(kCheckThreads) value_checks_kernel(ValueCheckT
                                                                      uint32_t* __restrict__ flags) {
     const r2s_value_check& c = table.c[blockIdx.y];
     const bool bad = c.dtype == R2S_F64 ? scan_check<double>(c) : scan_check<float>(c);
-    if (__ballot(bad) != 0 && threadIdx.x % kWave == 0) flags[blockIdx.y] = 1u;
+    // (the flags may lie in pinned host memory: a system-scope store)
+    if (__ballot(bad) != 0 && threadIdx.x % kWave == 0) {
+        __hip_atomic_store(flags + blockIdx.y, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __threadfence_system();
+    }
 }
 
 }  // namespace r2s
 
-extern "C" int r2s_value_checks(const r2s_value_check* checks, uint32_t n_checks, uint32_t* flags,
-                                r2s_stream_t stream) {
-    using namespace r2s;
-    if (n_checks == 0) return R2S_OK;
-    R2S_REQUIRE(checks && flags, "checks and flags must be non-null");
-    R2S_REQUIRE(n_checks <= R2S_MAX_VALUE_CHECKS, "at most %d value checks per call", R2S_MAX_VALUE_CHECKS);
+namespace r2s {
+
+static int launch_checks(const r2s_value_check* checks, uint32_t n_checks, uint32_t* flags, hipStream_t stream) {
     ValueCheckTable table = {};
     uint64_t most = 0;
     for (uint32_t i = 0; i < n_checks; ++i) {
@@ -115,11 +118,95 @@ extern "C" int r2s_value_checks(const r2s_value_check* checks, uint32_t n_checks
         table.c[i] = c;
         most = std::max<uint64_t>(most, c.kind >= R2S_CHECK_ZERO_ROW ? c.n / c.row : c.n);
     }
-    value_checks_clear_kernel<<<1, kWave, 0, stream>>>(n_checks, flags);
-    if (int rc = check_launch("value_checks_clear")) return rc;
     constexpr uint64_t kPerBlock = kCheckThreads * 4;
     const uint64_t want = std::max<uint64_t>(1, (most + kPerBlock - 1) / kPerBlock);
     const uint32_t blocks = uint32_t(std::min<uint64_t>(kCheckBlocks, want));
     value_checks_kernel<<<dim3(blocks, n_checks), kCheckThreads, 0, stream>>>(table, flags);
     return check_launch("value_checks");
+}
+
+// ---------------------------------------------------------------------------
+// Words handed to the host while the stream goes on: a one-wave kernel copies
+// them (or nothing: the value checks set their flags there themselves) to pinned
+// host memory and raises the first word, which the host polls. Against a copy
+// to pageable memory and a stream synchronisation this leaves out the copy
+// launch and the wake-up, and work launched after the hand-over runs while the
+// host waits.
+// ---------------------------------------------------------------------------
+constexpr uint32_t kMaxFetch = 64;
+
+__global__ void __launch_bounds__(kWave)
+fetch_kernel(const uint32_t* __restrict__ src, uint32_t n, uint32_t* host) {
+    if (threadIdx.x < n) __hip_atomic_store(host + 1 + threadIdx.x, src[threadIdx.x], __ATOMIC_RELAXED,
+                                            __HIP_MEMORY_SCOPE_SYSTEM);
+    __threadfence_system();  // one wave: every lane's words precede the first word
+    if (threadIdx.x == 0) __hip_atomic_store(host, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+static int fetch_begin(const uint32_t* src, uint32_t n, uint32_t* host, hipStream_t stream) {
+    __atomic_store_n(host, 0u, __ATOMIC_RELEASE);
+    fetch_kernel<<<1, kWave, 0, stream>>>(src, n, host);
+    return check_launch("fetch");
+}
+
+}  // namespace r2s
+
+extern "C" int r2s_value_checks(const r2s_value_check* checks, uint32_t n_checks, uint32_t* flags,
+                                r2s_stream_t stream) {
+    using namespace r2s;
+    if (n_checks == 0) return R2S_OK;
+    R2S_REQUIRE(checks && flags, "checks and flags must be non-null");
+    R2S_REQUIRE(n_checks <= R2S_MAX_VALUE_CHECKS, "at most %d value checks per call", R2S_MAX_VALUE_CHECKS);
+    value_checks_clear_kernel<<<1, kWave, 0, stream>>>(n_checks, flags);
+    if (int rc = check_launch("value_checks_clear")) return rc;
+    return launch_checks(checks, n_checks, flags, stream);
+}
+
+extern "C" int r2s_value_checks_begin(const r2s_value_check* checks, uint32_t n_checks, uint32_t* host,
+                                      r2s_stream_t stream) {
+    using namespace r2s;
+    R2S_REQUIRE(checks && host, "checks and host must be non-null");
+    R2S_REQUIRE(n_checks > 0 && n_checks <= R2S_MAX_VALUE_CHECKS, "1 to %d value checks per call",
+                R2S_MAX_VALUE_CHECKS);
+    for (uint32_t i = 0; i < n_checks; ++i) host[1 + i] = 0u;
+    if (int rc = launch_checks(checks, n_checks, host + 1, stream)) return rc;
+    return fetch_begin(nullptr, 0, host, stream);
+}
+
+extern "C" int r2s_fetch_begin(const uint32_t* src, uint32_t n, uint32_t* host, r2s_stream_t stream) {
+    using namespace r2s;
+    R2S_REQUIRE(src && host, "src and host must be non-null");
+    R2S_REQUIRE(n > 0 && n <= kMaxFetch, "1 to %u words per call", kMaxFetch);
+    return fetch_begin(src, n, host, stream);
+}
+
+// Polls the first word: without pause for 4 ms (a sleep of 20 us lasts 75 us
+// with the timer's slack: waits of 0.1-0.7 ms ended 45 us late with a spin of
+// 50 us), then every 50 us or so, asking the runtime whether the stream has ended
+// (an error, or all work done) so that a failed launch ends the wait.
+extern "C" int r2s_fetch_wait(const uint32_t* host, r2s_stream_t stream) {
+    using namespace r2s;
+    using clock = std::chrono::steady_clock;
+    R2S_REQUIRE(host, "host must be non-null");
+    const auto raised = [&] { return __atomic_load_n(host, __ATOMIC_ACQUIRE) != 0u; };
+    const auto spin_end = clock::now() + std::chrono::milliseconds(4);
+    do {
+        for (int k = 0; k < 64; ++k) {
+            if (raised()) return R2S_OK;
+            __builtin_ia32_pause();
+        }
+    } while (clock::now() < spin_end);
+    while (!raised()) {
+        const hipError_t e = hipStreamQuery(stream);
+        if (e == hipErrorNotReady) {
+            (void)hipGetLastError();
+            std::this_thread::sleep_for(std::chrono::microseconds(50));
+            continue;
+        }
+        if (e == hipSuccess && hipStreamSynchronize(stream) == hipSuccess && raised()) return R2S_OK;
+        (void)hipGetLastError();
+        set_error("fetch: %s", e == hipSuccess ? "the stream ended without the words" : hipGetErrorString(e));
+        return R2S_ERR_HIP;
+    }
+    return R2S_OK;
 }

@@ -111,8 +111,10 @@ class _Context:
         context._guard.verify()
         return context
 
-    def adjoints(self, named) -> list:
-        """Validates the output adjoints (None stays None) with one value check."""
+    def adjoints(self, named) -> tuple:
+        """The output adjoints (None stays None) and their launched value check,
+        which the backward reports after launching its own kernels (they read
+        any values safely)."""
         checks = check.ValueChecks()
         out = []
         for name, value in named:
@@ -120,8 +122,7 @@ class _Context:
                 value = check.tensor(name, value, self.shape, self.primitives[0])
                 checks.finite(name, value)
             out.append(value)
-        checks.run()
-        return out
+        return out, checks.begin()
 
     def zero_gradients(self) -> ParameterGradients:
         return ParameterGradients(*(None if p is None else torch.zeros_like(p) for p in self.primitives))
@@ -240,6 +241,26 @@ def _drop_state(buffers, eps, radius_clip):
     buffers["recompute"] = (eps, radius_clip)
 
 
+def _fused_config(prims, C, height, width):
+    """(tile edge, forward waves, backward waves) of the configuration for this
+    shape (the explicit calls take the waves; their tile edge stays the operators' 16)."""
+    return fused.config_for_shape(prims[0].shape[0], C, height, width, prims[4] is not None)
+
+
+def _raster_forward(prims, viewmats, Ks, shape, eps, radius_clip):
+    """(state for the VJP, output) of the rasterizer."""
+    means, quats, scales, densities, beta, uncertainty = prims
+    C, height, width = shape
+    if not _use_fused(means):
+        state = _raster_state(prims, viewmats, Ks, width, height, eps, radius_clip)
+        return state, _raster_render(state, prims, shape)
+    _, fwd_waves, bwd_waves = _fused_config(prims, C, height, width)
+    output, f = fused.forward(means, quats, scales, densities, viewmats, Ks, width, height, eps, radius_clip,
+                              waves=fwd_waves, beta=beta, uncertainty=uncertainty)
+    f.fwd_waves, f.bwd_waves = fwd_waves, bwd_waves
+    return {"fused": f}, output
+
+
 def _raster_state(prims, viewmats, Ks, width, height, eps, radius_clip) -> dict:
     """Projection and tile binning: everything the rasterizer and its VJP read."""
     means, quats, scales, densities, beta, uncertainty = prims
@@ -247,9 +268,7 @@ def _raster_state(prims, viewmats, Ks, width, height, eps, radius_clip) -> dict:
     if _use_fused(means):
         f = fused.prepare(means, quats, scales, densities, viewmats, Ks, width, height, eps, radius_clip, beta=beta,
                           uncertainty=uncertainty)
-        # the waves per tile of the configuration for this shape (the tile
-        # edge stays the operators' 16)
-        _, f.fwd_waves, f.bwd_waves = fused.config_for_shape(means.shape[0], C, height, width, beta is not None)
+        _, f.fwd_waves, f.bwd_waves = _fused_config(prims, C, height, width)
         return {"fused": f}
     T = RASTER_TILE
     with stage("project"):
@@ -275,8 +294,6 @@ def _raster_state(prims, viewmats, Ks, width, height, eps, radius_clip) -> dict:
 def _raster_render(b, prims, shape):
     means, _, _, _, beta, uncertainty = prims
     C, height, width = shape
-    if "fused" in b:
-        return fused.render(b["fused"], C, means.device, b["fused"].fwd_waves)
     T = RASTER_TILE
     prefix = "beta_" if beta is not None else ""
     args = (b["mapped"], b["conics"], b["opacity"], b["mus"]) + (() if beta is None else (b["beta2d"],))
@@ -328,8 +345,8 @@ def rasterize_fwd(
         image = means.new_zeros(shape)
         output = image if uncertainty is None else (image, image.clone())
     else:
-        buffers.update(_raster_state(prims, viewmats, Ks, width, height, eps, radius_clip))
-        output = _raster_render(buffers, prims, shape)
+        state, output = _raster_forward(prims, viewmats, Ks, shape, eps, radius_clip)
+        buffers.update(state)
         if recompute:
             _drop_state(buffers, eps, radius_clip)
     return output, _Context("rasterize", shape, prims, buffers, inputs, eps, mode, detach_variance)
@@ -342,15 +359,23 @@ def rasterize_bwd(context: _Context, v_image: Optional[Tensor], v_variance: Opti
     means, quats, scales, densities, beta, uncertainty = context.primitives
     if v_variance is not None and uncertainty is None:
         raise ValueError("v_variance requires uncertainty in the forward call")
-    v_image, v_variance = context.adjoints((("v_image", v_image), ("v_variance", v_variance)))
+    (v_image, v_variance), checks = context.adjoints((("v_image", v_image), ("v_variance", v_variance)))
+    with checks:
+        gradients = _raster_vjp(context, v_image, v_variance)
+    checks.report()
+    return context.close(gradients)
+
+
+def _raster_vjp(context: _Context, v_image, v_variance) -> ParameterGradients:
+    means, quats, scales, densities, beta, uncertainty = context.primitives
     if means.shape[0] == 0 or (v_image is None and v_variance is None):
-        return context.close(context.zero_gradients())
+        return context.zero_gradients()
     if v_image is None:
         v_image = means.new_zeros(context.shape)
     b = context.buffers
     if "recompute" in b:
         _, height, width = context.shape
-        b.update(_raster_state(context.primitives, b["viewmats"], b["Ks"], width, height, *b.pop("recompute")))
+        b = {**b, **_raster_state(context.primitives, b["viewmats"], b["Ks"], width, height, *b["recompute"])}
     if "fused" in b:
         grads = fused.backward(b["fused"], means, quats, scales, densities, b["viewmats"], b["Ks"], v_image,
                                waves=b["fused"].bwd_waves, v_variance=v_variance,
@@ -358,7 +383,7 @@ def rasterize_bwd(context: _Context, v_image: Optional[Tensor], v_variance: Opti
         v_means, v_quats, v_scales, v_densities = grads[:4]
         v_beta = grads[4] if beta is not None else None
         v_uncertainty = grads[-1] if uncertainty is not None else None
-        return context.close(ParameterGradients(v_means, v_quats, v_scales, v_densities, v_beta, v_uncertainty))
+        return ParameterGradients(v_means, v_quats, v_scales, v_densities, v_beta, v_uncertainty)
     _, height, width = context.shape
     T = RASTER_TILE
     prefix = "beta_" if beta is not None else ""
@@ -390,7 +415,7 @@ def rasterize_bwd(context: _Context, v_image: Optional[Tensor], v_variance: Opti
                                                               height, v_mapped.contiguous(), v_cov2d)
         v_quats, v_scales = ops.parameter_transform_bwd(quats, scales, v_covars)
         v_densities = v_opacity.sum(dim=0)
-    return context.close(ParameterGradients(v_means, v_quats, v_scales, v_densities, v_beta, v_uncertainty))
+    return ParameterGradients(v_means, v_quats, v_scales, v_densities, v_beta, v_uncertainty)
 
 
 # ---------------------------------------------------------------------------
@@ -492,14 +517,22 @@ def voxelize_bwd(context: _Context, v_volume: Optional[Tensor], v_variance: Opti
     means, quats, scales, densities, beta, uncertainty = context.primitives
     if v_variance is not None and uncertainty is None:
         raise ValueError("v_variance requires uncertainty in the forward call")
-    v_volume, v_variance = context.adjoints((("v_volume", v_volume), ("v_variance", v_variance)))
+    (v_volume, v_variance), checks = context.adjoints((("v_volume", v_volume), ("v_variance", v_variance)))
+    with checks:
+        gradients = _voxel_vjp(context, v_volume, v_variance)
+    checks.report()
+    return context.close(gradients)
+
+
+def _voxel_vjp(context: _Context, v_volume, v_variance) -> ParameterGradients:
+    means, quats, scales, densities, beta, uncertainty = context.primitives
     if means.shape[0] == 0 or (v_volume is None and v_variance is None):
-        return context.close(context.zero_gradients())
+        return context.zero_gradients()
     if v_volume is None:
         v_volume = means.new_zeros(context.shape)
     b = context.buffers
     if "recompute" in b:
-        b.update(_voxel_state(context.primitives, b, context.shape, *b.pop("recompute")))
+        b = {**b, **_voxel_state(context.primitives, b, context.shape, *b["recompute"])}
     depth, height, width = context.shape
     T = VOXEL_TILE
     prefix = "beta_" if beta is not None else ""
@@ -532,7 +565,7 @@ def voxelize_bwd(context: _Context, v_volume: Optional[Tensor], v_variance: Opti
                                                             height, depth, context.eps, v_mapped.contiguous(),
                                                             v_conics.contiguous())
         v_quats, v_scales = ops.parameter_transform_bwd(quats, scales, v_covars)
-    return context.close(ParameterGradients(v_means, v_quats, v_scales, v_densities, v_beta, v_uncertainty))
+    return ParameterGradients(v_means, v_quats, v_scales, v_densities, v_beta, v_uncertainty)
 
 
 __all__ = ["ParameterGradients", "rasterize_fwd", "rasterize_bwd", "voxelize_fwd", "voxelize_bwd"]

@@ -80,10 +80,27 @@ class FusedForward:
     # for this forward (0: the kernels' default, 8)
     fwd_waves: int = 0
     bwd_waves: int = 0
+    # the counters on their way to the host (a prepare with defer=True), and
+    # the capacity cache's key
+    pending: Optional[be.HostWords] = None
+    key: tuple = ()
 
     @property
     def is_beta(self) -> int:
         return int(self.beta is not None)
+
+    def settle(self) -> bool:
+        """Reads a deferred prepare's counters: whether the intersections fit
+        (if not, the next prepare of this shape has room for them)."""
+        words, self.pending = self.pending, None
+        if words is None:
+            return True
+        self.n_isects, overflow = words.wait()
+        if overflow:
+            CAPACITY.grow(self.key, self.n_isects)
+            return False
+        CAPACITY.settle(self.key, self.n_isects)
+        return True
 
     @property
     def kind(self) -> int:
@@ -120,7 +137,8 @@ def _scratch(C, N, width, height, tile_size, capacity, beta, device):
 
 
 def prepare(means, quats, scales, densities, viewmats, Ks, width, height, eps, radius_clip, *, capacity=None,
-            check=None, tile_size: int = TILE, beta=None, factors=None, uncertainty=None) -> FusedForward:
+            check=None, tile_size: int = TILE, beta=None, factors=None, uncertainty=None,
+            defer: bool = False) -> FusedForward:
     """Primitive order, projection and binning into tile lists (everything but the image). float32, one device.
 
     ``check`` (default: unless the stream is being captured into a graph)
@@ -128,7 +146,9 @@ def prepare(means, quats, scales, densities, viewmats, Ks, width, height, eps, r
     capacity of the last eager call with the same shapes is used and the flag
     is left on the device (``FusedForward.counters[1]``) for the caller.
     ``beta`` [N] selects Beta primitives; ``factors`` = beta_factors(beta)
-    may be passed in to reuse them; ``uncertainty`` [N] adds the variance."""
+    may be passed in to reuse them; ``uncertainty`` [N] adds the variance.
+    ``defer`` leaves the overflow flag (if it is to be read) to the caller:
+    FusedForward.settle(), which has to be called."""
     device = means.device
     C, N = viewmats.shape[0], means.shape[0]
     kind = _kind(beta, uncertainty)
@@ -151,7 +171,6 @@ def prepare(means, quats, scales, densities, viewmats, Ks, width, height, eps, r
     counters = torch.empty((2,), dtype=torch.int32, device=device)
     with torch.cuda.device(device):
         stream = be.stream_of(device)
-        n_isects = -1
         while True:
             scratch = _scratch(C, N, width, height, tile_size, cap, kind, device)
             packed = torch.empty((be.lib().r2s_fused_packed_bytes(C, N, cap, kind),), dtype=torch.uint8,
@@ -162,17 +181,17 @@ def prepare(means, quats, scales, densities, viewmats, Ks, width, height, eps, r
                      scratch.numel(), ptr(packed), ptr(offsets), ptr(tile_order), ptr(record_offsets), ptr(counters),
                      stream)
             del scratch
-            if not check:
+            fwd = FusedForward(packed, offsets, tile_order, record_offsets, counters, cap, -1, width, height,
+                               float(eps), tile_size, beta, ratio, log_grad, uncertainty, key=key)
+            if check:
+                fwd.pending = be.fetch(counters)
+            if defer or fwd.settle():
                 break
-            n_isects, overflow = (int(v) for v in counters.tolist())
-            if not overflow:
-                CAPACITY.settle(key, n_isects)
-                break
-            cap = CAPACITY.grow(key, n_isects)
+            cap = CAPACITY.grow(key, fwd.n_isects)
+            del fwd, packed
     global LAST_COUNTERS
     LAST_COUNTERS = counters
-    return FusedForward(packed, offsets, tile_order, record_offsets, counters, cap, n_isects, width, height,
-                        float(eps), tile_size, beta, ratio, log_grad, uncertainty)
+    return fwd
 
 
 def render(fwd: FusedForward, C: int, device, waves: int = 0):
@@ -192,9 +211,20 @@ def forward(means, quats, scales, densities, viewmats, Ks, width, height, eps, r
             check=None, tile_size: int = TILE, waves: int = 0, beta=None, uncertainty=None):
     """Renders [C, H, W] (with uncertainty: (image, variance)); returns
     (output, FusedForward). float32, contiguous, one device."""
-    fwd = prepare(means, quats, scales, densities, viewmats, Ks, width, height, eps, radius_clip,
-                  capacity=capacity, check=check, tile_size=tile_size, beta=beta, uncertainty=uncertainty)
-    return render(fwd, viewmats.shape[0], means.device, waves), fwd
+    args = (means, quats, scales, densities, viewmats, Ks, width, height, eps, radius_clip)
+    options = dict(check=check, tile_size=tile_size, beta=beta, uncertainty=uncertainty)
+    # the overflow flag travels to the host while the image is rendered (a list
+    # that did not fit counts as empty there)
+    fwd = prepare(*args, capacity=capacity, defer=True, **options)
+    try:
+        output = render(fwd, viewmats.shape[0], means.device, waves)
+    finally:
+        fits = fwd.settle()
+    if not fits:
+        del fwd, output
+        fwd = prepare(*args, **options)
+        output = render(fwd, viewmats.shape[0], means.device, waves)
+    return output, fwd
 
 
 def backward(fwd: FusedForward, means, quats, scales, densities, viewmats, Ks, v_image, waves: int = 0,

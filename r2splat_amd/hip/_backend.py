@@ -52,6 +52,9 @@ SIGNATURES = {
     "r2s_abi_version": [],
     "r2s_last_error": [],
     "r2s_value_checks": [P, U32, P, P],
+    "r2s_value_checks_begin": [P, U32, P, P],
+    "r2s_fetch_begin": [P, U32, P, P],
+    "r2s_fetch_wait": [P, P],
     "r2s_parameter_transform_fwd": [I32, P, P, P, P, U32, P],
     "r2s_parameter_transform_bwd": [I32, P, P, P, P, P, U32, P],
     "r2s_world_to_image_projection_fwd": [I32, P, P, P, P, U32, U32, F, F, P, P, P, U32, U32, P],
@@ -199,6 +202,32 @@ def dtype_code(dtype: torch.dtype) -> int:
 
 def stream_of(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
+
+
+class HostWords:
+    """n int32 words that a stream hands to the host (pinned memory; word 0 is
+    the sign that they are there). ``wait`` has to be called, also when what
+    was launched meanwhile failed: the memory must not be reused before."""
+
+    def __init__(self, n: int, device: torch.device):
+        self.device = device
+        self.stream = stream_of(device)
+        self.host = torch.empty((n + 1,), dtype=torch.int32, pin_memory=True)
+        self.ptr = self.host.data_ptr()
+
+    def wait(self) -> list:
+        with torch.cuda.device(self.device):
+            call("r2s_fetch_wait", self.ptr, self.stream)
+        return self.host.tolist()[1:]
+
+
+def fetch(words: torch.Tensor) -> HostWords:
+    """The int32 words of a small device tensor, on their way to the host after
+    the work launched so far; ``.wait()`` gives them as a list."""
+    out = HostWords(words.numel(), words.device)
+    with torch.cuda.device(words.device):
+        call("r2s_fetch_begin", words.data_ptr(), words.numel(), out.ptr, out.stream)
+    return out
 
 
 def ptr(t) -> int | None:

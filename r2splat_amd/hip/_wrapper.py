@@ -255,7 +255,7 @@ def isect_tiles(means2d, radii, tile_size, n_tiles_dim1, n_tiles_dim0):
         scan_ws = _workspace(be.lib().r2s_scan_workspace_bytes(total), dev)
         call("r2s_isect_tiles_count", dt, ptr(means2d), ptr(radii), rect, C, N, int(tile_size),
              int(n_tiles_dim1), int(n_tiles_dim0), ptr(tiles), ptr(cum), ptr(scan_ws), ptr(d_total), L.stream)
-        n_isects = int(d_total.item())
+        n_isects = be.fetch(d_total).wait()[0]
         isect_ids = torch.empty((n_isects,), dtype=torch.int64, device=dev)
         flatten_ids = torch.empty((n_isects,), dtype=torch.int32, device=dev)
         if n_isects > 0:
@@ -307,7 +307,7 @@ def _isect_tiles_3d(means3d, radii, tile_size, n_tiles_dim2, n_tiles_dim1, n_til
         scan_ws = _workspace(be.lib().r2s_scan_workspace_bytes(N), dev)
         call("r2s_isect_tiles_3d_count", dt, ptr(means3d), ptr(radii), N, int(tile_size), nx, ny, nz,
              ptr(tiles), ptr(cum), ptr(scan_ws), ptr(d_total), L.stream)
-        n_isects = int(d_total.item())
+        n_isects = be.fetch(d_total).wait()[0]
         isect_ids = torch.empty((n_isects,), dtype=torch.int64, device=dev)
         flatten_ids = torch.empty((n_isects,), dtype=torch.int32, device=dev)
         if n_isects > 0:

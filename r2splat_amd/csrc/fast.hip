@@ -246,22 +246,48 @@ __device__ __forceinline__ void row_span(const R& s, float y_base, int T, int& l
     hi = max(lo, int(fh));
 }
 
-// Tile rectangle and row reach of one projected record. The projection
-// writes the rectangle (uint2: x0 | x1 << 16, y0 | y1 << 16, tiles [x0, x1) x
-// [y0, y1), 0 when culled) and, for the direct-placement binning, the reach
-// (float2: the mean row and row_span's half-extent, -1 reaching no row and
-// +inf every row of a tile), so the binning never reads a record to classify
-// an intersection by height.
+// Columns [lo, hi) of a T-column tile starting at x_base that a record can
+// reach: row_span with x and y exchanged.
+template <typename R>
+__device__ __forceinline__ void col_span(const R& s, float x_base, int T, int& lo, int& hi) {
+    R t = s;
+    t.A = s.C;
+    t.C = s.A;
+    t.my = s.mx;
+    row_span(t, x_base, T, lo, hi);
+}
+
+// The raster backward's unit of Beta work: kSegment columns of one row. A record
+// that reaches the columns [lo, hi) of a tile takes `segments` of them from
+// column `first` (a multiple of four, for 16-byte LDS reads).
+constexpr int kSegment = 8;
+__device__ __forceinline__ void col_segments(int lo, int hi, int T, int& first, int& segments) {
+    first = lo & ~3;
+    segments = hi > lo ? (hi - first + kSegment - 1) / kSegment : 0;
+    first = min(first, T - segments * kSegment);
+}
+
+// Tile rectangle and reach of one projected record. The projection writes the
+// rectangle (uint2: x0 | x1 << 16, y0 | y1 << 16, tiles [x0, x1) x [y0, y1), 0
+// when culled) and the reach (the mean row and row_span's half-extent, -1
+// reaching no row and +inf every row of a tile; Beta records, float4: also the
+// mean column and col_span's), so the binning never reads a record to classify
+// an intersection by the work it gives the backward.
+template <bool BETA>
+using Reach = typename std::conditional<BETA, float4, float2>::type;
+
 struct SpanRect {
     uint32_t xr, yr;
-    float my, ext;
+    float my, ext, mx, ext_x;
 };
 
-__device__ __forceinline__ SpanRect load_span(const uint2* __restrict__ rects, const float2* __restrict__ reach,
+__device__ __forceinline__ SpanRect span_rect(uint2 r, float2 e) { return SpanRect{r.x, r.y, e.x, e.y, 0.f, 0.f}; }
+__device__ __forceinline__ SpanRect span_rect(uint2 r, float4 e) { return SpanRect{r.x, r.y, e.x, e.y, e.z, e.w}; }
+
+template <typename E>
+__device__ __forceinline__ SpanRect load_span(const uint2* __restrict__ rects, const E* __restrict__ reach,
                                               size_t i) {
-    const uint2 r = rects[i];
-    const float2 e = reach[i];
-    return SpanRect{r.x, r.y, e.x, e.y};
+    return span_rect(rects[i], reach[i]);
 }
 
 // row_span's extent of a record as a value (-1: no row; +inf: whole tile).
@@ -275,14 +301,37 @@ __device__ __forceinline__ float row_reach(const R& s) {
     return __builtin_amdgcn_sqrtf(e2) * 1.001f + 0.05f;
 }
 
-// Number of tile rows [lo, hi) of a record with mean row my and extent ext
-// that a T-row tile starting at y_base holds (row_span's result).
-__device__ __forceinline__ uint32_t rows_reached(float my, float ext, float y_base, uint32_t T) {
-    if (ext < 0.f) return 0u;
+// col_span's, likewise.
+template <typename R>
+__device__ __forceinline__ float col_reach(const R& s) {
+    R t = s;
+    t.A = s.C;
+    t.C = s.A;
+    return row_reach(t);
+}
+
+// Tile rows [lo, hi) of a record with mean row my and extent ext that a T-row
+// tile starting at y_base holds (row_span's result).
+__device__ __forceinline__ void reach_span(float my, float ext, float y_base, uint32_t T, int& lo, int& hi) {
     const float c = my - y_base - 0.5f;
     const float fl = fminf(fmaxf(ceilf(c - ext), 0.f), float(T));
     const float fh = fminf(fmaxf(floorf(c + ext) + 1.f, 0.f), float(T));
-    return fh > fl ? uint32_t(fh - fl) : 0u;
+    lo = int(fl);
+    hi = ext < 0.f ? lo : max(lo, int(fh));
+}
+
+__device__ __forceinline__ uint32_t rows_reached(float my, float ext, float y_base, uint32_t T) {
+    int lo, hi;
+    reach_span(my, ext, y_base, T, lo, hi);
+    return uint32_t(hi - lo);
+}
+
+// Segments (col_segments) of each row of the tile that a Beta record reaches.
+__device__ __forceinline__ uint32_t segments_reached(float mx, float ext_x, float x_base, uint32_t T) {
+    int lo, hi, first, segments;
+    reach_span(mx, ext_x, x_base, T, lo, hi);
+    col_segments(lo, hi, int(T), first, segments);
+    return uint32_t(segments);
 }
 
 // ---------------------------------------------------------------------------
@@ -611,7 +660,7 @@ fused_project_kernel(const float* __restrict__ means, const PrimFrame* __restric
                      const float* __restrict__ ratio, const float* __restrict__ unc,
                      const CamFrame* __restrict__ cams, uint32_t C, uint32_t W,
                      uint32_t H, float eps, float clip, uint32_t tile_size, uint32_t ntx, uint32_t nty, uint32_t N,
-                     Stored<BETA, VAR>* __restrict__ recs, uint2* __restrict__ rects, float2* __restrict__ reach,
+                     Stored<BETA, VAR>* __restrict__ recs, uint2* __restrict__ rects, Reach<BETA>* __restrict__ reach,
                      uint32_t* __restrict__ counts) {
     const uint32_t n = blockIdx.x * blockDim.x + threadIdx.x;
     if (n >= N) return;
@@ -628,7 +677,8 @@ fused_project_kernel(const float* __restrict__ means, const PrimFrame* __restric
         rec.g = int32_t(idx);
         if constexpr (VAR) rec.unc = uncertainty;
         uint2 rect = make_uint2(0u, 0u);
-        float2 rr = make_float2(0.f, -1.f);
+        Reach<BETA> rr = {};
+        rr.y = -1.f;
         uint32_t count = 0;
         double m2[2], c2[6];
         if (project_f64(cams[c], means + 3 * size_t(n), f.cov, m2, c2)) {
@@ -665,7 +715,12 @@ fused_project_kernel(const float* __restrict__ means, const PrimFrame* __restric
                 tile_span(m2[1], ry, tile_size, nty, y0, y1)) {
                 count = (x1 - x0) * (y1 - y0);
                 rect = make_uint2(x0 | (x1 << 16), y0 | (y1 << 16));
-                rr = make_float2(rec.my, row_reach(rec));
+                rr.x = rec.my;
+                rr.y = row_reach(rec);
+                if constexpr (BETA) {
+                    rr.z = rec.mx;
+                    rr.w = col_reach(rec);
+                }
             }
         }
         if constexpr (BETA)
@@ -834,19 +889,20 @@ fused_list_lengths_kernel(const uint32_t* __restrict__ tm, const uint32_t* __res
 // (row-major within the record's tile rectangle, the order fused_emit_kernel
 // wrote it in; w0 = the record's first emission index). The lists are
 // camera-major, the reference's list layout. Within each chunk of kPackChunk
-// intersections the entries are ordered by the number of tile rows their
-// records reach (descending; ties keep the primitive order), a stable
-// counting sort in LDS: the backward's waves then take 64 records of similar
-// height and loop over no more rows than their tallest record needs.
+// intersections the entries are ordered by the number of tile rows (Beta: of
+// row segments) their records reach (descending; ties keep the primitive order),
+// a stable counting sort in LDS: the backward's waves then take 64 records of
+// similar work and loop over no more rows than their largest record needs.
 constexpr int kPackItems = 4;
 constexpr int kPackThreads = 256;
 constexpr int kPackChunk = kPackItems * kPackThreads;
 constexpr int kPackWaves = kPackThreads / kWave;
-constexpr int kPackClasses = 34;  // rows 0..32 plus "not written"
+constexpr int kPackClasses = 34;  // rows (or segments) 0..32 plus "not written"
 constexpr int kPackSlots = kPackItems * kPackWaves;
 
+template <bool BETA>
 __global__ void __launch_bounds__(kPackThreads)
-fused_pack_kernel(const uint2* __restrict__ rects, const float2* __restrict__ reach,
+fused_pack_kernel(const uint2* __restrict__ rects, const Reach<BETA>* __restrict__ reach,
                   const uint32_t* __restrict__ cum, uint32_t n_recs, uint32_t C, uint32_t nt, uint32_t ntx,
                   uint32_t T, const uint32_t* __restrict__ vals, const uint32_t* __restrict__ tm,
                   const uint32_t* __restrict__ cm, const uint32_t* __restrict__ d_n, uint32_t capacity,
@@ -864,7 +920,10 @@ fused_pack_kernel(const uint2* __restrict__ rects, const float2* __restrict__ re
     const float y_base = float(ty * T);
     const uint32_t wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
     const uint64_t below = (uint64_t(1) << lane) - 1u;
-    const uint32_t skip_cls = T + 1u;
+    const float x_base = float(tx * T);
+    // Beta: up to T^2 / 8 row segments, in fours for 32-pixel tiles
+    const uint32_t shift = BETA && T == 32u ? 2u : 0u, most = BETA ? (T * T / kSegment) >> shift : T;
+    const uint32_t skip_cls = most + 1u;
     for (uint32_t r0 = 0; r0 < len; r0 += kPackChunk) {
         uint32_t v[kPackItems], cls[kPackItems], rank[kPackItems];
 #pragma unroll
@@ -880,8 +939,11 @@ fused_pack_kernel(const uint2* __restrict__ rects, const float2* __restrict__ re
             if (v[q] < n_recs) {
                 rc[q] = rects[v[q]];
                 w0[q] = cum[v[q]];
-                const float2 e = reach[v[q]];
-                cls[q] = T - rows_reached(e.x, e.y, y_base, T);
+                const Reach<BETA> e = reach[v[q]];
+                uint32_t work = rows_reached(e.x, e.y, y_base, T);
+                if constexpr (BETA)
+                    work = (work * segments_reached(e.z, e.w, x_base, T) + (1u << shift) - 1u) >> shift;
+                cls[q] = most - work;
             }
         }
         for (uint32_t i = threadIdx.x; i < uint32_t(kPackClasses * kPackSlots); i += kPackThreads) cnt[i] = 0u;
@@ -937,10 +999,11 @@ fused_pack_kernel(const uint2* __restrict__ rects, const float2* __restrict__ re
 
 // ---------------------------------------------------------------------------
 // Direct placement (the binning used when a camera's bins fit in a small LDS
-// table). Bin = (tile, height class) within a camera, class 0 the tallest
-// records; the packed lists are ordered (camera, tile, class, range, ...):
-// each camera-major tile list holds its records by decreasing height class
-// (the backward's waves take 64 records of similar height). One wave owns a
+// table). Bin = (tile, work class) within a camera, class 0 the records that
+// reach most rows (Beta: row segments) of the tile; the packed lists are ordered
+// (camera, tile, class, range, ...): each camera-major tile list holds its
+// records by decreasing class (the backward's waves take 64 records of similar
+// work). One wave owns a
 // range of R consecutive primitives of one camera, one lane per record, and
 // walks the records' tile rectangles in step (pair k of every lane's
 // rectangle, row-major, at step k):
@@ -955,17 +1018,25 @@ fused_pack_kernel(const uint2* __restrict__ rects, const float2* __restrict__ re
 // Everything is deterministic: counts do not depend on the order of the LDS
 // increments and the placement order is fixed.
 // ---------------------------------------------------------------------------
-constexpr uint32_t kBinClasses = 9;  // heights ceil(8 h / T) = 8 .. 1, then h = 0
+constexpr uint32_t kBinClasses = 9;  // ceil(8 h / T) = 8 .. 1 for h rows (Beta: of T^2 / 8 segments), then none
 
 // (T is 8, 16 or 32: the division is a shift)
-__device__ __forceinline__ uint32_t height_class(const SpanRect& r, uint32_t ty, uint32_t T) {
-    const uint32_t h = rows_reached(r.my, r.ext, float(ty * T), T);
-    return h == 0u ? kBinClasses - 1u : kBinClasses - 1u - ((8u * h + T - 1u) >> (__builtin_ctz(T)));
+__device__ __forceinline__ uint32_t work_class(uint32_t work, uint32_t log2_most) {
+    return work == 0u ? kBinClasses - 1u : kBinClasses - 1u - ((8u * work + (1u << log2_most) - 1u) >> log2_most);
 }
 
 // A lane's walk over its record's tile rectangle, row-major.
+template <bool BETA>
 struct RectWalk {
-    uint32_t x0, x1, tx, ty, cnt, row, cls;
+    uint32_t x0, x1, tx, ty, cnt, row, rows, cls;
+    __device__ __forceinline__ void classify(const SpanRect& r, uint32_t T, bool new_row) {
+        const uint32_t log2_T = uint32_t(__builtin_ctz(T));
+        if (new_row) rows = rows_reached(r.my, r.ext, float(ty * T), T);
+        if constexpr (BETA)
+            cls = work_class(rows * segments_reached(r.mx, r.ext_x, float(tx * T), T), 2u * log2_T - 3u);
+        else if (new_row)
+            cls = work_class(rows, log2_T);
+    }
     __device__ __forceinline__ void start(const SpanRect& r, uint32_t ntx, uint32_t T) {
         x0 = r.xr & 0xffffu;
         x1 = r.xr >> 16;
@@ -974,23 +1045,26 @@ struct RectWalk {
         tx = x0;
         ty = y0;
         row = ty * ntx;
-        cls = cnt ? height_class(r, ty, T) : 0u;
+        rows = cls = 0u;
+        if (cnt) classify(r, T, true);
     }
     __device__ __forceinline__ uint32_t bin() const { return (row + tx) * kBinClasses + cls; }
     __device__ __forceinline__ void advance(const SpanRect& r, uint32_t ntx, uint32_t T) {
-        if (++tx == x1) {
+        const bool new_row = ++tx == x1;
+        if (new_row) {
             tx = x0;
             ++ty;
             row += ntx;
-            cls = height_class(r, ty, T);
         }
+        if (BETA || new_row) classify(r, T, new_row);
     }
 };
 
 // grid (n_ranges, C), one wave; dynamic LDS: n_bins counters. range_totals:
 // the intersections of each (camera, range).
+template <bool BETA>
 __global__ void __launch_bounds__(kWave)
-fused_bin_count_kernel(const uint2* __restrict__ rects, const float2* __restrict__ reach, uint32_t N,
+fused_bin_count_kernel(const uint2* __restrict__ rects, const Reach<BETA>* __restrict__ reach, uint32_t N,
                        uint32_t range_len, uint32_t n_ranges, uint32_t ntx, uint32_t T, uint32_t n_bins,
                        uint32_t* __restrict__ range_counts, uint32_t* __restrict__ range_totals) {
     extern __shared__ uint32_t hist[];
@@ -1001,7 +1075,7 @@ fused_bin_count_kernel(const uint2* __restrict__ rects, const float2* __restrict
     uint32_t total = 0;
     for (uint32_t n = n0 + lane; n < n1; n += kWave) {
         const SpanRect sr = load_span(rects, reach, size_t(cam) * N + n);
-        RectWalk w;
+        RectWalk<BETA> w;
         w.start(sr, ntx, T);
         total += w.cnt;
         for (uint32_t k = 0; k < w.cnt; ++k) {
@@ -1130,8 +1204,9 @@ constexpr uint32_t kTableBatch = 16;  // table entries a lane loads at once
 // grid (n_ranges, C), one wave; dynamic LDS: the n_bins next free slots. Also
 // writes the record offsets: first_isect, the (camera, range)'s first emission
 // index, and a wave scan of the records' tile counts.
+template <bool BETA>
 __global__ void __launch_bounds__(kWave)
-fused_bin_place_kernel(const uint2* __restrict__ rects, const float2* __restrict__ reach,
+fused_bin_place_kernel(const uint2* __restrict__ rects, const Reach<BETA>* __restrict__ reach,
                        uint32_t* __restrict__ cum, uint32_t N, uint32_t range_len, uint32_t n_ranges,
                        uint32_t ntx, uint32_t T, uint32_t n_bins, uint32_t bin_bits,
                        const uint32_t* __restrict__ range_starts, const uint32_t* __restrict__ bin_starts,
@@ -1159,9 +1234,9 @@ fused_bin_place_kernel(const uint2* __restrict__ rects, const float2* __restrict
     for (uint32_t s = n0; s < n1; s += kWave) {
         const uint32_t n = s + lane;
         const size_t idx = size_t(cam) * N + n;
-        SpanRect sr = {0u, 0u, 0.f, -1.f};
+        SpanRect sr = {0u, 0u, 0.f, -1.f, 0.f, -1.f};
         if (n < n1) sr = load_span(rects, reach, idx);
-        RectWalk w;
+        RectWalk<BETA> w;
         w.start(sr, ntx, T);
         const uint32_t incl = wave_scan(w.cnt);
         const uint32_t g = emitted + incl - w.cnt;
@@ -1262,6 +1337,50 @@ __device__ __forceinline__ void settle(const R& s) {
     if constexpr (std::is_same<R, BetaSplat>::value) asm volatile("" ::"v"(s.b2d), "v"(s.unc), "v"(s.lx), "v"(s.ly));
 }
 
+// The Beta forward of a 16-pixel tile: a wave's sixteen groups of four lanes own
+// a 4 x 4 block of pixels each (lane = column, four rows) and walk lists of their
+// own: a batch's records are entered into the list of every block their support
+// can reach (in order, so each pixel's sum is the same as if the wave walked the
+// whole batch), and step k evaluates sixteen (record, block) pairs, one per
+// group. Supports are small against a tile (500k primitives over 512^2 images: 3
+// pixels to a side): walking each record's 4-row bands over all 16 columns
+// evaluates 1.43 bands a record, the lists take 0.28 steps of four pixels a lane.
+struct BlockWalk {
+    static constexpr uint32_t kBlocks = 16, kNone = kWave;  // kNone: the slot of an empty record
+
+    // The blocks (bit 4 band + column block) a record can reach.
+    static __device__ __forceinline__ uint32_t reached(const BetaSplat& s, float x_base, float y_base) {
+        int r_lo, r_hi, c_lo, c_hi;
+        row_span(s, y_base, 16, r_lo, r_hi);
+        col_span(s, x_base, 16, c_lo, c_hi);
+        if (r_lo >= r_hi || c_lo >= c_hi) return 0u;
+        const uint32_t rows = (0xfu >> (3 - ((r_hi - 1) >> 2))) & (0xfu << (r_lo >> 2));
+        const uint32_t cols = (0xfu >> (3 - ((c_hi - 1) >> 2))) & (0xfu << (c_lo >> 2));
+        const uint32_t spread = (rows & 1u) | ((rows & 2u) << 3) | ((rows & 4u) << 6) | ((rows & 8u) << 9);
+        return spread * cols;
+    }
+
+    // Fills lists[block][k] (bytes; kNone past a block's end) from the lanes'
+    // block masks; returns the longest list.
+    static __device__ __forceinline__ uint32_t fill(uint32_t blocks, uint32_t lane, uint8_t (*lists)[kWave]) {
+        constexpr uint32_t kFill = kNone * 0x01010101u;
+        reinterpret_cast<uint4*>(lists)[lane] = make_uint4(kFill, kFill, kFill, kFill);
+        wave_lds_sync();
+        uint32_t longest = 0;
+#pragma unroll
+        for (uint32_t b = 0; b < kBlocks; ++b) {
+            const bool in = (blocks >> b) & 1u;
+            const uint64_t members = __ballot(in);
+            const uint32_t at = __builtin_amdgcn_mbcnt_hi(uint32_t(members >> 32),
+                                                          __builtin_amdgcn_mbcnt_lo(uint32_t(members), 0u));
+            if (in) lists[b][at] = uint8_t(lane);
+            longest = max(longest, uint32_t(__popcll(members)));
+        }
+        wave_lds_sync();
+        return longest;
+    }
+};
+
 // One tile of the forward: the workgroup renders the tile at position `pos`
 // of the tile order (or tile `pos` without one).
 template <int T, int WAVES, bool BETA, bool VAR>
@@ -1274,9 +1393,15 @@ __device__ __forceinline__ void raster_fwd_tile(const uint2* __restrict__ entrie
                                                 float* __restrict__ out_var, uint32_t pos) {
     constexpr int PX = T * T / kWave, STEP = kWave / T;
     static_assert(PX * kWave == T * T && STEP * T == kWave, "tile must be 8, 16 or 32");
-    __shared__ float part[WAVES][T * T];  // the slices' partial images (mean, then variance)
+    constexpr bool BLOCKS = BETA && T == 16;  // blocks of 4 x 4 pixels with lists of their own (BlockWalk)
     using R = Rec<BETA, VAR>;
-    __shared__ R stage[WAVES][kWave];
+    __shared__ R stage[WAVES][kWave + (BLOCKS ? 1 : 0)];
+    // the slices' partial images (mean, then variance); with blocks in the stages'
+    // place (two workgroups of 16 waves then fit a compute unit)
+    __shared__ float own_part[BLOCKS ? 1 : WAVES][T * T];
+    auto* part = BLOCKS ? reinterpret_cast<float(*)[T * T]>(stage) : own_part;
+    static_assert(sizeof(stage) >= (BLOCKS ? WAVES * T * T * sizeof(float) : 0), "the partial images fit the stages");
+    __shared__ __align__(16) uint8_t lists[BLOCKS ? WAVES : 1][BLOCKS ? BlockWalk::kBlocks : 1][kWave];
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const uint32_t tile = order ? order[pos] : pos;
     const uint32_t n_live = live(d_n, capacity);
@@ -1290,12 +1415,15 @@ __device__ __forceinline__ void raster_fwd_tile(const uint2* __restrict__ entrie
     const int32_t lo = start + int32_t(wave) * kWave, hi = end;
     const uint32_t nt = ntx * nty, cam = tile / nt, t = tile - cam * nt;
     const uint32_t ty = t / ntx, tx = t - ty * ntx;
-    const uint32_t lane = threadIdx.x % kWave, col = lane % T, row0 = lane / T;
+    const uint32_t lane = threadIdx.x % kWave;
+    // the lane's pixels: column col, rows row0 + row_step k
+    const uint32_t col = BLOCKS ? lane % 16u : lane % T, row0 = BLOCKS ? lane / 16u * 4u : lane / T;
+    constexpr uint32_t row_step = BLOCKS ? 1u : uint32_t(STEP);
     const float px = float(tx * T + col) + 0.5f;
     float py[PX], acc[PX], acc_var[PX];
 #pragma unroll
     for (int k = 0; k < PX; ++k) {
-        py[k] = float(ty * T + row0 + STEP * k) + 0.5f;
+        py[k] = float(ty * T + row0 + row_step * k) + 0.5f;
         acc[k] = 0.f;
         acc_var[k] = 0.f;
     }
@@ -1305,15 +1433,22 @@ __device__ __forceinline__ void raster_fwd_tile(const uint2* __restrict__ entrie
     uint2 ahead = load_entry(entries, lo + int32_t(lane), hi);
     R next = gather_splat<R>(recs, ahead);
     ahead = load_entry(entries, lo + kStride + int32_t(lane), hi);
-    const float y_base = float(ty * T);
+    const float y_base = float(ty * T), x_base = float(tx * T);
+    if constexpr (BLOCKS) {
+        if (lane == 0) slot[BlockWalk::kNone] = R{};  // contributes nowhere (qlim = 0)
+    }
     for (int32_t base = lo; base < hi; base += kStride) {
         // row groups of the record this lane stages (lane rows are row0 + STEP k,
         // row0 < STEP); record j's span is read from lane j's register
-        int r_lo, r_hi;
-        row_span(next, y_base, T, r_lo, r_hi);
-        const int k_lo = r_lo / STEP, k_hi = (r_hi + STEP - 1) / STEP;  // groups [k_lo, k_hi)
-        const uint32_t spans = r_lo < r_hi ? ((k_hi >= 32 ? 0xffffffffu : (1u << k_hi) - 1u) & ~((1u << k_lo) - 1u))
-                                           : 0u;
+        uint32_t spans;
+        if constexpr (BLOCKS) {
+            spans = base + int32_t(lane) < hi ? BlockWalk::reached(next, x_base, y_base) : 0u;
+        } else {
+            int r_lo, r_hi;
+            row_span(next, y_base, T, r_lo, r_hi);
+            const int k_lo = r_lo / STEP, k_hi = (r_hi + STEP - 1) / STEP;  // groups [k_lo, k_hi)
+            spans = r_lo < r_hi ? ((k_hi >= 32 ? 0xffffffffu : (1u << k_hi) - 1u) & ~((1u << k_lo) - 1u)) : 0u;
+        }
         wave_lds_sync();  // every lane is done reading the previous batch
         if constexpr (VAR) {
             // the staged copy's uncertainty field carries the record's variance
@@ -1327,6 +1462,18 @@ __device__ __forceinline__ void raster_fwd_tile(const uint2* __restrict__ entrie
         wave_lds_sync();
         next = gather_splat<R>(recs, ahead);
         ahead = load_entry(entries, base + 2 * kStride + int32_t(lane), hi);
+        if constexpr (BLOCKS) {
+            // (block of lane = band lane / 16, column block lane % 16 / 4)
+            const uint32_t longest = BlockWalk::fill(spans, lane, lists[wave]);
+            const uint32_t* list = reinterpret_cast<const uint32_t*>(lists[wave][lane / 4u]);
+            for (uint32_t k = 0; k < longest; k += 4) {
+                uint32_t four = list[k / 4u];
+                const uint32_t steps = min(longest - k, 4u);
+                for (uint32_t j = 0; j < steps; ++j, four >>= 8)
+                    splat_accumulate<PX, BETA, VAR>(slot[four & 0xffu], (1u << PX) - 1u, px, py, acc, acc_var);
+            }
+            continue;
+        }
         const int32_t n = min(int32_t(kWave), hi - base);
         // LDS reads pipelined one record ahead in two registers that alternate
         // roles (no copies between them); the batch holds n >= 1 records
@@ -1344,8 +1491,9 @@ __device__ __forceinline__ void raster_fwd_tile(const uint2* __restrict__ entrie
             if (++j >= n) break;
         }
     }
+    if constexpr (BLOCKS) __syncthreads();  // every wave is done with its stage
 #pragma unroll
-    for (int k = 0; k < PX; ++k) part[wave][(row0 + STEP * k) * T + col] = acc[k];
+    for (int k = 0; k < PX; ++k) part[wave][(row0 + row_step * k) * T + col] = acc[k];
     __syncthreads();
     for (uint32_t p = threadIdx.x; p < uint32_t(T * T); p += WAVES * kWave) {
         float v = 0.f;
@@ -1357,7 +1505,7 @@ __device__ __forceinline__ void raster_fwd_tile(const uint2* __restrict__ entrie
     if constexpr (VAR) {
         __syncthreads();  // the mean's partial images are consumed
 #pragma unroll
-        for (int k = 0; k < PX; ++k) part[wave][(row0 + STEP * k) * T + col] = acc_var[k];
+        for (int k = 0; k < PX; ++k) part[wave][(row0 + row_step * k) * T + col] = acc_var[k];
         __syncthreads();
         for (uint32_t p = threadIdx.x; p < uint32_t(T * T); p += WAVES * kWave) {
             float v = 0.f;
@@ -1457,20 +1605,36 @@ __device__ __forceinline__ void raster_bwd_tile(const uint2* __restrict__ entrie
         if (active) row_span(s, y0 - 0.5f, T, r_lo, r_hi);
         // Beta: pairs below lim.x pass; those in [lim.x, lim.y) are settled in double
         const uint2 lim = (BETA && active) ? edge_limits(s) : make_uint2(0u, 0u);
-        // the columns' offsets and their squares are the same in every row
-        float dxc[T], dxsq[T];
-#pragma unroll
-        for (int j = 0; j < T; ++j) {
-            dxc[j] = dx0 + float(j);
-            dxsq[j] = dxc[j] * dxc[j];
+        // Beta: kSegment columns of a row at a time, segments from column c (a
+        // support of 500k primitives over 512^2 images covers 3 columns to a side,
+        // 20% of the 16-column rows it reaches)
+        int c = 0, segments = 1;
+        if constexpr (BETA) {
+            int c_lo = 0, c_hi = 0;
+            if (r_lo < r_hi) col_span(s, x0 - 0.5f, T, c_lo, c_hi);
+            col_segments(c_lo, c_hi, T, c, segments);
         }
-        for (int r = r_lo; r < r_hi; ++r) {
+        constexpr int COLS = BETA ? kSegment : T;
+        // the columns' offsets and their squares are the same in every row
+        float dxc[COLS], dxsq[COLS];
+        const auto columns = [&](float first) {
+#pragma unroll
+            for (int j = 0; j < COLS; ++j) {
+                dxc[j] = dx0 + (first + float(j));
+                dxsq[j] = dxc[j] * dxc[j];
+            }
+        };
+        columns(float(c));
+        const int c0 = c, c_end = c + segments * COLS;
+        int r = r_lo;
+        float r0 = 0.f, r1 = 0.f, r2 = 0.f;  // the row's moments in x, summed over its columns in order
+        for (int left = (r_hi - r_lo) * segments; left > 0; --left) {
             const float dy = offset_y<BETA>(s, y0 + float(r));
             const float bdy = s.B * dy, cdy2 = s.C * dy * dy;
-            const float4* row = reinterpret_cast<const float4*>(sv[0] + r * T);
-            float v[T], vv[VAR ? T : 1];
+            const float4* row = reinterpret_cast<const float4*>(sv[0] + r * T + c);
+            float v[COLS], vv[VAR ? COLS : 1];
 #pragma unroll
-            for (int k = 0; k < T / 4; ++k) {
+            for (int k = 0; k < COLS / 4; ++k) {
                 const float4 q4 = row[k];
                 v[4 * k] = q4.x;
                 v[4 * k + 1] = q4.y;
@@ -1478,9 +1642,9 @@ __device__ __forceinline__ void raster_bwd_tile(const uint2* __restrict__ entrie
                 v[4 * k + 3] = q4.w;
             }
             if constexpr (VAR) {
-                const float4* rowv = reinterpret_cast<const float4*>(sv[VAR ? 1 : 0] + r * T);
+                const float4* rowv = reinterpret_cast<const float4*>(sv[VAR ? 1 : 0] + r * T + c);
 #pragma unroll
-                for (int k = 0; k < T / 4; ++k) {
+                for (int k = 0; k < COLS / 4; ++k) {
                     const float4 q4 = rowv[k];
                     vv[4 * k] = q4.x;
                     vv[4 * k + 1] = q4.y;
@@ -1488,7 +1652,6 @@ __device__ __forceinline__ void raster_bwd_tile(const uint2* __restrict__ entrie
                     vv[4 * k + 3] = q4.w;
                 }
             }
-            float r0 = 0.f, r1 = 0.f, r2 = 0.f;
             // one Beta pair's terms (in: it passes the cut-off). h is clamped to
             // the smallest normal float (outside the support 1 - q <= 0), so log2 h
             // is finite and a pair that fails the cut-off (hb = 0, so ve = 0) adds
@@ -1514,15 +1677,15 @@ __device__ __forceinline__ void raster_bwd_tile(const uint2* __restrict__ entrie
                 r1 = fmaf(g, dx, r1);
                 r2 = fmaf(g, dxsq_j, r2);
             };
-            bool any_near = false;  // Beta: a pair of this row lies in the edge band
+            bool any_near = false;  // Beta: a pair of this segment lies in the edge band
 #pragma unroll
-            for (int j = 0; j < T; ++j) {
-                const float dx = dxc[j];
+            for (int j = 0; j < COLS; ++j) {
+                const float dx = dxc[j], dx2 = dxsq[j];
                 const float q = form_by_rows(s.A, dx, bdy, cdy2);
                 if constexpr (BETA) {
                     const bool in = contributes(q, lim.x);
                     any_near = any_near || (!in && contributes(q, lim.y));
-                    beta_pair(q, dx, dxsq[j], v[j], VAR ? vv[VAR ? j : 0] : 0.f, in);
+                    beta_pair(q, dx, dx2, v[j], VAR ? vv[VAR ? j : 0] : 0.f, in);
                 } else {
                     const float e = contributes(q, s.qlim) ? __builtin_amdgcn_exp2f(-q) : 0.f;
                     float g;
@@ -1536,14 +1699,14 @@ __device__ __forceinline__ void raster_bwd_tile(const uint2* __restrict__ entrie
                     }
                     r0 += g;
                     r1 = fmaf(g, dx, r1);
-                    r2 = fmaf(g, dxsq[j], r2);
+                    r2 = fmaf(g, dx2, r2);
                 }
             }
             if constexpr (BETA) {
-                // the pairs of this row in the edge band, settled in double (rare)
+                // the pairs of this segment in the edge band, settled in double (rare)
                 if (__builtin_expect(__ballot(any_near) != 0ull, 0) && any_near) {
 #pragma unroll 1
-                    for (int j = 0; j < T; ++j) {
+                    for (int j = c; j < c + COLS; ++j) {
                         const float dx = dx0 + float(j);
                         const float q = form_by_rows(s.A, dx, bdy, cdy2);
                         if (!contributes(q, lim.x) && contributes(q, lim.y) &&
@@ -1552,12 +1715,21 @@ __device__ __forceinline__ void raster_bwd_tile(const uint2* __restrict__ entrie
                     }
                 }
             }
+            if constexpr (BETA) {
+                c += COLS;
+                const bool more = c < c_end;  // another segment of this row
+                if (!more) c = c0;
+                if (segments > 1) columns(float(c));
+                if (more) continue;
+            }
             m0 += r0;
             mx += r1;
             mxx += r2;
             my = fmaf(dy, r0, my);
             mxy = fmaf(dy, r1, mxy);
             myy = fmaf(dy * dy, r0, myy);
+            r0 = r1 = r2 = 0.f;
+            ++r;
         }
         if (active && s.g >= 0 && uint32_t(s.g) < n_live) {
             float* out = isect_grads + kPartialStride * size_t(s.g);
@@ -1965,7 +2137,7 @@ static FusedScratch fused_scratch(uint32_t C, uint32_t N, uint32_t n_tiles, uint
     L.frames = o; o += al(size_t(N) * sizeof(PrimFrame));
     L.cams = o; o += al(size_t(C) * sizeof(CamFrame));
     L.rects = o; o += al(CN * sizeof(uint2));
-    L.reach = o; o += al(CN * sizeof(float2));
+    L.reach = o; o += al(CN * ((kind & kKindBeta) ? sizeof(Reach<true>) : sizeof(Reach<false>)));
     const uint64_t nt = C ? n_tiles / C : 0;
     const size_t table = nt * kBinClasses * sizeof(uint32_t);
     if (C > 0 && nt > 0 && table <= kPlaceLargeBytes) {
@@ -2173,7 +2345,7 @@ static int prepare_impl(const float* means, const float* quats, const float* sca
         dim3 grid(ceil_div(N, 256), ceil_div(C, kProjectCams));
         fused_project_kernel<BETA, VAR><<<grid, 256, 0, stream>>>(
             p_means, p_frames, p_dens, p_betas, p_ratio, p_unc, cams, C, width, height, eps, radius_clip,
-            tile_size, ntx, nty, N, recs, at<uint2>(scratch, L.rects), at<float2>(scratch, L.reach), L.place ? nullptr : cum);
+            tile_size, ntx, nty, N, recs, at<uint2>(scratch, L.rects), at<Reach<BETA>>(scratch, L.reach), L.place ? nullptr : cum);
         if (int rc = check_launch("fused_project")) return rc;
     }
     if (L.place) {
@@ -2183,8 +2355,8 @@ static int prepare_impl(const float* means, const float* quats, const float* sca
         const size_t lds = size_t(L.n_bins) * sizeof(uint32_t);
         const dim3 grid(L.n_ranges, C);
         if (CN > 0) {
-            fused_bin_count_kernel<<<grid, kWave, lds, stream>>>(
-                at<uint2>(scratch, L.rects), at<float2>(scratch, L.reach), N, L.range_len, L.n_ranges, ntx, tile_size,
+            fused_bin_count_kernel<BETA><<<grid, kWave, lds, stream>>>(
+                at<uint2>(scratch, L.rects), at<Reach<BETA>>(scratch, L.reach), N, L.range_len, L.n_ranges, ntx, tile_size,
                 L.n_bins, range_counts, range_totals);
             if (int rc = check_launch("fused_bin_count")) return rc;
         }
@@ -2194,8 +2366,8 @@ static int prepare_impl(const float* means, const float* quats, const float* sca
         fused_bin_starts_kernel<<<C, kScanThreads, 0, stream>>>(totals, L.n_bins, range_totals, L.n_ranges);
         if (int rc = check_launch("fused_bin_starts")) return rc;
         if (CN > 0) {
-            fused_bin_place_kernel<<<grid, kWave, lds, stream>>>(
-                at<uint2>(scratch, L.rects), at<float2>(scratch, L.reach), cum, N,
+            fused_bin_place_kernel<BETA><<<grid, kWave, lds, stream>>>(
+                at<uint2>(scratch, L.rects), at<Reach<BETA>>(scratch, L.reach), cum, N,
                 L.range_len, L.n_ranges, ntx, tile_size, L.n_bins, L.bin_bits, range_counts, totals, range_totals,
                 capacity, entries);
             if (int rc = check_launch("fused_bin_place")) return rc;
@@ -2233,8 +2405,8 @@ static int prepare_impl(const float* means, const float* quats, const float* sca
                                 stream))
         return rc;
     const uint32_t pack_blocks = (n_tiles + 7u) & ~7u;  // a multiple of the 8 XCDs
-    fused_pack_kernel<<<pack_blocks, kPackThreads, 0, stream>>>(
-        at<uint2>(scratch, L.rects), at<float2>(scratch, L.reach), cum, CN, C, ntx * nty, ntx, tile_size, vals, tm,
+    fused_pack_kernel<BETA><<<pack_blocks, kPackThreads, 0, stream>>>(
+        at<uint2>(scratch, L.rects), at<Reach<BETA>>(scratch, L.reach), cum, CN, C, ntx * nty, ntx, tile_size, vals, tm,
         cm, counters, capacity, entries, tile_offsets);
     if (int rc = check_launch("fused_pack")) return rc;
     }

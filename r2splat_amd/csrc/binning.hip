@@ -157,27 +157,27 @@ scan_reduce_kernel(const uint32_t* __restrict__ in, uint32_t n, uint32_t* __rest
 // *d_total when given).
 template <int THREADS, int ITEMS>
 __global__ void __launch_bounds__(THREADS)
-scan_tile_kernel(const uint32_t* __restrict__ in, uint32_t n, const uint32_t* __restrict__ base,
-                 uint32_t* __restrict__ out, uint32_t* __restrict__ d_total) {
+scan_tile_kernel(const uint32_t* in, uint32_t n, const uint32_t* __restrict__ base, uint32_t* out,
+                 uint32_t* __restrict__ d_total) {
     constexpr uint32_t kTile = uint32_t(THREADS) * ITEMS;
     __shared__ uint32_t lds[THREADS / kWave];
     const size_t tile0 = size_t(blockIdx.x) * kTile;
     const size_t t0 = tile0 + size_t(threadIdx.x) * ITEMS;
     uint32_t v[ITEMS], s = 0;
+    load_run<ITEMS>(in, t0, n, runs_aligned(in), v);
 #pragma unroll
-    for (int k = 0; k < ITEMS; ++k) {
-        v[k] = (t0 + k < n) ? in[t0 + k] : 0u;
-        s += v[k];
-    }
+    for (int k = 0; k < ITEMS; ++k) s += v[k];
     uint32_t excl;
     const uint32_t total = block_exclusive_scan(s, excl, lds);
     const uint32_t b = base ? base[blockIdx.x] : 0u;
     uint32_t run = b + excl;
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
-        if (t0 + k < n) out[t0 + k] = run;
-        run += v[k];
+        const uint32_t x = v[k];
+        v[k] = run;
+        run += x;
     }
+    store_run<ITEMS>(out, t0, n, runs_aligned(out), v);
     const bool last_block = (tile0 + kTile >= n);
     if (last_block && threadIdx.x == 0) {
         out[n] = b + total;

@@ -128,4 +128,43 @@ __device__ __forceinline__ uint64_t wave_match(uint32_t value, uint32_t bits, ui
 template <typename S>
 __device__ __forceinline__ void atomic_add(S* p, S v) { atomicAdd(p, v); }
 
+// ITEMS consecutive words of a thread's run, from word i of p (0 past word n), and
+// back. A run loaded word by word costs each instruction a cache line per lane
+// (a one-workgroup scan of 12k words took 10 us); where p + i and p + i + ITEMS are
+// 16-byte aligned (i is a multiple of ITEMS, so p decides) and the run is whole, it
+// moves in 16-byte pieces.
+__device__ __forceinline__ bool runs_aligned(const uint32_t* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
+
+template <int ITEMS>
+__device__ __forceinline__ void load_run(const uint32_t* __restrict__ p, size_t i, size_t n, bool aligned,
+                                         uint32_t (&v)[ITEMS]) {
+    static_assert(ITEMS % 4 == 0, "whole 16-byte pieces");
+    if (aligned && i + ITEMS <= n) {
+#pragma unroll
+        for (int k = 0; k < ITEMS; k += 4) {
+            const uint4 q = *reinterpret_cast<const uint4*>(p + i + k);
+            v[k] = q.x;
+            v[k + 1] = q.y;
+            v[k + 2] = q.z;
+            v[k + 3] = q.w;
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < ITEMS; ++k) v[k] = i + k < n ? p[i + k] : 0u;
+    }
+}
+template <int ITEMS>
+__device__ __forceinline__ void store_run(uint32_t* __restrict__ p, size_t i, size_t n, bool aligned,
+                                          const uint32_t (&v)[ITEMS]) {
+    if (aligned && i + ITEMS <= n) {
+#pragma unroll
+        for (int k = 0; k < ITEMS; k += 4)
+            *reinterpret_cast<uint4*>(p + i + k) = make_uint4(v[k], v[k + 1], v[k + 2], v[k + 3]);
+    } else {
+#pragma unroll
+        for (int k = 0; k < ITEMS; ++k)
+            if (i + k < n) p[i + k] = v[k];
+    }
+}
+
 }  // namespace r2s

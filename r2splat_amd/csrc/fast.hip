@@ -1096,16 +1096,15 @@ constexpr uint32_t kScanThreads = 512, kScanPer = 8;
 
 __device__ __forceinline__ uint32_t scan_in_place(uint32_t* __restrict__ v, uint32_t n, uint32_t base,
                                                   uint32_t* lds_waves) {
+    const bool aligned = runs_aligned(v);
     const uint32_t lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
     uint32_t carry = base;
     for (uint32_t r = 0; r < n; r += kScanThreads * kScanPer) {
         const uint32_t i0 = r + threadIdx.x * kScanPer;
         uint32_t x[kScanPer], sum = 0;
+        load_run<int(kScanPer)>(v, i0, n, aligned, x);
 #pragma unroll
-        for (uint32_t j = 0; j < kScanPer; ++j) {
-            x[j] = i0 + j < n ? v[i0 + j] : 0u;
-            sum += x[j];
-        }
+        for (uint32_t j = 0; j < kScanPer; ++j) sum += x[j];
         const uint32_t incl = wave_scan(sum);
         if (lane == kWave - 1) lds_waves[wave] = incl;
         __syncthreads();
@@ -1118,9 +1117,11 @@ __device__ __forceinline__ uint32_t scan_in_place(uint32_t* __restrict__ v, uint
         uint32_t run = carry + before + incl - sum;
 #pragma unroll
         for (uint32_t j = 0; j < kScanPer; ++j) {
-            if (i0 + j < n) v[i0 + j] = run;
-            run += x[j];
+            const uint32_t y = x[j];
+            x[j] = run;
+            run += y;
         }
+        store_run<int(kScanPer)>(v, i0, n, aligned, x);
         carry += total;
         __syncthreads();  // lds_waves is reused
     }

@@ -666,6 +666,28 @@ int r2s_image_l1_fwd_ordered(int dtype, const void* prediction, const void* targ
                              double divisor, double lambda, void* l1_map, void* l1, void* loss,
                              void* partials, r2s_stream_t stream);
 
+/* Voxelization in one call per phase: what r2s_parameter_transform_fwd,
+ * r2s_world_to_volume_mapping_fwd, r2s_voxel_frame (frame and its double-precision
+ * volume frame given: float32 only) and r2s_isect_tiles_3d_count (cum: N + 1 words)
+ * compute, the intersection count handed to the host (`host` as for
+ * r2s_fetch_begin, one word); then the sorted lists and their tile offsets; and the
+ * VJPs of the volume mapping and of the parameter transform (v_covars: N x 6
+ * workspace). */
+int r2s_voxel_prepare(int dtype, const void* means, const void* quats, const void* scales, const void* ranges,
+                      const void* centers, const double* ranges64, const double* centers64, uint32_t dim_x,
+                      uint32_t dim_y, uint32_t dim_z, double eps, double radius_clip, uint32_t tile_size,
+                      uint32_t n_tiles_x, uint32_t n_tiles_y, uint32_t n_tiles_z, uint32_t N, void* covars,
+                      void* means3d_v, void* conics, int32_t* radii, double* frame, uint32_t* cum, void* scan_ws,
+                      uint32_t* host, r2s_stream_t stream);
+int r2s_voxel_lists(int dtype, const void* means3d, const int32_t* radii, uint32_t N, uint32_t tile_size,
+                    uint32_t n_tiles_x, uint32_t n_tiles_y, uint32_t n_tiles_z, const uint32_t* cum,
+                    uint32_t n_isects, int64_t* isect_ids, int32_t* flatten_ids, void* sort_ws,
+                    size_t sort_ws_bytes, int32_t* offsets, r2s_stream_t stream);
+int r2s_voxel_param_vjp(int dtype, const void* means, const void* quats, const void* scales, const void* covars,
+                        const void* ranges, const void* centers, uint32_t dim_x, uint32_t dim_y, uint32_t dim_z,
+                        double eps, const void* v_means3d_v, const void* v_conics, void* v_covars, void* v_means,
+                        void* v_quats, void* v_scales, uint32_t N, r2s_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -555,3 +555,13 @@ extern "C" int r2s_isect_offset_encode(const int64_t* isect_ids, uint32_t n_isec
     offset_encode_kernel<<<ceil_div(n_keys, 256), 256, 0, stream>>>(isect_ids, n_isects, n_keys, offsets);
     return check_launch("isect_offset_encode");
 }
+
+extern "C" int r2s_voxel_lists(int dtype, const void* means3d, const int32_t* radii, uint32_t N, uint32_t tile_size,
+                               uint32_t n_tiles_x, uint32_t n_tiles_y, uint32_t n_tiles_z, const uint32_t* cum,
+                               uint32_t n_isects, int64_t* isect_ids, int32_t* flatten_ids, void* sort_ws,
+                               size_t sort_ws_bytes, int32_t* offsets, r2s_stream_t stream) {
+    if (int rc = r2s_isect_tiles_3d_emit(dtype, means3d, radii, N, tile_size, n_tiles_x, n_tiles_y, n_tiles_z, cum,
+                                         n_isects, isect_ids, flatten_ids, sort_ws, sort_ws_bytes, stream))
+        return rc;
+    return r2s_isect_offset_encode(isect_ids, n_isects, n_tiles_x * n_tiles_y * n_tiles_z, offsets, stream);
+}

@@ -30,6 +30,8 @@ constexpr uint32_t kIsectBlocks = 1u << 16;
 // ---------------------------------------------------------------------------
 void set_error(const char* fmt, ...);
 int check_launch(const char* where);
+// Copies n words of device memory to host[1..n] (pinned) behind the stream's work, then raises host[0].
+int fetch_begin(const uint32_t* src, uint32_t n, uint32_t* host, hipStream_t stream);
 
 #define R2S_REQUIRE(cond, ...)                 \
     do {                                       \

@@ -4,6 +4,9 @@
 //
 // Semantics follow the reference operators (files cited per kernel); the 2x2
 // and 3x3 covariance inversions run in double precision for every dtype.
+#include <type_traits>
+
+#include "binning.hpp"
 #include "common.hpp"
 #include "geometry_common.hpp"
 
@@ -173,6 +176,39 @@ beta_factors_kernel(const S* __restrict__ betas, uint64_t n, S* __restrict__ rat
     if (log_grad) log_grad[i] = S(g);
 }
 
+// The volume frame of one primitive: its voxel-frame mean, inverse covariance
+// (zeros when singular) and radii, from its mean and covariance.
+template <typename S>
+__device__ __forceinline__ void map_to_volume(const S* __restrict__ mean, const S s[6], const S* __restrict__ ranges,
+                                              const S* __restrict__ centers, uint32_t dx, uint32_t dy, uint32_t dz,
+                                              S eps, S clip, S mapped[3], S conic[6], int32_t radii[3]) {
+    const S D[3] = {S(dx), S(dy), S(dz)};
+    const S r[3] = {D[0] / ranges[0], D[1] / ranges[1], D[2] / ranges[2]};
+#pragma unroll
+    for (int k = 0; k < 3; ++k) mapped[k] = (mean[k] - centers[k]) * r[k] + D[k] * S(0.5);
+    // Voxel-frame covariance in the working precision (its diagonal sets the radii).
+    const S sv[6] = {r[0] * r[0] * s[0] + eps, r[0] * r[1] * s[1], r[0] * r[2] * s[2],
+                     r[1] * r[1] * s[3] + eps, r[1] * r[2] * s[4], r[2] * r[2] * s[5] + eps};
+    double a[6], inv[6];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) a[k] = double(sv[k]);
+    const bool ok = spd3_inverse(a, inv);
+#pragma unroll
+    for (int k = 0; k < 6; ++k) conic[k] = S(inv[k]);
+    radii[0] = radii[1] = radii[2] = 0;
+    if (ok) {
+        const S rad[3] = {ceil(clip * sqrt(max(S(0), sv[0]))), ceil(clip * sqrt(max(S(0), sv[3]))),
+                          ceil(clip * sqrt(max(S(0), sv[5])))};
+        bool good = true;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) good = good && isfinite(rad[k]) && rad[k] > S(0);
+        if (good) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) radii[k] = static_cast<int32_t>(rad[k]);
+        }
+    }
+}
+
 template <typename S>
 __global__ void __launch_bounds__(kGeomThreads)
 volume_mapping_fwd_kernel(const S* __restrict__ means, const S* __restrict__ covars,
@@ -182,35 +218,60 @@ volume_mapping_fwd_kernel(const S* __restrict__ means, const S* __restrict__ cov
                           int32_t* __restrict__ radii, uint32_t N) {
     const uint32_t n = blockIdx.x * blockDim.x + threadIdx.x;
     if (n >= N) return;
-    const S D[3] = {S(dx), S(dy), S(dz)};
-    const S r[3] = {D[0] / ranges[0], D[1] / ranges[1], D[2] / ranges[2]};
+    S cov[6], m[3], c[6];
+    int32_t r[3];
 #pragma unroll
-    for (int k = 0; k < 3; ++k)
-        mapped[3 * size_t(n) + k] = (means[3 * size_t(n) + k] - centers[k]) * r[k] + D[k] * S(0.5);
-    const S* s = covars + 6 * size_t(n);
-    // Voxel-frame covariance in the working precision (its diagonal sets the radii).
-    const S sv[6] = {r[0] * r[0] * s[0] + eps, r[0] * r[1] * s[1], r[0] * r[2] * s[2],
-                     r[1] * r[1] * s[3] + eps, r[1] * r[2] * s[4], r[2] * r[2] * s[5] + eps};
-    double a[6], inv[6];
+    for (int k = 0; k < 6; ++k) cov[k] = covars[6 * size_t(n) + k];
+    map_to_volume(means + 3 * size_t(n), cov, ranges, centers, dx, dy, dz, eps, clip, m, c, r);
 #pragma unroll
-    for (int k = 0; k < 6; ++k) a[k] = double(sv[k]);
-    const bool ok = spd3_inverse(a, inv);
-#pragma unroll
-    for (int k = 0; k < 6; ++k) conics[6 * size_t(n) + k] = S(inv[k]);
-    int32_t rr[3] = {0, 0, 0};
-    if (ok) {
-        const S rad[3] = {ceil(clip * sqrt(max(S(0), sv[0]))), ceil(clip * sqrt(max(S(0), sv[3]))),
-                          ceil(clip * sqrt(max(S(0), sv[5])))};
-        bool good = true;
-#pragma unroll
-        for (int k = 0; k < 3; ++k) good = good && isfinite(rad[k]) && rad[k] > S(0);
-        if (good) {
-#pragma unroll
-            for (int k = 0; k < 3; ++k) rr[k] = static_cast<int32_t>(rad[k]);
-        }
+    for (int k = 0; k < 3; ++k) {
+        mapped[3 * size_t(n) + k] = m[k];
+        radii[3 * size_t(n) + k] = r[k];
     }
 #pragma unroll
-    for (int k = 0; k < 3; ++k) radii[3 * size_t(n) + k] = rr[k];
+    for (int k = 0; k < 6; ++k) conics[6 * size_t(n) + k] = c[k];
+}
+
+// Everything a voxelization does per primitive before its lists: parameter
+// transform, volume mapping, double-precision frame (`frame` given) and tile
+// count. One launch in place of four, which a small volume spends on launching
+// (the operators of each stage remain entry points of their own).
+template <typename S>
+__global__ void __launch_bounds__(kGeomThreads)
+voxel_prepare_kernel(const S* __restrict__ means, const S* __restrict__ quats, const S* __restrict__ scales,
+                     const S* __restrict__ ranges, const S* __restrict__ centers,
+                     const double* __restrict__ ranges64, const double* __restrict__ centers64, uint32_t dx,
+                     uint32_t dy, uint32_t dz, double eps, double clip, uint32_t tile, uint32_t ntx, uint32_t nty,
+                     uint32_t ntz, uint32_t N, S* __restrict__ covars, S* __restrict__ mapped,
+                     S* __restrict__ conics, int32_t* __restrict__ radii, double* __restrict__ frame,
+                     uint32_t* __restrict__ counts) {
+    const uint32_t n = blockIdx.x * blockDim.x + threadIdx.x;
+    if (n >= N) return;
+    S q[4], mag, norm, R[9], cov[6], m[3], c[6];
+    unit_quat(quats + 4 * size_t(n), q, mag, norm);
+    quat_to_rot(q, R);
+    const S s[3] = {scales[3 * size_t(n)], scales[3 * size_t(n) + 1], scales[3 * size_t(n) + 2]};
+    covariance_from(R, s, cov);
+    int32_t r[3];
+    map_to_volume(means + 3 * size_t(n), cov, ranges, centers, dx, dy, dz, S(eps), S(clip), m, c, r);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        mapped[3 * size_t(n) + k] = m[k];
+        radii[3 * size_t(n) + k] = r[k];
+    }
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+        covars[6 * size_t(n) + k] = cov[k];
+        conics[6 * size_t(n) + k] = c[k];
+    }
+    uint32_t lo[3], hi[3];
+    counts[n] = box_3d(m, r, 0, tile, ntx, nty, ntz, lo, hi)
+                    ? (hi[0] - lo[0]) * (hi[1] - lo[1]) * (hi[2] - lo[2]) : 0u;
+    if constexpr (std::is_same<S, float>::value) {
+        if (frame)
+            voxel_frame(means + 3 * size_t(n), quats + 4 * size_t(n), scales + 3 * size_t(n), ranges64, centers64, dx,
+                        dy, dz, eps, frame + 9 * size_t(n));
+    }
 }
 
 // Inverse VJP: v_Sv = -P V P with V the upper-triangular packed adjoint.
@@ -394,4 +455,41 @@ extern "C" int r2s_beta_factors(int dtype, const void* betas, uint64_t n, void* 
                                                                                       (S*)log_grad);
         return check_launch("beta_factors");
     });
+}
+
+extern "C" int r2s_voxel_prepare(int dtype, const void* means, const void* quats, const void* scales,
+                                 const void* ranges, const void* centers, const double* ranges64,
+                                 const double* centers64, uint32_t dim_x, uint32_t dim_y, uint32_t dim_z, double eps,
+                                 double radius_clip, uint32_t tile_size, uint32_t n_tiles_x, uint32_t n_tiles_y,
+                                 uint32_t n_tiles_z, uint32_t N, void* covars, void* means3d_v, void* conics,
+                                 int32_t* radii, double* frame, uint32_t* cum, void* scan_ws, uint32_t* host,
+                                 r2s_stream_t stream) {
+    R2S_REQUIRE(means && quats && scales && ranges && centers && covars && means3d_v && conics && radii && cum &&
+                scan_ws && host, "voxel_prepare: null argument");
+    R2S_REQUIRE(N > 0 && N < (1u << 31), "N must be in (0, 2^31)");
+    R2S_REQUIRE(tile_size > 0, "tile_size must be positive");
+    R2S_REQUIRE(!frame || (dtype == R2S_F32 && ranges64 && centers64),
+                "the double-precision frame belongs to float32 primitives and needs the frame's vectors in double");
+    return dispatch_dtype(dtype, [&](auto tag) {
+        using S = decltype(tag);
+        voxel_prepare_kernel<S><<<ceil_div(N, kGeomThreads), kGeomThreads, 0, stream>>>(
+            (const S*)means, (const S*)quats, (const S*)scales, (const S*)ranges, (const S*)centers, ranges64,
+            centers64, dim_x, dim_y, dim_z, eps, radius_clip, tile_size, n_tiles_x, n_tiles_y, n_tiles_z, N,
+            (S*)covars, (S*)means3d_v, (S*)conics, radii, frame, cum);
+        if (int rc = check_launch("voxel_prepare")) return rc;
+        if (int rc = scan_exclusive(cum, N, cum, nullptr, scan_ws, stream)) return rc;
+        return fetch_begin(cum + N, 1, host, stream);
+    });
+}
+
+extern "C" int r2s_voxel_param_vjp(int dtype, const void* means, const void* quats, const void* scales,
+                                   const void* covars, const void* ranges, const void* centers, uint32_t dim_x,
+                                   uint32_t dim_y, uint32_t dim_z, double eps, const void* v_means3d_v,
+                                   const void* v_conics, void* v_covars, void* v_means, void* v_quats, void* v_scales,
+                                   uint32_t N, r2s_stream_t stream) {
+    // (one kernel for both rounds the quaternion gradient differently)
+    if (int rc = r2s_world_to_volume_mapping_bwd(dtype, means, covars, ranges, centers, dim_x, dim_y, dim_z, eps,
+                                                 v_means3d_v, v_conics, v_means, v_covars, N, stream))
+        return rc;
+    return r2s_parameter_transform_bwd(dtype, quats, scales, v_covars, v_quats, v_scales, N, stream);
 }

@@ -483,4 +483,29 @@ __device__ __forceinline__ void normalize_vjp(const S q[4], S mag, S norm, const
     for (int i = 0; i < 4; ++i) out[i] = ((g[i] - q[i] * qg) / norm) / mag;
 }
 
+// One float32 primitive's voxel-frame mean (x y z) and inverse covariance (xx xy
+// xz yy yz zz) in double: the operator chain parameter transform -> volume
+// mapping, in double.
+__device__ __forceinline__ void voxel_frame(const float* __restrict__ mean, const float* __restrict__ quat,
+                                            const float* __restrict__ scale, const double* __restrict__ ranges,
+                                            const double* __restrict__ centers, uint32_t dx, uint32_t dy, uint32_t dz,
+                                            double eps, double* __restrict__ f) {
+    const double raw[4] = {double(quat[0]), double(quat[1]), double(quat[2]), double(quat[3])};
+    double q[4], mag, norm, R[9], cov[6];
+    unit_quat(raw, q, mag, norm);
+    quat_to_rot(q, R);
+    const double s[3] = {double(scale[0]), double(scale[1]), double(scale[2])};
+    covariance_from(R, s, cov);
+    const double D[3] = {double(dx), double(dy), double(dz)};
+    const double r[3] = {D[0] / ranges[0], D[1] / ranges[1], D[2] / ranges[2]};
+#pragma unroll
+    for (int k = 0; k < 3; ++k) f[k] = (double(mean[k]) - centers[k]) * r[k] + D[k] * 0.5;
+    const double sv[6] = {r[0] * r[0] * cov[0] + eps, r[0] * r[1] * cov[1], r[0] * r[2] * cov[2],
+                          r[1] * r[1] * cov[3] + eps, r[1] * r[2] * cov[4], r[2] * r[2] * cov[5] + eps};
+    double inv[6];
+    spd3_inverse(sv, inv);  // zeros when singular (such primitives have zero radii and no tiles)
+#pragma unroll
+    for (int k = 0; k < 6; ++k) f[3 + k] = inv[k];
+}
+
 }  // namespace r2s

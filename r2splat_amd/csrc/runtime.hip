@@ -143,7 +143,7 @@ fetch_kernel(const uint32_t* __restrict__ src, uint32_t n, uint32_t* host) {
     if (threadIdx.x == 0) __hip_atomic_store(host, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-static int fetch_begin(const uint32_t* src, uint32_t n, uint32_t* host, hipStream_t stream) {
+int fetch_begin(const uint32_t* src, uint32_t n, uint32_t* host, hipStream_t stream) {
     __atomic_store_n(host, 0u, __ATOMIC_RELEASE);
     fetch_kernel<<<1, kWave, 0, stream>>>(src, n, host);
     return check_launch("fetch");

@@ -353,25 +353,8 @@ vox_frame_kernel(const float* __restrict__ means, const float* __restrict__ quat
                  uint32_t dz, double eps, uint32_t N, double* __restrict__ frame) {
     const uint32_t n = blockIdx.x * blockDim.x + threadIdx.x;
     if (n >= N) return;
-    const double raw[4] = {double(quats[4 * size_t(n)]), double(quats[4 * size_t(n) + 1]),
-                           double(quats[4 * size_t(n) + 2]), double(quats[4 * size_t(n) + 3])};
-    double q[4], mag, norm, R[9], cov[6];
-    unit_quat(raw, q, mag, norm);
-    quat_to_rot(q, R);
-    const double s[3] = {double(scales[3 * size_t(n)]), double(scales[3 * size_t(n) + 1]),
-                         double(scales[3 * size_t(n) + 2])};
-    covariance_from(R, s, cov);
-    const double D[3] = {double(dx), double(dy), double(dz)};
-    const double r[3] = {D[0] / ranges[0], D[1] / ranges[1], D[2] / ranges[2]};
-    double* f = frame + kFrame * size_t(n);
-#pragma unroll
-    for (int k = 0; k < 3; ++k) f[k] = (double(means[3 * size_t(n) + k]) - centers[k]) * r[k] + D[k] * 0.5;
-    const double sv[6] = {r[0] * r[0] * cov[0] + eps, r[0] * r[1] * cov[1], r[0] * r[2] * cov[2],
-                          r[1] * r[1] * cov[3] + eps, r[1] * r[2] * cov[4], r[2] * r[2] * cov[5] + eps};
-    double inv[6];
-    spd3_inverse(sv, inv);  // zeros when singular (such primitives have zero radii and no tiles)
-#pragma unroll
-    for (int k = 0; k < 6; ++k) f[3 + k] = inv[k];
+    voxel_frame(means + 3 * size_t(n), quats + 4 * size_t(n), scales + 3 * size_t(n), ranges, centers, dx, dy, dz, eps,
+                frame + kFrame * size_t(n));
 }
 
 // Mean of primitive G split into float hi + lo (lo = 0 without a frame).

@@ -428,6 +428,11 @@ def _voxel_state(prims, vol: dict, shape, eps, radius_clip) -> dict:
     extent, center = vol["extent"], vol["center"]
     depth, height, width = shape
     T = VOXEL_TILE
+    if BACKEND == "fused":
+        with stage("voxel_bin"):
+            return _ops_impl.voxel_prepare(means, quats, scales, extent, center, vol["extent64"], vol["center64"],
+                                           (width, height, depth), eps, radius_clip, T,
+                                           (-(-width // T), -(-height // T), -(-depth // T)))
     with stage("voxel_map"):
         covars, max_scales = ops.parameter_transform_fwd(quats, scales)
         mapped, conics, radii = ops.world_to_volume_mapping_fwd(means, covars, max_scales, extent, center, width,
@@ -436,13 +441,8 @@ def _voxel_state(prims, vol: dict, shape, eps, radius_clip) -> dict:
     with stage("voxel_bin"):
         _, isect_ids, flatten_ids, tile_cum = _ops_impl._isect_tiles_3d(mapped, radii, T, tx, ty, tz)
         offsets = ops.isect_offset_encode_3d(isect_ids, tx, ty, tz)
-    state = dict(covars=covars, mapped=mapped, conics=conics, radii=radii, tile_cum=tile_cum, offsets=offsets,
-                 isect_ids=isect_ids, flatten_ids=flatten_ids)
-    if _use_fused_voxels(means):
-        with stage("voxel_map"):
-            state["frame"] = fused.voxel_frame(means, quats, scales, vol["extent64"], vol["center64"],
-                                               (width, height, depth), eps)
-    return state
+    return dict(covars=covars, mapped=mapped, conics=conics, radii=radii, tile_cum=tile_cum, offsets=offsets,
+                isect_ids=isect_ids, flatten_ids=flatten_ids)
 
 
 def _voxel_render(b, prims, shape):
@@ -561,6 +561,11 @@ def _voxel_vjp(context: _Context, v_volume, v_variance) -> ParameterGradients:
     v_mapped, v_conics, v_densities = grads[:3]
     v_beta = None if beta is None else grads[3]
     with stage("voxel_map_bwd"):
+        if BACKEND == "fused":
+            v_means, v_quats, v_scales = _ops_impl.voxel_param_vjp(means, quats, scales, b["covars"], b["extent"],
+                                                                   b["center"], (width, height, depth), context.eps,
+                                                                   v_mapped.contiguous(), v_conics.contiguous())
+            return ParameterGradients(v_means, v_quats, v_scales, v_densities, v_beta, v_uncertainty)
         v_means, v_covars = ops.world_to_volume_mapping_bwd(means, b["covars"], b["extent"], b["center"], width,
                                                             height, depth, context.eps, v_mapped.contiguous(),
                                                             v_conics.contiguous())

@@ -102,6 +102,10 @@ SIGNATURES = {
     "r2s_voxel_partials_bytes": [U32],
     "r2s_voxelize_fused_vjp": [P, P, P, P, P, P, P, P, P, P, U32, U32, U32, U32, U32, U32, U32, U32, U32, P,
                                P, I32, P, SZ, P, P, P, P, P, P],
+    "r2s_voxel_prepare": [I32, P, P, P, P, P, P, P, U32, U32, U32, D, D, U32, U32, U32, U32, U32, P, P, P, P, P, P, P,
+                          P, P],
+    "r2s_voxel_lists": [I32, P, P, U32, U32, U32, U32, U32, P, U32, P, P, P, SZ, P, P],
+    "r2s_voxel_param_vjp": [I32, P, P, P, P, P, P, U32, U32, U32, D, P, P, P, P, P, P, U32, P],
     "r2s_mse_partials": [U64],
     "r2s_mse_adjoint": [P, P, U64, P, P, P, P],
     "r2s_mse_adjoint_noalloc": [P, P, U64, P, P, P],

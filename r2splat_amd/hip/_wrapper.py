@@ -326,6 +326,52 @@ def isect_offset_encode_3d(isect_ids, n_tiles_dim2, n_tiles_dim1, n_tiles_dim0):
 
 
 # ---------------------------------------------------------------------------
+# voxelization in one call per phase (validated inputs of the explicit API)
+# ---------------------------------------------------------------------------
+def voxel_prepare(means, quats, scales, extent, center, extent64, center64, dims, eps, radius_clip, tile_size,
+                  tiles) -> dict:
+    """parameter_transform_fwd, world_to_volume_mapping_fwd, isect_tiles_3d and
+    isect_offset_encode_3d (and, for float32, the double-precision frame of
+    fused.voxel_frame) of N > 0 primitives; dims and tiles in x, y, z order."""
+    N, dev, dt = means.size(0), means.device, be.dtype_code(means.dtype)
+    covars, conics, mapped = means.new_empty((N, 6)), means.new_empty((N, 6)), means.new_empty((N, 3))
+    radii = torch.empty((N, 3), dtype=torch.int32, device=dev)
+    cum = torch.empty((N + 1,), dtype=torch.int32, device=dev)
+    frame = torch.empty((N, 9), dtype=torch.float64, device=dev) if dt == be.F32 else None
+    nx, ny, nz = tiles
+    offsets = torch.empty((nz, ny, nx), dtype=torch.int32, device=dev)
+    with _Launch(means) as L:
+        scan_ws = _workspace(be.lib().r2s_scan_workspace_bytes(N), dev)
+        words = be.HostWords(1, dev)
+        call("r2s_voxel_prepare", dt, ptr(means), ptr(quats), ptr(scales), ptr(extent), ptr(center), ptr(extent64),
+             ptr(center64), *dims, float(eps), float(radius_clip), tile_size, nx, ny, nz, N, ptr(covars), ptr(mapped),
+             ptr(conics), ptr(radii), ptr(frame), ptr(cum), ptr(scan_ws), words.ptr, L.stream)
+        (n_isects,) = words.wait()
+        isect_ids = torch.empty((n_isects,), dtype=torch.int64, device=dev)
+        flatten_ids = torch.empty((n_isects,), dtype=torch.int32, device=dev)
+        nbytes = be.lib().r2s_sort_workspace_bytes(n_isects, 0)
+        sort_ws = _workspace(nbytes, dev)
+        call("r2s_voxel_lists", dt, ptr(mapped), ptr(radii), N, tile_size, nx, ny, nz, ptr(cum), n_isects,
+             ptr(isect_ids), ptr(flatten_ids), ptr(sort_ws), nbytes, ptr(offsets), L.stream)
+    state = dict(covars=covars, mapped=mapped, conics=conics, radii=radii, tile_cum=cum, offsets=offsets,
+                 isect_ids=isect_ids, flatten_ids=flatten_ids)
+    if frame is not None:
+        state["frame"] = frame
+    return state
+
+
+def voxel_param_vjp(means, quats, scales, covars, extent, center, dims, eps, v_mapped, v_conics):
+    """world_to_volume_mapping_bwd and parameter_transform_bwd -> (v_means, v_quats, v_scales)."""
+    v_means, v_quats, v_scales = torch.empty_like(means), torch.empty_like(quats), torch.empty_like(scales)
+    v_covars = torch.empty_like(covars)
+    with _Launch(means) as L:
+        call("r2s_voxel_param_vjp", be.dtype_code(means.dtype), ptr(means), ptr(quats), ptr(scales), ptr(covars),
+             ptr(extent), ptr(center), *dims, float(eps), ptr(v_mapped), ptr(v_conics), ptr(v_covars), ptr(v_means),
+             ptr(v_quats), ptr(v_scales), means.size(0), L.stream)
+    return v_means, v_quats, v_scales
+
+
+# ---------------------------------------------------------------------------
 # 2D rasterization
 # ---------------------------------------------------------------------------
 def _raster_inputs(means2d, conics, opacities, mus, betas, tile_offsets, flatten_ids):

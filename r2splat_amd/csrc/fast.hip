@@ -190,13 +190,6 @@ __device__ __forceinline__ bool edge_keep(const BetaEdge& e, float px, float py)
     return q >= 0.0 && q < 1.0 && q <= e.dmax;
 }
 
-// LDS written by some lanes of a wave is visible to its other lanes.
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // The record's quadratic form q (Gaussian: sigma log2 e; Beta: d^2) at one
 // pixel, in the two evaluation orders of the raster kernels. The forward
 // shares the column terms of a lane's pixels (adx2 = A dx dx, bdx = B dx with
@@ -950,15 +943,11 @@ fused_pack_kernel(const uint2* __restrict__ rects, const Reach<BETA>* __restrict
         __syncthreads();
 #pragma unroll
         for (int q = 0; q < kPackItems; ++q) {
-            // stable rank among this wave's items of the same class: one ballot per distinct class
-            uint64_t pending = __ballot(1);
-            while (pending) {
-                const uint32_t c = __shfl(cls[q], __builtin_ctzll(pending), kWave);
-                const uint64_t m = __ballot(cls[q] == c);
-                if (cls[q] == c) rank[q] = uint32_t(__popcll(m & below));
-                if (lane == 0) cnt[c * kPackSlots + q * kPackWaves + wave] = uint32_t(__popcll(m));
-                pending &= ~m;
-            }
+            // stable rank among this wave's items of the same class (a ballot per distinct
+            // class, 20 of them, took 2.28 ms for 274M entries, these ballots 2.19)
+            const uint64_t peers = wave_match(cls[q], 6, ~uint64_t(0));
+            rank[q] = uint32_t(__popcll(peers & below));
+            if (rank[q] == 0u) cnt[cls[q] * kPackSlots + q * kPackWaves + wave] = uint32_t(__popcll(peers));
         }
         __syncthreads();
         if (wave == 0) {  // exclusive scan of the counts, 9 per lane

@@ -1049,6 +1049,71 @@ struct RectWalk {
     }
 };
 
+// The placement's pairs of 64 records, compacted: the walk above, a record per
+// lane, has as many steps as its largest rectangle has tiles and few lanes in most
+// of them (27 of 64 for 100k Gaussians x 64 views of 256^2), and ranking and
+// writing a step's pairs is the long part. So each step only lists its (record,
+// pair) numbers in LDS, and 64 listed pairs are placed at a time, in the same order:
+// by pair number in the rectangle, then lane. (The count is short per pair and
+// keeps the walk: with pairs listed it took 143 us in place of 84 there.)
+struct __align__(16) PairBox {  // a record's rectangle (corner and width) and reach, and its first emission index
+    uint32_t first, x0, y0, w;
+    float my, ext, mx, ext_x;
+};
+struct PairList {
+    PairBox boxes[kWave];
+    uint32_t pairs[2 * kWave];  // lane of the record | pair number << 6
+};
+
+// The bin of a pair: (tile, work class).
+template <bool BETA>
+__device__ __forceinline__ uint32_t pair_bin(const PairBox& b, uint32_t tx, uint32_t ty, uint32_t ntx, uint32_t T) {
+    const uint32_t log2_T = uint32_t(__builtin_ctz(T));
+    const uint32_t rows = rows_reached(b.my, b.ext, float(ty * T), T);
+    uint32_t cls;
+    if constexpr (BETA)
+        cls = work_class(rows * segments_reached(b.mx, b.ext_x, float(tx * T), T), 2u * log2_T - 3u);
+    else
+        cls = work_class(rows, log2_T);
+    return (ty * ntx + tx) * kBinClasses + cls;
+}
+
+__device__ __forceinline__ uint32_t rect_pairs(const SpanRect& r) {
+    return ((r.xr >> 16) - (r.xr & 0xffffu)) * ((r.yr >> 16) - (r.yr & 0xffffu));
+}
+
+// Calls f(valid, lane of the record, pair number, box) for the pairs, a pair per
+// lane (valid = false for lanes past the last).
+template <typename F>
+__device__ __forceinline__ void place_pairs(const SpanRect& r, uint32_t cnt, uint32_t first, PairList& lds, F&& f) {
+    const uint32_t lane = threadIdx.x % kWave;
+    wave_lds_sync();  // every lane is done with the previous records
+    const uint32_t x0 = r.xr & 0xffffu;
+    lds.boxes[lane] = PairBox{first, x0, r.yr & 0xffffu, (r.xr >> 16) - x0, r.my, r.ext, r.mx, r.ext_x};
+    const auto place = [&](uint32_t n) {
+        wave_lds_sync();
+        const uint32_t pair = lds.pairs[lane], owner = pair % kWave;
+        f(lane < n, owner, pair / kWave, lds.boxes[owner]);
+    };
+    uint32_t listed = 0;
+    for (uint32_t k = 0;; ++k) {
+        const uint64_t members = __ballot(k < cnt);
+        if (members == 0ull) break;
+        const uint32_t at = __builtin_amdgcn_mbcnt_hi(uint32_t(members >> 32),
+                                                      __builtin_amdgcn_mbcnt_lo(uint32_t(members), listed));
+        if (k < cnt) lds.pairs[at] = lane | (k << 6);  // (k < 2^26: a rectangle of 2^26 tiles passes no grid limit)
+        listed += uint32_t(__popcll(members));
+        if (listed >= kWave) {
+            place(kWave);
+            listed -= kWave;
+            const uint32_t rest = lds.pairs[kWave + lane];
+            wave_lds_sync();
+            if (lane < listed) lds.pairs[lane] = rest;
+        }
+    }
+    if (listed > 0u) place(listed);
+}
+
 // grid (n_ranges, C), one wave; dynamic LDS: n_bins counters. range_totals:
 // the intersections of each (camera, range).
 template <bool BETA>
@@ -1202,6 +1267,7 @@ fused_bin_place_kernel(const uint2* __restrict__ rects, const Reach<BETA>* __res
                        const uint32_t* __restrict__ range_starts, const uint32_t* __restrict__ bin_starts,
                        const uint32_t* __restrict__ first_isect, uint32_t capacity, uint2* __restrict__ entries) {
     extern __shared__ uint32_t next_slot[];
+    __shared__ PairList list;
     const uint32_t range = blockIdx.x, cam = blockIdx.y, lane = threadIdx.x;
     const uint32_t* rs = range_starts + (size_t(cam) * n_ranges + range) * n_bins;
     const uint32_t* bs = bin_starts + size_t(cam) * n_bins;
@@ -1221,30 +1287,41 @@ fused_bin_place_kernel(const uint2* __restrict__ rects, const Reach<BETA>* __res
     __syncthreads();
     const uint64_t below = (uint64_t(1) << lane) - 1u;
     const uint32_t n0 = range * range_len, n1 = min(N, n0 + range_len);
+    SpanRect next = {0u, 0u, 0.f, -1.f, 0.f, -1.f};
+    if (n0 + lane < n1) next = load_span(rects, reach, size_t(cam) * N + n0 + lane);
     for (uint32_t s = n0; s < n1; s += kWave) {
-        const uint32_t n = s + lane;
-        const size_t idx = size_t(cam) * N + n;
-        SpanRect sr = {0u, 0u, 0.f, -1.f, 0.f, -1.f};
-        if (n < n1) sr = load_span(rects, reach, idx);
-        RectWalk<BETA> w;
-        w.start(sr, ntx, T);
-        const uint32_t incl = wave_scan(w.cnt);
-        const uint32_t g = emitted + incl - w.cnt;
+        const SpanRect sr = next;
+        next = SpanRect{0u, 0u, 0.f, -1.f, 0.f, -1.f};
+        if (s + kWave + lane < n1) next = load_span(rects, reach, size_t(cam) * N + s + kWave + lane);
+        const uint32_t cnt = rect_pairs(sr), incl = wave_scan(cnt);
+        const uint32_t first_rec = cam * N + s;  // (C N < 2^31)
+        if (s + lane < n1) cum[first_rec + lane] = emitted + incl - cnt;
+        place_pairs(sr, cnt, emitted + incl - cnt, list,
+                    [&](bool valid, uint32_t owner, uint32_t k, const PairBox& b) {
+                        uint32_t bin = 0u;
+                        if (valid) {
+                            // row and column of the pair in its rectangle: the quotient by a
+                            // hardware reciprocal is off by at most one
+                            uint32_t y = uint32_t(float(k) * __builtin_amdgcn_rcpf(float(b.w)));
+                            int32_t x = int32_t(k - y * b.w);
+                            if (x < 0) {
+                                --y;
+                                x += int32_t(b.w);
+                            } else if (x >= int32_t(b.w)) {
+                                ++y;
+                                x -= int32_t(b.w);
+                            }
+                            bin = pair_bin<BETA>(b, b.x0 + uint32_t(x), b.y0 + y, ntx, T);
+                        }
+                        // lanes of this step with the same bin, ranked by lane
+                        const uint64_t same = wave_match(bin, bin_bits, __ballot(valid));
+                        if (!valid) return;
+                        // every lane reads its bin's slot before the group's last lane advances it
+                        const uint32_t pos = next_slot[bin] + uint32_t(__popcll(same & below));
+                        if ((same >> lane) == 1u) next_slot[bin] = pos + 1u;
+                        if (pos < capacity) entries[pos] = make_uint2(first_rec + owner, b.first + k);
+                    });
         emitted += __builtin_amdgcn_readlane(incl, kWave - 1);
-        if (n < n1) cum[idx] = g;
-        for (uint32_t k = 0; __ballot(k < w.cnt); ++k) {
-            const bool act = k < w.cnt;
-            const uint32_t bin = act ? w.bin() : 0u;
-            // lanes of this step with the same bin, ranked by lane
-            const uint64_t same = wave_match(bin, bin_bits, __ballot(act));
-            if (act) {
-                // every lane reads its bin's slot before the group's last lane advances it
-                const uint32_t pos = next_slot[bin] + uint32_t(__popcll(same & below));
-                if ((same >> lane) == 1u) next_slot[bin] = pos + 1u;
-                if (pos < capacity) entries[pos] = make_uint2(uint32_t(idx), g + k);
-                w.advance(sr, ntx, T);
-            }
-        }
     }
 }
 
@@ -2141,7 +2218,7 @@ static FusedScratch fused_scratch(uint32_t C, uint32_t N, uint32_t n_tiles, uint
         L.range_len = uint32_t(std::max<uint64_t>(least, (per + 63) / 64 * 64));
         L.n_ranges = (N + L.range_len - 1) / L.range_len;
         L.place = table <= kPlaceLdsBytes ||
-                  uint64_t(C) * L.n_ranges <= kComputeUnits * (kLdsBytes / table);
+                  uint64_t(C) * L.n_ranges <= kComputeUnits * (kLdsBytes / (table + sizeof(PairList)));
         if (L.place) {
             L.range_counts = o; o += al(size_t(C) * L.n_ranges * L.n_bins * 4 + 4);
             L.range_totals = o; o += al(size_t(C) * L.n_ranges * 4 + 4);

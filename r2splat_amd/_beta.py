@@ -66,7 +66,7 @@ def beta_factors(gamma: torch.Tensor, ratio: torch.Tensor | None = None, log_gra
     gamma = gamma.contiguous()
     ratio = torch.empty_like(gamma) if ratio is None else ratio
     log_grad = torch.empty_like(gamma) if log_grad is None else log_grad
-    with torch.cuda.device(gamma.device):
+    with be.on(gamma.device):
         be.call("r2s_beta_factors", be.dtype_code(gamma.dtype), be.ptr(gamma), gamma.numel(), be.ptr(ratio),
                 be.ptr(log_grad), be.stream_of(gamma.device))
     return ratio, log_grad

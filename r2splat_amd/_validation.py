@@ -94,7 +94,7 @@ class ValueChecks:
         flags = torch.stack([pending[i][1]().reshape(()) for i in reduced]).to(torch.int32) if reduced else None
         words = []
         if native:
-            with torch.cuda.device(device):
+            with be.on(device):
                 for lo in range(0, len(native), be.MAX_VALUE_CHECKS):
                     chunk = native[lo: lo + be.MAX_VALUE_CHECKS]
                     table = (be.ValueCheck * len(chunk))()

@@ -166,7 +166,7 @@ class _MSE(torch.autograd.Function):
         partials = torch.empty((max(1, int(be.lib().r2s_mse_partials(n))),), dtype=torch.float32,
                                device=image.device)
         loss = torch.empty((), dtype=torch.float32, device=image.device)
-        with torch.cuda.device(image.device):
+        with be.on(image.device):
             be.call("r2s_mse_adjoint", be.ptr(image), be.ptr(target), n, be.ptr(v), be.ptr(partials), be.ptr(loss),
                     be.stream_of(image.device))
         ctx.save_for_backward(v)

@@ -16,13 +16,23 @@ __device__ __forceinline__ uint32_t clamp_bound(S v, uint32_t upper) {
 }
 
 template <typename S>
-__device__ __forceinline__ bool tile_span(S mean, int32_t radius, uint32_t tile, uint32_t n_tiles,
-                                          uint32_t& lo, uint32_t& hi) {
-    const S t = S(tile);
-    const S c = mean / t, r = S(radius) / t;
+__device__ __forceinline__ bool tile_span_of(S c, S r, uint32_t n_tiles, uint32_t& lo, uint32_t& hi) {
     lo = clamp_bound(floor(c - r), n_tiles);
     hi = clamp_bound(ceil(c + r), n_tiles);
     return hi > lo;
+}
+template <typename S>
+__device__ __forceinline__ bool tile_span(S mean, int32_t radius, uint32_t tile, uint32_t n_tiles,
+                                          uint32_t& lo, uint32_t& hi) {
+    const S t = S(tile);
+    return tile_span_of(mean / t, S(radius) / t, n_tiles, lo, hi);
+}
+// tile_span for a tile edge that is a power of two, inv_tile its reciprocal: the
+// products are exact, and a division in double is 15 instructions.
+template <typename S>
+__device__ __forceinline__ bool tile_span_inv(S mean, int32_t radius, S inv_tile, uint32_t n_tiles, uint32_t& lo,
+                                              uint32_t& hi) {
+    return tile_span_of(mean * inv_tile, S(radius) * inv_tile, n_tiles, lo, hi);
 }
 
 // Tile box of one 3D primitive (IsectTiles3DKernel.cu:36-45): per axis the

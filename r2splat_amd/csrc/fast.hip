@@ -658,6 +658,7 @@ fused_project_kernel(const float* __restrict__ means, const PrimFrame* __restric
     const uint32_t n = blockIdx.x * blockDim.x + threadIdx.x;
     if (n >= N) return;
     const PrimFrame f = frames[n];
+    const double inv_tile = 1.0 / double(tile_size);  // (8, 16 or 32)
     const float density = dens[n];
     const float beta = BETA ? betas[n] : 0.f, beta_ratio = BETA ? ratio[n] : 0.f;
     const float uncertainty = VAR ? unc[n] : 0.f;
@@ -704,8 +705,8 @@ fused_project_kernel(const float* __restrict__ means, const PrimFrame* __restric
                 rec.qlim = qlim_of(w);
             }
             uint32_t x0, x1, y0, y1;
-            if (rx > 0 && ry > 0 && tile_span(m2[0], rx, tile_size, ntx, x0, x1) &&
-                tile_span(m2[1], ry, tile_size, nty, y0, y1)) {
+            if (rx > 0 && ry > 0 && tile_span_inv(m2[0], rx, inv_tile, ntx, x0, x1) &&
+                tile_span_inv(m2[1], ry, inv_tile, nty, y0, y1)) {
                 count = (x1 - x0) * (y1 - y0);
                 rect = make_uint2(x0 | (x1 << 16), y0 | (y1 << 16));
                 rr.x = rec.my;

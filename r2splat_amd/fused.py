@@ -169,7 +169,7 @@ def prepare(means, quats, scales, densities, viewmats, Ks, width, height, eps, r
     # per-record intersection offsets (C*N + 1) followed by the primitive order (N)
     record_offsets = torch.empty((C * N + 1 + N,), dtype=torch.int32, device=device)
     counters = torch.empty((2,), dtype=torch.int32, device=device)
-    with torch.cuda.device(device):
+    with be.on(device):
         stream = be.stream_of(device)
         while True:
             scratch = _scratch(C, N, width, height, tile_size, cap, kind, device)
@@ -199,7 +199,7 @@ def render(fwd: FusedForward, C: int, device, waves: int = 0):
     carries uncertainties (`waves` per tile: 4, 8, 16; 0 = 8)."""
     image = torch.empty((C, fwd.height, fwd.width), dtype=torch.float32, device=device)
     var = torch.empty_like(image) if fwd.uncertainty is not None else None
-    with torch.cuda.device(device):
+    with be.on(device):
         with stage("rasterize_fwd"):
             call("r2s_fused_render", ptr(fwd.packed), ptr(fwd.offsets), ptr(fwd.tile_order), ptr(fwd.counters),
                  fwd.capacity, C, fwd.width, fwd.height, fwd.tile_size, waves, fwd.kind, ptr(image), ptr(var),
@@ -243,7 +243,7 @@ def backward(fwd: FusedForward, means, quats, scales, densities, viewmats, Ks, v
     v_dens = torch.empty_like(densities)
     v_beta = torch.empty_like(fwd.beta) if fwd.is_beta else None
     v_unc = torch.empty_like(fwd.uncertainty) if fwd.uncertainty is not None else None
-    with torch.cuda.device(device):
+    with be.on(device):
         stream = be.stream_of(device)
         with stage("rasterize_bwd"):
             call("r2s_fused_raster_vjp", ptr(fwd.packed), ptr(fwd.offsets), ptr(fwd.tile_order), ptr(fwd.counters),
@@ -270,7 +270,7 @@ def voxel_frame(means, quats, scales, extent, center, dims, eps: float) -> torch
     N = means.shape[0]
     W, H, D = dims
     frame = torch.empty((N, 9), dtype=torch.float64, device=means.device)
-    with torch.cuda.device(means.device):
+    with be.on(means.device):
         call("r2s_voxel_frame", ptr(means), ptr(quats), ptr(scales), ptr(extent), ptr(center), W, H, D, float(eps),
              N, ptr(frame), be.stream_of(means.device))
     return frame
@@ -298,7 +298,7 @@ def voxel_vjp(state: dict, densities, beta, v_volume, dims, tile_size: int = 8, 
     v_dens = torch.empty((N,), dtype=torch.float32, device=device)
     v_beta = torch.empty((N,), dtype=torch.float32, device=device) if beta is not None else None
     v_unc = torch.empty((N,), dtype=torch.float32, device=device) if v_variance is not None else None
-    with torch.cuda.device(device):
+    with be.on(device):
         call("r2s_voxelize_fused_vjp", ptr(mapped), ptr(state["frame"]), ptr(state["conics"]),
              ptr(densities), ptr(beta),
              ptr(uncertainty if v_variance is not None else None), ptr(state["radii"]), ptr(state["tile_cum"]),
@@ -323,7 +323,7 @@ def voxel_render(state: dict, densities, beta, dims, tile_size: int = 8, *, unce
     T = int(tile_size)
     out = torch.empty((D, H, W), dtype=torch.float32, device=device)
     var = torch.empty_like(out) if uncertainty is not None else None
-    with torch.cuda.device(device):
+    with be.on(device):
         call("r2s_voxelize_fused_fwd", ptr(mapped), ptr(state["frame"]), ptr(state["conics"]),
              ptr(densities), ptr(beta),
              ptr(uncertainty), ptr(state["offsets"]), ptr(state["flatten_ids"]), state["flatten_ids"].numel(),

@@ -59,7 +59,7 @@ class _Launch:
 
     def __init__(self, ref: Tensor):
         self.device = ref.device
-        self._guard = torch.cuda.device(ref.device)
+        self._guard = be.on(ref.device)
 
     def __enter__(self):
         self._guard.__enter__()

@@ -539,13 +539,9 @@ vox_bwd_moments_kernel(VoxArgs<float> A, const int64_t* __restrict__ isect_ids, 
             float m0 = 0.f, m_x = 0.f, m_y = 0.f, m_z = 0.f, mxx = 0.f, myy = 0.f, mzz = 0.f, mxy = 0.f, mxz = 0.f,
                   myz = 0.f, se = 0.f, sl = 0.f, vq = 0.f;
             const float dx0 = (x0 - f.hi[0]) - f.lo[0];
-            // the columns' offsets and their squares are the same in every row
-            float dxc[T], dxsq[T];
+            float dxc[T];  // the columns' offsets, the same in every row
 #pragma unroll
-            for (uint32_t x = 0; x < T; ++x) {
-                dxc[x] = dx0 + float(x);
-                dxsq[x] = dxc[x] * dxc[x];
-            }
+            for (uint32_t x = 0; x < T; ++x) dxc[x] = dx0 + float(x);
             while (rows) {
                 const uint32_t bit = uint32_t(__builtin_ctzll(rows)), z = bit / T, y = bit % T;
                 rows &= rows - 1ull;
@@ -575,7 +571,7 @@ vox_bwd_moments_kernel(VoxArgs<float> A, const int64_t* __restrict__ isect_ids, 
                     const double dx4 = dx0d + double(h4);
 #pragma unroll
                     for (int x = 0; x < kStep; ++x) {
-                        float dx, dx2, q, h;
+                        float dx, q, h;
                         bool in;
                         if constexpr (WIDE) {
                             const double dxd = dx4 + double(x);
@@ -584,10 +580,8 @@ vox_bwd_moments_kernel(VoxArgs<float> A, const int64_t* __restrict__ isect_ids, 
                             h = float(1.0 - qd);
                             q = 0.f;
                             dx = float(dxd);
-                            dx2 = dx * dx;
                         } else {
                             dx = dxc[x];
-                            dx2 = dxsq[x];
                             q = fmaf(dx, fmaf(f.a, dx, c1), c0);
                             in = __float_as_uint(q) < f.qlim;
                             h = 1.f - q;
@@ -620,8 +614,9 @@ vox_bwd_moments_kernel(VoxArgs<float> A, const int64_t* __restrict__ isect_ids, 
                             }
                         }
                         r0 += gv;
-                        r1 = fmaf(gv, dx, r1);
-                        r2 = fmaf(gv, dx2, r2);
+                        const float gx = gv * dx;
+                        r1 += gx;
+                        r2 = fmaf(gx, dx, r2);
                     }
                 }
                 m0 += r0;
@@ -928,49 +923,38 @@ vox_fwd_fused_kernel(VoxArgs<float> A, float* __restrict__ out, float* __restric
     }
 }
 
-// Per-primitive sums of the intersection partials [cum[n], cum[n+1]) in a fixed
-// order (deterministic; no atomics): 16 lanes per primitive, lane 4 p + c adding
-// float4 c (of three) of the partials p, p + 4, .. in order, then the four
-// phases pairwise. (One lane per primitive read its partials one after another:
-// 65 us for 2.9M partials of 100k primitives, now 24, and 21 us for 285k of 3k,
-// now 5.)
-constexpr uint32_t kReduceLanes = 16, kReduceThreads = 256;
+// Per-primitive sums of the intersection partials [cum[n], cum[n+1]) in emission
+// order (deterministic; no atomics): four lanes per primitive, lane c adding float4
+// c (of three) of its partials one after another, kBatch loads ahead of the sums.
+// (One lane per primitive, a partial's three loads at a time: 65 us for 2.9M
+// partials of 100k primitives, now 31, and 21 us for 285k of 3k, now 6.)
+constexpr uint32_t kReduceLanes = 4, kReduceThreads = 256;
 
 __global__ void __launch_bounds__(kReduceThreads)
 vox_partials_reduce_kernel(const uint32_t* __restrict__ cum, const float* __restrict__ partials, uint32_t N,
                            uint32_t n_isects, float* __restrict__ v_xyz, float* __restrict__ v_c,
                            float* __restrict__ v_opac, float* __restrict__ v_beta, float* __restrict__ v_unc) {
-    constexpr uint32_t kBatch = 4, kGroups = kReduceThreads / kReduceLanes;  // loads in flight; primitives per round
-    const uint32_t column = threadIdx.x % 4, phase = (threadIdx.x % kReduceLanes) / 4;
+    constexpr uint32_t kBatch = 16, kGroups = kReduceThreads / kReduceLanes;  // loads in flight; primitives per round
+    const uint32_t column = threadIdx.x % kReduceLanes;
     const float4* part = reinterpret_cast<const float4*>(partials);
     static_assert(kVoxPartial == 12, "a partial is three float4");
-    for (uint32_t n0 = blockIdx.x * kGroups; n0 < N; n0 += gridDim.x * kGroups) {
-        const uint32_t n = n0 + threadIdx.x / kReduceLanes;
+    if (column == 3) return;
+    for (uint32_t n = blockIdx.x * kGroups + threadIdx.x / kReduceLanes; n < N; n += gridDim.x * kGroups) {
         float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (n < N && column < 3) {
-            const uint32_t lo = min(cum[n], n_isects), hi = min(cum[n + 1], n_isects);
-            for (uint32_t j = lo + phase; j < hi; j += 4 * kBatch) {
-                float4 p[kBatch];
+        const uint32_t lo = min(cum[n], n_isects), hi = min(cum[n + 1], n_isects);
+        for (uint32_t j = lo; j < hi; j += kBatch) {
+            float4 p[kBatch];
 #pragma unroll
-                for (uint32_t k = 0; k < kBatch; ++k)
-                    p[k] = j + 4 * k < hi ? part[3 * size_t(j + 4 * k) + column] : make_float4(0.f, 0.f, 0.f, 0.f);
+            for (uint32_t k = 0; k < kBatch; ++k)
+                p[k] = j + k < hi ? part[3 * size_t(j + k) + column] : make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
-                for (uint32_t k = 0; k < kBatch; ++k) {
-                    acc.x += p[k].x;
-                    acc.y += p[k].y;
-                    acc.z += p[k].z;
-                    acc.w += p[k].w;
-                }
+            for (uint32_t k = 0; k < kBatch; ++k) {
+                acc.x += p[k].x;
+                acc.y += p[k].y;
+                acc.z += p[k].z;
+                acc.w += p[k].w;
             }
         }
-#pragma unroll
-        for (int off = 4; off < int(kReduceLanes); off *= 2) {
-            acc.x += __shfl_xor(acc.x, off, kWave);
-            acc.y += __shfl_xor(acc.y, off, kWave);
-            acc.z += __shfl_xor(acc.z, off, kWave);
-            acc.w += __shfl_xor(acc.w, off, kWave);
-        }
-        if (n >= N || phase != 0) continue;
         if (column == 0) {  // v_mean, v_conic xx
             v_xyz[3 * size_t(n)] = acc.x;
             v_xyz[3 * size_t(n) + 1] = acc.y;
@@ -981,7 +965,7 @@ vox_partials_reduce_kernel(const uint32_t* __restrict__ cum, const float* __rest
             v_c[6 * size_t(n) + 2] = acc.y;
             v_c[6 * size_t(n) + 3] = acc.z;
             v_c[6 * size_t(n) + 4] = acc.w;
-        } else if (column == 2) {  // v_conic zz, v_opac, v_beta, v_q
+        } else {  // v_conic zz, v_opac, v_beta, v_q
             v_c[6 * size_t(n) + 5] = acc.x;
             v_opac[n] = acc.y;
             if (v_beta) v_beta[n] = acc.z;

@@ -728,10 +728,8 @@ extern "C" int r2s_rasterize_to_pixels_bwd_per_gaussian(
         using S = decltype(tag);
         const size_t CN = size_t(C) * N;
         if (int rc = zero_grads_2d<S>(CN, v_means2d_abs, v_means2d, v_conics, v_opacities, v_mus,
-                                      beta ? v_betas : nullptr, stream))
+                                      beta ? v_betas : nullptr, stream, v_uncertainties, N))
             return rc;
-        if (v_uncertainties)
-            if (int rc = fill_zero<S>((S*)v_uncertainties, N, stream)) return rc;
         if (n_isects == 0 || CN == 0) return R2S_OK;
         auto A = make_args<S>(means2d, conics, opacities, mus, betas, nullptr, nullptr, flatten_ids,
                               n_isects, C, N, width, height, tile_size, n_tiles_x, n_tiles_y);

@@ -1309,11 +1309,9 @@ extern "C" int r2s_voxelize_to_voxels_bwd(int dtype, const void* means3d, const 
     R2S_REQUIRE(!beta || v_betas != nullptr, "v_betas is required with betas");
     return dispatch_dtype(dtype, [&](auto tag) {
         using S = decltype(tag);
-        if (int rc = fill_zero<S>((S*)v_means3d, 3 * size_t(N), stream)) return rc;
-        if (int rc = fill_zero<S>((S*)v_conics, 6 * size_t(N), stream)) return rc;
-        if (int rc = fill_zero<S>((S*)v_opacities, N, stream)) return rc;
-        if (beta)
-            if (int rc = fill_zero<S>((S*)v_betas, N, stream)) return rc;
+        if (int rc = fill_zeros<S>({{v_means3d, 3 * size_t(N)}, {v_conics, 6 * size_t(N)}, {v_opacities, N},
+                                    {beta ? v_betas : nullptr, N}}, stream))
+            return rc;
         const uint64_t blocks = uint64_t(n_tiles_x) * n_tiles_y * n_tiles_z;
         if (blocks == 0 || n_isects == 0 || N == 0) return R2S_OK;
         const uint32_t threads = vox_threads(tile_size);
@@ -1341,13 +1339,9 @@ extern "C" int r2s_voxelize_to_voxels_bwd_per_gaussian(
     R2S_REQUIRE(!beta || v_betas != nullptr, "v_betas is required with betas");
     return dispatch_dtype(dtype, [&](auto tag) {
         using S = decltype(tag);
-        if (int rc = fill_zero<S>((S*)v_means3d, 3 * size_t(N), stream)) return rc;
-        if (int rc = fill_zero<S>((S*)v_conics, 6 * size_t(N), stream)) return rc;
-        if (int rc = fill_zero<S>((S*)v_opacities, N, stream)) return rc;
-        if (beta)
-            if (int rc = fill_zero<S>((S*)v_betas, N, stream)) return rc;
-        if (v_uncertainties)
-            if (int rc = fill_zero<S>((S*)v_uncertainties, N, stream)) return rc;
+        if (int rc = fill_zeros<S>({{v_means3d, 3 * size_t(N)}, {v_conics, 6 * size_t(N)}, {v_opacities, N},
+                                    {beta ? v_betas : nullptr, N}, {v_uncertainties, N}}, stream))
+            return rc;
         if (n_isects == 0 || N == 0) return R2S_OK;
         auto A = make_vox_args<S>(means3d, conics, opacities, betas, nullptr, nullptr, flatten_ids,
                                   n_isects, N, dim_x, dim_y, dim_z, tile_size, n_tiles_x,

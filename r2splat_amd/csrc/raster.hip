@@ -246,7 +246,7 @@ raster_bwd_isect_kernel(RasterArgs<S> A, const int64_t* __restrict__ isect_ids,
 // cost, so rows outside the footprint are what there is to save: 20k Gaussians
 // on 8 views of 128^2 touch 9.8 of 16 rows per tile. A pixel per thread over
 // the whole list took 688 us there (four waves a tile, two a SIMD), a wave per
-// intersection with its nine wave reductions 494 us; these take 206 and 157. What
+// intersection with its nine wave reductions 494 us; these take 144 and 157. What
 // bounds them is double arithmetic in the few tiles that the object covers.
 // ---------------------------------------------------------------------------
 // Rows [lo, hi) of a T-row tile (first pixel centre at row y_base + 1/2) in which
@@ -286,6 +286,16 @@ __device__ __forceinline__ void reached_rows(const Prim2D<S>& p, S y_base, int T
     hi = max(lo, int(fminf(fmaxf(floorf(c + ext) + 1.f, 0.f), float(T))));
 }
 
+// Columns [lo, hi) in which |alpha| can reach 1e-5: reached_rows with x and y exchanged.
+template <typename S, bool BETA>
+__device__ __forceinline__ void reached_cols(const Prim2D<S>& p, S x_base, int T, int& lo, int& hi) {
+    Prim2D<S> t = p;
+    t.my = p.mx;
+    t.a = p.c;
+    t.c = p.a;
+    reached_rows<S, BETA>(t, x_base, T, lo, hi);
+}
+
 // The form at a pixel, from a dx, dx, b dx (twice that for Beta), c and dy, in the
 // roundings eval_profile compiles to: a thin footprint's float32 terms cancel, and any other order would give
 // such a primitive an exponent that differs from the general kernel's.
@@ -316,7 +326,9 @@ __device__ __forceinline__ Prim2D<S> load_prim(const RasterArgs<S>& A, int32_t g
 // skipped by scalar branches. The waves' partial images are summed in wave order.
 // SPLIT: a workgroup renders one row group of a tile (PX workgroups a tile), for
 // launches of few tiles, whose lists are long where the object is: 20k Gaussians
-// on 8 views of 128^2 have 128 tiles that matter, half the compute units.
+// on 8 views of 128^2 have 128 tiles that matter, half the compute units. Row groups
+// of 16-pixel tiles are four blocks of 4 x 4 pixels there, each with a list of the
+// batch's records that reach it (206 -> 144 us there).
 template <typename S>
 struct OpRec {
     S mx, my, a, b, c, w, beta, q;
@@ -332,8 +344,10 @@ __global__ void __launch_bounds__((op_waves<T, SPLIT>() * kWave))
 raster_fwd_rows_kernel(RasterArgs<S> A, S* __restrict__ out, S* __restrict__ out_var) {
     constexpr int WAVES = op_waves<T, SPLIT>(), STEP = kWave / T, GROUPS = T * T / kWave, PX = SPLIT ? 1 : GROUPS;
     constexpr uint32_t kPixels = PX * kWave;
-    __shared__ OpRec<S> stage[WAVES][kWave];
+    constexpr bool BLOCKS = SPLIT && T == 16;
+    __shared__ OpRec<S> stage[WAVES][kWave + (BLOCKS ? 1 : 0)];
     __shared__ S part[WAVES][kPixels];
+    __shared__ __align__(16) uint8_t lists[BLOCKS ? WAVES : 1][4][kWave];
     uint32_t cam, ty, tx;
     int32_t start, end;
     const uint32_t group = SPLIT ? blockIdx.x % GROUPS : 0u, y0 = group * STEP;  // the workgroup's first row
@@ -349,8 +363,9 @@ raster_fwd_rows_kernel(RasterArgs<S> A, S* __restrict__ out, S* __restrict__ out
         acc_var[k] = S(0);
     }
     OpRec<S>* slot = stage[wave];
+    if (BLOCKS && lane == 0) slot[kWave] = OpRec<S>{};  // the record past a list's end: no weight
     for (int32_t base = start + int32_t(wave) * kWave; base < end; base += WAVES * kWave) {
-        uint32_t groups = 0;
+        uint32_t groups = 0, blocks = 0;
         OpRec<S> r = {};
         if (base + int32_t(lane) < end) {
             const int32_t g = A.flatten[base + int32_t(lane)];
@@ -361,12 +376,23 @@ raster_fwd_rows_kernel(RasterArgs<S> A, S* __restrict__ out, S* __restrict__ out
                 const int k_lo = lo / STEP, k_hi = (hi + STEP - 1) / STEP;
                 if (lo < hi) groups = (((1u << k_hi) - 1u) & ~((1u << k_lo) - 1u)) >> group;
                 if constexpr (SPLIT) groups &= 1u;
+                if constexpr (BLOCKS) {
+                    if (groups != 0u) {
+                        int c_lo, c_hi;
+                        reached_cols<S, BETA>(p, S(tx * T), T, c_lo, c_hi);
+                        if (c_lo < c_hi) blocks = (0xfu >> (3 - ((c_hi - 1) >> 2))) & (0xfu << (c_lo >> 2));
+                    }
+                }
                 r = OpRec<S>{p.mx, p.my, p.a, p.b, p.c, p.opac * p.mu, p.beta, VAR ? A.unc[uint32_t(g) % A.N] : S(0)};
             }
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();  // every lane is done with the previous batch
         slot[lane] = r;
+        if constexpr (BLOCKS) {
+            constexpr uint32_t kFill = uint32_t(kWave) * 0x01010101u;
+            reinterpret_cast<uint32_t*>(lists[wave])[lane] = kFill;
+        }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
         const auto splat = [&](const OpRec<S>& s, uint32_t rows) {
@@ -391,6 +417,27 @@ raster_fwd_rows_kernel(RasterArgs<S> A, S* __restrict__ out, S* __restrict__ out
                 if constexpr (VAR) acc_var[k] += s.q * alpha * alpha;
             }
         };
+        if constexpr (BLOCKS) {
+            // each 4 x 4 block of the row group (16 lanes) walks the records that reach it
+            uint32_t longest = 0;
+#pragma unroll
+            for (uint32_t b = 0; b < 4; ++b) {
+                const uint64_t members = __ballot((blocks >> b) & 1u);
+                const uint32_t at = __builtin_amdgcn_mbcnt_hi(uint32_t(members >> 32),
+                                                              __builtin_amdgcn_mbcnt_lo(uint32_t(members), 0u));
+                if ((blocks >> b) & 1u) lists[wave][b][at] = uint8_t(lane);
+                longest = max(longest, uint32_t(__popcll(members)));
+            }
+            wave_lds_sync();
+            const uint8_t* list = lists[wave][(lane % 16u) / 4u];
+            OpRec<S> next = slot[list[0]];
+            for (uint32_t k = 0; k < longest; ++k) {
+                const OpRec<S> now = next;
+                next = slot[list[min(k + 1u, uint32_t(kWave) - 1u)]];  // read while this one is evaluated
+                splat(now, 1u);
+            }
+            continue;
+        }
         // the batch's records that reach a group, the next one read from LDS while
         // this one is evaluated (two registers that alternate roles)
         uint64_t todo = __ballot(groups != 0u);

@@ -20,7 +20,8 @@ namespace r2s {
 // indices come from 32-bit divisions per VEC elements instead of 64-bit ones
 // per element (anisotropic gradient 91 -> 30 us); and the isotropic gradient
 // marches along z, so that a voxel costs 2.25 square roots instead of four
-// (126 -> 66 us, bound by the correctly rounded square roots and divisions).
+// (126 -> 66 us, and by sharing terms between threads to 54, bound by the
+// correctly rounded square roots and divisions).
 constexpr int kLossThreads = 256;
 constexpr int kSumThreads = 1024;
 constexpr uint32_t kSumBlocks = 512;  // two per CU
@@ -200,21 +201,32 @@ tv_bwd_kernel(const S* __restrict__ vol, const S* __restrict__ grad_out, Volume<
 // d/dV(v) of sum_u t(u), t the isotropic term: -(dz + dy + dx)(v) / t(v) plus
 // dz(v - ez) / t(v - ez), dy(v - ey) / t(v - ey) and dx(v - ex) / t(v - ex)
 // where those voxels exist. A thread takes a pack's column over kMarch planes:
-// plane d's dz / t is what plane d + 1 needs, and the pack's own dx / t what
-// its next columns need, so a voxel costs its own term, the one below it in y
-// and 1 / VEC of the one to its left. `total` counts (plane chunk, row, pack).
+// plane d's dz / t is what plane d + 1 needs, a pack's last dx / t what the next
+// lane needs, and its dy / t what the thread of the row above needs (through LDS,
+// `quads` threads on), so that a voxel costs one correctly rounded square root and
+// four divisions, which bound the kernel; only a workgroup's first row, a wave's
+// first lane and a march's first plane evaluate a neighbour's terms (each thread
+// evaluating its neighbours: 67 us for 256^3 floats, now 54). `total` counts
+// (plane chunk, row, pack).
+constexpr int kMarchThreads = 512;
+
 template <typename S, typename I, int VEC>
-__global__ void __launch_bounds__(kLossThreads)
+__global__ void __launch_bounds__(kMarchThreads)
 tv_iso_bwd_kernel(const S* __restrict__ vol, const S* __restrict__ grad_out, Volume<I> g, uint32_t chunks, S eps,
                   S scale, S* __restrict__ grad) {
-    const I i = I(blockIdx.x) * kLossThreads + threadIdx.x;
-    if (i >= g.total) return;
+    __shared__ Pack<S, VEC> shared_y[2][kMarchThreads];  // dy / t, by the parity of the plane
+    const I mine = I(blockIdx.x) * kMarchThreads + threadIdx.x;
+    const bool valid = mine < g.total;  // (the others repeat the last pack and store nothing)
+    const I i = valid ? mine : g.total - 1;
     const I row = i / g.quads, slab = row / I(g.H);
     const uint32_t x = uint32_t(i - row * g.quads) * VEC, h = uint32_t(row - slab * I(g.H));
     const I b = slab / I(chunks);
     const uint32_t d0 = uint32_t(slab - b * I(chunks)) * kMarch, d1 = min(g.D, d0 + kMarch);
     const size_t sd = size_t(g.H) * g.W, sh = g.W;
     const bool has_yn = h + 1 < g.H, has_yp = h > 0, has_xn = x + VEC < g.W, has_xp = x > 0;
+    // the threads of the packs to the left and in the row above, if in this wave and workgroup
+    const bool left_lane = valid && has_xp && threadIdx.x % kWave != 0;
+    const bool row_thread = valid && has_yp && I(threadIdx.x) >= g.quads;
     const S gs = grad_out[0] * scale;
     size_t o = ((size_t(b) * g.D + d0) * g.H + h) * g.W + x;
     Pack<S, VEC> c = load_pack<S, VEC>(vol + o);
@@ -231,48 +243,70 @@ tv_iso_bwd_kernel(const S* __restrict__ vol, const S* __restrict__ grad_out, Vol
 #pragma unroll
         for (int k = 0; k < VEC; ++k) below[k] = dz[k] / sqrt(dz[k] * dz[k] + dy[k] * dy[k] + dx[k] * dx[k] + eps);
     }
-    for (uint32_t d = d0; d < d1; ++d, o += sd) {
+    for (uint32_t step = 0; step < kMarch; ++step, o += sd) {  // every thread takes every step: barriers
+        const uint32_t d = d0 + step;
+        const bool active = d < d1;
+        Pack<S, VEC> zn = c, yt;
+        S out[VEC], xt[VEC], carry_x = S(0);  // -(dz + dy + dx) / t, dx / t; dx / t of the voxel to the left
         const bool has_z = d + 1 < g.D;
-        const Pack<S, VEC> zn = has_z ? load_pack<S, VEC>(vol + o + sd) : c;
-        const Pack<S, VEC> yn = has_yn ? load_pack<S, VEC>(vol + o + sh) : c;
-        const S right = has_xn ? vol[o + VEC] : S(0);
-        S dz[VEC], dy[VEC], dx[VEC];
-        differences<S, VEC>(c, zn, yn, right, has_z, has_yn, has_xn, dz, dy, dx);
-        S carry_x = S(0);  // dx / t of the voxel to the left
-        if (has_xp) {
-            const S l = vol[o - 1];
-            const S lz = has_z ? vol[o + sd - 1] - l : S(0), ly = has_yn ? vol[o + sh - 1] - l : S(0);
-            const S lx = c.v[0] - l;
-            carry_x = lx / sqrt(lz * lz + ly * ly + lx * lx + eps);
-        }
-        S from_y[VEC];  // dy / t of the voxel at y - 1
+        if (active) {
+            if (has_z) zn = load_pack<S, VEC>(vol + o + sd);
+            const Pack<S, VEC> yn = has_yn ? load_pack<S, VEC>(vol + o + sh) : c;
+            const S right = has_xn ? vol[o + VEC] : S(0);
+            S dz[VEC], dy[VEC], dx[VEC];
+            differences<S, VEC>(c, zn, yn, right, has_z, has_yn, has_xn, dz, dy, dx);
 #pragma unroll
-        for (int k = 0; k < VEC; ++k) from_y[k] = S(0);
-        if (has_yp) {
-            const size_t q = o - sh;
-            const Pack<S, VEC> p = load_pack<S, VEC>(vol + q);
-            const Pack<S, VEC> pz = has_z ? load_pack<S, VEC>(vol + q + sd) : p;
-            const S pr = has_xn ? vol[q + VEC] : S(0);
-            S az[VEC], ay[VEC], ax[VEC];
-            differences<S, VEC>(p, pz, c, pr, has_z, true, has_xn, az, ay, ax);
-#pragma unroll
-            for (int k = 0; k < VEC; ++k)
-                from_y[k] = ay[k] / sqrt(az[k] * az[k] + ay[k] * ay[k] + ax[k] * ax[k] + eps);
+            for (int k = 0; k < VEC; ++k) {
+                const S t = sqrt(dz[k] * dz[k] + dy[k] * dy[k] + dx[k] * dx[k] + eps);
+                out[k] = -(dz[k] + dy[k] + dx[k]) / t;
+                out[k] += below[k];
+                below[k] = dz[k] / t;
+                yt.v[k] = dy[k] / t;
+                xt[k] = dx[k] / t;
+            }
+            shared_y[step % 2][threadIdx.x] = yt;
+            carry_x = __shfl_up(xt[VEC - 1], 1, kWave);  // (the left pack's lane takes the same steps)
+            if (!left_lane) {
+                carry_x = S(0);
+                if (has_xp) {
+                    const S l = vol[o - 1];
+                    const S lz = has_z ? vol[o + sd - 1] - l : S(0), ly = has_yn ? vol[o + sh - 1] - l : S(0);
+                    const S lx = c.v[0] - l;
+                    carry_x = lx / sqrt(lz * lz + ly * ly + lx * lx + eps);
+                }
+            }
         }
-        Pack<S, VEC> out;
+        __syncthreads();  // (the other buffer's readers passed it before the last one)
+        if (active) {
+            S from_y[VEC];  // dy / t of the voxel at y - 1
 #pragma unroll
-        for (int k = 0; k < VEC; ++k) {
-            const S t = sqrt(dz[k] * dz[k] + dy[k] * dy[k] + dx[k] * dx[k] + eps);
-            S s = -(dz[k] + dy[k] + dx[k]) / t;
-            s += below[k];
-            s += from_y[k];
-            s += carry_x;
-            out.v[k] = s * gs;
-            below[k] = dz[k] / t;
-            carry_x = dx[k] / t;
+            for (int k = 0; k < VEC; ++k) from_y[k] = S(0);
+            if (row_thread) {
+                const Pack<S, VEC> p = shared_y[step % 2][threadIdx.x - uint32_t(g.quads)];
+#pragma unroll
+                for (int k = 0; k < VEC; ++k) from_y[k] = p.v[k];
+            } else if (has_yp) {
+                const size_t q = o - sh;
+                const Pack<S, VEC> p = load_pack<S, VEC>(vol + q);
+                const Pack<S, VEC> pz = has_z ? load_pack<S, VEC>(vol + q + sd) : p;
+                const S pr = has_xn ? vol[q + VEC] : S(0);
+                S az[VEC], ay[VEC], ax[VEC];
+                differences<S, VEC>(p, pz, c, pr, has_z, true, has_xn, az, ay, ax);
+#pragma unroll
+                for (int k = 0; k < VEC; ++k)
+                    from_y[k] = ay[k] / sqrt(az[k] * az[k] + ay[k] * ay[k] + ax[k] * ax[k] + eps);
+            }
+            Pack<S, VEC> w;
+#pragma unroll
+            for (int k = 0; k < VEC; ++k) {
+                S s = out[k];
+                s += from_y[k];
+                s += k > 0 ? xt[k > 0 ? k - 1 : 0] : carry_x;
+                w.v[k] = s * gs;
+            }
+            if (valid) store_pack<S, VEC>(grad + o, w);
+            c = zn;
         }
-        store_pack<S, VEC>(grad + o, out);
-        c = zn;
     }
 }
 
@@ -445,7 +479,7 @@ extern "C" int r2s_volume_tv_iso_bwd(int dtype, const void* volume, const void* 
             using I = decltype(index);
             constexpr int VEC = decltype(vec)::value;
             const Volume<I> g{I(W / VEC), I(rows * (W / VEC)), D, H, W};
-            tv_iso_bwd_kernel<S, I, VEC><<<ceil_div(g.total, kLossThreads), kLossThreads, 0, stream>>>(
+            tv_iso_bwd_kernel<S, I, VEC><<<ceil_div(g.total, kMarchThreads), kMarchThreads, 0, stream>>>(
                 (const S*)volume, (const S*)grad_output, g, chunks, S(eps), S(lambda_tv / double(total)),
                 (S*)grad_volume);
             return check_launch("volume_tv_iso_bwd");

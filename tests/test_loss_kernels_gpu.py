@@ -62,3 +62,19 @@ def test_image_l1_at_pack_edges(n, offset, dtype):
     assert torch.equal(l1_map.cpu(), expected)
     t = 2e-6 if dtype == torch.float32 else 1e-12
     assert abs(l1.item() - expected.double().mean().item()) <= t * expected.double().mean().item()
+
+
+# rows of fewer, as many and more packs than a workgroup has threads, and workgroups
+# whose threads lie in several plane chunks of different lengths
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("shape", [(1, 9, 7, 20), (2, 3, 33, 6), (1, 20, 3, 2048), (1, 10, 2, 2052), (1, 11, 5, 1031),
+                                   (3, 17, 2, 4)])
+def test_isotropic_gradient_where_threads_share_terms(shape, dtype):
+    device = torch.device("cuda:0")
+    g = torch.Generator().manual_seed(sum(shape))
+    vol = torch.randn(*shape, generator=g, dtype=torch.float64).to(dtype)
+    ref = vol.double().requires_grad_()
+    (grad,) = torch.autograd.grad(O.volume_tv_iso(ref, 1e-8), ref)
+    got = ops.volume_loss_iso_bwd(vol.to(device), torch.ones(1, device=device, dtype=dtype), 1.0)
+    t = 1e-5 if dtype == torch.float32 else 5e-12  # as above: five roundings of a short chain
+    assert O.relative_error(got, grad) <= t

@@ -441,16 +441,20 @@ __device__ __forceinline__ VoxForm vox_form(const VoxArgs<float>& A, size_t G, c
 // the mean shifted by (xs, ys) dz; its extent in y over the row's eight columns
 // is that of its upper and lower branches y(x) = (+-sqrt(4 cyy S - den x^2) - bxy
 // x) / 2 cyy, den = 4 a cyy - bxy^2, at their extremes clamped to the columns. S
-// is widened by 2e-3 and the columns and rows by 0.05 voxels, which covers the
-// rounding of q and of this bound where den and k do not cancel (to 1e-3);
-// other forms get every row, and a form no term of which passes none.
+// is widened by 2e-3 and the columns and rows by 0.05 voxels. That covers the
+// float32 rounding of q and of this bound while the determinant k den of the form
+// is at least 1e-3 of the product of its diagonal: k is formed with den's error,
+// so two cancellations of 1e-3 each, as in a thin disc's form, leave an error of
+// a few percent of k. Forms that cancel further get every row, and a form no term
+// of which passes none.
 __device__ __forceinline__ uint64_t vox_row_mask(const VoxForm& f, float S, float x0, float y0, float z0) {
     if (f.qlim == 0u) return 0ull;
     const float ac4 = 4.f * f.a * f.cyy, den = ac4 - f.bxy * f.bxy, inv = __builtin_amdgcn_rcpf(den);
     const float xs = (f.bxy * f.cyz - 2.f * f.cyy * f.bxz) * inv, ys = (f.bxy * f.bxz - 2.f * f.a * f.cyz) * inv;
     const float k = f.czz + 0.5f * (f.bxz * xs + f.cyz * ys);
     const float wide = S * 1.002f;
-    if (!(f.a > 0.f) || !(f.cyy > 0.f) || !(den > 1e-3f * ac4) || !(k > 1e-3f * f.czz) || !(wide * inv < 1e30f))
+    if (!(f.a > 0.f) || !(f.cyy > 0.f) || !(den > 1e-3f * ac4) || !(k * den > 1e-3f * f.czz * ac4) ||
+        !(wide * inv < 1e30f))
         return ~0ull;
     const float reach_x = __builtin_amdgcn_sqrtf(4.f * f.cyy * inv) * 1.001f;      // per sqrt of the plane's bound
     const float top = -0.5f * f.bxy * __builtin_amdgcn_rcpf(f.a) * __builtin_amdgcn_sqrtf(4.f * f.a * inv);

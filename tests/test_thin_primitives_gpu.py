@@ -1,0 +1,74 @@
+"""Bounds on what a thin primitive reaches: kernels that skip rows, octants, blocks
+or columns against every voxel or pixel that a primitive's own form covers."""
+
+import pytest
+import torch
+
+from r2splat_amd import fused, hip as ops
+from r2splat_amd.hip._wrapper import _isect_tiles_3d
+
+pytestmark = pytest.mark.gpu
+
+# ---------------------------------------------------------------------------
+# voxel VJPs: discs of 40:1 to 100:1 tilted off the axes, half-axes of 15 to 60
+# voxels, at beta 1/2. Both minors of such a form cancel, each by less than 1e-3,
+# their product by more. The adjoint is 1 on the outer tenth of the support, so
+# that a voxel of a dropped row shows in the sums. The reference sums the
+# definition in double over the whole volume.
+# ---------------------------------------------------------------------------
+SIDE, DISCS = 96, 60
+
+
+def _discs(seed):
+    g = torch.Generator().manual_seed(seed)
+    r = lambda *s: torch.rand(*s, generator=g, dtype=torch.float64)  # noqa: E731
+    q, _ = torch.linalg.qr(r(DISCS, 3, 3) - 0.5)
+    long = 15.0 + 45.0 * r(DISCS, 1)
+    s = torch.cat([long / (40.0 + 60.0 * r(DISCS, 1)), long, long * (0.8 + 0.2 * r(DISCS, 1))], 1)
+    P = q @ torch.diag_embed(s ** -2) @ q.transpose(1, 2)
+    means = SIDE * (0.3 + 0.4 * r(DISCS, 3))
+    return means, torch.stack([P[:, 0, 0], P[:, 0, 1], P[:, 0, 2], P[:, 1, 1], P[:, 1, 2], P[:, 2, 2]], 1)
+
+
+def _disc_reference(mean, conic, beta, w):
+    """(adjoint, sum v h^beta, sum v w h^beta log h) over the volume, in double."""
+    axis = torch.arange(SIDE, device=mean.device, dtype=torch.float64) + 0.5
+    z, y, x = torch.meshgrid(axis, axis, axis, indexing="ij")
+    dx, dy, dz = x - mean[0], y - mean[1], z - mean[2]
+    h = 1.0 - (conic[0] * dx * dx + conic[3] * dy * dy + conic[5] * dz * dz +
+               2.0 * (conic[1] * dx * dy + conic[2] * dx * dz + conic[4] * dy * dz))
+    shell = (h > 1e-4) & (h < 0.1)  # (the float32 form of the innermost 1e-4 carries no digits)
+    vis = torch.where(shell, h, torch.ones_like(h)).pow(beta) * shell
+    return shell.to(torch.float32), vis.sum(), (w * vis * torch.where(shell, h, torch.ones_like(h)).log()).sum()
+
+
+@pytest.mark.parametrize("seed", [1, 2])
+@pytest.mark.parametrize("kernel", ["fused", "operator"])
+def test_voxel_vjps_of_thin_discs(device, kernel, seed):
+    means, conics = (t.to(device) for t in _discs(seed))
+    n = -(-SIDE // 8)
+    radii = torch.full((1, 3), 4 * SIDE, dtype=torch.int32, device=device)
+    for k in range(DISCS):
+        mean, conic = means[k:k + 1].contiguous(), conics[k:k + 1].contiguous()
+        if kernel == "fused":  # float32 weights; the form is double in both
+            mean32 = mean.float()
+            _, ids, flat, cum = _isect_tiles_3d(mean32, radii, 8, n, n, n)
+            beta = torch.full((1,), 0.5, device=device)
+            w = torch.full((1,), 0.7, device=device)
+            v, v_w, v_beta = _disc_reference(means[k], conics[k], 0.5, float(w))
+            state = dict(mapped=mean32, frame=torch.cat([mean, conic], 1).contiguous(), conics=conic.float(),
+                         radii=radii, tile_cum=cum, isect_ids=ids, flatten_ids=flat)
+            got = fused.voxel_vjp(state, w, beta, v, (SIDE, SIDE, SIDE))
+            tol = 1e-5  # float32 sums of up to a few thousand terms of one sign
+        else:
+            _, ids, flat = ops.isect_tiles_3d(mean, radii, 8, n, n, n)
+            off = ops.isect_offset_encode_3d(ids, n, n, n)
+            beta = torch.full((1,), 0.5, device=device, dtype=torch.float64)
+            w = torch.full((1,), 0.7, device=device, dtype=torch.float64)
+            v, v_w, v_beta = _disc_reference(means[k], conics[k], 0.5, float(w))
+            got = ops.beta_voxelize_to_voxels_bwd_per_gaussian(mean, conic, w, beta, off, ids, flat, v.double(), SIDE,
+                                                               SIDE, SIDE, 8)
+            tol = 1e-9
+        assert ids.numel() == n ** 3
+        for name, a, b in (("opacity", got[2][0], v_w), ("beta", got[3][0], v_beta)):
+            assert abs(float(a) - float(b)) <= tol * abs(float(b)), (k, name, float(a), float(b))

@@ -4,7 +4,7 @@ or columns against every voxel or pixel that a primitive's own form covers."""
 import pytest
 import torch
 
-from r2splat_amd import fused, hip as ops
+from r2splat_amd import fused, hip as ops, parity
 from r2splat_amd.hip._wrapper import _isect_tiles_3d
 
 pytestmark = pytest.mark.gpu
@@ -72,3 +72,70 @@ def test_voxel_vjps_of_thin_discs(device, kernel, seed):
         assert ids.numel() == n ** 3
         for name, a, b in (("opacity", got[2][0], v_w), ("beta", got[3][0], v_beta)):
             assert abs(float(a) - float(b)) <= tol * abs(float(b)), (k, name, float(a), float(b))
+
+
+# ---------------------------------------------------------------------------
+# Beta rasterizer: needles of 1000:1 to 3000:1, hundreds of pixels long, whose end
+# lies in the image. The 16-pixel forward walks 4 x 4 blocks and the backward
+# segments of 8 columns, so each has a bound on columns beside the one on rows;
+# the keep masks know the rows alone. A pixel is lit exactly where the forward's
+# mask keeps the primitive, and an adjoint of one kept pixel reaches the density.
+# ---------------------------------------------------------------------------
+IMAGE, VIEWS = 160, 4096
+
+
+def _needle(seed, device):
+    g = torch.Generator().manual_seed(seed)
+    r = lambda *s: torch.rand(*s, generator=g, dtype=torch.float64)  # noqa: E731
+    f = 1.2 * IMAGE
+    px = 2.5 / f  # world units of a pixel at the needle's depth
+    half = 460.0
+    theta, end = 6.2832 * r(VIEWS), IMAGE * (0.05 + 0.9 * r(VIEWS, 2)) - IMAGE / 2
+    c, s = torch.cos(theta), torch.sin(theta)
+    views = torch.zeros(VIEWS, 4, 4, dtype=torch.float64)
+    views[:, 0, 0], views[:, 0, 1], views[:, 1, 0], views[:, 1, 1] = c, -s, s, c
+    views[:, 2, 2] = views[:, 3, 3] = 1.0
+    views[:, :2, 3] = (end - half * torch.stack([c, s], 1)) * px  # the needle's mean is the world origin
+    views[:, 2, 3] = 2.5
+    Ks = torch.tensor([[f, 0.0, IMAGE / 2], [0.0, f, IMAGE / 2], [0.0, 0.0, 1.0]], dtype=torch.float64)
+    thin = half * px / (1000.0 + 2000.0 * float(r(1)))
+    prims = [torch.zeros(1, 3), torch.tensor([[1.0, 0.0, 0.0, 0.0]]), torch.tensor([[half * px, thin, thin]]),
+             torch.ones(1)]
+    return ([t.to(device, torch.float32).contiguous() for t in prims],
+            views.to(device, torch.float32), Ks.expand(VIEWS, 3, 3).to(device, torch.float32).contiguous())
+
+
+def _pixels(table, words, device):
+    """Which pixels [view, y, x] a keep mask keeps (one primitive)."""
+    n, T = table.cam.numel(), table.tile
+    bits = (words[:, :, None] >> torch.arange(32, device=device, dtype=torch.int32)) & 1
+    e, p = bits.reshape(n, T * T).bool().nonzero(as_tuple=True)
+    kept = torch.zeros(VIEWS, IMAGE, IMAGE, dtype=torch.bool, device=device)
+    kept[table.cam[e], table.ty[e] * T + p // T, table.tx[e] * T + p % T] = True
+    return kept
+
+
+@pytest.mark.parametrize("seed", [1, 2, 3])
+def test_beta_rasterizer_of_needles(device, seed):
+    prims, views, Ks = _needle(seed, device)
+    beta = torch.full((1,), 0.6, device=device)
+    args = (*prims, views, Ks)
+    image, fwd = fused.forward(*args, IMAGE, IMAGE, 1e-8, 1.0, beta=beta)
+    table = parity.pair_table(fwd, VIEWS, 1)
+    kept = _pixels(table, table.mask_fwd, device)
+    assert int(kept.sum()) > VIEWS
+    lit = image != 0
+    strays, lost = int((lit & ~kept).sum()), int((kept & ~lit).sum())
+    assert (strays, lost) == (0, 0)
+    # the kept pixels nearest the needle's ends in x, one adjoint per view; views one by one
+    both = kept & _pixels(table, table.mask_bwd, device) & (image > 1e-3)
+    cols = both.any(1)
+    first, last = cols.int().argmax(1), IMAGE - 1 - cols.flip(1).int().argmax(1)
+    v = torch.zeros(1, IMAGE, IMAGE, device=device)
+    for k in cols.any(1).nonzero().flatten().tolist()[:1500]:
+        _, one = fused.forward(*prims, views[k:k + 1], Ks[k:k + 1], IMAGE, IMAGE, 1e-8, 1.0, beta=beta)
+        for x in (int(first[k]), int(last[k])):
+            y = int(both[k, :, x].int().argmax())
+            v.zero_()[0, y, x] = 1.0
+            grads = fused.backward(one, *prims, views[k:k + 1], Ks[k:k + 1], v)
+            assert float(grads[3][0]) > 0.0, (k, y, x)

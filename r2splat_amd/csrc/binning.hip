@@ -390,8 +390,10 @@ static SortLayout sort_layout(uint64_t n) {
     L.off_a_vals = o; o += kb;
     L.off_b_keys = o; o += kb;
     L.off_b_vals = o; o += kb;
-    // (a workspace never shrinks as n grows past 2^20, where the tiles get larger)
-    const size_t hist_n = size_t(kRadix) * std::max<size_t>(L.n_blocks, n > (1u << 20) ? 1024 : 0);
+    // (the workspace never shrinks as n grows: past 2^16, 2^17 and 2^20 keys, where the
+    // tiles get larger, it has room for the workgroups of the counts below)
+    const uint32_t most = std::max(L.n_blocks, n > (1u << 20) ? 1024u : n > (1u << 16) ? 64u : 0u);
+    const size_t hist_n = size_t(kRadix) * most;
     L.off_hist = o; o += align256((hist_n + 1) * 4);
     L.off_scan = o; o += align256(scan_levels_bytes(hist_n));
     L.total = o;

@@ -102,6 +102,17 @@ def test_fused_size_queries_need_no_gpu():
     assert b - a >= 8 * 10**6
 
 
+def test_sort_workspace_never_shrinks_as_the_count_grows():
+    """A caller that sizes its workspace once, for the largest count it expects,
+    may sort any smaller count with it: the tiles a sort is cut into grow with
+    the count, its workspace does not shrink."""
+    lib = _backend.lib(require_gpu=False)
+    counts = sorted({max(0, (1 << k) + d) for k in range(9, 23) for d in (-4097, -1, 0, 1, 1000, 4097)})
+    for query in (lambda n: lib.r2s_sort_workspace_bytes(n, 0), lib.r2s_scan_workspace_bytes):
+        sizes = [query(n) for n in counts]
+        assert sizes == sorted(sizes)
+
+
 def test_workspace_growth_is_all_or_nothing(monkeypatch):
     """A capacity growth that runs out of memory part way leaves every buffer
     and the version (which graphs captured on the workspace check) as they

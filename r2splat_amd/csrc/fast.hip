@@ -2235,7 +2235,8 @@ static size_t packed_bytes(uint32_t C, uint32_t N, uint32_t capacity, int kind) 
 // once do (one view of 333 x 517 with 30k primitives: 100 us of binning kernels
 // against 145 us of sort and pack), and larger grids or more waves sort and pack (500k
 // primitives x 256 views of 512^2 took 49.6 ms a step placing, 44.7 sorting).
-// Calls of the middle kind have scratch for either.
+// Which of the two a call of the middle kind takes depends on C and N, so its scratch
+// has room for either, in one place.
 constexpr size_t kPlaceLdsBytes = 16384, kPlaceLargeBytes = 40960, kLdsBytes = 163840;
 constexpr uint64_t kComputeUnits = 256;
 constexpr uint32_t kPlaceWaves = 4096;  // target number of ranges (waves) per binning pass
@@ -2259,6 +2260,7 @@ static FusedScratch fused_scratch(uint32_t C, uint32_t N, uint32_t n_tiles, uint
     L.reach = o; o += al(CN * ((kind & kKindBeta) ? sizeof(Reach<true>) : sizeof(Reach<false>)));
     const uint64_t nt = C ? n_tiles / C : 0;
     const size_t table = nt * kBinClasses * sizeof(uint32_t);
+    size_t p = o;  // the placement's tables, where the sort's buffers lie otherwise
     if (C > 0 && nt > 0 && table <= kPlaceLargeBytes) {
         L.n_bins = uint32_t(nt) * kBinClasses;
         L.bin_bits = 32u - uint32_t(__builtin_clz(L.n_bins - 1u));
@@ -2272,25 +2274,23 @@ static FusedScratch fused_scratch(uint32_t C, uint32_t N, uint32_t n_tiles, uint
         L.place = table <= kPlaceLdsBytes ||
                   uint64_t(C) * L.n_ranges <= kComputeUnits * (kLdsBytes / (table + sizeof(PairList)));
         if (L.place) {
-            L.range_counts = o; o += al(size_t(C) * L.n_ranges * L.n_bins * 4 + 4);
-            L.range_totals = o; o += al(size_t(C) * L.n_ranges * 4 + 4);
-            L.bin_totals = o; o += al(size_t(C) * L.n_bins * 4 + 4);
+            L.range_counts = p; p += al(size_t(C) * L.n_ranges * L.n_bins * 4 + 4);
+            L.range_totals = p; p += al(size_t(C) * L.n_ranges * 4 + 4);
+            L.bin_totals = p; p += al(size_t(C) * L.n_bins * 4 + 4);
         }
     }
-    if (table <= kPlaceLdsBytes && L.place) {
-        L.bytes = o;
-        return L;
+    if (table > kPlaceLdsBytes || !L.place) {
+        L.scan = o; o += al(scan_workspace_bytes(CN));
+        L.sort_bytes = sort_workspace_bytes(capacity);
+        L.sort = o; o += al(L.sort_bytes);
+        L.keys = o; o += al(size_t(capacity) * 4 + 4);
+        L.vals = o; o += al(size_t(capacity) * 4 + 4);
+        L.tm = o; o += al(size_t(n_tiles) * 4 + 4);
+        L.lengths = o; o += al(size_t(n_tiles) * 4 + 4);
+        L.cm = o; o += al(size_t(n_tiles) * 4 + 8);
+        L.tile_scan = o; o += al(scan_workspace_bytes(n_tiles));
     }
-    L.scan = o; o += al(scan_workspace_bytes(CN));
-    L.sort_bytes = sort_workspace_bytes(capacity);
-    L.sort = o; o += al(L.sort_bytes);
-    L.keys = o; o += al(size_t(capacity) * 4 + 4);
-    L.vals = o; o += al(size_t(capacity) * 4 + 4);
-    L.tm = o; o += al(size_t(n_tiles) * 4 + 4);
-    L.lengths = o; o += al(size_t(n_tiles) * 4 + 4);
-    L.cm = o; o += al(size_t(n_tiles) * 4 + 8);
-    L.tile_scan = o; o += al(scan_workspace_bytes(n_tiles));
-    L.bytes = o;
+    L.bytes = std::max(o, p);
     return L;
 }
 

@@ -113,6 +113,14 @@ def test_sort_workspace_never_shrinks_as_the_count_grows():
         assert sizes == sorted(sizes)
 
 
+def test_fused_scratch_holds_the_tables_or_the_sort():
+    """A camera of 1024 tiles may place or sort, by its primitives: the scratch
+    has room for the larger of the two, not for both (1152 tiles always sort)."""
+    size = _backend.lib(require_gpu=False).r2s_fused_scratch_bytes
+    for C, N, capacity in ((1, 30_000, 10**6), (2, 200_000, 4 * 10**6), (4, 1000, 10**6)):
+        assert size(C, N, 512, 512, 16, capacity, 0) <= size(C, N, 512, 576, 16, capacity, 0)
+
+
 def test_workspace_growth_is_all_or_nothing(monkeypatch):
     """A capacity growth that runs out of memory part way leaves every buffer
     and the version (which graphs captured on the workspace check) as they

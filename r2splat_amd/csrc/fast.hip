@@ -2271,13 +2271,19 @@ static FusedScratch fused_scratch(uint32_t C, uint32_t N, uint32_t n_tiles, uint
         while (least < 256 && uint64_t(C) * ((N + least - 1) / least) * table > kRangeTables) least *= 2;
         L.range_len = uint32_t(std::max<uint64_t>(least, (per + 63) / 64 * 64));
         L.n_ranges = (N + L.range_len - 1) / L.range_len;
-        L.place = table <= kPlaceLdsBytes ||
-                  uint64_t(C) * L.n_ranges <= kComputeUnits * (kLdsBytes / (table + sizeof(PairList)));
-        if (L.place) {
-            L.range_counts = p; p += al(size_t(C) * L.n_ranges * L.n_bins * 4 + 4);
-            L.range_totals = p; p += al(size_t(C) * L.n_ranges * 4 + 4);
-            L.bin_totals = p; p += al(size_t(C) * L.n_bins * 4 + 4);
-        }
+        const bool small = table <= kPlaceLdsBytes;
+        const uint64_t resident = kComputeUnits * (kLdsBytes / (table + sizeof(PairList)));
+        L.place = small || uint64_t(C) * L.n_ranges <= resident;
+        // room for the most (camera, range) pairs of up to N primitives and C cameras
+        // (their number falls where the ranges get longer), so that a buffer sized for
+        // the largest call holds every smaller one: by the rule above a range has 64
+        // records or more, 256 unless the tables are few, and C N / kPlaceWaves
+        uint64_t most = std::min(std::max<uint64_t>(kRangeTables / table, C * ((uint64_t(N) + 255) / 256)),
+                                 std::min<uint64_t>(C * ((uint64_t(N) + 63) / 64), uint64_t(kPlaceWaves) + C));
+        if (!small) most = std::min(most, resident);
+        L.range_counts = p; p += al(most * table + 4);
+        L.range_totals = p; p += al(most * 4 + 4);
+        L.bin_totals = p; p += al(size_t(C) * L.n_bins * 4 + 4);
     }
     if (table > kPlaceLdsBytes || !L.place) {
         L.scan = o; o += al(scan_workspace_bytes(CN));

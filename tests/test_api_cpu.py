@@ -121,6 +121,26 @@ def test_fused_scratch_holds_the_tables_or_the_sort():
         assert size(C, N, 512, 512, 16, capacity, 0) <= size(C, N, 512, 576, 16, capacity, 0)
 
 
+@pytest.mark.parametrize("kind", [0, 3])
+@pytest.mark.parametrize("width,height,tile", [(64, 64, 16), (128, 128, 8), (256, 256, 16), (517, 333, 16),
+                                               (512, 512, 16), (512, 576, 16)])
+def test_fused_scratch_never_shrinks_for_a_larger_call(width, height, tile, kind):
+    """Scratch sized once, for the most primitives, cameras and intersections a
+    caller expects, serves every smaller call (grids that place, that may do
+    either, and that sort)."""
+    size = _backend.lib(require_gpu=False).r2s_fused_scratch_bytes
+    counts = sorted({int(64 * 1.07 ** k) for k in range(150)} | {(1 << k) + d for k in range(6, 21) for d in (-1, 0, 1)})
+    for C in (1, 2, 8, 64):
+        for capacity in (1000, 10**6):
+            sizes = [size(C, N, width, height, tile, capacity, kind) for N in counts]
+            assert sizes == sorted(sizes)
+    for N in (64, 3000, 100_000):
+        sizes = [size(C, N, width, height, tile, 1000, kind) for C in range(1, 400)]
+        assert sizes == sorted(sizes)
+    sizes = [size(4, 30_000, width, height, tile, capacity, kind) for capacity in counts]
+    assert sizes == sorted(sizes)
+
+
 def test_workspace_growth_is_all_or_nothing(monkeypatch):
     """A capacity growth that runs out of memory part way leaves every buffer
     and the version (which graphs captured on the workspace check) as they

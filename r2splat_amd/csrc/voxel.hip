@@ -448,6 +448,7 @@ __device__ __forceinline__ VoxForm vox_form(const VoxArgs<float>& A, size_t G, c
 // a few percent of k. Forms that cancel further get every row, and a form no term
 // of which passes none.
 __device__ __forceinline__ uint64_t vox_row_mask(const VoxForm& f, float S, float x0, float y0, float z0) {
+    if (!(fabsf(f.hi[0]) + fabsf(f.hi[1]) + fabsf(f.hi[2]) < 1e30f)) return ~0ull;  // (a NaN reaches every row)
     if (f.qlim == 0u) return 0ull;
     const float ac4 = 4.f * f.a * f.cyy, den = ac4 - f.bxy * f.bxy, inv = __builtin_amdgcn_rcpf(den);
     const float xs = (f.bxy * f.cyz - 2.f * f.cyy * f.bxz) * inv, ys = (f.bxy * f.bxz - 2.f * f.a * f.cyz) * inv;
@@ -985,9 +986,19 @@ vox_partials_reduce_kernel(const uint32_t* __restrict__ cum, const float* __rest
 // thread over the whole list took 210 us there and a wave per intersection 373 us;
 // these take 166 and 160.
 // ---------------------------------------------------------------------------
-// The float form of a primitive and the bound S on its q (Gaussian: q = sigma)
-// beyond which no term passes the cut-off; false when none can (its weight is
-// surely below it).
+// Whether every parameter of a primitive is finite. Others get every voxel of a
+// tile, so that a NaN shows where their pairs pass the cut-off.
+template <typename S, bool BETA>
+__device__ __forceinline__ bool all_finite(const Prim3D<S>& p) {
+    bool ok = isfinite(p.x) && isfinite(p.y) && isfinite(p.z) && isfinite(p.opac) && (!BETA || isfinite(p.beta));
+#pragma unroll
+    for (int k = 0; k < 6; ++k) ok = ok && isfinite(p.c[k]);
+    return ok;
+}
+
+// The float form of a finite primitive and the bound S on its q (Gaussian: q =
+// sigma) beyond which no term passes the cut-off; false when none can (its weight
+// is surely below it).
 template <typename S, bool BETA>
 __device__ __forceinline__ bool op_form(const Prim3D<S>& p, VoxForm& f, float& bound) {
     const float w = fabsf(float(p.opac)), cut = BETA ? 1e-5f : 1e-6f;
@@ -1079,7 +1090,9 @@ vox_fwd_octants_kernel(VoxArgs<S> A, S* __restrict__ out, S* __restrict__ out_va
                 if constexpr (VAR) q = A.unc[g];
                 VoxForm f;
                 float bound;
-                if (op_form<S, BETA>(r, f, bound))
+                if (!all_finite<S, BETA>(r))
+                    octants = 0xffu;
+                else if (op_form<S, BETA>(r, f, bound))
                     octants = form_octants(f, bound, float(tx * T), float(ty * T), float(tz * T));
             }
         }
@@ -1097,10 +1110,11 @@ vox_fwd_octants_kernel(VoxArgs<S> A, S* __restrict__ out, S* __restrict__ out_va
             for (uint32_t o = 0; o < 8; ++o) {
                 if (!((reach >> o) & 1u)) continue;
                 S vis, alpha;
-                if (!eval_profile3<S, BETA>(p, px + S(4 * (o & 1u)), py + S(2 * (o & 2u)), pz + S(o & 4u), vis, alpha))
-                    alpha = S(0);
+                const bool keep =
+                    eval_profile3<S, BETA>(p, px + S(4 * (o & 1u)), py + S(2 * (o & 2u)), pz + S(o & 4u), vis, alpha);
+                if (!keep) alpha = S(0);
                 acc[o] += alpha;
-                if constexpr (VAR) acc_var[o] += unc * alpha * alpha;
+                if constexpr (VAR) acc_var[o] += (keep ? unc : S(0)) * alpha * alpha;
             }
         }
     }
@@ -1156,10 +1170,16 @@ vox_bwd_rows_kernel(VoxArgs<S> A, const int64_t* __restrict__ isect_ids, const S
         [&](uint32_t e, uint32_t tile, uint64_t& mask, double&) {
             const int32_t g = A.flatten[e];
             if (g < 0 || uint32_t(g) >= A.N) return false;
+            const Prim3D<S> p = load_prim3(A, g, BETA);
+            const uint32_t tx = tile % A.ntx, rest = tile / A.ntx;
+            if (!all_finite<S, BETA>(p)) {  // the rows inside the volume (a pair past it is none)
+                const uint32_t ny = min(T, A.dy - (rest % A.nty) * T), nz = min(T, A.dz - (rest / A.nty) * T);
+                mask = (0x0101010101010101ull * ((1u << ny) - 1u)) & (~0ull >> (8u * (T - nz)));
+                return true;
+            }
             VoxForm f;
             float bound;
-            if (!op_form<S, BETA>(load_prim3(A, g, BETA), f, bound)) return false;
-            const uint32_t tx = tile % A.ntx, rest = tile / A.ntx;
+            if (!op_form<S, BETA>(p, f, bound)) return false;
             mask = vox_row_mask(f, bound, float(tx * T) + 0.5f, float((rest % A.nty) * T) + 0.5f,
                                 float((rest / A.nty) * T) + 0.5f);
             return mask != 0ull;
@@ -1171,6 +1191,8 @@ vox_bwd_rows_kernel(VoxArgs<S> A, const int64_t* __restrict__ isect_ids, const S
             const S q2 = VAR && unc ? S(2) * unc[g] : S(0);
             S m0 = S(0), m_x = S(0), m_y = S(0), m_z = S(0), mxx = S(0), myy = S(0), mzz = S(0), mxy = S(0), mxz = S(0),
               myz = S(0), sl = S(0), vq = S(0);
+            bool any = false;  // a pair of the volume passed the cut-off
+            const uint32_t columns = A.dx - tx * T;
             while (rows) {
                 const uint32_t bit = uint32_t(__builtin_ctzll(rows)), z = bit / T, y = bit % T;
                 rows &= rows - 1ull;
@@ -1188,6 +1210,7 @@ vox_bwd_rows_kernel(VoxArgs<S> A, const int64_t* __restrict__ isect_ids, const S
                         if (q < S(0) || q >= S(1)) continue;
                         const S h = S(1) - q, vis = Math<S>::pow(h, p.beta), alpha = p.opac * vis;
                         if (fabs(alpha) < S(1e-5)) continue;
+                        any = any || j < columns;
                         if constexpr (VAR) {
                             vq += vv * alpha * alpha;
                             v += q2 * alpha * vv;
@@ -1201,6 +1224,7 @@ vox_bwd_rows_kernel(VoxArgs<S> A, const int64_t* __restrict__ isect_ids, const S
                     } else {
                         const S vis = Math<S>::exp(-q), alpha = p.opac * vis;
                         const bool keep = !(q < S(0) || fabs(alpha) < S(1e-6));
+                        any = any || (keep && j < columns);
                         if constexpr (VAR) {
                             vq += keep ? vv * alpha * alpha : S(0);
                             v += q2 * alpha * vv;
@@ -1222,7 +1246,7 @@ vox_bwd_rows_kernel(VoxArgs<S> A, const int64_t* __restrict__ isect_ids, const S
                 mxy += dy * r1;
                 mxz += dz * r1;
             }
-            if (!active) return;
+            if (!active || !any) return;  // (no pair: an infinite parameter times an empty sum would be a NaN)
             const size_t G = size_t(g);
             const S k = BETA ? S(2) * p.opac * p.beta : p.opac, kc = BETA ? -p.opac * p.beta : S(-0.5) * p.opac;
             atomic_add(v_xyz + 3 * G, k * (p.c[0] * m_x + p.c[1] * m_y + p.c[2] * m_z));

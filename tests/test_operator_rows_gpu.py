@@ -136,3 +136,101 @@ def test_voxel_8_tiles_match_the_general_kernel(device, N, dims, beta, var, dtyp
         return img, [] if moments else grads
 
     _compare(run, case, 8, 7)
+
+
+def _same_marks(got, general, image, what):
+    """Images: NaN and either infinity in the same places; gradients: the same values
+    finite (an infinite sum may be infinite or NaN by its order). The finite values
+    are one sum in two orders."""
+    for k, (a, b) in enumerate(zip(got, general)):
+        for mark in (torch.isnan, torch.isposinf, torch.isneginf) if image else (torch.isfinite,):
+            assert torch.equal(mark(a), mark(b)), (*what, k, int(mark(a).sum()), int(mark(b).sum()))
+        x, y = a[b.isfinite()], b[b.isfinite()]
+        if y.numel():
+            assert float((x - y).abs().max()) <= 1e-11 * float(y.abs().max()), (*what, k)
+
+
+NONFINITE = [float("nan"), float("inf"), float("-inf")]
+
+
+@pytest.mark.parametrize("beta,var", [(False, True), (True, True)])
+@pytest.mark.parametrize("T", [8, 16, 32])
+def test_row_kernels_keep_nonfinite_parameters_to_their_pairs(device, T, beta, var):
+    """A primitive with a NaN or an infinity marks the pixels and gradients that the
+    general kernel marks: those of its own pairs past the cut-off."""
+    W, H, N = 70, 45, 20
+    for value in NONFINITE:
+        for field in ("mean", "conic a", "conic b", "opacity", "mu", "beta", "uncertainty"):
+            if field == "beta" and not beta:
+                continue
+            (means, conics, opac, mus), betas, unc, v, vv = _case(device, torch.float64, 1, N, W, H, 11, beta, var)
+            target = {"mean": means[0, 7], "conic a": conics[0, 7], "conic b": conics[0, 7, 1:], "opacity": opac[0, 7:],
+                      "mu": mus[0, 7:], "beta": None if betas is None else betas[0, 7:], "uncertainty": unc[7:]}[field]
+            target[0] = value
+            case = ((means, conics, opac, mus), betas, unc, v, vv)
+            (img, grads), (ref, expected) = (_run_lists(case, W, H, t) for t in (T, 10))
+            _same_marks(img, ref, True, (value, field, "image"))
+            _same_marks(grads, expected, False, (value, field, "gradient"))
+
+
+def _run_lists(case, W, H, T):
+    """_run with every primitive in every tile whatever its mean holds."""
+    (means, conics, opac, mus), betas, unc, v, vv = case
+    C, N = opac.shape
+    nt = -(-W // T) * -(-H // T)
+    dev = means.device
+    flat = torch.arange(N, dtype=torch.int32, device=dev).repeat(nt)
+    ids = torch.arange(nt, device=dev).repeat_interleave(N)
+    off = ops.isect_offset_encode(ids, C, -(-W // T), -(-H // T))
+    args = (means, conics, opac, mus) + (() if betas is None else (betas,))
+    pre = "" if betas is None else "beta_"
+    img = getattr(ops, pre + "rasterize_to_pixels_mean_var_fwd")(*args, unc, off, flat, W, H, T)
+    grads = getattr(ops, pre + "rasterize_to_pixels_mean_var_bwd_per_gaussian")(
+        *args, off, ids, flat, v, vv, unc, False, W, H, T, False)
+    return img, [g for g in grads if g is not None]
+
+
+@pytest.mark.parametrize("beta", [False, True])
+def test_voxel_8_tiles_keep_nonfinite_parameters_to_their_pairs(device, beta):
+    dims, N = (21, 17, 30), 20
+    for value in NONFINITE:
+        for field in ("mean", "conic xx", "conic xy", "opacity", "beta", "uncertainty"):
+            if field == "beta" and not beta:
+                continue
+            (means, conics, opac), betas, unc, v, vv = _voxel_case(device, torch.float64, N, dims, 11, beta, True)
+            target = {"mean": means[7], "conic xx": conics[7], "conic xy": conics[7, 1:], "opacity": opac[7:],
+                      "beta": None if betas is None else betas[7:], "uncertainty": unc[7:]}[field]
+            target[0] = value
+            args = (means, conics, opac) + (() if betas is None else (betas,))
+            pre = "beta_" if beta else ""
+            out = []
+            for T in (8, 7):
+                n = [-(-d // T) for d in dims]
+                nt = n[0] * n[1] * n[2]
+                flat = torch.arange(N, dtype=torch.int32, device=device).repeat(nt)
+                ids = torch.arange(nt, device=device).repeat_interleave(N)
+                off = ops.isect_offset_encode_3d(ids, *n)
+                img = getattr(ops, pre + "voxelize_to_voxels_mean_var_fwd")(*args, unc, off, flat, *dims, T)
+                grads = getattr(ops, pre + "voxelize_to_voxels_mean_var_bwd_per_gaussian")(
+                    *args, off, ids, flat, v, vv, unc, False, *dims, T)
+                out.append((img, [g for g in grads if g is not None]))
+            _same_marks(out[0][0], out[1][0], True, (value, field, "volume"))
+            _same_marks(out[0][1], out[1][1], False, (value, field, "gradient"))
+
+
+@pytest.mark.parametrize("beta", [False, True])
+def test_float32_moments_show_a_nan_mean(device, beta):
+    dims, N = (21, 17, 30), 20
+    (means, conics, opac), betas, _, v, _ = _voxel_case(device, torch.float32, N, dims, 11, beta, False)
+    means[7, 1] = float("nan")
+    n = [-(-d // 8) for d in dims]
+    nt = n[0] * n[1] * n[2]
+    flat = torch.arange(N, dtype=torch.int32, device=device).repeat(nt)
+    ids = torch.arange(nt, device=device).repeat_interleave(N)
+    off = ops.isect_offset_encode_3d(ids, *n)
+    args = (means, conics, opac) + (() if betas is None else (betas,))
+    grads = getattr(ops, ("beta_" if beta else "") + "voxelize_to_voxels_bwd_per_gaussian")(*args, off, ids, flat, v,
+                                                                                            *dims, 8)
+    for k, g in enumerate(grads[:2]):  # mean and conic
+        rows = g.isnan().any(-1)
+        assert rows.nonzero().flatten().tolist() == [7], k

@@ -93,18 +93,22 @@ class ValueChecks:
         reduced = [i for i, (_, c) in enumerate(pending) if callable(c)]
         flags = torch.stack([pending[i][1]().reshape(()) for i in reduced]).to(torch.int32) if reduced else None
         words = []
-        if native:
-            with be.on(device):
-                for lo in range(0, len(native), be.MAX_VALUE_CHECKS):
-                    chunk = native[lo: lo + be.MAX_VALUE_CHECKS]
-                    table = (be.ValueCheck * len(chunk))()
-                    for entry, i in zip(table, chunk):
-                        value, kind, row = pending[i][1]
-                        entry.data, entry.n, entry.dtype = value.data_ptr(), value.numel(), be.dtype_code(value.dtype)
-                        entry.kind, entry.row = kind, row
+        try:
+            for lo in range(0, len(native), be.MAX_VALUE_CHECKS):
+                chunk = native[lo: lo + be.MAX_VALUE_CHECKS]
+                table = (be.ValueCheck * len(chunk))()
+                for entry, i in zip(table, chunk):
+                    value, kind, row = pending[i][1]
+                    entry.data, entry.n, entry.dtype = value.data_ptr(), value.numel(), be.dtype_code(value.dtype)
+                    entry.kind, entry.row = kind, row
+                with be.on(device):
                     batch = be.HostWords(len(chunk), device)
                     be.call("r2s_value_checks_begin", ctypes.addressof(table), len(chunk), batch.ptr, batch.stream)
-                    words.append(batch)
+                words.append(batch)
+        except BaseException:
+            for batch in words:  # the launched batches still write to their memory
+                batch.wait()
+            raise
         return PendingChecks(pending, native + reduced, words, flags)
 
 

@@ -189,7 +189,9 @@ extern "C" int r2s_value_checks_begin(const r2s_value_check* checks, uint32_t n_
                 R2S_MAX_VALUE_CHECKS);
     for (uint32_t i = 0; i < n_checks; ++i) host[1 + i] = 0u;
     if (int rc = launch_checks(checks, n_checks, host + 1, stream)) return rc;
-    return fetch_begin(nullptr, 0, host, stream);
+    const int rc = fetch_begin(nullptr, 0, host, stream);
+    if (rc) (void)hipStreamSynchronize(stream);  // the checks write to `host`, which the caller takes back
+    return rc;
 }
 
 extern "C" int r2s_fetch_begin(const uint32_t* src, uint32_t n, uint32_t* host, r2s_stream_t stream) {

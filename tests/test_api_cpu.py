@@ -102,6 +102,36 @@ def test_fused_size_queries_need_no_gpu():
     assert b - a >= 8 * 10**6
 
 
+def test_launched_check_batches_are_waited_for_when_a_later_one_fails(monkeypatch):
+    """The first 16 checks write to pinned words of their own while the next
+    batch is launched; a failure there must not free them before they arrive."""
+    from r2splat_amd import _validation
+
+    events = []
+
+    class Words:
+        def __init__(self, n, device):
+            self.ptr, self.stream, self.name = 0, 0, f"batch of {n}"
+
+        def wait(self):
+            events.append(("waited", self.name))
+            return []
+
+    def call(name, table, n, host, stream):
+        if n < 16:
+            raise RuntimeError("launch failed")
+        events.append(("launched", f"batch of {n}"))
+
+    monkeypatch.setattr(_validation.be, "HostWords", Words)
+    monkeypatch.setattr(_validation.be, "call", call)
+    checks = _validation.ValueChecks()
+    for k in range(19):
+        checks.finite(f"x{k}", torch.ones(4))
+    with pytest.raises(RuntimeError, match="launch failed"):
+        checks.begin()
+    assert events == [("launched", "batch of 16"), ("waited", "batch of 16")]
+
+
 def test_sort_workspace_never_shrinks_as_the_count_grows():
     """A caller that sizes its workspace once, for the largest count it expects,
     may sort any smaller count with it: the tiles a sort is cut into grow with

@@ -218,14 +218,16 @@ extern "C" int r2s_fetch_wait(const uint32_t* host, r2s_stream_t stream) {
         }
     } while (clock::now() < spin_end);
     while (!raised()) {
-        const hipError_t e = hipStreamQuery(stream);
+        hipError_t e = hipStreamQuery(stream);
         if (e == hipErrorNotReady) {
-            (void)hipGetLastError();
+            // (the query's own state alone: an earlier call's error stays for its reader)
+            if (hipPeekAtLastError() == hipErrorNotReady) (void)hipGetLastError();
             std::this_thread::sleep_for(std::chrono::microseconds(50));
             continue;
         }
-        if (e == hipSuccess && hipStreamSynchronize(stream) == hipSuccess && raised()) return R2S_OK;
-        (void)hipGetLastError();
+        if (e == hipSuccess) e = hipStreamSynchronize(stream);
+        if (e == hipSuccess && raised()) return R2S_OK;
+        if (e != hipSuccess) (void)hipGetLastError();  // reported here
         set_error("fetch: %s", e == hipSuccess ? "the stream ended without the words" : hipGetErrorString(e));
         return R2S_ERR_HIP;
     }

@@ -2,6 +2,7 @@
 long and short work, on several streams and threads, and when the work
 launched meanwhile raises."""
 
+import ctypes
 import threading
 
 import pytest
@@ -81,3 +82,23 @@ def test_forward_rendered_before_its_overflow_is_known(device):
     image, g = fused.forward(*args, capacity=64)  # does not fit: rendered again with room
     assert f.n_isects == g.n_isects > 64
     assert torch.equal(image, expected)
+
+
+def test_a_long_wait_keeps_another_calls_error(device):
+    """The wait asks the runtime whether the stream has ended; an error that the
+    thread has yet to read is not its own to clear."""
+    path = next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line)
+    hip = ctypes.CDLL(path)
+    x = torch.zeros(1 << 24, device=device)
+    src = torch.arange(2, device=device, dtype=torch.int32)
+    torch.cuda.synchronize(device)
+    for _ in range(600):  # some 20 ms: past the wait's spin
+        x.add_(1.0)
+    words = be.fetch(src)
+    invalid = hip.hipSetDevice(10_000)
+    assert invalid != 0 and hip.hipPeekAtLastError() == invalid
+    try:
+        assert words.wait() == [0, 1]
+        assert hip.hipPeekAtLastError() == invalid
+    finally:
+        hip.hipGetLastError()

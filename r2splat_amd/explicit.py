@@ -429,10 +429,9 @@ def _voxel_state(prims, vol: dict, shape, eps, radius_clip) -> dict:
     depth, height, width = shape
     T = VOXEL_TILE
     if BACKEND == "fused":
-        with stage("voxel_bin"):
-            return _ops_impl.voxel_prepare(means, quats, scales, extent, center, vol["extent64"], vol["center64"],
-                                           (width, height, depth), eps, radius_clip, T,
-                                           (-(-width // T), -(-height // T), -(-depth // T)))
+        return _ops_impl.voxel_prepare(means, quats, scales, extent, center, vol["extent64"], vol["center64"],
+                                       (width, height, depth), eps, radius_clip, T,
+                                       (-(-width // T), -(-height // T), -(-depth // T)))
     with stage("voxel_map"):
         covars, max_scales = ops.parameter_transform_fwd(quats, scales)
         mapped, conics, radii = ops.world_to_volume_mapping_fwd(means, covars, max_scales, extent, center, width,

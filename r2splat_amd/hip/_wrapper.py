@@ -18,6 +18,7 @@ import torch
 
 from . import _backend as be
 from ._backend import call, ptr
+from ..profiling import stage
 
 Tensor = torch.Tensor
 
@@ -341,18 +342,21 @@ def voxel_prepare(means, quats, scales, extent, center, extent64, center64, dims
     nx, ny, nz = tiles
     offsets = torch.empty((nz, ny, nx), dtype=torch.int32, device=dev)
     with _Launch(means) as L:
-        scan_ws = _workspace(be.lib().r2s_scan_workspace_bytes(N), dev)
-        words = be.HostWords(1, dev)
-        call("r2s_voxel_prepare", dt, ptr(means), ptr(quats), ptr(scales), ptr(extent), ptr(center), ptr(extent64),
-             ptr(center64), *dims, float(eps), float(radius_clip), tile_size, nx, ny, nz, N, ptr(covars), ptr(mapped),
-             ptr(conics), ptr(radii), ptr(frame), ptr(cum), ptr(scan_ws), words.ptr, L.stream)
-        (n_isects,) = words.wait()
-        isect_ids = torch.empty((n_isects,), dtype=torch.int64, device=dev)
-        flatten_ids = torch.empty((n_isects,), dtype=torch.int32, device=dev)
-        nbytes = be.lib().r2s_sort_workspace_bytes(n_isects, 0)
-        sort_ws = _workspace(nbytes, dev)
-        call("r2s_voxel_lists", dt, ptr(mapped), ptr(radii), N, tile_size, nx, ny, nz, ptr(cum), n_isects,
-             ptr(isect_ids), ptr(flatten_ids), ptr(sort_ws), nbytes, ptr(offsets), L.stream)
+        with stage("voxel_map"):  # (and the tile counts, which come from the same launch)
+            scan_ws = _workspace(be.lib().r2s_scan_workspace_bytes(N), dev)
+            words = be.HostWords(1, dev)
+            call("r2s_voxel_prepare", dt, ptr(means), ptr(quats), ptr(scales), ptr(extent), ptr(center),
+                 ptr(extent64), ptr(center64), *dims, float(eps), float(radius_clip), tile_size, nx, ny, nz, N,
+                 ptr(covars), ptr(mapped), ptr(conics), ptr(radii), ptr(frame), ptr(cum), ptr(scan_ws), words.ptr,
+                 L.stream)
+        with stage("voxel_bin"):
+            (n_isects,) = words.wait()
+            isect_ids = torch.empty((n_isects,), dtype=torch.int64, device=dev)
+            flatten_ids = torch.empty((n_isects,), dtype=torch.int32, device=dev)
+            nbytes = be.lib().r2s_sort_workspace_bytes(n_isects, 0)
+            sort_ws = _workspace(nbytes, dev)
+            call("r2s_voxel_lists", dt, ptr(mapped), ptr(radii), N, tile_size, nx, ny, nz, ptr(cum), n_isects,
+                 ptr(isect_ids), ptr(flatten_ids), ptr(sort_ws), nbytes, ptr(offsets), L.stream)
     state = dict(covars=covars, mapped=mapped, conics=conics, radii=radii, tile_cum=cum, offsets=offsets,
                  isect_ids=isect_ids, flatten_ids=flatten_ids)
     if frame is not None:

@@ -4,7 +4,7 @@ stand for (bitwise), and the exclusive scan around its 16-byte runs."""
 import pytest
 import torch
 
-from r2splat_amd import explicit, fused, hip as ops, workloads
+from r2splat_amd import explicit, fused, hip as ops, profiling, workloads
 from r2splat_amd.hip import _backend as be, _wrapper
 
 pytestmark = pytest.mark.gpu
@@ -47,6 +47,23 @@ def test_voxelize_of_primitives_that_reach_no_tile(device):
     out, ctx = explicit.voxelize_fwd(sc.means + 5.0, *sc.params()[1:], (9, 10, 11), volume_extent=(1.0, 1.0, 1.0))
     assert not bool(out.any())
     assert not bool(explicit.voxelize_bwd(ctx, torch.ones_like(out)).densities.any())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("backend", ["fused", "ops"])
+def test_voxelize_reports_its_stages(device, monkeypatch, backend, dtype):
+    sc = workloads.scene(50, 1, 8, 8, scale_range=(0.05, 0.1), seed=1, device=device, dtype=dtype)
+    monkeypatch.setattr(explicit, "BACKEND", backend)
+    profiling.reset()
+    profiling.enable()
+    try:
+        out, ctx = explicit.voxelize_fwd(*sc.params(), (9, 10, 11), volume_extent=(1.0, 1.0, 1.0))
+        explicit.voxelize_bwd(ctx, torch.ones_like(out))
+        stages = set(profiling.collect())
+    finally:
+        profiling.enable(False)
+        profiling.reset()
+    assert {"voxel_map", "voxel_bin", "voxel_map_bwd"} <= stages
 
 
 # a one-launch scan of either kind and a scan of levels, whole and cut 16-byte runs

@@ -7,6 +7,7 @@ import torch
 
 from oracle import splat as O
 from r2splat_amd import hip as ops
+from r2splat_amd.hip import _backend as be
 
 pytestmark = pytest.mark.gpu
 
@@ -78,3 +79,29 @@ def test_isotropic_gradient_where_threads_share_terms(shape, dtype):
     got = ops.volume_loss_iso_bwd(vol.to(device), torch.ones(1, device=device, dtype=dtype), 1.0)
     t = 1e-5 if dtype == torch.float32 else 5e-12  # as above: five roundings of a short chain
     assert O.relative_error(got, grad) <= t
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("shape", [(1, 1, 1, 1), (2, 9, 3, 8), (3, 7, 5, 13), (1, 130, 128, 132)])
+def test_plain_sums_of_the_c_entries(shape, dtype):
+    """r2s_volume_tv_fwd, r2s_volume_tv_iso_fwd and r2s_image_l1_fwd, which add
+    their workgroups' sums by atomics: one workgroup and several, twice into one
+    result, against the maps they leave and the operators' maps."""
+    device = torch.device("cuda:0")
+    g = torch.Generator().manual_seed(sum(shape))
+    x, y = (torch.randn(*shape, generator=g, dtype=torch.float64).to(device, dtype) for _ in range(2))
+    code, stream = be.dtype_code(dtype), be.stream_of(device)
+    # sums of n positive terms: chains of at most 512 in the dtype, then in double;
+    # one rounding to the dtype for each of at most 512 workgroups
+    t = 5e-5 if dtype == torch.float32 else 1e-12
+    calls = (("r2s_volume_tv_fwd", (x.data_ptr(), *shape), ops.volume_loss_fwd(x, 1.0)[2]),
+             ("r2s_volume_tv_iso_fwd", (x.data_ptr(), *shape, 1e-8), ops.volume_loss_iso_fwd(x, 1.0)[2]),
+             ("r2s_image_l1_fwd", (x.data_ptr(), y.data_ptr(), x.numel()),
+              ops.image_loss_l1_fwd(x.flatten(0, 1), y.flatten(0, 1), 1.0)[2]))
+    for name, args, expected in calls:
+        out, total = torch.empty_like(x), torch.full((1,), 7.0, device=device, dtype=dtype)
+        for _ in range(2):
+            be.call(name, code, *args, out.data_ptr(), total.data_ptr(), stream)
+            assert torch.equal(out.flatten(), expected.flatten())
+            exact = out.double().sum().item()
+            assert abs(total.item() - exact) <= t * exact

@@ -314,6 +314,14 @@ __device__ __forceinline__ S pair_form(S adx, S dx, S bdx, S c, S dy) {
     return Math<S>::fma(bdx, dy, S(0.5) * Math<S>::fma(adx, dx, c * dy * dy));
 }
 
+// The Gaussian VJP's form. The general VJP rounds the other square first, and a thin
+// footprint's gradient keeps that float32 exponent.
+template <typename S>
+__device__ __forceinline__ S vjp_sigma(S adx, S dx, S bdx, S c, S dy) {
+    if constexpr (sizeof(S) == sizeof(double)) return pair_form<S, false>(adx, dx, bdx, c, dy);
+    return Math<S>::fma(bdx, dy, S(0.5) * Math<S>::fma(c * dy, dy, adx * dx));
+}
+
 template <typename S>
 __device__ __forceinline__ Prim2D<S> load_prim(const RasterArgs<S>& A, int32_t g, bool beta) {
     Prim2D<S> p;
@@ -508,7 +516,7 @@ raster_bwd_rows_kernel(RasterArgs<S> A, const int64_t* __restrict__ isect_ids, c
                        const S* __restrict__ v_var, const S* __restrict__ unc, S* __restrict__ v_xy,
                        S* __restrict__ v_conic, S* __restrict__ v_opac, S* __restrict__ v_mu,
                        S* __restrict__ v_beta, S* __restrict__ v_q) {
-    constexpr uint32_t kPixels = T * T;
+    constexpr uint32_t kPixels = T * T, kRun = std::is_same<S, float>::value ? 8 : T;  // columns of a row sum
     __shared__ __align__(16) S sv[op_tiles<T>() * kPixels];
     __shared__ __align__(16) S svv[VAR ? op_tiles<T>() * kPixels : 2];
     const uint32_t nt = A.ntx * A.nty;
@@ -539,80 +547,86 @@ raster_bwd_rows_kernel(RasterArgs<S> A, const int64_t* __restrict__ isect_ids, c
             const Prim2D<S> p = load_prim(A, g, BETA);
             const uint32_t n = uint32_t(g) % A.N;
             const S w = p.opac * p.mu, q2 = VAR && unc ? S(2) * unc[n] : S(0);
-            S m0 = S(0), mx = S(0), my = S(0), mxx = S(0), mxy = S(0), myy = S(0), sl = S(0), vq = S(0);
+            double m0 = 0.0, mx = 0.0, my = 0.0, mxx = 0.0, mxy = 0.0, myy = 0.0, sl = 0.0, vq = 0.0;
             bool any = false;  // a pair of the image passed the cut-off
             const uint32_t columns = A.W - tx * T;
             while (rows) {
                 const uint32_t r = uint32_t(__builtin_ctzll(rows));
                 rows &= rows - 1ull;
                 const S py = S(ty * T + r) + S(0.5), dy = BETA ? p.my - py : py - p.my;
-                S r0 = S(0), r1 = S(0), r2 = S(0);
                 const S* row = sv + slot * kPixels + r * T;
                 const S* rowv = svv + (VAR ? slot * kPixels + r * T : 0);
+#pragma unroll 1
+                for (uint32_t j0 = 0; j0 < uint32_t(T); j0 += kRun) {
+                    S r0 = S(0), r1 = S(0), r2 = S(0), rm = S(0), rl = S(0), rq = S(0);
 #pragma unroll 2
-                for (uint32_t j = 0; j < uint32_t(T); ++j) {
-                    const S px = S(tx * T + j) + S(0.5), dx = BETA ? p.mx - px : px - p.mx;
-                    S v = row[j];
-                    const S vv = VAR ? rowv[VAR ? j : 0] : S(0);
-                    if constexpr (BETA) {
-                        const S q = pair_form<S, BETA>(p.a * dx, dx, S(2) * p.b * dx, p.c, dy);
-                        if (q < S(0) || q >= S(1)) continue;
-                        const S h = S(1) - q, vis = Math<S>::pow(h, p.beta), alpha = w * vis;
-                        if (fabs(alpha) < S(1e-5)) continue;
-                        any = any || j < columns;
-                        if constexpr (VAR) {
-                            vq += vv * alpha * alpha;
-                            v += q2 * alpha * vv;
+                    for (uint32_t j = j0; j < j0 + kRun; ++j) {
+                        const S px = S(tx * T + j) + S(0.5), dx = BETA ? p.mx - px : px - p.mx;
+                        S v = row[j];
+                        const S vv = VAR ? rowv[VAR ? j : 0] : S(0);
+                        if constexpr (BETA) {
+                            const S q = pair_form<S, BETA>(p.a * dx, dx, S(2) * p.b * dx, p.c, dy);
+                            if (q < S(0) || q >= S(1)) continue;
+                            const S h = S(1) - q, vis = Math<S>::pow(h, p.beta), alpha = w * vis;
+                            if (fabs(alpha) < S(1e-5)) continue;
+                            any = any || j < columns;
+                            if constexpr (VAR) {
+                                row_sum(rq, vq, vv * alpha * alpha);
+                                v += q2 * alpha * vv;
+                            }
+                            const S gv = v * (vis / h);
+                            row_sum(rm, m0, v * vis);
+                            row_sum(rl, sl, v * alpha * Math<S>::log(h));
+                            r0 += gv;
+                            r1 += gv * dx;
+                            r2 += gv * dx * dx;
+                        } else {
+                            const S sigma = vjp_sigma(p.a * dx, dx, p.b * dx, p.c, dy);
+                            const S vis = Math<S>::exp(-sigma), alpha = w * vis;
+                            const bool keep = !(sigma < S(0) || fabs(alpha) < S(1e-5));
+                            any = any || (keep && j < columns);
+                            if constexpr (VAR) {
+                                row_sum(rq, vq, keep ? vv * alpha * alpha : S(0));
+                                v += q2 * alpha * vv;
+                            }
+                            const S gv = keep ? v * alpha : S(0);
+                            row_sum(rm, m0, keep ? v * vis : S(0));
+                            r0 += gv;
+                            r1 += gv * dx;
+                            r2 += gv * dx * dx;
                         }
-                        const S gv = v * (vis / h);
-                        m0 += v * vis;
-                        sl += v * alpha * Math<S>::log(h);
-                        r0 += gv;
-                        r1 += gv * dx;
-                        r2 += gv * dx * dx;
-                    } else {
-                        const S sigma = pair_form<S, BETA>(p.a * dx, dx, p.b * dx, p.c, dy);
-                        const S vis = Math<S>::exp(-sigma), alpha = w * vis;
-                        const bool keep = !(sigma < S(0) || fabs(alpha) < S(1e-5));
-                        any = any || (keep && j < columns);
-                        if constexpr (VAR) {
-                            vq += keep ? vv * alpha * alpha : S(0);
-                            v += q2 * alpha * vv;
-                        }
-                        const S gv = keep ? v * alpha : S(0);
-                        m0 += keep ? v * vis : S(0);
-                        r0 += gv;
-                        r1 += gv * dx;
-                        r2 += gv * dx * dx;
                     }
+                    mx += r1;
+                    mxx += r2;
+                    my += double(dy) * r0;
+                    mxy += double(dy) * r1;
+                    myy += double(dy) * dy * r0;
+                    m0 += rm;
+                    sl += rl;
+                    vq += rq;
                 }
-                mx += r1;
-                mxx += r2;
-                my += dy * r0;
-                mxy += dy * r1;
-                myy += dy * dy * r0;
             }
             if (!active || !any) return;  // (no pair: an infinite parameter times an empty sum would be a NaN)
             const size_t G = size_t(g);
             if constexpr (BETA) {
-                const S k = -w * p.beta;
-                atomic_add(v_xy + 2 * G, S(2) * k * (p.a * mx + p.b * my));
-                atomic_add(v_xy + 2 * G + 1, S(2) * k * (p.b * mx + p.c * my));
-                atomic_add(v_conic + 3 * G, k * mxx);
-                atomic_add(v_conic + 3 * G + 1, S(2) * k * mxy);
-                atomic_add(v_conic + 3 * G + 2, k * myy);
-                atomic_add(v_beta + G, sl);
+                const double k = -w * p.beta;
+                atomic_add(v_xy + 2 * G, S(2.0 * k * (p.a * mx + p.b * my)));
+                atomic_add(v_xy + 2 * G + 1, S(2.0 * k * (p.b * mx + p.c * my)));
+                atomic_add(v_conic + 3 * G, S(k * mxx));
+                atomic_add(v_conic + 3 * G + 1, S(2.0 * k * mxy));
+                atomic_add(v_conic + 3 * G + 2, S(k * myy));
+                atomic_add(v_beta + G, S(sl));
             } else {
-                atomic_add(v_xy + 2 * G, p.a * mx + p.b * my);
-                atomic_add(v_xy + 2 * G + 1, p.b * mx + p.c * my);
-                atomic_add(v_conic + 3 * G, S(-0.5) * mxx);
-                atomic_add(v_conic + 3 * G + 1, -mxy);
-                atomic_add(v_conic + 3 * G + 2, S(-0.5) * myy);
+                atomic_add(v_xy + 2 * G, S(p.a * mx + p.b * my));
+                atomic_add(v_xy + 2 * G + 1, S(p.b * mx + p.c * my));
+                atomic_add(v_conic + 3 * G, S(-0.5 * mxx));
+                atomic_add(v_conic + 3 * G + 1, S(-mxy));
+                atomic_add(v_conic + 3 * G + 2, S(-0.5 * myy));
             }
-            atomic_add(v_opac + G, p.mu * m0);
-            atomic_add(v_mu + G, p.opac * m0);
+            atomic_add(v_opac + G, S(p.mu * m0));
+            atomic_add(v_mu + G, S(p.opac * m0));
             if constexpr (VAR)
-                if (v_q) atomic_add(v_q + n, vq);
+                if (v_q) atomic_add(v_q + n, S(vq));
         });
 }
 

@@ -120,4 +120,14 @@ __device__ __forceinline__ void sorted_chunk(const int64_t* __restrict__ ids, ui
     }
 }
 
+// The sums of work(): a lane adds a whole tile's terms by itself, so float terms are
+// summed over eight columns of a row and those sums in double (one float sum over a
+// 16- or 32-pixel tile was 2.5 to 6 times as far from 64 bits as a wave's tree of
+// sums, these are as near). Double terms go straight to the total.
+template <typename S>
+__device__ __forceinline__ void row_sum(S& row, double& total, S term) {
+    if constexpr (sizeof(S) == sizeof(double)) total += term;
+    else row += term;
+}
+
 }  // namespace r2s

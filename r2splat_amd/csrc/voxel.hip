@@ -1189,15 +1189,15 @@ vox_bwd_rows_kernel(VoxArgs<S> A, const int64_t* __restrict__ isect_ids, const S
             const int32_t g = A.flatten[e];
             const Prim3D<S> p = load_prim3(A, g, BETA);
             const S q2 = VAR && unc ? S(2) * unc[g] : S(0);
-            S m0 = S(0), m_x = S(0), m_y = S(0), m_z = S(0), mxx = S(0), myy = S(0), mzz = S(0), mxy = S(0), mxz = S(0),
-              myz = S(0), sl = S(0), vq = S(0);
+            double m0 = 0.0, m_x = 0.0, m_y = 0.0, m_z = 0.0, mxx = 0.0, myy = 0.0, mzz = 0.0, mxy = 0.0, mxz = 0.0,
+                   myz = 0.0, sl = 0.0, vq = 0.0;
             bool any = false;  // a pair of the volume passed the cut-off
             const uint32_t columns = A.dx - tx * T;
             while (rows) {
                 const uint32_t bit = uint32_t(__builtin_ctzll(rows)), z = bit / T, y = bit % T;
                 rows &= rows - 1ull;
                 const S dy = (S(ty * T + y) + S(0.5)) - p.y, dz = (S(tz * T + z) + S(0.5)) - p.z;
-                S r0 = S(0), r1 = S(0), r2 = S(0);
+                S r0 = S(0), r1 = S(0), r2 = S(0), rm = S(0), rl = S(0), rq = S(0);
                 const S* row = sv + slot * T3 + bit * T;
                 const S* rowv = svv + (VAR ? slot * T3 + bit * T : 0);
 #pragma unroll 2
@@ -1212,12 +1212,12 @@ vox_bwd_rows_kernel(VoxArgs<S> A, const int64_t* __restrict__ isect_ids, const S
                         if (fabs(alpha) < S(1e-5)) continue;
                         any = any || j < columns;
                         if constexpr (VAR) {
-                            vq += vv * alpha * alpha;
+                            row_sum(rq, vq, vv * alpha * alpha);
                             v += q2 * alpha * vv;
                         }
                         const S gv = v * (vis / h);
-                        m0 += v * vis;
-                        sl += v * alpha * Math<S>::log(h);
+                        row_sum(rm, m0, v * vis);
+                        row_sum(rl, sl, v * alpha * Math<S>::log(h));
                         r0 += gv;
                         r1 += gv * dx;
                         r2 += gv * dx * dx;
@@ -1226,7 +1226,7 @@ vox_bwd_rows_kernel(VoxArgs<S> A, const int64_t* __restrict__ isect_ids, const S
                         const bool keep = !(q < S(0) || fabs(alpha) < S(1e-6));
                         any = any || (keep && j < columns);
                         if constexpr (VAR) {
-                            vq += keep ? vv * alpha * alpha : S(0);
+                            row_sum(rq, vq, keep ? vv * alpha * alpha : S(0));
                             v += q2 * alpha * vv;
                         }
                         const S gv = keep ? v * vis : S(0);
@@ -1235,33 +1235,36 @@ vox_bwd_rows_kernel(VoxArgs<S> A, const int64_t* __restrict__ isect_ids, const S
                         r2 += gv * dx * dx;
                     }
                 }
-                if constexpr (!BETA) m0 += r0;
+                m0 += BETA ? rm : r0;
                 m_x += r1;
                 mxx += r2;
-                m_y += dy * r0;
-                m_z += dz * r0;
-                myy += dy * dy * r0;
-                mzz += dz * dz * r0;
-                myz += dy * dz * r0;
-                mxy += dy * r1;
-                mxz += dz * r1;
+                const double ey = dy, ez = dz;
+                m_y += ey * r0;
+                m_z += ez * r0;
+                myy += ey * ey * r0;
+                mzz += ez * ez * r0;
+                myz += ey * ez * r0;
+                mxy += ey * r1;
+                mxz += ez * r1;
+                sl += rl;
+                vq += rq;
             }
             if (!active || !any) return;  // (no pair: an infinite parameter times an empty sum would be a NaN)
             const size_t G = size_t(g);
-            const S k = BETA ? S(2) * p.opac * p.beta : p.opac, kc = BETA ? -p.opac * p.beta : S(-0.5) * p.opac;
-            atomic_add(v_xyz + 3 * G, k * (p.c[0] * m_x + p.c[1] * m_y + p.c[2] * m_z));
-            atomic_add(v_xyz + 3 * G + 1, k * (p.c[1] * m_x + p.c[3] * m_y + p.c[4] * m_z));
-            atomic_add(v_xyz + 3 * G + 2, k * (p.c[2] * m_x + p.c[4] * m_y + p.c[5] * m_z));
-            atomic_add(v_c + 6 * G, kc * mxx);
-            atomic_add(v_c + 6 * G + 1, S(2) * kc * mxy);
-            atomic_add(v_c + 6 * G + 2, S(2) * kc * mxz);
-            atomic_add(v_c + 6 * G + 3, kc * myy);
-            atomic_add(v_c + 6 * G + 4, S(2) * kc * myz);
-            atomic_add(v_c + 6 * G + 5, kc * mzz);
-            atomic_add(v_opac + G, m0);
-            if constexpr (BETA) atomic_add(v_beta + G, sl);
+            const double k = BETA ? S(2) * p.opac * p.beta : p.opac, kc = BETA ? -p.opac * p.beta : S(-0.5) * p.opac;
+            atomic_add(v_xyz + 3 * G, S(k * (p.c[0] * m_x + p.c[1] * m_y + p.c[2] * m_z)));
+            atomic_add(v_xyz + 3 * G + 1, S(k * (p.c[1] * m_x + p.c[3] * m_y + p.c[4] * m_z)));
+            atomic_add(v_xyz + 3 * G + 2, S(k * (p.c[2] * m_x + p.c[4] * m_y + p.c[5] * m_z)));
+            atomic_add(v_c + 6 * G, S(kc * mxx));
+            atomic_add(v_c + 6 * G + 1, S(2.0 * kc * mxy));
+            atomic_add(v_c + 6 * G + 2, S(2.0 * kc * mxz));
+            atomic_add(v_c + 6 * G + 3, S(kc * myy));
+            atomic_add(v_c + 6 * G + 4, S(2.0 * kc * myz));
+            atomic_add(v_c + 6 * G + 5, S(kc * mzz));
+            atomic_add(v_opac + G, S(m0));
+            if constexpr (BETA) atomic_add(v_beta + G, S(sl));
             if constexpr (VAR)
-                if (v_q) atomic_add(v_q + G, vq);
+                if (v_q) atomic_add(v_q + G, S(vq));
         });
 }
 

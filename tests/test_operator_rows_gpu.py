@@ -234,3 +234,31 @@ def test_float32_moments_show_a_nan_mean(device, beta):
     for k, g in enumerate(grads[:2]):  # mean and conic
         rows = g.isnan().any(-1)
         assert rows.nonzero().flatten().tolist() == [7], k
+
+
+@pytest.mark.parametrize("beta,var", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("T", [8, 16, 32])
+def test_float32_vjp_sums_are_as_near_as_the_general_kernels(device, T, beta, var):
+    """Round footprints, whose terms carry no cancellation: what is left is how the
+    VJP adds them. The root mean square error over 1200 primitives and four scenes
+    varies by a few percent (the largest error by half); a quarter more than the
+    general kernel's is a longer chain of float sums."""
+    C, N, W, H = 3, 400, 150, 110
+    new, old = 0.0, 0.0
+    for seed in range(4):
+        g = torch.Generator().manual_seed(seed)
+        r = lambda *s: torch.rand(*s, generator=g, dtype=torch.float64)  # noqa: E731
+        means = torch.stack([r(C, N) * W, r(C, N) * H], -1)
+        s = 1.5 + 4.5 * r(C, N)
+        conics = torch.stack([s**-2, 0.1 * s**-2, s**-2], -1)
+        prims = [t.to(device, torch.float32) for t in (means, conics, r(C, N), r(C, N) + 0.05)]
+        betas = (0.6 + 3 * r(C, N)).to(device, torch.float32) if beta else None
+        unc = (0.1 * r(N)).to(device, torch.float32) if var else None
+        v, vv = ((r(C, H, W) - 0.5).to(device, torch.float32) for _ in range(2))
+        case = (prims, betas, unc, v, vv if var else None)
+        wide = [t.double() for t in prims], *(None if t is None else t.double() for t in case[1:])
+        exact = _run(wide, W, H, 10)[1]
+        errors = lambda tile: torch.tensor(  # noqa: E731
+            [float((a.double() - b).norm() / b.norm()) for a, b in zip(_run(case, W, H, tile)[1], exact)])
+        new, old = new + errors(T), old + errors(10)
+    assert bool((new <= 1.25 * old).all()), (new / old).tolist()

@@ -593,8 +593,8 @@ __device__ __forceinline__ void camera_frame(const float* __restrict__ viewmats,
 // index), and each primitive's PrimFrame; workgroup 0 also writes the C
 // camera frames and clears the counters.
 __global__ void __launch_bounds__(256)
-permute_params_kernel(const uint32_t* __restrict__ perm, uint32_t* __restrict__ counters, uint32_t N, const float* __restrict__ means,
-                      const float* __restrict__ quats, const float* __restrict__ scales,
+permute_params_kernel(const uint32_t* __restrict__ perm, uint32_t* __restrict__ counters, uint32_t N,
+                      const float* __restrict__ means, const float* __restrict__ quats, const float* __restrict__ scales,
                       const float* __restrict__ dens, const float* __restrict__ betas,
                       const float* __restrict__ ratio, const float* __restrict__ unc, float* __restrict__ o_means,
                       float* __restrict__ o_dens, float* __restrict__ o_betas, float* __restrict__ o_ratio,
@@ -2470,7 +2470,8 @@ static int prepare_impl(const float* means, const float* quats, const float* sca
         dim3 grid(ceil_div(N, 256), ceil_div(C, kProjectCams));
         fused_project_kernel<BETA, VAR><<<grid, 256, 0, stream>>>(
             p_means, p_frames, p_dens, p_betas, p_ratio, p_unc, cams, C, width, height, eps, radius_clip,
-            tile_size, ntx, nty, N, recs, at<uint2>(scratch, L.rects), at<Reach<BETA>>(scratch, L.reach), L.place ? nullptr : cum);
+            tile_size, ntx, nty, N, recs, at<uint2>(scratch, L.rects), at<Reach<BETA>>(scratch, L.reach),
+            L.place ? nullptr : cum);
         if (int rc = check_launch("fused_project")) return rc;
     }
     if (L.place) {
@@ -2481,8 +2482,8 @@ static int prepare_impl(const float* means, const float* quats, const float* sca
         const dim3 grid(L.n_ranges, C);
         if (CN > 0) {
             fused_bin_count_kernel<BETA><<<grid, kWave, lds, stream>>>(
-                at<uint2>(scratch, L.rects), at<Reach<BETA>>(scratch, L.reach), N, L.range_len, L.n_ranges, ntx, tile_size,
-                L.n_bins, range_counts, range_totals);
+                at<uint2>(scratch, L.rects), at<Reach<BETA>>(scratch, L.reach), N, L.range_len, L.n_ranges, ntx,
+                tile_size, L.n_bins, range_counts, range_totals);
             if (int rc = check_launch("fused_bin_count")) return rc;
         }
         fused_bin_scan_ranges_kernel<<<ceil_div(size_t(C) * L.n_bins, kScanCols) + 1, kScanThreads, 0, stream>>>(
@@ -2505,35 +2506,35 @@ static int prepare_impl(const float* means, const float* quats, const float* sca
         fused_bin_tile_offsets_kernel<<<ceil_div(n_tiles, 256), 256, 0, stream>>>(totals, n_tiles, tile_offsets);
         if (int rc = check_launch("fused_bin_tile_offsets")) return rc;
     } else {
-    if (int rc = scan_exclusive(cum, CN, cum, counters, at<void>(scratch, L.scan), stream)) return rc;
-    void* sort_ws = at<void>(scratch, L.sort);
-    if (CN > 0) {
-        fused_emit_kernel<<<ceil_div(CN, 256), 256, 0, stream>>>(
-            at<uint2>(scratch, L.rects), cum, CN, ntx, capacity, sort_keys_buffer(sort_ws),
-            sort_vals_buffer(sort_ws, capacity), counters + 1);
-        if (int rc = check_launch("fused_emit")) return rc;
-    }
-    uint32_t* keys = at<uint32_t>(scratch, L.keys);
-    uint32_t* vals = at<uint32_t>(scratch, L.vals);
-    if (int rc = sort_pairs_u32(sort_ws, L.sort_bytes, capacity, counters, key_end_bit(ntx * nty - 1), keys, vals,
-                                stream))
-        return rc;
-    uint32_t* tm = at<uint32_t>(scratch, L.tm);
-    uint32_t* cm = at<uint32_t>(scratch, L.cm);
-    fused_offsets_kernel<<<ceil_div(n_tiles, 256), 256, 0, stream>>>(keys, vals, counters, capacity, C, N, n_tiles,
-                                                                     reinterpret_cast<int32_t*>(tm));
-    if (int rc = check_launch("fused_offsets")) return rc;
-    fused_list_lengths_kernel<<<ceil_div(n_tiles, 256), 256, 0, stream>>>(tm, counters, capacity, C, ntx * nty,
-                                                                          at<uint32_t>(scratch, L.lengths));
-    if (int rc = check_launch("fused_list_lengths")) return rc;
-    if (int rc = scan_exclusive(at<uint32_t>(scratch, L.lengths), n_tiles, cm, nullptr, at<void>(scratch, L.tile_scan),
-                                stream))
-        return rc;
-    const uint32_t pack_blocks = (n_tiles + 7u) & ~7u;  // a multiple of the 8 XCDs
-    fused_pack_kernel<BETA><<<pack_blocks, kPackThreads, 0, stream>>>(
-        at<uint2>(scratch, L.rects), at<Reach<BETA>>(scratch, L.reach), cum, CN, C, ntx * nty, ntx, tile_size, vals, tm,
-        cm, counters, capacity, entries, tile_offsets);
-    if (int rc = check_launch("fused_pack")) return rc;
+        if (int rc = scan_exclusive(cum, CN, cum, counters, at<void>(scratch, L.scan), stream)) return rc;
+        void* sort_ws = at<void>(scratch, L.sort);
+        if (CN > 0) {
+            fused_emit_kernel<<<ceil_div(CN, 256), 256, 0, stream>>>(
+                at<uint2>(scratch, L.rects), cum, CN, ntx, capacity, sort_keys_buffer(sort_ws),
+                sort_vals_buffer(sort_ws, capacity), counters + 1);
+            if (int rc = check_launch("fused_emit")) return rc;
+        }
+        uint32_t* keys = at<uint32_t>(scratch, L.keys);
+        uint32_t* vals = at<uint32_t>(scratch, L.vals);
+        if (int rc = sort_pairs_u32(sort_ws, L.sort_bytes, capacity, counters, key_end_bit(ntx * nty - 1), keys, vals,
+                                    stream))
+            return rc;
+        uint32_t* tm = at<uint32_t>(scratch, L.tm);
+        uint32_t* cm = at<uint32_t>(scratch, L.cm);
+        fused_offsets_kernel<<<ceil_div(n_tiles, 256), 256, 0, stream>>>(keys, vals, counters, capacity, C, N, n_tiles,
+                                                                         reinterpret_cast<int32_t*>(tm));
+        if (int rc = check_launch("fused_offsets")) return rc;
+        fused_list_lengths_kernel<<<ceil_div(n_tiles, 256), 256, 0, stream>>>(tm, counters, capacity, C, ntx * nty,
+                                                                              at<uint32_t>(scratch, L.lengths));
+        if (int rc = check_launch("fused_list_lengths")) return rc;
+        if (int rc = scan_exclusive(at<uint32_t>(scratch, L.lengths), n_tiles, cm, nullptr,
+                                    at<void>(scratch, L.tile_scan), stream))
+            return rc;
+        const uint32_t pack_blocks = (n_tiles + 7u) & ~7u;  // a multiple of the 8 XCDs
+        fused_pack_kernel<BETA><<<pack_blocks, kPackThreads, 0, stream>>>(
+            at<uint2>(scratch, L.rects), at<Reach<BETA>>(scratch, L.reach), cum, CN, C, ntx * nty, ntx, tile_size, vals,
+            tm, cm, counters, capacity, entries, tile_offsets);
+        if (int rc = check_launch("fused_pack")) return rc;
     }
     if (tile_order && n_tiles > 0) {
         fused_tile_order_kernel<<<8, kTileOrderThreads, 0, stream>>>(reinterpret_cast<const uint32_t*>(tile_offsets),

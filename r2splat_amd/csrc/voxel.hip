@@ -329,12 +329,6 @@ vox_bwd_isect_kernel(VoxArgs<S> A, const int64_t* __restrict__ isect_ids, const 
 // ---------------------------------------------------------------------------
 constexpr uint32_t kMomT = 8;
 
-__device__ __forceinline__ void wave_sync_lds() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // The fused float32 kernels read each primitive's voxel-frame mean and
 // inverse covariance from a double-precision frame, kFrame doubles per
 // primitive (mean x y z, then the conic xx xy xz yy yz zz), computed from the
@@ -850,10 +844,10 @@ vox_fwd_fused_kernel(VoxArgs<float> A, float* __restrict__ out, float* __restric
     R next = load_vox_rec<BETA>(A, lo + int32_t(lane), hi, x0, y0, z0);
     float next_q = VAR ? load_vox_unc(A, lo + int32_t(lane), hi) : 0.f;
     for (int32_t base = lo; base < hi; base += kWave) {
-        wave_sync_lds();
+        wave_lds_sync();
         slot[lane] = next;
         if constexpr (VAR) stage_q[wave][lane] = next_q;
-        wave_sync_lds();
+        wave_lds_sync();
         next = load_vox_rec<BETA>(A, base + kWave + int32_t(lane), hi, x0, y0, z0);
         if constexpr (VAR) next_q = load_vox_unc(A, base + kWave + int32_t(lane), hi);
         const int32_t n = min(int32_t(kWave), hi - base);
@@ -1096,10 +1090,10 @@ vox_fwd_octants_kernel(VoxArgs<S> A, S* __restrict__ out, S* __restrict__ out_va
                     octants = form_octants(f, bound, float(tx * T), float(ty * T), float(tz * T));
             }
         }
-        wave_sync_lds();
+        wave_lds_sync();
         stage[wave][lane] = r;
         if constexpr (VAR) stage_q[wave][lane] = q;
-        wave_sync_lds();
+        wave_lds_sync();
         const int32_t n = min(int32_t(kWave), end - base);
         for (int32_t j = 0; j < n; ++j) {
             const uint32_t reach = __builtin_amdgcn_readlane(octants, j);

@@ -249,8 +249,7 @@ raster_bwd_isect_kernel(RasterArgs<S> A, const int64_t* __restrict__ isect_ids,
 // intersection with its nine wave reductions 494 us; these take 144 and 157. What
 // bounds them is double arithmetic in the few tiles that the object covers.
 // ---------------------------------------------------------------------------
-// Whether every parameter of a primitive is finite. The bounds below give others
-// every pixel of a tile, so that a NaN shows where their pairs pass the cut-off.
+// Whether every parameter of a primitive is finite.
 template <typename S, bool BETA>
 __device__ __forceinline__ bool all_finite(const Prim2D<S>& p) {
     return isfinite(p.mx) && isfinite(p.my) && isfinite(p.a) && isfinite(p.b) && isfinite(p.c) && isfinite(p.opac) &&
@@ -260,16 +259,16 @@ __device__ __forceinline__ bool all_finite(const Prim2D<S>& p) {
 // Rows [lo, hi) of a T-row tile (first pixel centre at row y_base + 1/2) in which
 // |alpha| can reach 1e-5: dy^2 <= 4 A S / (4 A C - B^2) for the form A dx^2 + B dx
 // dy + C dy^2 <= S, widened by 1e-3 and 0.05 px (the bound is formed in float).
-// Forms that are flat, not positive definite or not finite get every row; only a
-// weight surely below the cut-off gets none.
+// Forms that are flat, not positive definite or not finite get every row, and so do
+// means that are not finite: their NaN shows where their pairs pass the cut-off. Only
+// a finite primitive whose weight is surely below it gets none.
 template <typename S, bool BETA>
 __device__ __forceinline__ void reached_rows(const Prim2D<S>& p, S y_base, int T, int& lo, int& hi) {
     lo = 0;
     hi = T;
-    if (!all_finite<S, BETA>(p)) return;
     const float w = fabsf(float(p.opac * p.mu));
     if (w < 0.999e-5f) {
-        hi = 0;
+        hi = all_finite<S, BETA>(p) ? 0 : T;
         return;
     }
     float A, B, C, bound;
@@ -290,7 +289,7 @@ __device__ __forceinline__ void reached_rows(const Prim2D<S>& p, S y_base, int T
     if (!(A > 0.f) || !(den > 1e-3f * ac4) || !(e2 >= 0.f) || !(e2 < 1e30f)) return;
     const float ext = __builtin_amdgcn_sqrtf(e2) * 1.001f + 0.05f;
     const float c = float(p.my - y_base) - 0.5f;
-    if (!(fabsf(c) < 1e9f)) return;
+    if (!(fabsf(c) < 1e9f) || !(fabsf(float(p.mx)) < 1e30f)) return;
     lo = int(fminf(fmaxf(ceilf(c - ext), 0.f), float(T)));
     hi = max(lo, int(fminf(fmaxf(floorf(c + ext) + 1.f, 0.f), float(T))));
 }
@@ -299,6 +298,7 @@ __device__ __forceinline__ void reached_rows(const Prim2D<S>& p, S y_base, int T
 template <typename S, bool BETA>
 __device__ __forceinline__ void reached_cols(const Prim2D<S>& p, S x_base, int T, int& lo, int& hi) {
     Prim2D<S> t = p;
+    t.mx = p.my;
     t.my = p.mx;
     t.a = p.c;
     t.c = p.a;
@@ -502,16 +502,11 @@ raster_fwd_rows_kernel(RasterArgs<S> A, S* __restrict__ out, S* __restrict__ out
 //     v_conic = -(Mxx / 2, Mxy, Myy / 2), v_opac = mu sum v vis, v_mu = opac sum v vis;
 //   Beta, delta = mean - pixel, G = v vis / h, k = -opac mu beta: v_mean = 2k (a Mx +
 //     b My, b Mx + c My), v_conic = k (Mxx, 2 Mxy, Myy), v_beta = sum v alpha log h.
-// Waves a SIMD: the plain Gaussian form of short launches fits the 96 registers of
-// five without a spill; the other forms take 102 to 168.
-template <uint32_t CHUNK, bool BETA, bool VAR>
-constexpr int op_bwd_waves() { return !BETA && !VAR && CHUNK == 256 ? 5 : 3; }
-
 template <int T>
 constexpr uint32_t op_tiles() { return T == 8 ? 16 : T == 16 ? 8 : 2; }
 
 template <typename S, int T, uint32_t CHUNK, bool BETA, bool VAR>
-__global__ void __launch_bounds__(kChunkThreads) __attribute__((amdgpu_waves_per_eu(op_bwd_waves<CHUNK, BETA, VAR>())))
+__global__ void __launch_bounds__(kChunkThreads) __attribute__((amdgpu_waves_per_eu(3)))
 raster_bwd_rows_kernel(RasterArgs<S> A, const int64_t* __restrict__ isect_ids, const S* __restrict__ v_render,
                        const S* __restrict__ v_var, const S* __restrict__ unc, S* __restrict__ v_xy,
                        S* __restrict__ v_conic, S* __restrict__ v_opac, S* __restrict__ v_mu,
@@ -535,9 +530,8 @@ raster_bwd_rows_kernel(RasterArgs<S> A, const int64_t* __restrict__ isect_ids, c
             if (g < 0 || uint32_t(g) >= A.C * A.N) return false;
             int lo, hi;
             const uint32_t y0 = ((key % nt) / A.ntx) * T;
-            const Prim2D<S> p = load_prim(A, g, BETA);
-            reached_rows<S, BETA>(p, S(y0), T, lo, hi);
-            if (!all_finite<S, BETA>(p)) hi = int(min(uint32_t(T), A.H - y0));  // (a pair past the image is none)
+            reached_rows<S, BETA>(load_prim(A, g, BETA), S(y0), T, lo, hi);
+            hi = max(lo, min(hi, int(A.H) - int(y0)));  // (a pair past the image is none)
             mask = ((1ull << hi) - 1ull) & ~((1ull << lo) - 1ull);
             return hi > lo;
         },
@@ -548,8 +542,6 @@ raster_bwd_rows_kernel(RasterArgs<S> A, const int64_t* __restrict__ isect_ids, c
             const uint32_t n = uint32_t(g) % A.N;
             const S w = p.opac * p.mu, q2 = VAR && unc ? S(2) * unc[n] : S(0);
             double m0 = 0.0, mx = 0.0, my = 0.0, mxx = 0.0, mxy = 0.0, myy = 0.0, sl = 0.0, vq = 0.0;
-            bool any = false;  // a pair of the image passed the cut-off
-            const uint32_t columns = A.W - tx * T;
             while (rows) {
                 const uint32_t r = uint32_t(__builtin_ctzll(rows));
                 rows &= rows - 1ull;
@@ -569,7 +561,6 @@ raster_bwd_rows_kernel(RasterArgs<S> A, const int64_t* __restrict__ isect_ids, c
                             if (q < S(0) || q >= S(1)) continue;
                             const S h = S(1) - q, vis = Math<S>::pow(h, p.beta), alpha = w * vis;
                             if (fabs(alpha) < S(1e-5)) continue;
-                            any = any || j < columns;
                             if constexpr (VAR) {
                                 row_sum(rq, vq, vv * alpha * alpha);
                                 v += q2 * alpha * vv;
@@ -584,7 +575,6 @@ raster_bwd_rows_kernel(RasterArgs<S> A, const int64_t* __restrict__ isect_ids, c
                             const S sigma = vjp_sigma(p.a * dx, dx, p.b * dx, p.c, dy);
                             const S vis = Math<S>::exp(-sigma), alpha = w * vis;
                             const bool keep = !(sigma < S(0) || fabs(alpha) < S(1e-5));
-                            any = any || (keep && j < columns);
                             if constexpr (VAR) {
                                 row_sum(rq, vq, keep ? vv * alpha * alpha : S(0));
                                 v += q2 * alpha * vv;
@@ -606,7 +596,9 @@ raster_bwd_rows_kernel(RasterArgs<S> A, const int64_t* __restrict__ isect_ids, c
                     vq += rq;
                 }
             }
-            if (!active || !any) return;  // (no pair: an infinite parameter times an empty sum would be a NaN)
+            if (!active) return;
+            // no pair: an infinite parameter times an empty sum would be a NaN
+            if (m0 == 0.0 && vq == 0.0 && !all_finite<S, BETA>(p)) return;
             const size_t G = size_t(g);
             if constexpr (BETA) {
                 const double k = -w * p.beta;

@@ -980,8 +980,7 @@ vox_partials_reduce_kernel(const uint32_t* __restrict__ cum, const float* __rest
 // thread over the whole list took 210 us there and a wave per intersection 373 us;
 // these take 166 and 160.
 // ---------------------------------------------------------------------------
-// Whether every parameter of a primitive is finite. Others get every voxel of a
-// tile, so that a NaN shows where their pairs pass the cut-off.
+// Whether every parameter of a primitive is finite.
 template <typename S, bool BETA>
 __device__ __forceinline__ bool all_finite(const Prim3D<S>& p) {
     bool ok = isfinite(p.x) && isfinite(p.y) && isfinite(p.z) && isfinite(p.opac) && (!BETA || isfinite(p.beta));
@@ -990,13 +989,14 @@ __device__ __forceinline__ bool all_finite(const Prim3D<S>& p) {
     return ok;
 }
 
-// The float form of a finite primitive and the bound S on its q (Gaussian: q =
-// sigma) beyond which no term passes the cut-off; false when none can (its weight
-// is surely below it).
+// The float form of a primitive and the bound S on its q (Gaussian: q = sigma)
+// beyond which no term passes the cut-off; false when none can (a finite primitive
+// whose weight is surely below it). The bounds by rows and octants give a primitive
+// with a NaN or an infinity every voxel, so that it shows where its pairs pass.
 template <typename S, bool BETA>
 __device__ __forceinline__ bool op_form(const Prim3D<S>& p, VoxForm& f, float& bound) {
     const float w = fabsf(float(p.opac)), cut = BETA ? 1e-5f : 1e-6f;
-    if (w < 0.999f * cut) return false;
+    if (w < 0.999f * cut && all_finite<S, BETA>(p)) return false;
     const float s = BETA ? 1.f : 0.5f, t2 = BETA ? 2.f : 1.f;
     f.hi[0] = float(p.x);
     f.hi[1] = float(p.y);
@@ -1027,13 +1027,16 @@ __device__ __forceinline__ uint32_t form_octants(const VoxForm& f, float S, floa
     if (!(f.a > 0.f) || !(det > 1e-3f * f.a * f.cyy * f.czz) || !(S >= 0.f)) return 0xffu;
     const float m[3] = {f.hi[0] - x0, f.hi[1] - y0, f.hi[2] - z0};
     uint32_t part[3];
+    bool far = false;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
         const float e = __builtin_amdgcn_sqrtf(S * c[k] * __builtin_amdgcn_rcpf(det)) * 1.002f + 0.05f;
         const float lo = m[k] - e, hi = m[k] + e;  // voxel centres of the tile at 0.5 .. 7.5
         part[k] = (lo <= 3.5f && hi >= 0.5f ? 1u : 0u) | (lo <= 7.5f && hi >= 4.5f ? 2u : 0u);
-        if (!(e < 1e9f) || !(fabsf(m[k]) < 1e9f)) part[k] = 3u;
+        if (!(e < 1e9f)) part[k] = 3u;
+        far = far || !(fabsf(m[k]) < 1e9f);
     }
+    if (far) return 0xffu;
     const uint32_t row = part[0], plane = (part[1] & 1u ? row : 0u) | (part[1] & 2u ? row << 2 : 0u);
     return (part[2] & 1u ? plane : 0u) | (part[2] & 2u ? plane << 4 : 0u);
 }
@@ -1084,9 +1087,7 @@ vox_fwd_octants_kernel(VoxArgs<S> A, S* __restrict__ out, S* __restrict__ out_va
                 if constexpr (VAR) q = A.unc[g];
                 VoxForm f;
                 float bound;
-                if (!all_finite<S, BETA>(r))
-                    octants = 0xffu;
-                else if (op_form<S, BETA>(r, f, bound))
+                if (op_form<S, BETA>(r, f, bound))
                     octants = form_octants(f, bound, float(tx * T), float(ty * T), float(tz * T));
             }
         }
@@ -1164,18 +1165,14 @@ vox_bwd_rows_kernel(VoxArgs<S> A, const int64_t* __restrict__ isect_ids, const S
         [&](uint32_t e, uint32_t tile, uint64_t& mask, double&) {
             const int32_t g = A.flatten[e];
             if (g < 0 || uint32_t(g) >= A.N) return false;
-            const Prim3D<S> p = load_prim3(A, g, BETA);
-            const uint32_t tx = tile % A.ntx, rest = tile / A.ntx;
-            if (!all_finite<S, BETA>(p)) {  // the rows inside the volume (a pair past it is none)
-                const uint32_t ny = min(T, A.dy - (rest % A.nty) * T), nz = min(T, A.dz - (rest / A.nty) * T);
-                mask = (0x0101010101010101ull * ((1u << ny) - 1u)) & (~0ull >> (8u * (T - nz)));
-                return true;
-            }
             VoxForm f;
             float bound;
-            if (!op_form<S, BETA>(p, f, bound)) return false;
-            mask = vox_row_mask(f, bound, float(tx * T) + 0.5f, float((rest % A.nty) * T) + 0.5f,
-                                float((rest / A.nty) * T) + 0.5f);
+            if (!op_form<S, BETA>(load_prim3(A, g, BETA), f, bound)) return false;
+            const uint32_t tx = tile % A.ntx, rest = tile / A.ntx, ty = rest % A.nty, tz = rest / A.nty;
+            mask = vox_row_mask(f, bound, float(tx * T) + 0.5f, float(ty * T) + 0.5f, float(tz * T) + 0.5f);
+            // the rows of the volume (a pair past it is none)
+            const uint32_t ny = ty * T < A.dy ? min(T, A.dy - ty * T) : 0u, nz = tz * T < A.dz ? min(T, A.dz - tz * T) : 0u;
+            mask &= nz == 0u ? 0ull : (0x0101010101010101ull * ((1u << ny) - 1u)) & (~0ull >> (8u * (T - nz)));
             return mask != 0ull;
         },
         [&](uint32_t e, uint32_t tile, uint32_t slot, uint64_t rows, double, bool active) {
@@ -1185,8 +1182,6 @@ vox_bwd_rows_kernel(VoxArgs<S> A, const int64_t* __restrict__ isect_ids, const S
             const S q2 = VAR && unc ? S(2) * unc[g] : S(0);
             double m0 = 0.0, m_x = 0.0, m_y = 0.0, m_z = 0.0, mxx = 0.0, myy = 0.0, mzz = 0.0, mxy = 0.0, mxz = 0.0,
                    myz = 0.0, sl = 0.0, vq = 0.0;
-            bool any = false;  // a pair of the volume passed the cut-off
-            const uint32_t columns = A.dx - tx * T;
             while (rows) {
                 const uint32_t bit = uint32_t(__builtin_ctzll(rows)), z = bit / T, y = bit % T;
                 rows &= rows - 1ull;
@@ -1204,7 +1199,6 @@ vox_bwd_rows_kernel(VoxArgs<S> A, const int64_t* __restrict__ isect_ids, const S
                         if (q < S(0) || q >= S(1)) continue;
                         const S h = S(1) - q, vis = Math<S>::pow(h, p.beta), alpha = p.opac * vis;
                         if (fabs(alpha) < S(1e-5)) continue;
-                        any = any || j < columns;
                         if constexpr (VAR) {
                             row_sum(rq, vq, vv * alpha * alpha);
                             v += q2 * alpha * vv;
@@ -1218,7 +1212,6 @@ vox_bwd_rows_kernel(VoxArgs<S> A, const int64_t* __restrict__ isect_ids, const S
                     } else {
                         const S vis = Math<S>::exp(-q), alpha = p.opac * vis;
                         const bool keep = !(q < S(0) || fabs(alpha) < S(1e-6));
-                        any = any || (keep && j < columns);
                         if constexpr (VAR) {
                             row_sum(rq, vq, keep ? vv * alpha * alpha : S(0));
                             v += q2 * alpha * vv;
@@ -1243,7 +1236,9 @@ vox_bwd_rows_kernel(VoxArgs<S> A, const int64_t* __restrict__ isect_ids, const S
                 sl += rl;
                 vq += rq;
             }
-            if (!active || !any) return;  // (no pair: an infinite parameter times an empty sum would be a NaN)
+            if (!active) return;
+            // no pair: an infinite parameter times an empty sum would be a NaN
+            if (m0 == 0.0 && vq == 0.0 && !all_finite<S, BETA>(p)) return;
             const size_t G = size_t(g);
             const double k = BETA ? S(2) * p.opac * p.beta : p.opac, kc = BETA ? -p.opac * p.beta : S(-0.5) * p.opac;
             atomic_add(v_xyz + 3 * G, S(k * (p.c[0] * m_x + p.c[1] * m_y + p.c[2] * m_z)));

@@ -644,6 +644,35 @@ RasterArgs<S> make_args(const void* means2d, const void* conics, const void* opa
                          ntx, nty};
 }
 
+// Whether a forward takes the row kernel. It gives a tile several waves, so it wins
+// where tiles are few (float32, 137k intersections on 9 16-pixel tiles: 119 us, one
+// wave per pixel group 7113) or their lists long, the longer the more tiles there
+// are to fill the chip without it; it loses on short lists of many tiles (4096 tiles,
+// 2778 intersections: 51 us against 10; 65536 8-pixel tiles of 11 each: 164 against 43).
+inline bool fwd_by_rows(uint32_t n_isects, uint64_t prims, uint64_t tiles) {
+    const double list = std::min(80.0, 4.0 + double(tiles) / 40.0) * (0.5 + 2.0 * tile_overhang(n_isects, prims, 2));
+    return tiles <= 64 || double(n_isects) >= list * double(tiles);
+}
+
+// Whether a per-primitive VJP takes the row kernel, a lane per intersection: it needs
+// intersections enough to fill the chip, more where each fills its tile (a lane then
+// walks all T^2 pixels alone), and lists long enough that a chunk meets few tiles. On
+// the other side the general kernel has a wave per intersection. float64 Beta, 32-pixel
+// tiles: 1.9M intersections on 64 tiles 228 us against 3361; 545 on 256 tiles 5325
+// against 25. float32, 16-pixel tiles: 2.2M on 144 tiles 343 against 1068; 718 on 1024
+// 267 against 13.
+template <typename S>
+inline bool vjp_by_rows(uint32_t n_isects, uint64_t prims, uint64_t tiles, uint32_t T, bool beta) {
+    constexpr bool kDouble = std::is_same<S, double>::value;
+    const double over = tile_overhang(n_isects, prims, 2);
+    double few, few_wide, list, list_wide;  // intersections and mean list at no overhang, and what a whole tile adds
+    if (T == 8) few = 0, few_wide = 16e3, list = 8, list_wide = 0;
+    else if (T == 16) few = 0, few_wide = kDouble && beta ? 128e3 : 32e3, list = 24, list_wide = kDouble && !beta ? 32 : 128;
+    else if (T == 32) few = 8e3, few_wide = beta ? 256e3 : 160e3, list = 48, list_wide = kDouble && beta ? 512 : 96;
+    else return false;
+    return n_isects >= few + few_wide * over && double(n_isects) >= (list + list_wide * over) * double(tiles);
+}
+
 int launch_fwd(int dtype, bool beta, bool var, const void* means2d, const void* conics,
                const void* opac, const void* mus, const void* betas, const void* unc,
                const int32_t* offsets, const int32_t* flatten, uint32_t n_isects, uint32_t C,
@@ -672,9 +701,11 @@ int launch_fwd(int dtype, bool beta, bool var, const void* means2d, const void* 
             };
             return blocks <= kSplitTiles ? launch(std::true_type{}) : launch(std::false_type{});
         };
-        if (T == 8) return rows(std::integral_constant<int, 8>{});
-        if (T == 16) return rows(std::integral_constant<int, 16>{});
-        if (T == 32) return rows(std::integral_constant<int, 32>{});
+        if (fwd_by_rows(n_isects, uint64_t(C) * N, blocks)) {
+            if (T == 8) return rows(std::integral_constant<int, 8>{});
+            if (T == 16) return rows(std::integral_constant<int, 16>{});
+            if (T == 32) return rows(std::integral_constant<int, 32>{});
+        }
         auto k = beta ? (var ? raster_fwd_kernel<S, true, true> : raster_fwd_kernel<S, true, false>)
                       : (var ? raster_fwd_kernel<S, false, true> : raster_fwd_kernel<S, false, false>);
         k<<<uint32_t(blocks), threads, shm, stream>>>(A, (S*)out, (S*)out_var);
@@ -826,7 +857,8 @@ extern "C" int r2s_rasterize_to_pixels_bwd_per_gaussian(
             else launch(std::integral_constant<uint32_t, 512>{});
             return check_launch("rasterize_to_pixels_bwd_per_gaussian");
         };
-        if (!v_means2d_abs && uint64_t(C) * n_tiles_x * n_tiles_y < (1ull << 32) - 1) {
+        const uint64_t tiles = uint64_t(C) * n_tiles_x * n_tiles_y;
+        if (!v_means2d_abs && tiles < (1ull << 32) - 1 && vjp_by_rows<S>(n_isects, CN, tiles, tile_size, beta)) {
             if (tile_size == 8) return rows(std::integral_constant<int, 8>{});
             if (tile_size == 16) return rows(std::integral_constant<int, 16>{});
             if (tile_size == 32) return rows(std::integral_constant<int, 32>{});

@@ -14,6 +14,15 @@ constexpr uint32_t kNoTile = 0xffffffffu;
 // against 66; 2.9M: 534 us against 479, their rows sorted less finely).
 constexpr uint32_t kFewIsects = 1u << 19;
 
+// How far the mean primitive reaches beyond one tile along an axis, in tiles, at
+// most one, from n_isects intersections of `prims` primitives on tiles of `axes`
+// dimensions. The operator kernels that work row by row are chosen by it and by
+// the lengths of the lists: a primitive that fills its tiles has no rows to skip.
+inline double tile_overhang(uint32_t n_isects, uint64_t prims, int axes) {
+    const double tiles = prims ? double(n_isects) / double(prims) : 0.0;
+    return std::min(1.0, std::max(0.0, (axes == 2 ? std::sqrt(tiles) : std::cbrt(tiles)) - 1.0));
+}
+
 // Takes intersections [e0, e0 + CHUNK) of the list (ids: their tile ids,
 // ascending; those outside [0, n_tiles) are skipped), for at most TILES distinct
 // tiles at a time:

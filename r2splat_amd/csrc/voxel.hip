@@ -1276,6 +1276,33 @@ VoxArgs<S> make_vox_args(const void* means3d, const void* conics, const void* op
                       (const S*)unc, offsets, flatten, n_isects, N, dx, dy, dz, T, ntx, nty, ntz};
 }
 
+// Whether an operator forward of 8^3 tiles takes the octant kernel, whose waves share
+// a tile's list and skip the octants a primitive does not reach. It wins on long lists
+// (142k intersections on 8 tiles, Beta: float32 609 us against 2674, float64 684 against
+// 3050) and loses where lists are short for what a primitive covers: float32, 18.7k
+// intersections on 512 tiles, primitives reaching into the next tile, 31 us against 23.
+// Launches of up to 600 tiles need longer lists for it (float64, 3604 intersections on
+// 125 tiles: 51 us against 21).
+template <typename S>
+inline bool fwd_by_octants(uint32_t n_isects, uint64_t prims, uint64_t tiles) {
+    const double wide = std::is_same<S, double>::value ? 64.0 : 24.0;
+    double list = 4.0 + wide * tile_overhang(n_isects, prims, 3);
+    if (tiles <= 600) list = 2.0 * list + 32.0;
+    return double(n_isects) >= list * double(tiles);
+}
+
+// Whether an operator VJP of 8^3 tiles takes the kernel with a lane per intersection:
+// it needs intersections enough to fill the chip, more where a lane walks its whole
+// tile of 512 voxels, and lists long enough that a chunk meets few tiles; the general
+// kernel has a wave per intersection. float64 Beta: 142k intersections on 8 tiles 20 us
+// against 280, 1895 on 4096 tiles 8698 against 26.
+template <typename S>
+inline bool vjp_by_rows(uint32_t n_isects, uint64_t prims, uint64_t tiles, bool beta) {
+    const double over = tile_overhang(n_isects, prims, 3);
+    const double wide = std::is_same<S, double>::value && !beta ? 32.0 : 64.0;
+    return n_isects >= 4e3 + 48e3 * over && double(n_isects) >= (4.0 + wide * over) * double(tiles);
+}
+
 }  // namespace r2s
 
 using namespace r2s;
@@ -1301,7 +1328,7 @@ extern "C" int r2s_voxelize_to_voxels_fwd(int dtype, const void* means3d, const 
         auto A = make_vox_args<S>(means3d, conics, opacities, betas, uncertainties, tile_offsets,
                                   flatten_ids, n_isects, N, dim_x, dim_y, dim_z, tile_size,
                                   n_tiles_x, n_tiles_y, n_tiles_z);
-        if (tile_size == kMomT) {
+        if (tile_size == kMomT && fwd_by_octants<S>(n_isects, N, blocks)) {
             auto k = beta ? (var ? vox_fwd_octants_kernel<S, true, true> : vox_fwd_octants_kernel<S, true, false>)
                           : (var ? vox_fwd_octants_kernel<S, false, true> : vox_fwd_octants_kernel<S, false, false>);
             k<<<uint32_t(blocks), kVoxFwdWaves * kWave, 0, stream>>>(A, (S*)render, (S*)render_var);
@@ -1380,7 +1407,8 @@ extern "C" int r2s_voxelize_to_voxels_bwd_per_gaussian(
                 return check_launch("voxelize_to_voxels_bwd_per_gaussian");
             }
         }
-        if (tile_size == kMomT && uint64_t(n_tiles_x) * n_tiles_y * n_tiles_z < (1ull << 31)) {
+        const uint64_t tiles = uint64_t(n_tiles_x) * n_tiles_y * n_tiles_z;
+        if (tile_size == kMomT && tiles < (1ull << 31) && vjp_by_rows<S>(n_isects, N, tiles, beta)) {
             const bool var = v_render_var != nullptr;
             const auto launch = [&](auto chunk) {
                 constexpr uint32_t CHUNK = decltype(chunk)::value;

@@ -33,13 +33,16 @@ def _case(device, dtype, C, N, W, H, seed, beta, var):
     return out, betas, unc, v, vv
 
 
-def _run(case, W, H, T):
+def _run(case, W, H, T, listed=None):
+    """Every primitive in every tile, or the first `listed` of each camera."""
     (means, conics, opac, mus), betas, unc, v, vv = case
     C, N = opac.shape
+    listed = N if listed is None else listed
     nx, ny = -(-W // T), -(-H // T)
-    radii = torch.full((C, N, 2), 4 * (W + H), dtype=torch.int32, device=means.device)
+    radii = torch.zeros((C, N, 2), dtype=torch.int32, device=means.device)
+    radii[:, :listed] = 4 * (W + H)
     _, ids, flat = ops.isect_tiles(means, radii, T, nx, ny)
-    assert ids.numel() == C * N * nx * ny
+    assert ids.numel() == C * listed * nx * ny
     off = ops.isect_offset_encode(ids, C, nx, ny)
     args = (means, conics, opac, mus) + (() if betas is None else (betas,))
     pre = "" if betas is None else "beta_"
@@ -65,6 +68,27 @@ SHAPES = [(2, 7, 40, 24, 8), (12, 100, 200, 160, 8), (1, 70, 61, 47, 16), (36, 9
 def test_row_kernels_match_the_general_kernel(device, C, N, W, H, T, beta, var, dtype):
     case = _case(device, dtype, C, N, W, H, C + N, beta, var)
     _compare(lambda c, t: _run(c, W, H, t), case, T, 10)
+
+
+# A small launch of short lists takes the general kernel: these are of the sizes, for
+# primitives that fill their tiles, from which the VJP's row kernels are chosen.
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("beta,var", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("C,N,W,H,T", [(2, 150, 77, 90, 8), (2, 600, 200, 157, 16), (3, 1000, 320, 319, 32)])
+def test_row_kernels_of_long_lists(device, C, N, W, H, T, beta, var, dtype):
+    case = _case(device, dtype, C, N, W, H, C + N, beta, var)
+    _compare(lambda c, t: _run(c, W, H, t), case, T, 10)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("beta,var", [(False, True), (True, True)])
+@pytest.mark.parametrize("W,H,T", [(200, 160, 8), (390, 319, 16), (799, 620, 32)])
+def test_forward_row_kernels_of_many_tiles(device, W, H, T, beta, var, dtype):
+    """4500 tiles, more than the forward splits over workgroups; primitives that stand
+    in no list beside the 50 of each camera, so that lists are long for the footprints."""
+    C, listed = 9, 50
+    case = _case(device, dtype, C, listed * 500, W, H, T, beta, var)
+    _compare(lambda c, t: (_run(c, W, H, t, listed)[0], []), case, T, 10)
 
 
 def _compare(run, case, tile, other):
@@ -138,6 +162,21 @@ def test_voxel_8_tiles_match_the_general_kernel(device, N, dims, beta, var, dtyp
     _compare(run, case, 8, 7)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("beta,var", [(False, False), (False, True), (True, False), (True, True)])
+def test_voxel_8_tiles_of_long_lists(device, beta, var, dtype):
+    """Fewer than 2^19 intersections, from which the kernels take the longer chunk."""
+    N, dims = 420, (40, 47, 37)
+    case = _voxel_case(device, dtype, N, dims, N, beta, var)
+    moments = dtype == torch.float32 and not (beta or var)  # its VJP is another kernel
+
+    def run(c, t):
+        img, grads = _voxel_run(c, dims, t)
+        return img, [] if moments else grads
+
+    _compare(run, case, 8, 7)
+
+
 def _same_marks(got, general, image, what):
     """Images: NaN and either infinity in the same places; gradients: the same values
     finite (an infinite sum may be infinite or NaN by its order). The finite values
@@ -154,29 +193,31 @@ NONFINITE = [float("nan"), float("inf"), float("-inf")]
 
 
 @pytest.mark.parametrize("beta,var", [(False, True), (True, True)])
-@pytest.mark.parametrize("T", [8, 16, 32])
-def test_row_kernels_keep_nonfinite_parameters_to_their_pairs(device, T, beta, var):
+@pytest.mark.parametrize("T,N,pad", [(8, 20, 0), (16, 20, 0), (32, 20, 0),
+                                     (8, 20, 2000), (16, 30, 500), (32, 1400, 8000)])  # padded: long lists for the size
+def test_row_kernels_keep_nonfinite_parameters_to_their_pairs(device, T, N, pad, beta, var):
     """A primitive with a NaN or an infinity marks the pixels and gradients that the
-    general kernel marks: those of its own pairs past the cut-off."""
-    W, H, N = 70, 45, 20
+    general kernel marks: those of its own pairs past the cut-off. `pad` primitives
+    stand in no list, as off-screen ones do."""
+    W, H = 70, 45
     for value in NONFINITE:
         for field in ("mean", "conic a", "conic b", "opacity", "mu", "beta", "uncertainty"):
             if field == "beta" and not beta:
                 continue
-            (means, conics, opac, mus), betas, unc, v, vv = _case(device, torch.float64, 1, N, W, H, 11, beta, var)
+            (means, conics, opac, mus), betas, unc, v, vv = _case(device, torch.float64, 1, N + pad, W, H, 11, beta, var)
             target = {"mean": means[0, 7], "conic a": conics[0, 7], "conic b": conics[0, 7, 1:], "opacity": opac[0, 7:],
                       "mu": mus[0, 7:], "beta": None if betas is None else betas[0, 7:], "uncertainty": unc[7:]}[field]
             target[0] = value
             case = ((means, conics, opac, mus), betas, unc, v, vv)
-            (img, grads), (ref, expected) = (_run_lists(case, W, H, t) for t in (T, 10))
+            (img, grads), (ref, expected) = (_run_lists(case, W, H, t, N) for t in (T, 10))
             _same_marks(img, ref, True, (value, field, "image"))
             _same_marks(grads, expected, False, (value, field, "gradient"))
 
 
-def _run_lists(case, W, H, T):
-    """_run with every primitive in every tile whatever its mean holds."""
+def _run_lists(case, W, H, T, N):
+    """_run with the first N primitives in every tile whatever their means hold."""
     (means, conics, opac, mus), betas, unc, v, vv = case
-    C, N = opac.shape
+    C = opac.shape[0]
     nt = -(-W // T) * -(-H // T)
     dev = means.device
     flat = torch.arange(N, dtype=torch.int32, device=dev).repeat(nt)
@@ -191,13 +232,14 @@ def _run_lists(case, W, H, T):
 
 
 @pytest.mark.parametrize("beta", [False, True])
-def test_voxel_8_tiles_keep_nonfinite_parameters_to_their_pairs(device, beta):
-    dims, N = (21, 17, 30), 20
+@pytest.mark.parametrize("N,pad", [(20, 0), (120, 6000)])  # padded: long lists for the size
+def test_voxel_8_tiles_keep_nonfinite_parameters_to_their_pairs(device, N, pad, beta):
+    dims = (21, 17, 30)
     for value in NONFINITE:
         for field in ("mean", "conic xx", "conic xy", "opacity", "beta", "uncertainty"):
             if field == "beta" and not beta:
                 continue
-            (means, conics, opac), betas, unc, v, vv = _voxel_case(device, torch.float64, N, dims, 11, beta, True)
+            (means, conics, opac), betas, unc, v, vv = _voxel_case(device, torch.float64, N + pad, dims, 11, beta, True)
             target = {"mean": means[7], "conic xx": conics[7], "conic xy": conics[7, 1:], "opacity": opac[7:],
                       "beta": None if betas is None else betas[7:], "uncertainty": unc[7:]}[field]
             target[0] = value
@@ -244,6 +286,7 @@ def test_float32_vjp_sums_are_as_near_as_the_general_kernels(device, T, beta, va
     varies by a few percent (the largest error by half); a quarter more than the
     general kernel's is a longer chain of float sums."""
     C, N, W, H = 3, 400, 150, 110
+    total = 8000 if T == 32 else N  # of which N in the lists: the row kernel from 24k intersections
     new, old = 0.0, 0.0
     for seed in range(4):
         g = torch.Generator().manual_seed(seed)
@@ -255,10 +298,45 @@ def test_float32_vjp_sums_are_as_near_as_the_general_kernels(device, T, beta, va
         betas = (0.6 + 3 * r(C, N)).to(device, torch.float32) if beta else None
         unc = (0.1 * r(N)).to(device, torch.float32) if var else None
         v, vv = ((r(C, H, W) - 0.5).to(device, torch.float32) for _ in range(2))
+        extra = total - N
+        prims = [torch.cat([t, t[:, :1].expand(C, extra, *t.shape[2:])], 1).contiguous() for t in prims]
+        betas = None if betas is None else torch.cat([betas, betas[:, :1].expand(C, extra)], 1).contiguous()
+        unc = None if unc is None else torch.cat([unc, unc[:1].expand(extra)]).contiguous()
         case = (prims, betas, unc, v, vv if var else None)
         wide = [t.double() for t in prims], *(None if t is None else t.double() for t in case[1:])
-        exact = _run(wide, W, H, 10)[1]
+        exact = _run(wide, W, H, 10, N)[1]
         errors = lambda tile: torch.tensor(  # noqa: E731
-            [float((a.double() - b).norm() / b.norm()) for a, b in zip(_run(case, W, H, tile)[1], exact)])
+            [float((a.double() - b).norm() / b.norm()) for a, b in zip(_run(case, W, H, tile, N)[1], exact)])
         new, old = new + errors(T), old + errors(10)
     assert bool((new <= 1.25 * old).all()), (new / old).tolist()
+
+
+def _vjp_time(run):
+    """Least of ten timed calls after one untimed, in ms."""
+    run()
+    times = []
+    for _ in range(10):
+        start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        start.record()
+        run()
+        end.record()
+        end.synchronize()
+        times.append(start.elapsed_time(end))
+    return min(times)
+
+
+@pytest.mark.parametrize("kind", ["raster", "voxel"])
+def test_vjps_of_sparse_lists_take_no_lane_per_intersection(device, kind):
+    """A few hundred Beta primitives that fill their tiles, in float64: a wave each takes
+    some 30 us beside the call's own, a lane each 2 to 5 ms. The general kernel of a tile
+    edge that has no other is the measure; four times it is far from both."""
+    if kind == "raster":
+        case, W, H = _case(device, torch.float64, 1, 8, 256, 256, 5, True, False), 256, 256
+        run = lambda T: _run(case, W, H, T)  # noqa: E731
+        tiles = (32, 31)
+    else:
+        case, dims = _voxel_case(device, torch.float64, 8, (48, 48, 48), 5, True, False), (48, 48, 48)
+        run = lambda T: _voxel_run(case, dims, T)  # noqa: E731
+        tiles = (8, 7)
+    new, general = (_vjp_time(lambda: run(T)) for T in tiles)
+    assert new <= 4.0 * general, (new, general)

@@ -43,7 +43,7 @@ def _disc_reference(mean, conic, beta, w):
 
 
 @pytest.mark.parametrize("seed", [1, 2])
-@pytest.mark.parametrize("kernel", ["fused", "operator"])
+@pytest.mark.parametrize("kernel", ["fused", "operator", "operator, long lists"])
 def test_voxel_vjps_of_thin_discs(device, kernel, seed):
     means, conics = (t.to(device) for t in _discs(seed))
     n = -(-SIDE // 8)
@@ -61,15 +61,20 @@ def test_voxel_vjps_of_thin_discs(device, kernel, seed):
             got = fused.voxel_vjp(state, w, beta, v, (SIDE, SIDE, SIDE))
             tol = 1e-5  # float32 sums of up to a few thousand terms of one sign
         else:
-            _, ids, flat = ops.isect_tiles_3d(mean, radii, 8, n, n, n)
+            # long lists for the size: four of the disc among primitives that are in no list
+            copies, total = (4, 8000) if kernel != "operator" else (1, 1)
+            mean, conic = mean.repeat(total, 1), conic.repeat(total, 1)
+            reach = radii.repeat(total, 1)
+            reach[copies:] = 0
+            _, ids, flat = ops.isect_tiles_3d(mean, reach, 8, n, n, n)
             off = ops.isect_offset_encode_3d(ids, n, n, n)
-            beta = torch.full((1,), 0.5, device=device, dtype=torch.float64)
-            w = torch.full((1,), 0.7, device=device, dtype=torch.float64)
-            v, v_w, v_beta = _disc_reference(means[k], conics[k], 0.5, float(w))
+            beta = torch.full((total,), 0.5, device=device, dtype=torch.float64)
+            w = torch.full((total,), 0.7, device=device, dtype=torch.float64)
+            v, v_w, v_beta = _disc_reference(means[k], conics[k], 0.5, 0.7)
             got = ops.beta_voxelize_to_voxels_bwd_per_gaussian(mean, conic, w, beta, off, ids, flat, v.double(), SIDE,
                                                                SIDE, SIDE, 8)
             tol = 1e-9
-        assert ids.numel() == n ** 3
+        assert ids.numel() == (4 if "long" in kernel else 1) * n ** 3
         for name, a, b in (("opacity", got[2][0], v_w), ("beta", got[3][0], v_beta)):
             assert abs(float(a) - float(b)) <= tol * abs(float(b)), (k, name, float(a), float(b))
 

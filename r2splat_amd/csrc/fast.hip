@@ -2231,10 +2231,17 @@ static size_t packed_bytes(uint32_t C, uint32_t N, uint32_t capacity, int kind) 
 
 // Bin tables of the direct placement: its waves hold one table each in LDS, so
 // larger tables cost occupancy. Up to kPlaceLdsBytes every call places; up to
-// kPlaceLargeBytes (1024 tiles a camera) those whose waves are all resident at
-// once do (one view of 333 x 517 with 30k primitives: 100 us of binning kernels
-// against 145 us of sort and pack), and larger grids or more waves sort and pack (500k
-// primitives x 256 views of 512^2 took 49.6 ms a step placing, 44.7 sorting).
+// kPlaceLargeBytes (1024 tiles a camera) those do whose waves are all resident at
+// once and that have two primitives a tile or more, and the others sort and pack, as
+// larger grids do (500k primitives x 256 views of 512^2 took 49.6 ms a step placing,
+// 44.7 sorting). A wave walks its records' rectangles one after another, a sort
+// spreads the pairs over the chip, so wide rectangles sort sooner; and few primitives
+// fill an image only with wide ones. A forward pass of one view, placing and sorting:
+// 100 primitives at 740 tiles each on 512^2: 677 us and 279; 1600 at 8: 81 and 97;
+// 30k on 333 x 517 at 6.5 tiles each: 121 and 135, at 29: 306 and 277, at 139: 1124
+// and 887. How many tiles a record reaches is known on the device alone, and the two
+// order the lists differently, so the choice follows from the call's sizes and not
+// from the capacity, which depends on earlier calls.
 // Which of the two a call of the middle kind takes depends on C and N, so its scratch
 // has room for either, in one place.
 constexpr size_t kPlaceLdsBytes = 16384, kPlaceLargeBytes = 40960, kLdsBytes = 163840;
@@ -2273,7 +2280,7 @@ static FusedScratch fused_scratch(uint32_t C, uint32_t N, uint32_t n_tiles, uint
         L.n_ranges = (N + L.range_len - 1) / L.range_len;
         const bool small = table <= kPlaceLdsBytes;
         const uint64_t resident = kComputeUnits * (kLdsBytes / (table + sizeof(PairList)));
-        L.place = small || uint64_t(C) * L.n_ranges <= resident;
+        L.place = small || (N >= 2 * nt && uint64_t(C) * L.n_ranges <= resident);
         // room for the most (camera, range) pairs of up to N primitives and C cameras
         // (their number falls where the ranges get longer), so that a buffer sized for
         // the largest call holds every smaller one: by the rule above a range has 64

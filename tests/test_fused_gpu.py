@@ -601,3 +601,22 @@ def test_fused_float32_degenerate_scenes(device, case):
             assert (got.double() - exp).abs().max() <= 1e-4 * float(exp.abs().max()), name
         else:  # nothing drawn: exact zeros on both paths
             assert torch.count_nonzero(got) == 0 and torch.count_nonzero(exp) == 0, name
+
+
+def test_few_records_of_many_tiles_are_not_placed(device):
+    """100 primitives over most of 1024 tiles: a wave that walks 64 such rectangles takes
+    twice what the sort of the whole call does. 1056 tiles always sort: the measure."""
+    times = []
+    for H in (512, 528):
+        sc = workloads.scene(100, 1, H, 512, scale_range=(0.2, 0.5), seed=3, device=device)
+        args = (*sc.params(), sc.viewmats, sc.Ks, 512, H, 1e-8, 3.0)
+        best = []
+        for _ in range(12):
+            start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            start.record()
+            fused.forward(*args)
+            end.record()
+            end.synchronize()
+            best.append(start.elapsed_time(end))
+        times.append(min(best))
+    assert times[0] <= 1.5 * times[1], times

@@ -2231,7 +2231,7 @@ static size_t packed_bytes(uint32_t C, uint32_t N, uint32_t capacity, int kind) 
 
 // Bin tables of the direct placement: its waves hold one table each in LDS, so
 // larger tables cost occupancy. Up to kPlaceLdsBytes every call places; up to
-// kPlaceLargeBytes (1024 tiles a camera) those do whose waves are all resident at
+// kPlaceLargeBytes (1137 tiles a camera) those do whose waves are all resident at
 // once and that have two primitives a tile or more, and the others sort and pack, as
 // larger grids do (500k primitives x 256 views of 512^2 took 49.6 ms a step placing,
 // 44.7 sorting). A wave walks its records' rectangles one after another, a sort

@@ -168,7 +168,9 @@ int r2s_world_to_volume_mapping_bwd(int dtype, const void* means, const void* co
 /* ------------------------------------------------------------------------ */
 
 /* Workspace sizes (bytes) for the device scan over `n` counts and for the
- * stable radix sort of `n_isects` (key, value) pairs over `end_bit` key bits. */
+ * stable radix sort of `n_isects` (key, value) pairs over `end_bit` key bits.
+ * Neither falls as its first argument grows: a workspace of the largest call
+ * serves every smaller one. */
 size_t r2s_scan_workspace_bytes(uint64_t n);
 size_t r2s_sort_workspace_bytes(uint64_t n_isects, uint32_t end_bit);
 
@@ -400,6 +402,8 @@ int r2s_voxelize_to_voxels_bwd_per_gaussian(
  * RasterizeToPixelsFwd.cu mean_var kernels) and its VJP: the pixel adjoint
  * becomes v_image + 2 q alpha v_image_var unless `detach` (the reference's
  * detach_variance), and v_uncertainties = sum v_image_var alpha^2.
+ * r2s_fused_scratch_bytes does not fall as C, N or capacity grows, the other
+ * arguments equal: a scratch of the largest call serves every smaller one.
  * `kind` (bit 0 Beta, bit 1 uncertainty) selects the record layout in
  * r2s_fused_scratch_bytes / r2s_fused_record_bytes / r2s_fused_render /
  * r2s_fused_raster_vjp and must match the forward. */

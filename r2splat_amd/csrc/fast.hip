@@ -2249,7 +2249,11 @@ constexpr uint64_t kComputeUnits = 256;
 constexpr uint32_t kPlaceWaves = 4096;  // target number of ranges (waves) per binning pass
 // Bytes of count tables up to which ranges shorter than 256 records pay: a wave
 // walks its range's rectangles one step after another (0.4 us a step), while a
-// table is written, scanned twice and read once.
+// table is written, scanned twice and read once. Ranges of 256 and of 64, the whole
+// binning on 256^2: 1 view of 1000 primitives 47 us and 40, of 256k 139 and 198;
+// 4 views of 4000 62 and 52, of 64k 86 and 101. Over 80 such calls on 64^2 to 320^2
+// this line is within 12% of the better one but for 1 view of 64^2 with 256k (173 us
+// against 130).
 constexpr uint64_t kRangeTables = 8ull << 20;
 
 static FusedScratch fused_scratch(uint32_t C, uint32_t N, uint32_t n_tiles, uint32_t capacity, int kind) {
